@@ -911,8 +911,9 @@ int64_t* dense_gather(dxg2_plan* p, const void* d_frames, int64_t* d_sums, hipSt
     const bool wide = p->dtype == DXG2_U16;
     int64_t* gsums = wide ? p->d_psums : sums;
     const int64_t nbn = (int64_t)p->n_bins * p->N;
-    launch_fill_i64(gsums, (wide ? 2 : 1) * nbn, s);
-    launch_fill_i64(p->d_ugram, (wide ? 3 : 1) * nbn, s);
+    // the queue heads of the persistent Gram are cleared here too
+    launch_clear_call(gsums, (wide ? 2 : 1) * nbn, p->d_ugram, (wide ? 3 : 1) * nbn, p->d_heads,
+                      16, s);
     const int64_t hw = (int64_t)p->H * p->W;
     uint32_t* flagw = wide && wide_first ? reinterpret_cast<uint32_t*>(p->d_wflag) : nullptr;
     if (flagw) launch_fill_u32(flagw, (hw + 3) / 4, s);
@@ -939,13 +940,11 @@ int64_t* dense_gather(dxg2_plan* p, const void* d_frames, int64_t* d_sums, hipSt
 }
 
 // The Gram of every bin: the persistent launch over the per-XCD work queues (heads
-// cleared by a fill kernel, so the sequence can be captured in a graph), or one
-// workgroup per tile.
+// cleared by dense_gather), or one workgroup per tile.
 void dense_gram(dxg2_plan* p, int64_t* gsums, hipStream_t s, bool wide_first = false) {
     const int biased = p->dtype == DXG2_I8 ? 0 : 1;
     const int* nwkb = wide_first && p->dtype == DXG2_U16 ? p->d_nwkb : nullptr;
     if (p->use_queue) {
-        launch_fill_i32(p->d_heads, 16, s);
         launch_gram_i8_queue(p->gram_tile, false, p->d_slab, p->d_bins, p->d_qmwork,
                              (int)p->qm_work.size(), p->d_qoff, p->d_heads, p->N, p->nrows,
                              biased, nwkb, p->d_ugram, gsums, s);
@@ -1844,9 +1843,7 @@ int dxg2_batch_correlate_events(dxg2_batch* b, int32_t n, dxg2_plan* const* plan
         dxg2_plan* p = plans[i];
         const int64_t nbn = (int64_t)p->n_bins * p->N;
         int64_t* sums = d_sums && d_sums[i] ? d_sums[i] : p->d_sums;
-        launch_fill_i64(sums, nbn, s);
-        launch_fill_i64(p->d_ugram, nbn, s);
-        launch_fill_i32(p->d_err, 1, s);
+        launch_clear_call(sums, nbn, p->d_ugram, nbn, p->d_err, 1, s);
         jobs[i] = EventJob{d_times[i], d_data[i], d_offsets[i], p->d_pix, p->d_bins, nnz[i],
                            p->d_ugram, sums, p->d_err, p->N, 0};
         if (p->n_bins == 0) continue;
@@ -1951,9 +1948,7 @@ int dxg2_correlate_events_csr(dxg2_plan* p, const int32_t* d_times, const void* 
     hipStream_t s = (hipStream_t)stream;
     (void)hipGetLastError();
     const int64_t nbn = (int64_t)p->n_bins * p->N;
-    launch_fill_i64(d_sums ? d_sums : p->d_sums, nbn, s);
-    launch_fill_i64(p->d_ugram, nbn, s);
-    launch_fill_i32(p->d_err, 1, s);
+    launch_clear_call(d_sums ? d_sums : p->d_sums, nbn, p->d_ugram, nbn, p->d_err, 1, s);
     hipEvent_t* ev = nullptr;
     if (p->profiling && (rc = next_events(p, &ev))) return rc;
     if (ev) {
@@ -1980,9 +1975,7 @@ int dxg2_correlate_events_coo(dxg2_plan* p, const uint32_t* d_pixel, const uint3
     hipStream_t s = (hipStream_t)stream;
     (void)hipGetLastError();
     const int64_t nbn = (int64_t)p->n_bins * p->N;
-    launch_fill_i64(d_sums ? d_sums : p->d_sums, nbn, s);
-    launch_fill_i64(p->d_ugram, nbn, s);
-    launch_fill_i32(p->d_err, 1, s);
+    launch_clear_call(d_sums ? d_sums : p->d_sums, nbn, p->d_ugram, nbn, p->d_err, 1, s);
     hipEvent_t* ev = nullptr;
     if (p->profiling && (rc = next_events(p, &ev))) return rc;
     if (ev) DXG2_HIP(hipEventRecord(ev[0], s));

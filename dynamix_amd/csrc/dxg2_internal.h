@@ -141,6 +141,9 @@ struct KbWork {          // one k-block (64 pixels) of one bin
 // ------------------------------------------------------------------ launchers
 void launch_lds_atomic_rate(int mode, int blocks, int iters, uint32_t* out, hipStream_t s);
 void launch_fill_i64(int64_t* p, int64_t n, hipStream_t s);
+// a[0, na), b[0, nb) and c[0, nc) (nc <= 256) zeroed by one launch.
+void launch_clear_call(int64_t* a, int64_t na, int64_t* b, int64_t nb, int* c, int nc,
+                       hipStream_t s);
 void launch_gather_slots(const uint8_t* frames, int dtype, int64_t hw, int nframes, int nrows,
                          const int32_t* pix_idx, const BinDev* bins, const KbWork* kbl,
                          int n_items, int tf, int8_t* slab, hipStream_t s, uint32_t* flagw);

@@ -179,11 +179,10 @@ __global__ __launch_bounds__(PREP_THREADS) void sums_prep_kernel(
     }
 }
 
-// smax zeroed, then the chunks of every bin.
+// The chunks of every bin (smax zeroed by the caller).
 template <int PLANES>
 static void launch_sums_prep(const int64_t* plane_sums, int64_t* sums, int n_bins, int nframes,
                              int64_t* prefix, int64_t* smax, hipStream_t s) {
-    launch_fill_i64(smax, n_bins, s);
     const dim3 grid((unsigned)n_bins, (unsigned)((nframes + PREP_CHUNK - 1) / PREP_CHUNK));
     sums_prep_kernel<PLANES><<<grid, dim3(PREP_THREADS), 0, s>>>(plane_sums, sums, nframes,
                                                                  prefix, smax);
@@ -383,6 +382,33 @@ __device__ __forceinline__ int64_t edge_sums(const int64_t* P, int nframes, int 
     return P[nframes - tau] + P[nframes] - P[tau];
 }
 
+// The numerator of entry o from the raw Gram diagonals: n as stored in `num`, nd its FP64
+// value.  `stride` separates the rows of the digit products; pairs = padded pixel pairs on
+// the diagonal, pairs_w the same of the wide k-blocks (mode 3); edges(p) the edge sums of
+// plane p.  Modes as in finalize_kernel.
+template <typename NumT, typename Edges>
+__device__ __forceinline__ void complete_numerator(const NumT* __restrict__ ugram, int64_t o,
+                                                   int64_t stride, int mode, int64_t pairs,
+                                                   int64_t pairs_w, Edges edges, NumT& n,
+                                                   double& nd) {
+    if (mode >= 2) {
+        // biased digit products: (h-128)(h'-128) etc.; padding entries are -128 too
+        const int64_t eh = edges(0), el = edges(1);
+        const int64_t elx = mode == 3 ? edges(2) : el;
+        const int64_t pairs_h = mode == 3 ? pairs_w : pairs;
+        const int64_t hh = (int64_t)ugram[o] + 128 * eh - 16384 * pairs_h;
+        const int64_t ll = (int64_t)ugram[o + stride] + 128 * el - 16384 * pairs;
+        const int64_t x = (int64_t)ugram[o + 2 * stride] + 128 * (eh + elx) - 32768 * pairs_h;
+        const __int128 v = (__int128)hh * 65536 + (__int128)x * 256 + ll;
+        n = (NumT)(int64_t)v;
+        nd = i128_to_double(v);
+    } else {
+        n = ugram[o];
+        if (mode == 1) n += (NumT)(128 * edges(0) - 16384 * pairs);
+        nd = (double)n;
+    }
+}
+
 // grid (ceil(N / FIN_SPAN), n_bins), FIN_THREADS threads.  NumT is int64_t (exact
 // numerators of the Gram and event paths) or double (FFT path).  mode 0: numerators as
 // accumulated; 1: uint8 bias correction; 2: uint16 digit planes (ugram rows b, n_bins + b,
@@ -404,7 +430,6 @@ __global__ __launch_bounds__(FIN_THREADS) void finalize_kernel(
     const int tau0 = blockIdx.x * FIN_SPAN;
     const int tid = threadIdx.x;
     const int64_t* S = sums + (int64_t)b * nframes;
-    const int64_t* P = prefix + (int64_t)b * (nframes + 1);
 
     double d[FIN_LAGS];
     const double m = (double)smax[b];
@@ -433,42 +458,210 @@ __global__ __launch_bounds__(FIN_THREADS) void finalize_kernel(
         const int64_t pairs = kpad * (nframes - tau);  // padded pixel pairs on the diagonal
         double nd;
         NumT n;
-        if (mode >= 2) {
-            // biased digit products: (h-128)(h'-128) etc.; padding entries are -128 too
-            const int64_t* P1 = prefix + (int64_t)(nb + b) * (nframes + 1);
-            const int64_t eh = edge_sums(P, nframes, tau), el = edge_sums(P1, nframes, tau);
-            int64_t elx = el, pairs_h = pairs;
-            if (mode == 3) {
-                const int64_t* P2 = prefix + (int64_t)(2 * nb + b) * (nframes + 1);
-                elx = edge_sums(P2, nframes, tau);
-                pairs_h = (int64_t)nwkb[b] * KB * (nframes - tau);
-            }
-            const int64_t stride = (int64_t)nb * nframes;
-            const int64_t hh = (int64_t)ugram[o] + 128 * eh - 16384 * pairs_h;
-            const int64_t ll = (int64_t)ugram[o + stride] + 128 * el - 16384 * pairs;
-            const int64_t x = (int64_t)ugram[o + 2 * stride] + 128 * (eh + elx) - 32768 * pairs_h;
-            const __int128 v = (__int128)hh * 65536 + (__int128)x * 256 + ll;
-            n = (NumT)(int64_t)v;
-            nd = i128_to_double(v);
-        } else {
-            n = ugram[o];
-            if (mode == 1) n += (NumT)(128 * edge_sums(P, nframes, tau) - 16384 * pairs);
-            nd = (double)n;
-        }
+        complete_numerator<NumT>(
+            ugram, o, (int64_t)nb * nframes, mode, pairs,
+            mode == 3 ? (int64_t)nwkb[b] * KB * (nframes - tau) : 0,
+            [&](int p) {
+                return edge_sums(prefix + ((int64_t)p * nb + b) * (nframes + 1), nframes, tau);
+            },
+            n, nd);
         if (num) num[o] = n;
         if (den) den[o] = d[j];
         g2[o] = (float)(bd.scale * (nd / d[j]));
     }
 }
 
+// Short series (finish_is_small): prefix sums, Den and g2 in one launch instead of the
+// seven of sums_prep, den_mfma (two), den_i16, den_fp64, finalize and their fills, each
+// of which costs about 5 us of launch and drain whatever its work.  Block (x, bin) owns
+// FS_LAGS = 256 lags from tau0 = 256 x; every block loads the whole series of its bin
+// (L2-resident, at most 32 KiB) into LDS as doubles, S at index i + i / 4 so that the
+// lanes' windows, 4 frames apart, spread over the banks.  Lane l of wave q holds the 4 lags tau0 + 4 l + j
+// over the q-th quarter of the frames: per frame one broadcast S(t) and one new window
+// value feed 4 FMAs.  |S| <= 2^31 x 2^16 is exact in a double; when N M^2 < 2^52 (M =
+// max |S|) the FMAs are exact, otherwise the products go to 128 bits, as in
+// finalize_kernel.  What bounds it is the LDS reads of the N^2 / 2 products per bin, while
+// the chain it replaces is flat (about 50 us, most of it gaps between launches).  Stage
+// times, chain -> this: 47 -> 9 us (5 bins, N = 500), 51 -> 13 (10 bins, N = 1,000),
+// 56 -> 21 (20 bins, N = 2,000), 62 -> 46 (20 bins, N = 4,000), but 60 -> 82 (50 bins,
+// N = 4,096): the line lies at n_bins N^2 = 4e8, with N bounded by the staged series.
+constexpr int FINISH_SMALL = 4096;
+constexpr double FINISH_SMALL_WORK = 4e8;            // n_bins N^2
+constexpr int FS_LAGS = 256;
+constexpr int FS_LEN = FINISH_SMALL + FS_LAGS + 8;   // frames staged, zeros past the end
+
+__device__ __forceinline__ int fs_pad(int i) { return i + (i >> 2); }
+
+// PLANES as in sums_prep_kernel: 1 (S = plane_sums), 2 or 3 (uint16 digit planes; the
+// combined S goes to `sums`).  mode, nwkb, num, den, g2 as in finalize_kernel.
+template <typename NumT, int PLANES>
+__global__ __launch_bounds__(256) void finish_small_kernel(
+    const int64_t* __restrict__ plane_sums, int64_t* __restrict__ sums,
+    const NumT* __restrict__ ugram, const BinDev* __restrict__ bins, int nframes, int mode,
+    const int* __restrict__ nwkb, NumT* __restrict__ num, double* __restrict__ den,
+    float* __restrict__ g2) {
+    __shared__ double sS[FS_LEN + FS_LEN / 4];
+    __shared__ __attribute__((aligned(16))) unsigned char sred[4 * FS_LAGS * 8];
+    __shared__ int64_t sP[3][257];   // sums of the chunks before chunk i of each plane
+    __shared__ int64_t wtot[3][4];
+    __shared__ long long smax4[4];
+    const int b = blockIdx.y, nb = gridDim.y;
+    const int tau0 = blockIdx.x * FS_LAGS;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t* X[3] = {plane_sums + (int64_t)b * nframes,
+                           plane_sums + (int64_t)(nb + b) * nframes,
+                           plane_sums + (int64_t)(2 * nb + b) * nframes};
+    // S into LDS, its largest magnitude
+    long long mx = 0;
+    const int len = (nframes + FS_LAGS + 7) & ~3;
+    for (int t = tid; t < len; t += 256) {
+        int64_t v = 0;
+        if (t < nframes) {
+            v = X[0][t];
+            if (PLANES >= 2) {
+                v = 256 * v + X[1][t];
+                if (blockIdx.x == 0) sums[(int64_t)b * nframes + t] = v;
+            }
+        }
+        sS[fs_pad(t)] = (double)v;
+        mx = max(mx, (long long)(v < 0 ? -v : v));
+    }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) mx = max(mx, (long long)__shfl_xor(mx, d, 64));
+    if (lane == 0) smax4[wave] = mx;
+    // chunk sums of each plane and their exclusive scan (bias corrections only)
+    const int ch = (nframes + 255) / 256;
+    if (mode != 0) {
+        int64_t v[PLANES], x[PLANES];
+#pragma unroll
+        for (int p = 0; p < PLANES; ++p) {
+            v[p] = 0;
+            for (int t = tid * ch; t < min(nframes, (tid + 1) * ch); ++t) v[p] += X[p][t];
+            x[p] = v[p];
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const int64_t y = __shfl_up(x[p], d, 64);
+                if (lane >= d) x[p] += y;
+            }
+            if (lane == 63) wtot[p][wave] = x[p];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int p = 0; p < PLANES; ++p) {
+            int64_t before = 0;
+            for (int w = 0; w < wave; ++w) before += wtot[p][w];
+            sP[p][tid] = before + x[p] - v[p];
+            if (tid == 255) sP[p][256] = before + x[p];
+        }
+    }
+    __syncthreads();
+    const double m = (double)max(max(smax4[0], smax4[1]), max(smax4[2], smax4[3]));
+    const bool fp = (double)nframes * m * m < 4503599627370496.0;  // 2^52
+
+    // frames [ta, te) of this wave: a quarter of [0, N - tau0), starts multiples of 4
+    const int span = nframes - tau0;
+    const int q = ((span + 15) / 16) * 4;
+    const int ta = wave * q, te = min(span, ta + q);
+    double d = 0.0;  // Den(tau0 + tid)
+    if (fp) {
+        double acc[4] = {0.0, 0.0, 0.0, 0.0};
+        if (ta < te) {
+            const double* px = sS + fs_pad(ta);
+            const double* py = sS + fs_pad(tau0 + ta) + 5 * lane;
+            double y0 = py[0], y1 = py[1], y2 = py[2];
+#pragma unroll 4
+            for (int t = ta; t < te; t += 4, px += 5, py += 5) {
+                // windows of frames t .. t + 3: y[j + step], j < 4 (S past N is zero)
+                const double y3 = py[3], y4 = py[5], y5 = py[6], y6 = py[7];
+                const double x0 = px[0], x1 = px[1], x2 = px[2], x3 = px[3];
+                acc[0] = __builtin_fma(x0, y0, acc[0]);
+                acc[1] = __builtin_fma(x0, y1, acc[1]);
+                acc[2] = __builtin_fma(x0, y2, acc[2]);
+                acc[3] = __builtin_fma(x0, y3, acc[3]);
+                acc[0] = __builtin_fma(x1, y1, acc[0]);
+                acc[1] = __builtin_fma(x1, y2, acc[1]);
+                acc[2] = __builtin_fma(x1, y3, acc[2]);
+                acc[3] = __builtin_fma(x1, y4, acc[3]);
+                acc[0] = __builtin_fma(x2, y2, acc[0]);
+                acc[1] = __builtin_fma(x2, y3, acc[1]);
+                acc[2] = __builtin_fma(x2, y4, acc[2]);
+                acc[3] = __builtin_fma(x2, y5, acc[3]);
+                acc[0] = __builtin_fma(x3, y3, acc[0]);
+                acc[1] = __builtin_fma(x3, y4, acc[1]);
+                acc[2] = __builtin_fma(x3, y5, acc[2]);
+                acc[3] = __builtin_fma(x3, y6, acc[3]);
+                y0 = y4;
+                y1 = y5;
+                y2 = y6;
+            }
+        }
+        double* red = reinterpret_cast<double*>(sred) + wave * FS_LAGS + 4 * lane;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) red[j] = acc[j];
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < 4; ++w) d += reinterpret_cast<double*>(sred)[w * FS_LAGS + tid];
+    } else {
+        // 128-bit products of lag tau0 + tid over every frame (dense data with large sums)
+        __int128 acc = 0;
+        for (int t = 0; t < span - tid; ++t)
+            acc += (__int128)(int64_t)sS[fs_pad(t)] * (int64_t)sS[fs_pad(tau0 + t + tid)];
+        d = i128_to_double(acc);
+    }
+    const int tau = tau0 + tid;
+    if (tau >= nframes) return;
+    // sum_{t < N - tau} X(t) + sum_{t >= tau} X(t) of a plane
+    auto edges = [&](int p) -> int64_t {
+        auto P = [&](int t) -> int64_t {
+            const int c = t / ch;
+            int64_t v = sP[p][c];
+            for (int k = c * ch; k < t; ++k) v += X[p][k];
+            return v;
+        };
+        return P(nframes - tau) + P(nframes) - P(tau);
+    };
+    const BinDev bd = bins[b];
+    const int64_t o = (int64_t)b * nframes + tau;
+    double nd;
+    NumT n;
+    complete_numerator<NumT>(ugram, o, (int64_t)nb * nframes, mode,
+                             (int64_t)bd.nkb * KB * (nframes - tau),
+                             mode == 3 ? (int64_t)nwkb[b] * KB * (nframes - tau) : 0,
+                             [&](int p) { return edges(PLANES > p ? p : 0); }, n, nd);
+    if (num) num[o] = n;
+    if (den) den[o] = d;
+    g2[o] = (float)(bd.scale * (nd / d));
+}
+
+static bool finish_is_small(int n_bins, int nframes) {
+    return nframes <= FINISH_SMALL && (double)n_bins * nframes * nframes <= FINISH_SMALL_WORK;
+}
+
+template <typename NumT>
+static void launch_finish_small(const int64_t* plane_sums, int64_t* sums, const NumT* ugram,
+                                const BinDev* bins, int n_bins, int nframes, int mode,
+                                const int* nwkb, NumT* num, double* den, float* g2,
+                                hipStream_t s) {
+    const dim3 grid((unsigned)((nframes + FS_LAGS - 1) / FS_LAGS), (unsigned)n_bins);
+    if (mode == 3)
+        finish_small_kernel<NumT, 3><<<grid, 256, 0, s>>>(plane_sums, sums, ugram, bins, nframes,
+                                                          mode, nwkb, num, den, g2);
+    else if (mode == 2)
+        finish_small_kernel<NumT, 2><<<grid, 256, 0, s>>>(plane_sums, sums, ugram, bins, nframes,
+                                                          mode, nwkb, num, den, g2);
+    else
+        finish_small_kernel<NumT, 1><<<grid, 256, 0, s>>>(sums, sums, ugram, bins, nframes, mode,
+                                                          nwkb, num, den, g2);
+}
+
 // Den for every bin with N M^2 < 2^52: i8 MFMA for the bins whose |S| fits two digits
-// (k_den.hip), packed 16-bit dot products for |S| <= DEN_I16_MAX, FP64 above.
+// (k_den.hip), packed 16-bit dot products for |S| <= DEN_I16_MAX, FP64 above.  dpre was
+// zeroed (with smax) before sums_prep_kernel.
 static void launch_den_fp64(const int64_t* sums, int n_bins, int nframes, const int64_t* smax,
                             const int64_t* prefix, int planes, const DenMfma& dm, double* dpre,
                             hipStream_t s) {
     // bins with max |S| <= skip are den_mfma_kernel's
     const int skip = dm.v && dm.umax > 0 ? den_mfma_max() : -1;
-    launch_fill_i64(reinterpret_cast<int64_t*>(dpre), (int64_t)n_bins * nframes, s);  // +0.0
     launch_den_mfma(sums, n_bins, nframes, smax, prefix, planes, dm, dpre, s);
     const int64_t lag_blocks = (nframes + DEN_SPAN - 1) / DEN_SPAN;
     const int64_t chunks = (nframes + DEN_CH - 1) / DEN_CH;
@@ -488,6 +681,13 @@ void launch_finalize(const int64_t* plane_sums, int64_t* sums, const int64_t* ug
                      int64_t* smax, double* dpre, const int* nwkb, int64_t* num, double* den,
                      float* g2, const DenMfma& dm, hipStream_t s) {
     if (n_bins <= 0 || nframes <= 0) return;
+    if (finish_is_small(n_bins, nframes)) {
+        launch_finish_small<int64_t>(plane_sums, sums, ugram, bins, n_bins, nframes, mode, nwkb,
+                                     num, den, g2, s);
+        return;
+    }
+    launch_clear_call(smax, n_bins, reinterpret_cast<int64_t*>(dpre), (int64_t)n_bins * nframes,
+                      nullptr, 0, s);
     if (mode == 3)
         launch_sums_prep<3>(plane_sums, sums, n_bins, nframes, prefix, smax, s);
     else if (mode == 2)
@@ -504,6 +704,13 @@ void launch_finalize_f64(const int64_t* sums, const double* fnum, const BinDev* 
                          int nframes, int64_t* prefix, int64_t* smax, double* dpre, double* num,
                          double* den, float* g2, const DenMfma& dm, hipStream_t s) {
     if (n_bins <= 0 || nframes <= 0) return;
+    if (finish_is_small(n_bins, nframes)) {
+        launch_finish_small<double>(sums, const_cast<int64_t*>(sums), fnum, bins, n_bins, nframes,
+                                    0, nullptr, num, den, g2, s);
+        return;
+    }
+    launch_clear_call(smax, n_bins, reinterpret_cast<int64_t*>(dpre), (int64_t)n_bins * nframes,
+                      nullptr, 0, s);
     launch_sums_prep<1>(sums, const_cast<int64_t*>(sums), n_bins, nframes, prefix, smax, s);
     launch_den_fp64(sums, n_bins, nframes, smax, prefix, 1, dm, dpre, s);
     dim3 grid((unsigned)((nframes + FIN_SPAN - 1) / FIN_SPAN), (unsigned)n_bins);

@@ -49,6 +49,26 @@ void launch_fill_i32(int* p, int64_t n, hipStream_t s) {
     fill_i32_kernel<<<dim3((unsigned)blocks), dim3(256), 0, s>>>(p, n);
 }
 
+// The accumulators of one correlate call zeroed by one launch: two int64 ranges and a few
+// ints.
+__global__ void clear_call_kernel(int64_t* __restrict__ a, int64_t na, int64_t* __restrict__ b,
+                                  int64_t nb, int* __restrict__ c, int nc) {
+    const int64_t i0 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t i = i0; i < na; i += stride) a[i] = 0;
+    for (int64_t i = i0; i < nb; i += stride) b[i] = 0;
+    if (i0 < nc) c[i0] = 0;
+}
+
+void launch_clear_call(int64_t* a, int64_t na, int64_t* b, int64_t nb, int* c, int nc,
+                       hipStream_t s) {
+    const int64_t n = na > nb ? na : nb;
+    int64_t blocks = (n + 255) / 256;
+    if (blocks < 1) blocks = 1;
+    if (blocks > 4096) blocks = 4096;
+    clear_call_kernel<<<dim3((unsigned)blocks), dim3(256), 0, s>>>(a, na, b, nb, c, nc);
+}
+
 constexpr int GATHER_TF = 64;  // frames per workgroup tile
 
 // Broadcast lane j of every quad to the whole quad (DPP quad_perm [j, j, j, j]).
