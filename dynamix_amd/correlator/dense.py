@@ -228,7 +228,7 @@ class PlainMatMulCorrelator(_DenseHIP):
         return g2.cpu().numpy()
 
 
-# Half-lengths L (complex points) of the in-LDS FFT plans: 2^a 5^b, 1024 <= L <= 16384.
+# Half-lengths L up to 16384 frames: 2^a 5^b, 1024 <= L <= 16384.
 FFT_HALF_LENGTHS = (1024, 1280, 2048, 2560, 4096, 5120, 8192, 10240, 16384)
 
 
@@ -253,8 +253,7 @@ class FFTCorrelator(_DenseHIP):
     """Drop-in for FFTWCorrelator / CUFFTCorrelator (dense.py:275-369, cuda.py:129-219).
 
     Frames of any dtype the exact paths take (uint8, int8, uint16, or wider types
-    narrowed to them), nframes <= 131072 (above 16384 the transform is a four-step FFT
-    through an HBM scratch of at most DXG2_FFT_SCRATCH_MB MiB).  `weights` and `precompute_fft_plans` are accepted;
+    narrowed to them), nframes <= 131072.  `weights` and `precompute_fft_plans` are accepted;
     weights are ignored as in the reference FFT correlators (dense.py:277-285), and the
     FFT needs no plan.  scale_factor is ignored (the reference divides by the pixel count,
     dense.py:366).  Numerators carry FP32 FFT rounding: |Num - Num_exact| <= 2e-7 * Num(0)

@@ -299,14 +299,11 @@ struct dxg2_plan {
     std::vector<int32_t> fft_qkb;
     int32_t* d_pixfft = nullptr;
     int32_t* d_fftqkb = nullptr;
-    uint8_t* d_xs = nullptr;       // pixel-major bytes, same size as the slab
-    float2* d_tw = nullptr;        // exp(-2 pi i m / L), m < L; then exp(-pi i k / L), k <= L
+    uint8_t* d_xs = nullptr;       // series pairs (fft_series_bytes)
+    float2* d_tw = nullptr;        // twiddles (launch_fft_power)
     double* d_power = nullptr;     // (n_bins, L + 1)
     double* d_fnum = nullptr;      // (n_bins, N)
-    int fft_L = 0;
-    int fft_L1 = 0, fft_L2 = 0;    // long series: L = L1 L2 through the scratch below
-    int fft_chunk = 0;             // k-blocks per four-step chunk
-    float2* d_fy = nullptr;        // four-step scratch: fft_chunk * 64 * L complex
+    FftShape fft{};
 
     // Profiling: each correlate call records 4 events on its stream (no host sync);
     // dxg2_plan_stage_times() waits for the last one and averages every recorded call.
@@ -649,38 +646,21 @@ int next_events(dxg2_plan* p, hipEvent_t** out) {
 // Pixels of one bin's list handled by one event work item.
 constexpr int EVENT_ITEM_PIXELS = 1024;
 
-// FFT length: Nf = 2L with L the smallest length of the mixed-radix set (2^a 5^b, at
-// least 1024) with L >= N; any Nf >= 2N - 1 gives the linear autocorrelation.  Up to
-// 16384 a series is transformed in LDS; above, L = L1 L2 goes through the four-step
-// path (L <= 131072).  *L1 / *L2 are 0 for the in-LDS path.
-int fft_length(int n, int* L1 = nullptr, int* L2 = nullptr) {
-    int l1 = 0, l2 = 0;
-    int L = fft_lds_length(std::max(n, 1));
-    if (L == 0) L = fft_four_step_length(n, &l1, &l2);
-    if (L1) *L1 = l1;
-    if (L2) *L2 = l2;
-    return L;
-}
-
-// k-blocks per four-step chunk: the scratch holds 64 series of L complex points per
-// k-block, at most DXG2_FFT_SCRATCH_MB MiB (default 1024).
-int fft_chunk_kblocks(int L, int total_kb) {
-    const size_t cap = (size_t)std::max(1, env_int("DXG2_FFT_SCRATCH_MB", 1024)) << 20;
-    const size_t per = (size_t)KB * L * sizeof(float2);
-    return (int)std::max<size_t>(1, std::min<size_t>((size_t)std::max(total_kb, 1), cap / per));
+// Bytes of the FFT path's series: L elements per entry of the (padded) pixel lists.
+size_t fft_series_bytes(const dxg2_plan* p, int L) {
+    const size_t size = p->dtype == DXG2_U16 ? 2 : 1;
+    return std::max<size_t>(16, p->pix_idx.size() * (size_t)L * size);
 }
 
 int ensure_fft_buffers(dxg2_plan* p, hipStream_t s) {
     if (p->d_power) return DXG2_OK;
     p->kb_work.clear();
-    int L1 = 0, L2 = 0;
-    const int L = fft_length(p->N, &L1, &L2);
-    if (L == 0)
+    FftShape shape{};
+    if (!fft_shape(std::max(p->N, 1), &shape))
         return set_error(DXG2_EUNSUPPORTED, "FFT path supports up to 131072 frames (got %d)",
                          p->N);
-    p->fft_L = L;
-    p->fft_L1 = L1;
-    p->fft_L2 = L2;
+    p->fft = shape;
+    const int L = shape.L, H = shape.H;
     for (int b = 0; b < p->n_bins; ++b)
         for (int kb = 0; kb < p->bins[b].nkb; ++kb) p->kb_work.push_back(KbWork{b, kb});
     // quads are loaded as aligned 4-byte words, which needs 4 | H W (and a 4-aligned
@@ -728,18 +708,17 @@ int ensure_fft_buffers(dxg2_plan* p, hipStream_t s) {
         p->kb_gather.clear();
         for (const Item& it : items) p->kb_gather.insert(p->kb_gather.end(), it.begin(), it.end());
     }
-    p->fft_chunk = L1 ? fft_chunk_kblocks(L, (int)p->kb_work.size()) : 0;
-    // [0, L): exp(-2 pi i m / L), the transform's twiddles; [L, 2L]: exp(-pi i k / L),
-    // k = 0..L, the factor that unpacks the half-length complex transform
-    p->twiddles.resize(2 * (size_t)L + 1);
-    for (int m = 0; m < L; ++m) {
-        const double a = -2.0 * M_PI * (double)m / (double)L;
-        p->twiddles[m] = make_float2((float)std::cos(a), (float)std::sin(a));
-    }
-    for (int k = 0; k <= L; ++k) {
-        const double a = -M_PI * (double)k / (double)L;
-        p->twiddles[L + k] = make_float2((float)std::cos(a), (float)std::sin(a));
-    }
+    p->twiddles.resize(2 * (size_t)H + L + 1);
+    auto root = [](int64_t m, int64_t n) {  // exp(-2 pi i m / n)
+        const double a = -2.0 * M_PI * (double)m / (double)n;
+        return make_float2((float)std::cos(a), (float)std::sin(a));
+    };
+    const int stride = H / shape.last;  // butterflies of the last pass
+    for (int m = 0; m < H; ++m) p->twiddles[m] = root(m, H);
+    for (int r = 0; r < shape.last; ++r)
+        for (int b = 0; b < stride; ++b)
+            p->twiddles[H + r * stride + b] = root((int64_t)r * b, H);
+    for (int m = 0; m <= L; ++m) p->twiddles[2 * H + m] = root(m, 2 * (int64_t)L);
     // d_power is allocated last: it marks the workspace complete.  A failure releases
     // what this call allocated, so a later call starts again from nothing.
     uint8_t* xs = nullptr;
@@ -747,16 +726,13 @@ int ensure_fft_buffers(dxg2_plan* p, hipStream_t s) {
     double *power = nullptr, *fnum = nullptr;
     KbWork* kbw = nullptr;
     KbWork* kbg = nullptr;
-    float2* fy = nullptr;
     int32_t* pixf = nullptr;
     int32_t* qkb = nullptr;
-    if ((L1 && dev_alloc(p->alloc, (void**)&fy, (size_t)p->fft_chunk * KB * L * sizeof(float2),
-                         s) != hipSuccess) ||
-        (!p->pix_fft.empty() &&
+    if ((!p->pix_fft.empty() &&
          dev_alloc(p->alloc, (void**)&pixf, p->pix_fft.size() * sizeof(int32_t), s) !=
              hipSuccess) ||
         dev_alloc(p->alloc, (void**)&qkb, p->fft_qkb.size() * sizeof(int32_t), s) != hipSuccess ||
-        dev_alloc(p->alloc, (void**)&xs, p->slab_bytes, s) != hipSuccess ||
+        dev_alloc(p->alloc, (void**)&xs, fft_series_bytes(p, L), s) != hipSuccess ||
         dev_alloc(p->alloc, (void**)&tw, p->twiddles.size() * sizeof(float2), s) != hipSuccess ||
         dev_alloc(p->alloc, (void**)&fnum, (size_t)std::max(p->n_bins, 1) * p->N * sizeof(double), s) !=
             hipSuccess ||
@@ -767,11 +743,10 @@ int ensure_fft_buffers(dxg2_plan* p, hipStream_t s) {
         dev_alloc(p->alloc, (void**)&power, (size_t)std::max(p->n_bins, 1) * (L + 1) * sizeof(double), s) !=
             hipSuccess) {
         for (void* b : {(void*)xs, (void*)tw, (void*)fnum, (void*)kbw, (void*)kbg, (void*)power,
-                        (void*)fy, (void*)pixf, (void*)qkb})
+                        (void*)pixf, (void*)qkb})
             dev_free(p->alloc, b, s);
         return set_error(DXG2_ENOMEM, "cannot allocate FFT workspace");
     }
-    p->d_fy = fy;
     p->d_pixfft = pixf;
     p->d_fftqkb = qkb;
     p->d_xs = xs;
@@ -1288,7 +1263,7 @@ static void plan_release(dxg2_plan* p, hipStream_t s) {
                     p->d_ework, p->d_err,  p->d_cnt,   p->d_scan,  p->d_off,
                     p->d_etimes, p->d_edata, p->d_kbwork, p->d_kbgather, p->d_xs, p->d_tw,
                     p->d_pixfft, p->d_fftqkb,
-                    p->d_power, p->d_fnum, p->d_fy, p->d_qmwork, p->d_qxwork, p->d_qoff,
+                    p->d_power, p->d_fnum, p->d_qmwork, p->d_qxwork, p->d_qoff,
                     p->d_heads, p->d_gband, p->d_gband_kb, p->d_gfall,
                     p->coo_sort.keys, p->coo_sort.vals0, p->coo_sort.vals1, p->coo_sort.tmp,
                     p->d_wflag, p->d_pixw, p->d_nwkb};
@@ -1348,13 +1323,13 @@ int dxg2_plan_footprint(const dxg2_plan* p, int32_t path, size_t* bytes) {
             return DXG2_OK;
         }
         case 2: {
-            int L1 = 0, L2 = 0;
-            const int L = fft_length(p->N, &L1, &L2);
+            FftShape shape{};
+            (void)fft_shape(std::max(p->N, 1), &shape);
+            const int L = shape.L;
             int64_t nkb = 0;
             for (const auto& bd : p->bins) nkb += bd.nkb;
-            const size_t scratch =
-                L1 ? (size_t)fft_chunk_kblocks(L, (int)nkb) * KB * L * sizeof(float2) : 0;
-            *bytes = common + p->slab_bytes + (2 * (size_t)L + 1) * sizeof(float2) + scratch +
+            *bytes = common + fft_series_bytes(p, L) +
+                     (2 * (size_t)shape.H + L + 1) * sizeof(float2) +
                      (size_t)std::max(p->n_bins, 1) * ((L + 1) + p->N) * sizeof(double) +
                      (2 * (size_t)nkb + (size_t)N_XCD * PM_XCD_GROUP) * sizeof(KbWork) +
                      (p->pix_idx.size() + (size_t)std::max(p->n_bins, 1)) * sizeof(int32_t);
@@ -2001,27 +1976,16 @@ int dxg2_correlate_fft(dxg2_plan* p, const void* d_frames, double* d_num, int64_
     hipEvent_t* ev = nullptr;
     if (p->profiling && (rc = next_events(p, &ev))) return rc;
     if (ev) DXG2_HIP(hipEventRecord(ev[0], s));
-    launch_fill_i64(reinterpret_cast<int64_t*>(p->d_power), (int64_t)p->n_bins * (p->fft_L + 1), s);
+    launch_fill_i64(reinterpret_cast<int64_t*>(p->d_power), (int64_t)p->n_bins * (p->fft.L + 1), s);
     const bool quads = reinterpret_cast<uintptr_t>(d_frames) % 4 == 0;
-    launch_gather_pm((const uint8_t*)d_frames, p->dtype, (int64_t)p->H * p->W, p->N, p->nrows,
+    launch_gather_pm((const uint8_t*)d_frames, p->dtype, (int64_t)p->H * p->W, p->N, p->fft,
                      p->d_pixfft, quads ? p->d_fftqkb : nullptr, p->d_bins, p->n_bins,
                      p->d_kbgather, (int)(p->kb_gather.size() / PM_KPB), p->d_xs, sums, s);
     if (ev) DXG2_HIP(hipEventRecord(ev[1], s));
-    if (p->fft_L1) {
-        const int total = (int)p->kb_work.size();
-        for (int kb0 = 0; kb0 < total; kb0 += p->fft_chunk)
-            if (launch_fft_four_step(p->fft_L1, p->fft_L2, p->dtype, p->d_xs, p->d_bins,
-                                     p->d_kbwork, kb0, std::min(p->fft_chunk, total - kb0),
-                                     p->nrows, p->d_tw, p->d_tw + p->fft_L, p->d_fy,
-                                     p->d_power, s))
-                return set_error(DXG2_EUNSUPPORTED, "no FFT kernel for length %d x %d",
-                                 p->fft_L1, p->fft_L2);
-    } else if (launch_fft_power(p->fft_L, p->dtype, p->d_xs, p->d_bins, p->d_kbwork,
-                                (int)p->kb_work.size(), p->nrows, p->d_tw, p->d_tw + p->fft_L,
-                                p->d_power, s)) {
-        return set_error(DXG2_EUNSUPPORTED, "no FFT kernel for length %d", p->fft_L);
-    }
-    launch_fft_inverse(p->d_power, p->fft_L, p->n_bins, p->N, p->d_fnum, s);
+    if (launch_fft_power(p->fft, p->dtype, p->d_xs, p->d_bins, p->d_kbwork,
+                         (int)p->kb_work.size(), p->d_tw, p->d_power, s))
+        return set_error(DXG2_EUNSUPPORTED, "no FFT kernel for length %d", p->fft.L);
+    launch_fft_inverse(p->d_power, p->fft.L, p->n_bins, p->N, p->d_fnum, s);
     if (ev) DXG2_HIP(hipEventRecord(ev[2], s));
     launch_finalize_f64(sums, p->d_fnum, p->d_bins, p->n_bins, p->N, p->d_prefix, p->d_smax,
                         p->d_dpre, d_num, d_den, d_g2, p->dmf, s);

@@ -234,21 +234,25 @@ void launch_fill_i32(int* p, int64_t n, hipStream_t s);
 void launch_finalize_f64(const int64_t* sums, const double* fnum, const BinDev* bins, int n_bins,
                          int nframes, int64_t* prefix, int64_t* smax, double* dpre, double* num,
                          double* den, float* g2, const DenMfma& dm, hipStream_t s);
-// Pixel-major copy xs of every bin's series (in the order of pix_idx) and the exact frame
-// sums (sums[b][t] for t < nframes, zeroed here first).  work: n_work items of PM_KPB
-// k-blocks (kb -1: none).  quad_kb (8-bit frames; may be null): per bin, the leading
+// A transform length of the FFT path: series of up to L = G H / 2 frames, Nf = 2 L = G H,
+// in G / 2 + 1 classes of transforms of length H; last = radix of a transform's last pass.
+struct FftShape {
+    int L, H, G, last;
+};
+// The shape of the smallest L >= n; false above 131072.
+bool fft_shape(int n, FftShape* out);
+// Series of every bin in pairs (pairs of pix_idx's entries; H G elements a pair) and the
+// exact frame sums (sums[b][t] for t < nframes, zeroed here first).  work: n_work items of
+// PM_KPB k-blocks (kb -1: none).  quad_kb (8-bit frames; may be null): per bin, the leading
 // k-blocks whose entries are 16 aligned pixel quads.
-void launch_gather_pm(const uint8_t* frames, int dtype, int64_t hw, int nframes, int nrows,
-                      const int32_t* pix_idx, const int32_t* quad_kb, const BinDev* bins,
-                      int n_bins, const KbWork* work, int n_work, uint8_t* xs, int64_t* sums,
-                      hipStream_t s);
-int fft_lds_length(int n);
-int fft_four_step_length(int n, int* L1, int* L2);
-int launch_fft_four_step(int L1, int L2, int dtype, const uint8_t* xs, const BinDev* bins,
-                         const KbWork* work, int kb0, int n_kb, int nrows, const float2* tw,
-                         const float2* uw, float2* y, double* power, hipStream_t s);
-int launch_fft_power(int L, int dtype, const uint8_t* xs, const BinDev* bins, const KbWork* work,
-                     int n_work, int nrows, const float2* tw, const float2* uw, double* power,
+void launch_gather_pm(const uint8_t* frames, int dtype, int64_t hw, int nframes,
+                      const FftShape& shape, const int32_t* pix_idx, const int32_t* quad_kb,
+                      const BinDev* bins, int n_bins, const KbWork* work, int n_work,
+                      uint8_t* xs, int64_t* sums, hipStream_t s);
+// tw: exp(-2 pi i m / H), m < H; the same by (r, b) = r * H / last + b: exp(-2 pi i r b / H);
+// exp(-pi i m / L), m <= L.
+int launch_fft_power(const FftShape& shape, int dtype, const uint8_t* xs, const BinDev* bins,
+                     const KbWork* work, int n_work, const float2* tw, double* power,
                      hipStream_t s);
 void launch_fft_inverse(const double* power, int L, int n_bins, int nframes, double* num,
                         hipStream_t s);

@@ -11,22 +11,26 @@
 // (the product with the reversed series is the same autocorrelation; the inverse is
 // linear, so one inverse per bin replaces one per pixel).  Nf = 2L with L >= N from a
 // set of mixed-radix lengths (2^a 5^b), so a linear autocorrelation needs no more.
-//  * gather_pm_kernel<E>: frames -> pixel-major series xs[k][t] of the frame element
-//    type E (uint8, int8 or uint16; k in the bin's raster list order, t < nrows, zero
-//    past the last frame), 64 pixels x 256 frames per workgroup through an LDS transpose;
-//    the same workgroup adds its 64 pixels per frame from the LDS tile and sends each
-//    frame's total to the exact S_b(t) with one 64-bit atomic.
-//  * fft_spectra_kernel<E, L, T, R...>: one workgroup per (bin, k-block of 64 series);
-//    each series is packed as z[n] = x[2n] + i x[2n+1] (L complex points) and
-//    transformed by an FP32 mixed-radix Stockham FFT (Govindaraju et al., "High
-//    performance discrete Fourier transforms on graphics processors", SC 2008) with
-//    register DFTs of radix 4, 5, 8 or 16, then unpacked to X[k], k = 0..L, and |X[k]|^2
-//    is accumulated in FP64 per thread.  The first pass reads its inputs straight from
-//    HBM into registers (the next series' are loaded while the current one is
-//    transformed); the twiddles of the middle passes come from small LDS tables and those
-//    of the last pass and the unpacking factors are held in registers, so the series
-//    loop issues no other global load.  The last pass works in place (each butterfly
-//    writes the points it read).
+//
+// A series is never transformed whole.  Nf = G H, and the bins f = G k + c of one class c
+// are a transform of length H of the folded and modulated series
+//   z_c[n] = exp(-2 pi i n c / Nf) sum_{m < G/2} x[n + H m] exp(-2 pi i m c / G),  n < H
+// (the terms m >= G/2 are the zero padding).  |X(f)| = |X(Nf - f)| leaves the classes
+// c = 0 .. G/2.  For 0 < c < G/2 one transform serves one series, and its H points are all
+// of class c (and of class G - c by symmetry).  For c = 0 and G/2 z_c is a real sequence
+// times a modulation, so two series share a transform as its real and imaginary parts:
+// |Z(f)|^2 + |Z(-f)|^2 = 2 (|X_1|^2 + |X_2|^2), which the symmetric sum at the end undoes.
+// No transform is unpacked, none is longer than LDS holds, and nothing goes through HBM
+// between passes, up to N = 131,072.
+//  * gather_pm_kernel<E>: frames -> series in pairs, D[pair][n][series][m] of the frame
+//    element type E (n < H, m < G/2; zero past the last frame), so one load gives a thread
+//    what a point of every class needs; 64 pixels x 256 frames per workgroup through an LDS
+//    transpose; the same workgroup adds its 64 pixels per frame from the LDS tile and sends
+//    each frame's total to the exact S_b(t) with one 64-bit atomic.
+//  * fft_spectra_kernel<E, Plan, G>: one workgroup per (k-block of 64 series, class); an
+//    FP32 mixed-radix Stockham FFT (Govindaraju et al., "High performance discrete Fourier
+//    transforms on graphics processors", SC 2008) with register DFTs; |Z|^2 of the last
+//    pass's outputs is accumulated in FP64 registers straight from the DFT.
 //  * fft_inverse_kernel: Num(tau) = (P_0 + (-1)^tau P_L + 2 sum_{k=1}^{L-1} P_k
 //    cos(2 pi k tau / Nf)) / Nf in FP64, the cosines by four interleaved FP64 rotation
 //    recurrences.
@@ -93,6 +97,37 @@ struct Dft<5> {
     }
 };
 
+// exp(-2 pi i m / 10) for m < 5
+__device__ __forceinline__ c32 w10(int m) {
+    constexpr float C1 = 0.80901699437494742f, S1 = 0.58778525229247314f;
+    constexpr float C2 = 0.30901699437494745f, S2 = 0.95105651629515353f;
+    switch (m) {
+        case 1: return c32{C1, -S1};
+        case 2: return c32{C2, -S2};
+        case 3: return c32{-C2, -S2};
+        case 4: return c32{-C1, -S1};
+        default: return c32{1.f, 0.f};
+    }
+}
+
+template <>
+struct Dft<10> {
+    // n = 2 m + p: E_p = DFT5 over m of a[2m + p]; a[k] = E0[k] + w10^k E1[k],
+    // a[k + 5] = E0[k] - w10^k E1[k]
+    __device__ __forceinline__ static void run(c32* a) {
+        c32 e0[5] = {a[0], a[2], a[4], a[6], a[8]};
+        c32 e1[5] = {a[1], a[3], a[5], a[7], a[9]};
+        Dft<5>::run(e0);
+        Dft<5>::run(e1);
+#pragma unroll
+        for (int k = 0; k < 5; ++k) {
+            const c32 t = k ? cmul(w10(k), e1[k]) : e1[k];
+            a[k] = cadd(e0[k], t);
+            a[k + 5] = csub(e0[k], t);
+        }
+    }
+};
+
 // exp(-2 pi i m / 8) for m < 4
 __device__ __forceinline__ c32 w8(int m) {
     constexpr float H = 0.70710678118654752f;
@@ -151,21 +186,6 @@ struct Dft<16> {
         }
         twist(e, a);
     }
-    // a[8..15] zero (the zero-padded half of a series): the first DFT4s see
-    // (a[p], a[4 + p], 0, 0), and Dft<4> on them gives these sums and differences (its
-    // terms with the zeros are exact), so the result is the same as run()'s.
-    __device__ __forceinline__ static void run_lo8(c32* a) {
-        c32 e[4][4];
-#pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            const c32 x0 = a[p], x1 = a[4 + p], y1 = negi(x1);
-            e[p][0] = cadd(x0, x1);
-            e[p][1] = cadd(x0, y1);
-            e[p][2] = csub(x0, x1);
-            e[p][3] = csub(x0, y1);
-        }
-        twist(e, a);
-    }
     // second stage: a[k + 4q] = DFT4 over p of (w16^(p k) E_p[k]), output q
     __device__ __forceinline__ static void twist(c32 (&e)[4][4], c32* a) {
 #pragma unroll
@@ -196,38 +216,50 @@ __device__ __forceinline__ int sw_step(int base, int r) {
 }
 
 // ----------------------------------------------------------- series layout
-// Raw load of complex point i of a series: elements 2i and 2i + 1 (one 16-bit word for
-// 8-bit frames, one 32-bit word for 16-bit frames), zero past the row.
-template <typename E>
-struct Elem;
-template <>
-struct Elem<uint8_t> {
-    static constexpr int SIZE = 1;
-    __device__ __forceinline__ static uint32_t load(const uint8_t* row, int i, int nrows) {
-        return 2 * i < nrows ? (uint32_t) reinterpret_cast<const uint16_t*>(row)[i] : 0u;
+// One point n of a pair of series: G elements (series p, fold m) at index p G/2 + m.
+template <typename E, int G>
+struct RawPoint {
+    static constexpr int NW = G * (int)sizeof(E) / 4;
+    uint32_t w[NW];
+    __device__ __forceinline__ void load(const uint8_t* row, int n) {
+        const uint8_t* src = row + (int64_t)n * (4 * NW);
+        if constexpr (NW == 1) {
+            w[0] = *reinterpret_cast<const uint32_t*>(src);
+        } else if constexpr (NW == 2) {
+            const uint2 v = *reinterpret_cast<const uint2*>(src);
+            w[0] = v.x;
+            w[1] = v.y;
+        } else {
+#pragma unroll
+            for (int i = 0; i < NW; i += 4) {
+                const uint4 v = *reinterpret_cast<const uint4*>(src + 4 * i);
+                w[i] = v.x;
+                w[i + 1] = v.y;
+                w[i + 2] = v.z;
+                w[i + 3] = v.w;
+            }
+        }
     }
-    __device__ __forceinline__ static c32 value(uint32_t r) {
-        return c32{(float)(r & 0xFFu), (float)(r >> 8)};
+    __device__ __forceinline__ int value(int e) const {
+        if constexpr (sizeof(E) == 1)
+            return (int)(E)((w[e >> 2] >> (8 * (e & 3))) & 0xFFu);
+        else
+            return (int)(E)((w[e >> 1] >> (16 * (e & 1))) & 0xFFFFu);
     }
-};
-template <>
-struct Elem<int8_t> {
-    static constexpr int SIZE = 1;
-    __device__ __forceinline__ static uint32_t load(const uint8_t* row, int i, int nrows) {
-        return 2 * i < nrows ? (uint32_t) reinterpret_cast<const uint16_t*>(row)[i] : 0u;
-    }
-    __device__ __forceinline__ static c32 value(uint32_t r) {
-        return c32{(float)(int8_t)(r & 0xFFu), (float)(int8_t)((r >> 8) & 0xFFu)};
-    }
-};
-template <>
-struct Elem<uint16_t> {
-    static constexpr int SIZE = 2;
-    __device__ __forceinline__ static uint32_t load(const uint8_t* row, int i, int nrows) {
-        return 2 * i < nrows ? reinterpret_cast<const uint32_t*>(row)[i] : 0u;
-    }
-    __device__ __forceinline__ static c32 value(uint32_t r) {
-        return c32{(float)(r & 0xFFFFu), (float)(r >> 16)};
+    // Series p's elements in the first half: one shift or mask a word, p known at run time.
+    __device__ __forceinline__ RawPoint series(int p) const {
+        RawPoint r;
+        if constexpr (NW == 1) {
+            r.w[0] = w[0] >> (p * 16);
+        } else {
+#pragma unroll
+            for (int i = 0; i < NW / 2; ++i) {
+                const uint32_t m = 0u - (uint32_t)p;
+                r.w[i] = (w[NW / 2 + i] & m) | (w[i] & ~m);
+                r.w[NW / 2 + i] = 0u;
+            }
+        }
+        return r;
     }
 };
 
@@ -236,9 +268,10 @@ struct Elem<uint16_t> {
 // load instruction reads one frame of the 64 pixels (the k-block's stretch of detector
 // row).  A lane packs 4 / sizeof(E) consecutive frames into one 32-bit word and writes
 // it to its pixel's row of an LDS tile whose row stride is an odd number of words, so
-// the 64 lanes' column writes fall in distinct banks; then each thread reads 16
-// contiguous bytes of one row and stores them to xs, so consecutive threads write
-// consecutive 16-byte pieces of a pixel's series.  The frame sums S_b(t) (zeroed first)
+// the 64 lanes' column writes fall in distinct banks.  The tile's frames are G / 2 runs,
+// run m at frames H m + n0 .., so it holds every element of SEG points of the pairs: a
+// thread reads the G words (series, run) of a few points of one pair, transposes them in
+// registers and stores 4 G contiguous bytes.  The frame sums S_b(t) (zeroed first)
 // come from the same tile: a thread adds one word (4 frames of 8-bit values in 16-bit
 // halves, or 2 of 16-bit values in 32-bit registers) down 16 or 32 pixel rows, the row
 // groups meet in LDS, and each frame's total over the 64 pixels (below 2^31) goes to
@@ -254,10 +287,10 @@ struct Elem<uint16_t> {
 // pixels' words of the tile.
 // A workgroup takes KPB k-blocks that are neighbours in detector order (work item
 // blockIdx.x; kb -1: none) over 256 / KPB frames, so that the workgroups in flight read
-// a larger share of each frame row, and still stores whole 128-byte lines of each series.
-template <typename E, bool SGN, int KPB>
+// a larger share of each frame row, and still stores whole 128-byte lines of each pair.
+template <typename E, bool SGN, int KPB, int G>
 __global__ __launch_bounds__(256) void gather_pm_kernel(const uint8_t* __restrict__ frames,
-                                                        int64_t hw, int nframes, int nrows,
+                                                        int64_t hw, int nframes, int H,
                                                         const int32_t* __restrict__ pix_idx,
                                                         const int32_t* __restrict__ quad_kb,
                                                         const BinDev* __restrict__ bins,
@@ -272,6 +305,8 @@ __global__ __launch_bounds__(256) void gather_pm_kernel(const uint8_t* __restric
     constexpr int ROWS = KPB * KB;     // pixel rows of the tile
     constexpr int RG = 256 / WPR;      // row groups of the sums (threads = WPR x RG)
     constexpr int RPG = ROWS / RG;     // rows per group: within one k-block
+    constexpr int SEG = FT / (G / 2);  // frames per run
+    static_assert(SEG % 4 == 0 && SEG % FPW == 0, "a word lies in one run");
     static_assert(KB % RPG == 0 && FT * KPB == 256 && WPR % 16 == 0, "gather shape");
     __shared__ __attribute__((aligned(16))) uint32_t tile[ROWS * STRIDE];
     static_assert(RG * FT <= ROWS * STRIDE, "partials fit the tile");
@@ -279,8 +314,8 @@ __global__ __launch_bounds__(256) void gather_pm_kernel(const uint8_t* __restric
     if (item[0].kb < 0) return;  // padding of the gather order (the first slot is filled first)
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
-    const int t0 = blockIdx.y * FT;
-    const int ntq = max(0, min(FT, nframes - t0));  // frames present
+    const int n0 = blockIdx.y * SEG;
+    auto frame_of = [&](int f) { return (f / SEG) * H + n0 + f % SEG; };  // of tile column f
     constexpr uint32_t MASK = ES == 1 ? 0xFFu : 0xFFFFu;
 #pragma unroll
     for (int j = 0; j < KPB; ++j) {
@@ -297,10 +332,10 @@ __global__ __launch_bounds__(256) void gather_pm_kernel(const uint8_t* __restric
                 uint32_t v[4];
 #pragma unroll
                 for (int f4 = 0; f4 < 4; ++f4) {
-                    const int f = 4 * k + f4;
-                    v[f4] = f < ntq ? *reinterpret_cast<const uint32_t*>(
-                                          frames + (int64_t)(t0 + f) * hw + q0)
-                                    : 0u;
+                    const int t = frame_of(4 * k) + f4;
+                    v[f4] = t < nframes ? *reinterpret_cast<const uint32_t*>(
+                                              frames + (int64_t)t * hw + q0)
+                                        : 0u;
                 }
                 // v[f] byte b = pixel 4g + b at frame 4k + f  ->  word k of pixel 4g + b
                 const uint32_t l01 = __builtin_amdgcn_perm(v[1], v[0], 0x05010400u);
@@ -316,15 +351,15 @@ __global__ __launch_bounds__(256) void gather_pm_kernel(const uint8_t* __restric
         } else {
             const int p = pix_idx[bd.idx_off + (int64_t)w.kb * KB + lane];
             const E* fr = reinterpret_cast<const E*>(frames) + (p >= 0 ? p : 0);
-            const int nt = p >= 0 ? ntq : 0;
+            const int nt = p >= 0 ? nframes : 0;
 #pragma unroll
             for (int i = 0; i < WPR / 4; ++i) {
-                const int k = wave + 4 * i;  // word k: frames t0 + FPW k ..
+                const int k = wave + 4 * i;  // word k: tile columns FPW k ..
+                const int tk = frame_of(FPW * k);
                 uint32_t word = 0u;
 #pragma unroll
                 for (int q = 0; q < FPW; ++q) {
-                    const int f = FPW * k + q;
-                    const uint32_t v = f < nt ? (uint32_t)fr[(int64_t)(t0 + f) * hw] : 0u;
+                    const uint32_t v = tk + q < nt ? (uint32_t)fr[(int64_t)(tk + q) * hw] : 0u;
                     word |= (v & MASK) << (8 * ES * q);
                 }
                 rows[lane * STRIDE + k] = word;
@@ -332,16 +367,41 @@ __global__ __launch_bounds__(256) void gather_pm_kernel(const uint8_t* __restric
         }
     }
     __syncthreads();
-    constexpr int CHUNKS = WPR / 4;  // 16-byte pieces per pixel row
-    for (int c = threadIdx.x; c < ROWS * CHUNKS; c += 256) {
-        const int r = c / CHUNKS;
-        const KbWork w = item[r / KB];
+    // pair r of the tile (rows 2r, 2r + 1), word k of every run: FPW points, 4 G bytes
+    constexpr int WPS = SEG / FPW;  // words per run
+    for (int c = threadIdx.x; c < ROWS / 2 * WPS; c += 256) {
+        const int r = c / WPS, k = c % WPS;
+        const KbWork w = item[2 * r / KB];
         if (w.kb < 0) continue;
-        const int o = (c % CHUNKS) * 4;
-        const uint32_t* src = tile + r * STRIDE + o;
-        uint8_t* dst = xs + bins[w.bin].slab_off +
-                       (((int64_t)w.kb * KB + r % KB) * nrows + t0) * ES + 4 * o;
-        *reinterpret_cast<uint4*>(dst) = make_uint4(src[0], src[1], src[2], src[3]);
+        uint32_t v[G], o[G];  // v[p G/2 + m]: series p, run m
+#pragma unroll
+        for (int i = 0; i < G; ++i)
+            v[i] = tile[(2 * r + i / (G / 2)) * STRIDE + (i % (G / 2)) * WPS + k];
+        if constexpr (ES == 1) {
+#pragma unroll
+            for (int i = 0; i < G; i += 4) {  // 4 x 4 bytes: element i + j of point q
+                const uint32_t l01 = __builtin_amdgcn_perm(v[i + 1], v[i], 0x05010400u);
+                const uint32_t h01 = __builtin_amdgcn_perm(v[i + 1], v[i], 0x07030602u);
+                const uint32_t l23 = __builtin_amdgcn_perm(v[i + 3], v[i + 2], 0x05010400u);
+                const uint32_t h23 = __builtin_amdgcn_perm(v[i + 3], v[i + 2], 0x07030602u);
+                o[i / 4] = __builtin_amdgcn_perm(l23, l01, 0x05040100u);
+                o[G / 4 + i / 4] = __builtin_amdgcn_perm(l23, l01, 0x07060302u);
+                o[G / 2 + i / 4] = __builtin_amdgcn_perm(h23, h01, 0x05040100u);
+                o[3 * G / 4 + i / 4] = __builtin_amdgcn_perm(h23, h01, 0x07060302u);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < G; i += 2) {  // 2 x 2 halves
+                o[i / 2] = __builtin_amdgcn_perm(v[i + 1], v[i], 0x05040100u);
+                o[G / 2 + i / 2] = __builtin_amdgcn_perm(v[i + 1], v[i], 0x07060302u);
+            }
+        }
+        const int64_t pair = (bins[w.bin].idx_off + (int64_t)w.kb * KB) / 2 + r % (KB / 2);
+        uint8_t* dst = xs + (pair * H + n0 + FPW * k) * (G * ES);
+#pragma unroll
+        for (int i = 0; i < G; i += 4)
+            *reinterpret_cast<uint4*>(dst + 4 * i) =
+                make_uint4(o[i], o[i + 1], o[i + 2], o[i + 3]);
     }
     const int k = threadIdx.x % WPR, g = threadIdx.x / WPR;  // word k, rows RPG g ..
     const uint32_t* col = tile + RPG * g * STRIDE + k;
@@ -373,10 +433,10 @@ __global__ __launch_bounds__(256) void gather_pm_kernel(const uint8_t* __restric
     else
         *reinterpret_cast<int2*>(part + FT * g + 2 * k) = make_int2((int)s0, (int)s1);
     __syncthreads();
-    // thread (j, f): frame t0 + f of k-block j, from the RG / KPB row groups of that k-block
+    // thread (j, f): column f of k-block j, from the RG / KPB row groups of that k-block
     const int jb = threadIdx.x / FT, f = threadIdx.x % FT;
     const KbWork w = item[jb];
-    const int t = t0 + f;
+    const int t = frame_of(f);
     if (w.kb >= 0 && t < nframes) {
         constexpr int GPK = RG / KPB;  // row groups per k-block
         int64_t tot = SGN ? -(int64_t)KB * 128 : 0;
@@ -389,15 +449,14 @@ __global__ __launch_bounds__(256) void gather_pm_kernel(const uint8_t* __restric
 }
 
 // ------------------------------------------------------------------- spectra
-// A plan: L complex points, T threads, radices R1..R4 (R4 = 1 when there are three
-// passes).  The last pass's twiddles are held in registers, the middle passes' in LDS
-// tables (pass p's table holds exp(-2 pi i m / P_p), m < P_p = R1 ... R_p).
+// A plan: L complex points (the H of a series length G H / 2), T threads, radices R1..R4
+// (R4 = 1 when there are three passes).  The middle passes' twiddles are in LDS tables
+// (pass p's table holds exp(-2 pi i m / P_p), m < P_p = R1 ... R_p).
 template <int L_, int T_, int R1_, int R2_, int R3_, int R4_>
 struct FftPlan {
     static constexpr int L = L_, T = T_, R1 = R1_, R2 = R2_, R3 = R3_, R4 = R4_;
     static constexpr int NP = R4 > 1 ? 4 : 3;
     static constexpr int RL = NP == 4 ? R4 : R3;        // radix of the last pass
-    static constexpr int NSL = L / RL;                   // its stride
     static constexpr int P2 = R1 * R2;                   // table of pass 2
     static constexpr int P3 = NP == 4 ? R1 * R2 * R3 : 1;  // table of pass 3 (4 passes)
     static_assert(R1 * R2 * R3 * R4 == L, "radices must multiply to L");
@@ -437,91 +496,114 @@ __device__ __forceinline__ void mid_pass(c32* z, const c32* tab, int tid) {
     __syncthreads();
 }
 
-template <typename E, typename Plan>
-__global__ __launch_bounds__(Plan::T) void fft_spectra_kernel(
-    const uint8_t* __restrict__ xs, const BinDev* __restrict__ bins,
-    const KbWork* __restrict__ work, int nrows, const float2* __restrict__ tw,
-    const float2* __restrict__ uw, double* __restrict__ power) {
-    constexpr int L = Plan::L, T = Plan::T;
+// What a class's transforms are made of.
+enum FftClass {
+    PAIR_PLAIN,  // class 0: two series as real and imaginary parts
+    PAIR_MOD,    // class G/2: the same, modulated
+    SINGLE       // classes between: one series each
+};
+
+// The transforms of one k-block (npair pairs from `rows`, nser series) and one class; the
+// sums of |Z[k]|^2 over them go to prow[f], f = G k + cls folded into [0, L].
+template <typename E, typename Plan, int G, FftClass MODE>
+__device__ __forceinline__ void spectra_class(const uint8_t* __restrict__ rows, int nser, int cls,
+                                              const float2* __restrict__ twl,
+                                              const float2* __restrict__ uw,
+                                              double* __restrict__ prow, c32* z, const c32* tab2,
+                                              const c32* tab3) {
+    constexpr int H = Plan::L, T = Plan::T, L = H * (G / 2);
     constexpr int R1 = Plan::R1, R2 = Plan::R2, R3 = Plan::R3, RL = Plan::RL;
-    constexpr int NB1 = L / R1, M1 = (NB1 + T - 1) / T;       // first pass
-    constexpr int NBL = L / RL, ML = (NBL + T - 1) / T;       // last pass
-    constexpr int HP = L / 2;                                 // k = HP pairs with itself
-    constexpr int MH = (HP + T - 1) / T;                      // pairs (k, L - k), k < HP
-    __shared__ c32 z[L];
-    __shared__ c32 tab2[Plan::P2];
-    __shared__ c32 tab3[Plan::P3];
-    const KbWork w = work[blockIdx.x];
-    const BinDev bd = bins[w.bin];
+    constexpr int NB1 = H / R1, M1 = (NB1 + T - 1) / T;  // first pass
+    constexpr int NBL = H / RL, ML = (NBL + T - 1) / T;  // last pass
+    using Raw = RawPoint<E, G>;
     const int tid = threadIdx.x;
-
-    for (int m = tid; m < Plan::P2; m += T) tab2[m] = c_of(tw[m * (L / Plan::P2)]);
-    if (Plan::NP == 4)
-        for (int m = tid; m < Plan::P3; m += T) tab3[m] = c_of(tw[m * (L / Plan::P3)]);
-    double acc_lo[MH], acc_hi[MH], acc_mid = 0.0;  // |X|^2 at k, L - k, HP
+    const int npair = (nser + 1) / 2;
+    double acc[ML][RL];
 #pragma unroll
-    for (int m = 0; m < MH; ++m) acc_lo[m] = acc_hi[m] = 0.0;
-
-    const int kend = min(KB, bd.npix - w.kb * KB);
-    const uint8_t* rows = xs + bd.slab_off + (int64_t)w.kb * KB * nrows * Elem<E>::SIZE;
-    const int64_t row_bytes = (int64_t)nrows * Elem<E>::SIZE;
-    // Points from L / 2 on are frames from L on, past every row (the launcher checks
-    // nrows <= L): the zero padding.  With R1 = 16 they are the first pass's inputs
-    // r >= 8, which are neither loaded nor added.
-    constexpr int RLD = R1 == 16 ? 8 : R1;   // inputs loaded per first-pass butterfly
-    static_assert(R1 != 16 || 8 * NB1 == L / 2, "zero half");
-    uint32_t raw[M1][RLD];
+    for (int m = 0; m < ML; ++m)
 #pragma unroll
-    for (int m = 0; m < M1; ++m)
+        for (int q = 0; q < RL; ++q) acc[m][q] = 0.0;
+    c32 fold[G / 2];  // exp(-2 pi i m cls / G)
 #pragma unroll
-        for (int r = 0; r < RLD; ++r) {
-            const int b = tid + m * T;
-            raw[m][r] = (NB1 % T == 0 || b < NB1) ? Elem<E>::load(rows, b + r * NB1, nrows) : 0u;
-        }
-    __syncthreads();   // tables
+    for (int m = 0; m < G / 2; ++m) sincospif(-2.0f * (m * cls) / G, &fold[m].y, &fold[m].x);
+    auto modn = [&](int b, int r) { return c_of(uw[(b + r * NB1) * cls]); };
+    const int64_t row_bytes = (int64_t)H * G * sizeof(E);
+    // A pair's points are loaded while the transform before it runs, where the registers
+    // allow it.
+    constexpr bool AHEAD = M1 * R1 * Raw::NW <= (T > 768 ? 8 : 32);
+    Raw raw[AHEAD ? M1 : 1][R1];
+    auto load = [&](const uint8_t* row, int t) {
+#pragma unroll
+        for (int m = 0; m < (AHEAD ? M1 : 0); ++m)
+#pragma unroll
+            for (int r = 0; r < R1; ++r) {
+                const int b = t + m * T;
+                if (NB1 % T == 0 || b < NB1) raw[m][r].load(row, b + r * NB1);
+            }
+    };
+    load(rows, tid);
+    __syncthreads();  // tables
 
-    for (int j = 0; j < kend; ++j) {
-        // Every address, twiddle and factor below depends on the thread only; an opaque
-        // copy of the thread index per series keeps the compiler from holding them all
-        // in registers across the series loop (which spills): they are recomputed and
-        // the last pass's twiddles and the unpacking factors re-read from L1/L2.  By
-        // then the next series' loads issued after the first pass have landed.
+    const int count = MODE == SINGLE ? nser : npair;
+    for (int j = 0; j < count; ++j) {
+        // Every address and twiddle below depends on the thread only; an opaque copy of
+        // the thread index per transform keeps the compiler from holding them all in
+        // registers across the loop (which spills).
         int t = tid;
         asm volatile("" : "+v"(t));
-        // first pass (stride 1, no twiddles) from the registers loaded during the
-        // previous series: z[b + r NB1] -> outputs q at b R1 + q
+        // first pass (stride 1) from the registers loaded during the previous transform:
+        // point b + r NB1 -> outputs q at b R1 + q
 #pragma unroll
         for (int m = 0; m < M1; ++m) {
             const int b = t + m * T;
             if (NB1 % T == 0 || b < NB1) {
                 c32 v[R1];
 #pragma unroll
-                for (int r = 0; r < RLD; ++r) v[r] = Elem<E>::value(raw[m][r]);
-                if constexpr (R1 == 16)
-                    Dft<16>::run_lo8(v);
-                else
-                    Dft<R1>::run(v);
+                for (int r = 0; r < R1; ++r) {
+                    Raw& x0 = raw[AHEAD ? m : 0][r];
+                    if (!AHEAD) x0.load(rows + (MODE == SINGLE ? j / 2 : j) * row_bytes, b + r * NB1);
+                    if (MODE == SINGLE) {
+                        const Raw x = x0.series(j & 1);
+                        if (G == 4) {  // fold[1] = -i
+                            const float a0 = x.value(0), a1 = x.value(1);
+                            const c32 w = modn(b, r);
+                            v[r] = c32{a0 * w.x + a1 * w.y, a0 * w.y - a1 * w.x};
+                        } else {
+                            c32 a{0.f, 0.f};
+#pragma unroll
+                            for (int i = 0; i < G / 2; ++i) {
+                                const float xi = x.value(i);
+                                a.x += xi * fold[i].x;
+                                a.y += xi * fold[i].y;
+                            }
+                            v[r] = cmul(a, modn(b, r));
+                        }
+                    } else {  // integer sums, alternating in class G/2
+                            const Raw& x = x0;
+                        int s0 = 0, s1 = 0;
+#pragma unroll
+                        for (int i = 0; i < G / 2; ++i) {
+                            const bool neg = MODE == PAIR_MOD && (i & 1);
+                            s0 += neg ? -x.value(i) : x.value(i);
+                            s1 += neg ? -x.value(G / 2 + i) : x.value(G / 2 + i);
+                        }
+                        v[r] = c32{(float)s0, (float)s1};
+                        if (MODE == PAIR_MOD) v[r] = cmul(v[r], modn(b, r));
+                    }
+                }
+                Dft<R1>::run(v);
 #pragma unroll
                 for (int q = 0; q < R1; ++q) z[sw(b * R1 + q)] = v[q];
             }
         }
-        // the next series' inputs, in flight during this series' passes
-        if (j + 1 < kend) {
-            const uint8_t* nxt = rows + (int64_t)(j + 1) * row_bytes;
-#pragma unroll
-            for (int m = 0; m < M1; ++m)
-#pragma unroll
-                for (int r = 0; r < RLD; ++r) {
-                    const int b = t + m * T;
-                    if (NB1 % T == 0 || b < NB1)
-                        raw[m][r] = Elem<E>::load(nxt, b + r * NB1, nrows);
-                }
-        }
+        // the next pair's inputs, in flight during this transform's passes
+        const int next = MODE == SINGLE ? (j + 1) / 2 : j + 1;
+        if ((MODE != SINGLE || (j & 1)) && next < npair) load(rows + next * row_bytes, t);
         __syncthreads();
         mid_pass<Plan, R2, R1, Plan::P2>(z, tab2, t);
         if (Plan::NP == 4) mid_pass<Plan, R3, R1 * R2, Plan::P3>(z, tab3, t);
-        // last pass, in place: butterfly b reads and writes z[b + r NSL]; its twiddles
-        // are exp(-2 pi i r b / L) (k = b < NSL)
+        // last pass: butterfly b reads z[b + r NBL], twiddles exp(-2 pi i r b / H) (its
+        // table is r-major), and its outputs q are the bins k = b + q NBL
 #pragma unroll
         for (int m = 0; m < ML; ++m) {
             const int b = t + m * T;
@@ -530,269 +612,69 @@ __global__ __launch_bounds__(Plan::T) void fft_spectra_kernel(
 #pragma unroll
                 for (int r = 0; r < RL; ++r) {
                     const c32 a = z[sw_step<NBL>(b, r)];
-                    v[r] = r ? cmul(a, c_of(tw[r * b])) : a;
+                    v[r] = r ? cmul(a, c_of(twl[r * NBL + b])) : a;
                 }
                 Dft<RL>::run(v);
 #pragma unroll
-                for (int q = 0; q < RL; ++q) z[sw_step<NBL>(b, q)] = v[q];
+                for (int q = 0; q < RL; ++q) {
+                    const double xr = v[q].x, xi = v[q].y;
+                    acc[m][q] = fma(xi, xi, fma(xr, xr, acc[m][q]));
+                }
             }
         }
-        __syncthreads();
-        // unpack X[k] = S + D with S = (Z[k] + conj Z[L-k]) / 2 and
-        // D = -i W^k (Z[k] - conj Z[L-k]) / 2, W = exp(-pi i / L), Z[L] = Z[0].  As
-        // W^(L-k) = -conj W^k, the same S and D give conj X[L-k] = S - D, so each pair
-        // (k, L - k), k < L/2, is read and unpacked once (k = L/2 pairs with itself), and
-        // |X|^2 accumulates at both ends.  With t < T only m = 0 meets k = 0, and only
-        // the last m can pass L/2: the other points need no test.  The halves of S and D
-        // are left out here, and the accumulated |2X|^2 is scaled by 1/4 (exact) when it
-        // is flushed.
-        auto unpack = [&](c32 a, c32 c, int k, double& lo, double* hi) {
-            const c32 s2 = c32{a.x + c.x, a.y - c.y};
-            const c32 d = c32{a.x - c.x, a.y + c.y};
-            const c32 wd = cmul(c_of(uw[k]), d);
-            const double xr = s2.x + wd.y, xi = s2.y - wd.x;  // 2 X[k], rounded in FP32
-            lo = fma(xi, xi, fma(xr, xr, lo));
-            if (hi) {
-                const double yr = s2.x - wd.y, yi = s2.y + wd.x;  // 2 conj X[L-k]
-                *hi = fma(yi, yi, fma(yr, yr, *hi));
-            }
-        };
-#pragma unroll
-        for (int m = 0; m < MH; ++m) {
-            const int k = t + m * T;
-            if (HP % T == 0 || m < MH - 1 || k < HP) {
-                const c32 a = z[sw_step<T>(t, m)];
-                const c32 c = z[m == 0 ? sw(k == 0 ? 0 : L - k) : sw_step<T>(L - t, -m)];
-                unpack(a, c, k, acc_lo[m], &acc_hi[m]);
-            }
-        }
-        if (t == 0) {
-            const c32 a = z[sw(HP)];
-            unpack(a, a, HP, acc_mid, nullptr);
-        }
-        __syncthreads();
+        __syncthreads();  // z is rewritten by the next transform
     }
-    double* prow = power + (int64_t)w.bin * (L + 1);
-#pragma unroll
-    for (int m = 0; m < MH; ++m) {
-        const int k = tid + m * T;
-        if (k < HP) {
-            if (acc_lo[m] != 0.0) atomicAdd(prow + k, 0.25 * acc_lo[m]);
-            if (acc_hi[m] != 0.0) atomicAdd(prow + L - k, 0.25 * acc_hi[m]);
-        }
-    }
-    if (tid == 0 && acc_mid != 0.0) atomicAdd(prow + HP, 0.25 * acc_mid);
-}
-
-// ------------------------------------------------- long series: four-step through HBM
-// For N > 16384 the half-length is L = L1 L2 (L1 a plan length up to 8192, L2 in
-// {2, 4, 5, 8, 16}) and the transform is split (Bailey's four-step FFT):
-//   n = n1 + L1 n2, k = k2 + L2 k1,
-//   Y[k2][n1] = exp(-2 pi i n1 k2 / L) DFT_L2 over n2 of z[n1 + L1 n2]   (four_step_cols)
-//   Z[k2 + L2 k1] = DFT_L1 over n1 of Y[k2][n1]                          (four_step_rows)
-// through a scratch Y of L complex values per series, for a chunk of k-blocks at a time.
-// Z[k] pairs with Z[L - k] = Z[(L2 - k2) + L2 (L1 - 1 - k1)] for k2 > 0 (and with
-// Z[L2 ((L1 - k1) mod L1)] for k2 = 0), so a workgroup of four_step_rows transforms the
-// two rows k2 and L2 - k2 of a series and unpacks them together.
-
-// grid (series of the chunk, ceil(L1 / 256)); thread = n1.  Series s of the chunk is row
-// j = s % 64 of k-block work[kb0 + s / 64].
-template <typename E, int L2>
-__global__ __launch_bounds__(256) void four_step_cols_kernel(
-    const uint8_t* __restrict__ xs, const BinDev* __restrict__ bins,
-    const KbWork* __restrict__ work, int kb0, int nrows, int L1,
-    const float2* __restrict__ tw, float2* __restrict__ y) {
-    const int s = blockIdx.x;
-    const KbWork w = work[kb0 + s / KB];
-    const BinDev bd = bins[w.bin];
-    const int j = s % KB;
-    if (j >= bd.npix - w.kb * KB) return;     // padding rows of a bin's last k-block
-    const int n1 = blockIdx.y * 256 + threadIdx.x;
-    if (n1 >= L1) return;
-    const uint8_t* row = xs + bd.slab_off +
-                         ((int64_t)w.kb * KB + j) * nrows * Elem<E>::SIZE;
-    c32 v[L2];
-#pragma unroll
-    for (int n2 = 0; n2 < L2; ++n2) v[n2] = Elem<E>::value(Elem<E>::load(row, n1 + L1 * n2, nrows));
-    Dft<L2>::run(v);
-    float2* out = y + (int64_t)s * L1 * L2;
-#pragma unroll
-    for (int k2 = 0; k2 < L2; ++k2) {
-        const c32 r = k2 ? cmul(v[k2], c_of(tw[n1 * k2])) : v[k2];
-        out[(int64_t)k2 * L1 + n1] = make_float2(r.x, r.y);
-    }
-}
-
-template <int L2>
-struct RowPairs {   // (row A, row B) with B = L2 - A, or B = A for a row that pairs itself
-    static constexpr int N = L2 / 2 + 1;
-    __device__ __forceinline__ static void get(int i, int& a, int& b) {
-        a = i;
-        b = (i == 0 || 2 * i == L2) ? i : L2 - i;
-    }
-};
-
-// First pass of one row from registers (complex values loaded from Y).
-template <typename Plan>
-__device__ __forceinline__ void first_pass_c(c32* z, const c32 (&raw)[(Plan::L / Plan::R1 + Plan::T - 1) / Plan::T][Plan::R1], int t) {
-    constexpr int L = Plan::L, T = Plan::T, R1 = Plan::R1;
-    constexpr int NB1 = L / R1, M1 = (NB1 + T - 1) / T;
-#pragma unroll
-    for (int m = 0; m < M1; ++m) {
-        const int b = t + m * T;
-        if (NB1 % T == 0 || b < NB1) {
-            c32 v[R1];
-#pragma unroll
-            for (int r = 0; r < R1; ++r) v[r] = raw[m][r];
-            Dft<R1>::run(v);
-#pragma unroll
-            for (int q = 0; q < R1; ++q) z[sw(b * R1 + q)] = v[q];
-        }
-    }
-}
-
-template <typename Plan>
-__device__ __forceinline__ void load_row(c32 (&raw)[(Plan::L / Plan::R1 + Plan::T - 1) / Plan::T][Plan::R1],
-                                         const float2* __restrict__ src, int t) {
-    constexpr int L = Plan::L, T = Plan::T, R1 = Plan::R1;
-    constexpr int NB1 = L / R1, M1 = (NB1 + T - 1) / T;
-#pragma unroll
-    for (int m = 0; m < M1; ++m)
-#pragma unroll
-        for (int r = 0; r < R1; ++r) {
-            const int b = t + m * T;
-            if (NB1 % T == 0 || b < NB1) raw[m][r] = c_of(src[b + r * NB1]);
-        }
-}
-
-// Last pass of one row in place; twiddles exp(-2 pi i r b / L1) = tw[r b L2].
-template <typename Plan>
-__device__ __forceinline__ void last_pass_row(c32* z, const float2* __restrict__ tw, int l2,
-                                              int t) {
-    constexpr int L = Plan::L, T = Plan::T, RL = Plan::RL;
-    constexpr int NBL = L / RL, ML = (NBL + T - 1) / T;
+    // f and Nf - f are the same bin.  A pair class sees every bin but f = 0 and L twice.
 #pragma unroll
     for (int m = 0; m < ML; ++m) {
-        const int b = t + m * T;
-        if (NBL % T == 0 || b < NBL) {
-            c32 v[RL];
+        const int b = tid + m * T;
+        if (b >= NBL) continue;
 #pragma unroll
-            for (int r = 0; r < RL; ++r) {
-                const c32 a = z[sw(b + r * NBL)];
-                v[r] = r ? cmul(a, c_of(tw[r * b * l2])) : a;
-            }
-            Dft<RL>::run(v);
-#pragma unroll
-            for (int q = 0; q < RL; ++q) z[sw(b + q * NBL)] = v[q];
+        for (int q = 0; q < RL; ++q) {
+            const int f = G * (b + q * NBL) + cls;
+            const int g = f <= L ? f : 2 * L - f;
+            const double w = MODE == SINGLE || g == 0 || g == L ? 1.0 : 0.5;
+            if (acc[m][q] != 0.0) atomicAdd(prow + g, w * acc[m][q]);
         }
     }
 }
 
-// grid (k-blocks of the chunk, row pairs); Plan is the row plan (L = L1 <= 8192).  The
-// power of bin b is accumulated at k = k2 + L2 k1 (and k = L by the row-0 workgroup).
-template <typename Plan, int L2>
-__global__ __launch_bounds__(Plan::T) void four_step_rows_kernel(
-    const float2* __restrict__ y, const BinDev* __restrict__ bins,
-    const KbWork* __restrict__ work, int kb0, const float2* __restrict__ tw,
-    const float2* __restrict__ uw, double* __restrict__ power) {
-    constexpr int L1 = Plan::L, T = Plan::T, R1 = Plan::R1, R2 = Plan::R2, R3 = Plan::R3;
-    constexpr int L = L1 * L2;
-    constexpr int M1 = (L1 / R1 + T - 1) / T;
-    constexpr int MU = (L1 + T - 1) / T;
-    __shared__ c32 za[L1];
-    __shared__ c32 zb[L1];
+// G / 2 + 1 workgroups (classes) per k-block, the classes of a k-block 8 apart so that they
+// share an XCD's L2.  What bounds the kernel is VALU issue and, with the barriers of each
+// pass, the wavefronts a CU holds: at H = L / 2 twice the workgroups fit that one transform
+// of L points allowed.  Against such transforms with an unpacking step (and, above 16,384
+// frames, a scratch in HBM): 14.2 -> 13.7 ms at 479,980 series of 10,000 frames, 55 -> 15.1
+// ms at 262,144 of 20,000; error of g2 against 64 bits 7e-6 -> 8e-7 and 4e-6 -> 1.3e-6.
+template <typename E, typename Plan, int G>
+__global__ __launch_bounds__(Plan::T, Plan::T > 512 ? 1 : 4) void fft_spectra_kernel(
+    const uint8_t* __restrict__ xs, const BinDev* __restrict__ bins,
+    const KbWork* __restrict__ work, int n_work, const float2* __restrict__ tw,
+    double* __restrict__ power) {
+    constexpr int H = Plan::L, T = Plan::T, L = H * (G / 2), NC = G / 2 + 1;
+    __shared__ c32 z[H];
     __shared__ c32 tab2[Plan::P2];
     __shared__ c32 tab3[Plan::P3];
-    const int kbl = blockIdx.x;
-    const KbWork w = work[kb0 + kbl];
+    const int bx = blockIdx.x;
+    const int i = bx / (8 * NC) * 8 + (bx & 7);
+    const int cls = NC - 1 - (bx >> 3) % NC;
+    if (i >= n_work) return;
+    const KbWork w = work[i];
     const BinDev bd = bins[w.bin];
-    int ra, rb;
-    RowPairs<L2>::get(blockIdx.y, ra, rb);
-    const bool self = ra == rb;
-    const int tid = threadIdx.x;
-    for (int m = tid; m < Plan::P2; m += T) tab2[m] = c_of(tw[m * (L1 / Plan::P2) * L2]);
-    if (Plan::NP == 4)
-        for (int m = tid; m < Plan::P3; m += T) tab3[m] = c_of(tw[m * (L1 / Plan::P3) * L2]);
-    double acc_a[MU], acc_b[MU];
-    double acc_last = 0.0;   // k = L (row 0 only)
-#pragma unroll
-    for (int m = 0; m < MU; ++m) acc_a[m] = acc_b[m] = 0.0;
-    const int kend = min(KB, bd.npix - w.kb * KB);
-    const float2* ybase = y + (int64_t)kbl * KB * L;
-    c32 raw_a[M1][R1], raw_b[M1][R1];
-    load_row<Plan>(raw_a, ybase + (int64_t)ra * L1, tid);
-    if (!self) load_row<Plan>(raw_b, ybase + (int64_t)rb * L1, tid);
-    __syncthreads();
-    for (int j = 0; j < kend; ++j) {
-        int t = tid;
-        asm volatile("" : "+v"(t));
-        first_pass_c<Plan>(za, raw_a, t);
-        if (!self) first_pass_c<Plan>(zb, raw_b, t);
-        if (j + 1 < kend) {
-            const float2* nxt = ybase + (int64_t)(j + 1) * L;
-            load_row<Plan>(raw_a, nxt + (int64_t)ra * L1, t);
-            if (!self) load_row<Plan>(raw_b, nxt + (int64_t)rb * L1, t);
-        }
-        __syncthreads();
-        mid_pass<Plan, R2, R1, Plan::P2>(za, tab2, t);
-        if (!self) mid_pass<Plan, R2, R1, Plan::P2>(zb, tab2, t);
-        if (Plan::NP == 4) {
-            mid_pass<Plan, R3, R1 * R2, Plan::P3>(za, tab3, t);
-            if (!self) mid_pass<Plan, R3, R1 * R2, Plan::P3>(zb, tab3, t);
-        }
-        last_pass_row<Plan>(za, tw, L2, t);
-        if (!self) last_pass_row<Plan>(zb, tw, L2, t);
-        __syncthreads();
-        // unpack: X[k] = (Z[k] + conj Z[L-k]) / 2 - i W^k (Z[k] - conj Z[L-k]) / 2
-        const c32* zo = self ? za : zb;   // the row holding the partners of row A
-#pragma unroll
-        for (int m = 0; m < MU; ++m) {
-            const int k1 = t + m * T;
-            if (k1 < L1) {
-                // row A point k1 and its partner
-                {
-                    const int ka = ra + L2 * k1;
-                    const int pk = ra == 0 ? (L1 - k1) % L1 : L1 - 1 - k1;
-                    const c32 a = za[sw(k1)];
-                    const c32 c = zo[sw(pk)];
-                    const c32 s2 = c32{a.x + c.x, a.y - c.y};
-                    const c32 d = c32{a.x - c.x, a.y + c.y};
-                    const c32 wd = cmul(c_of(uw[ka]), d);
-                    const float xr = 0.5f * (s2.x + wd.y), xi = 0.5f * (s2.y - wd.x);
-                    acc_a[m] += (double)xr * xr + (double)xi * xi;
-                }
-                if (!self) {   // row B point k1, partner in row A
-                    const int kb_ = rb + L2 * k1;
-                    const c32 a = zb[sw(k1)];
-                    const c32 c = za[sw(L1 - 1 - k1)];
-                    const c32 s2 = c32{a.x + c.x, a.y - c.y};
-                    const c32 d = c32{a.x - c.x, a.y + c.y};
-                    const c32 wd = cmul(c_of(uw[kb_]), d);
-                    const float xr = 0.5f * (s2.x + wd.y), xi = 0.5f * (s2.y - wd.x);
-                    acc_b[m] += (double)xr * xr + (double)xi * xi;
-                }
-            }
-        }
-        if (ra == 0 && t == 0) {   // k = L: Z[L] = Z[0]
-            const c32 a = za[sw(0)];
-            const c32 s2 = c32{a.x + a.x, 0.f};
-            const c32 d = c32{0.f, a.y + a.y};
-            const c32 wd = cmul(c_of(uw[L]), d);
-            const float xr = 0.5f * (s2.x + wd.y), xi = 0.5f * (s2.y - wd.x);
-            acc_last += (double)xr * xr + (double)xi * xi;
-        }
-        __syncthreads();
-    }
+    const int nser = min(KB, bd.npix - w.kb * KB);
+    const int64_t kb = (bd.idx_off + (int64_t)w.kb * KB) / KB;
+    const uint8_t* rows = xs + kb * (KB / 2) * ((int64_t)H * G * sizeof(E));
+    const float2* twl = tw + H;
+    const float2* uw = tw + 2 * H;
     double* prow = power + (int64_t)w.bin * (L + 1);
-#pragma unroll
-    for (int m = 0; m < MU; ++m) {
-        const int k1 = tid + m * T;
-        if (k1 < L1) {
-            if (acc_a[m] != 0.0) atomicAdd(prow + ra + L2 * k1, acc_a[m]);
-            if (!self && acc_b[m] != 0.0) atomicAdd(prow + rb + L2 * k1, acc_b[m]);
-        }
-    }
-    if (ra == 0 && tid == 0 && acc_last != 0.0) atomicAdd(prow + L, acc_last);
+    for (int m = threadIdx.x; m < Plan::P2; m += T) tab2[m] = c_of(tw[m * (H / Plan::P2)]);
+    if (Plan::NP == 4)
+        for (int m = threadIdx.x; m < Plan::P3; m += T) tab3[m] = c_of(tw[m * (H / Plan::P3)]);
+    if (cls == 0)
+        spectra_class<E, Plan, G, PAIR_PLAIN>(rows, nser, 0, twl, uw, prow, z, tab2, tab3);
+    else if (cls == G / 2)
+        spectra_class<E, Plan, G, PAIR_MOD>(rows, nser, cls, twl, uw, prow, z, tab2, tab3);
+    else
+        spectra_class<E, Plan, G, SINGLE>(rows, nser, cls, twl, uw, prow, z, tab2, tab3);
 }
 
 // Num(tau) from the power spectrum, FP64; grid (ceil(N / 256), n_bins).  Every
@@ -859,38 +741,9 @@ __global__ __launch_bounds__(256) void fft_inverse_kernel(const double* __restri
 }
 
 // ------------------------------------------------------------------ launchers
-template <typename E, bool SGN>
-static void gather_pm_typed(const uint8_t* frames, int64_t hw, int nframes, int nrows,
-                            const int32_t* pix_idx, const int32_t* quad_kb, const BinDev* bins,
-                            const KbWork* work, int n_work, uint8_t* xs, int64_t* sums,
-                            hipStream_t s) {
-    constexpr int FT = 256 / PM_KPB;  // nrows is a multiple of 256
-    gather_pm_kernel<E, SGN, PM_KPB>
-        <<<dim3((unsigned)n_work, (unsigned)(nrows / FT)), 256, 0, s>>>(
-            frames, hw, nframes, nrows, pix_idx, quad_kb, bins, work, xs, sums);
-}
-
-void launch_gather_pm(const uint8_t* frames, int dtype, int64_t hw, int nframes, int nrows,
-                      const int32_t* pix_idx, const int32_t* quad_kb, const BinDev* bins,
-                      int n_bins, const KbWork* work, int n_work, uint8_t* xs, int64_t* sums,
-                      hipStream_t s) {
-    if (n_bins <= 0) return;
-    launch_fill_i64(sums, (int64_t)n_bins * nframes, s);
-    if (n_work <= 0) return;
-    // aligned quad loads need 4 | hw and a 4-aligned frame pointer
-    if (hw % 4 != 0 || reinterpret_cast<uintptr_t>(frames) % 4 != 0) quad_kb = nullptr;
-    if (dtype == DXG2_U16)
-        gather_pm_typed<uint16_t, false>(frames, hw, nframes, nrows, pix_idx, nullptr, bins,
-                                         work, n_work, xs, sums, s);
-    else if (dtype == DXG2_I8)
-        gather_pm_typed<uint8_t, true>(frames, hw, nframes, nrows, pix_idx, quad_kb, bins, work,
-                                       n_work, xs, sums, s);
-    else
-        gather_pm_typed<uint8_t, false>(frames, hw, nframes, nrows, pix_idx, quad_kb, bins,
-                                        work, n_work, xs, sums, s);
-}
-
-// Lengths with a plan: L (complex points), threads, radices.
+// Plans: H points, threads, radices.
+using Plan512 = FftPlan<512, 64, 8, 8, 8, 1>;
+using Plan640 = FftPlan<640, 64, 10, 8, 8, 1>;
 using Plan1024 = FftPlan<1024, 64, 16, 16, 4, 1>;
 using Plan1280 = FftPlan<1280, 128, 16, 16, 5, 1>;
 using Plan2048 = FftPlan<2048, 128, 16, 16, 8, 1>;
@@ -899,141 +752,102 @@ using Plan4096 = FftPlan<4096, 256, 16, 16, 16, 1>;
 using Plan5120 = FftPlan<5120, 320, 16, 16, 5, 4>;
 using Plan8192 = FftPlan<8192, 512, 16, 16, 8, 4>;
 using Plan10240 = FftPlan<10240, 640, 16, 16, 5, 8>;
+using Plan12800 = FftPlan<12800, 832, 16, 16, 10, 5>;
 using Plan16384 = FftPlan<16384, 1024, 16, 16, 4, 16>;
 
-static const int kFftLengths[] = {1024, 1280, 2048, 2560, 4096, 5120, 8192, 10240, 16384};
+// Series lengths L = G H / 2 with their plan.  Each L is one of the lengths a series of N
+// frames may be padded to (the smallest with L >= N).
+#define DXG2_FFT_SHAPES(X)                                                              \
+    X(512, 4) X(640, 4) X(1024, 4) X(1280, 4) X(2048, 4) X(2560, 4) X(4096, 4) X(5120, 4) \
+    X(8192, 4) X(10240, 4) X(12800, 4) X(16384, 4) X(10240, 8) X(16384, 8) X(10240, 16)  \
+    X(16384, 16)
 
-int fft_lds_length(int n) {
-    for (int L : kFftLengths)
-        if (L >= n) return L;
-    return 0;
+bool fft_shape(int n, FftShape* out) {
+    int best = 0;
+#define DXG2_FFT_SHAPE(HH, GG)                                     \
+    if (HH * GG / 2 >= n && (!best || HH * GG / 2 < best)) {       \
+        best = HH * GG / 2;                                        \
+        *out = FftShape{best, HH, GG, Plan##HH::RL};               \
+    }
+    DXG2_FFT_SHAPES(DXG2_FFT_SHAPE)
+#undef DXG2_FFT_SHAPE
+    return best > 0;
 }
 
-template <typename E, typename Plan>
-static void spectra_typed(const uint8_t* xs, const BinDev* bins, const KbWork* work, int n_work,
-                          int nrows, const float2* tw, const float2* uw, double* power,
-                          hipStream_t s) {
-    fft_spectra_kernel<E, Plan><<<dim3((unsigned)n_work), Plan::T, 0, s>>>(xs, bins, work, nrows,
-                                                                          tw, uw, power);
+template <typename E, bool SGN, int G>
+static void gather_pm_typed(const uint8_t* frames, int64_t hw, int nframes, int H,
+                            const int32_t* pix_idx, const int32_t* quad_kb, const BinDev* bins,
+                            const KbWork* work, int n_work, uint8_t* xs, int64_t* sums,
+                            hipStream_t s) {
+    constexpr int SEG = 256 / PM_KPB / (G / 2);  // divides every plan length (multiples of 128)
+    gather_pm_kernel<E, SGN, PM_KPB, G>
+        <<<dim3((unsigned)n_work, (unsigned)(H / SEG)), 256, 0, s>>>(
+            frames, hw, nframes, H, pix_idx, quad_kb, bins, work, xs, sums);
 }
 
-template <typename Plan>
-static void spectra_dtype(int dtype, const uint8_t* xs, const BinDev* bins, const KbWork* work,
-                          int n_work, int nrows, const float2* tw, const float2* uw,
-                          double* power, hipStream_t s) {
+template <int G>
+static void gather_pm_fold(const uint8_t* frames, int dtype, int64_t hw, int nframes, int H,
+                           const int32_t* pix_idx, const int32_t* quad_kb, const BinDev* bins,
+                           const KbWork* work, int n_work, uint8_t* xs, int64_t* sums,
+                           hipStream_t s) {
     if (dtype == DXG2_U16)
-        spectra_typed<uint16_t, Plan>(xs, bins, work, n_work, nrows, tw, uw, power, s);
+        gather_pm_typed<uint16_t, false, G>(frames, hw, nframes, H, pix_idx, nullptr, bins, work,
+                                            n_work, xs, sums, s);
     else if (dtype == DXG2_I8)
-        spectra_typed<int8_t, Plan>(xs, bins, work, n_work, nrows, tw, uw, power, s);
+        gather_pm_typed<uint8_t, true, G>(frames, hw, nframes, H, pix_idx, quad_kb, bins, work,
+                                          n_work, xs, sums, s);
     else
-        spectra_typed<uint8_t, Plan>(xs, bins, work, n_work, nrows, tw, uw, power, s);
+        gather_pm_typed<uint8_t, false, G>(frames, hw, nframes, H, pix_idx, quad_kb, bins, work,
+                                           n_work, xs, sums, s);
 }
 
-int launch_fft_power(int L, int dtype, const uint8_t* xs, const BinDev* bins, const KbWork* work,
-                     int n_work, int nrows, const float2* tw, const float2* uw, double* power,
+void launch_gather_pm(const uint8_t* frames, int dtype, int64_t hw, int nframes,
+                      const FftShape& shape, const int32_t* pix_idx, const int32_t* quad_kb,
+                      const BinDev* bins, int n_bins, const KbWork* work, int n_work,
+                      uint8_t* xs, int64_t* sums, hipStream_t s) {
+    if (n_bins <= 0) return;
+    launch_fill_i64(sums, (int64_t)n_bins * nframes, s);
+    if (n_work <= 0) return;
+    // aligned quad loads need 4 | hw and a 4-aligned frame pointer
+    if (hw % 4 != 0 || reinterpret_cast<uintptr_t>(frames) % 4 != 0) quad_kb = nullptr;
+    if (shape.G == 4)
+        gather_pm_fold<4>(frames, dtype, hw, nframes, shape.H, pix_idx, quad_kb, bins, work,
+                          n_work, xs, sums, s);
+    else if (shape.G == 8)
+        gather_pm_fold<8>(frames, dtype, hw, nframes, shape.H, pix_idx, quad_kb, bins, work,
+                          n_work, xs, sums, s);
+    else
+        gather_pm_fold<16>(frames, dtype, hw, nframes, shape.H, pix_idx, quad_kb, bins, work,
+                           n_work, xs, sums, s);
+}
+
+template <typename Plan, int G>
+static void spectra_dtype(int dtype, const uint8_t* xs, const BinDev* bins, const KbWork* work,
+                          int n_work, const float2* tw, double* power, hipStream_t s) {
+    const dim3 grid((unsigned)((n_work + 7) / 8 * 8 * (G / 2 + 1)));
+    if (dtype == DXG2_U16)
+        fft_spectra_kernel<uint16_t, Plan, G>
+            <<<grid, Plan::T, 0, s>>>(xs, bins, work, n_work, tw, power);
+    else if (dtype == DXG2_I8)
+        fft_spectra_kernel<int8_t, Plan, G>
+            <<<grid, Plan::T, 0, s>>>(xs, bins, work, n_work, tw, power);
+    else
+        fft_spectra_kernel<uint8_t, Plan, G>
+            <<<grid, Plan::T, 0, s>>>(xs, bins, work, n_work, tw, power);
+}
+
+int launch_fft_power(const FftShape& shape, int dtype, const uint8_t* xs, const BinDev* bins,
+                     const KbWork* work, int n_work, const float2* tw, double* power,
                      hipStream_t s) {
     if (n_work <= 0) return 0;
-    if (nrows > L) return -1;  // the spectra kernels take frames from L on as zero
-#define DXG2_FFT_CASE(LL)                                                                  \
-    case LL:                                                                               \
-        spectra_dtype<Plan##LL>(dtype, xs, bins, work, n_work, nrows, tw, uw, power, s);   \
-        return 0;
-    switch (L) {
-        DXG2_FFT_CASE(1024)
-        DXG2_FFT_CASE(1280)
-        DXG2_FFT_CASE(2048)
-        DXG2_FFT_CASE(2560)
-        DXG2_FFT_CASE(4096)
-        DXG2_FFT_CASE(5120)
-        DXG2_FFT_CASE(8192)
-        DXG2_FFT_CASE(10240)
-        DXG2_FFT_CASE(16384)
-        default:
-            return -1;
+#define DXG2_FFT_CASE(HH, GG)                                                        \
+    if (shape.H == HH && shape.G == GG) {                                            \
+        spectra_dtype<Plan##HH, GG>(dtype, xs, bins, work, n_work, tw, power, s);    \
+        return 0;                                                                    \
     }
+    DXG2_FFT_SHAPES(DXG2_FFT_CASE)
 #undef DXG2_FFT_CASE
-}
-
-// Long series: L = L1 L2 with L1 a row plan (<= 8192) and L2 in {2, 4, 5, 8, 16}; the
-// smallest such L >= n above 16384, the larger L1 on ties.  Returns 0 past 131072.
-static const int kRowLengths[] = {8192, 5120, 4096, 2560, 2048, 1280, 1024};
-static const int kColLengths[] = {2, 4, 5, 8, 16};
-
-int fft_four_step_length(int n, int* L1, int* L2) {
-    int best = 0;
-    for (int l1 : kRowLengths)
-        for (int l2 : kColLengths) {
-            const int L = l1 * l2;
-            if (L >= n && L > 16384 && (best == 0 || L < best)) {
-                best = L;
-                *L1 = l1;
-                *L2 = l2;
-            }
-        }
-    return best;
-}
-
-template <typename E, int L2>
-static void cols_typed(const uint8_t* xs, const BinDev* bins, const KbWork* work, int kb0,
-                       int n_kb, int nrows, int L1, const float2* tw, float2* y, hipStream_t s) {
-    four_step_cols_kernel<E, L2><<<dim3((unsigned)(n_kb * KB), (unsigned)((L1 + 255) / 256)),
-                                   256, 0, s>>>(xs, bins, work, kb0, nrows, L1, tw, y);
-}
-
-template <int L2>
-static void cols_dtype(int dtype, const uint8_t* xs, const BinDev* bins, const KbWork* work,
-                       int kb0, int n_kb, int nrows, int L1, const float2* tw, float2* y,
-                       hipStream_t s) {
-    if (dtype == DXG2_U16)
-        cols_typed<uint16_t, L2>(xs, bins, work, kb0, n_kb, nrows, L1, tw, y, s);
-    else if (dtype == DXG2_I8)
-        cols_typed<int8_t, L2>(xs, bins, work, kb0, n_kb, nrows, L1, tw, y, s);
-    else
-        cols_typed<uint8_t, L2>(xs, bins, work, kb0, n_kb, nrows, L1, tw, y, s);
-}
-
-template <typename Plan, int L2>
-static void rows_launch(const float2* y, const BinDev* bins, const KbWork* work, int kb0,
-                        int n_kb, const float2* tw, const float2* uw, double* power,
-                        hipStream_t s) {
-    four_step_rows_kernel<Plan, L2><<<dim3((unsigned)n_kb, (unsigned)RowPairs<L2>::N), Plan::T,
-                                      0, s>>>(y, bins, work, kb0, tw, uw, power);
-}
-
-template <int L2>
-static int rows_plan(int L1, const float2* y, const BinDev* bins, const KbWork* work, int kb0,
-                     int n_kb, const float2* tw, const float2* uw, double* power,
-                     hipStream_t s) {
-    switch (L1) {
-        case 1024: rows_launch<Plan1024, L2>(y, bins, work, kb0, n_kb, tw, uw, power, s); return 0;
-        case 1280: rows_launch<Plan1280, L2>(y, bins, work, kb0, n_kb, tw, uw, power, s); return 0;
-        case 2048: rows_launch<Plan2048, L2>(y, bins, work, kb0, n_kb, tw, uw, power, s); return 0;
-        case 2560: rows_launch<Plan2560, L2>(y, bins, work, kb0, n_kb, tw, uw, power, s); return 0;
-        case 4096: rows_launch<Plan4096, L2>(y, bins, work, kb0, n_kb, tw, uw, power, s); return 0;
-        case 5120: rows_launch<Plan5120, L2>(y, bins, work, kb0, n_kb, tw, uw, power, s); return 0;
-        case 8192: rows_launch<Plan8192, L2>(y, bins, work, kb0, n_kb, tw, uw, power, s); return 0;
-        default: return -1;
-    }
-}
-
-// One chunk of k-blocks [kb0, kb0 + n_kb) through the scratch y (n_kb * 64 * L complex).
-int launch_fft_four_step(int L1, int L2, int dtype, const uint8_t* xs, const BinDev* bins,
-                         const KbWork* work, int kb0, int n_kb, int nrows, const float2* tw,
-                         const float2* uw, float2* y, double* power, hipStream_t s) {
-    if (n_kb <= 0) return 0;
-    switch (L2) {
-        case 2: cols_dtype<2>(dtype, xs, bins, work, kb0, n_kb, nrows, L1, tw, y, s);
-                return rows_plan<2>(L1, y, bins, work, kb0, n_kb, tw, uw, power, s);
-        case 4: cols_dtype<4>(dtype, xs, bins, work, kb0, n_kb, nrows, L1, tw, y, s);
-                return rows_plan<4>(L1, y, bins, work, kb0, n_kb, tw, uw, power, s);
-        case 5: cols_dtype<5>(dtype, xs, bins, work, kb0, n_kb, nrows, L1, tw, y, s);
-                return rows_plan<5>(L1, y, bins, work, kb0, n_kb, tw, uw, power, s);
-        case 8: cols_dtype<8>(dtype, xs, bins, work, kb0, n_kb, nrows, L1, tw, y, s);
-                return rows_plan<8>(L1, y, bins, work, kb0, n_kb, tw, uw, power, s);
-        case 16: cols_dtype<16>(dtype, xs, bins, work, kb0, n_kb, nrows, L1, tw, y, s);
-                 return rows_plan<16>(L1, y, bins, work, kb0, n_kb, tw, uw, power, s);
-        default: return -1;
-    }
+    return -1;
 }
 
 void launch_fft_inverse(const double* power, int L, int n_bins, int nframes, double* num,

@@ -169,3 +169,31 @@ def test_fft_aligned_quads_ring_bins(dtype, offset):
     c = FFTCorrelator(shape, n, q)
     g2 = c.correlate(view)
     _check(c, g2, f, q)
+
+
+# (frames, half-length L) of series longer than 16,384: transforms of length L/2, L/4 and L/8
+LONG = [(16385, 20480), (25599, 25600), (25601, 32768), (32769, 40960), (50001, 65536),
+        (65537, 81920), (131072, 131072)]
+
+
+@pytest.mark.parametrize("dtype", [np.uint8, np.int8, np.uint16])
+@pytest.mark.parametrize("n,L", LONG)
+def test_fft_long_series_every_length(n, L, dtype):
+    """Every folded shape above 16,384 frames, with an odd number of pixels in a bin (its
+    last pair has one series) and the first and last frame of the longest series occupied."""
+    from dynamix_amd.correlator.dense import FFTCorrelator, fft_length
+    _announce("fft long n=%d L=%d %s" % (n, L, np.dtype(dtype).name))
+    assert fft_length(n) == 2 * L
+    shape = (3, 5)
+    rng = np.random.default_rng(n)
+    f = (rng.random((n,) + shape) < 0.02) * rng.integers(1, 9, size=(n,) + shape)
+    if dtype == np.int8:
+        f = f * rng.choice([-1, 1], size=f.shape)
+    f[0] = f[-1] = 3
+    if dtype == np.uint16:
+        f[:: n // 7, 1, 1] = 50000
+    f = f.astype(dtype)
+    q = np.ones(shape, np.int32)
+    q[0, :4] = 2
+    c = FFTCorrelator(shape, n, q)
+    _check(c, c.correlate(f), f, q, _sparse_ref(f, q))
