@@ -301,7 +301,7 @@ struct dxg2_plan {
     int32_t* d_fftqkb = nullptr;
     uint8_t* d_xs = nullptr;       // series pairs (fft_series_bytes)
     float2* d_tw = nullptr;        // twiddles (launch_fft_power)
-    double* d_power = nullptr;     // (n_bins, L + 1)
+    double* d_power = nullptr;     // n_bins rows of fft_power_row doubles
     double* d_fnum = nullptr;      // (n_bins, N)
     FftShape fft{};
 
@@ -652,6 +652,9 @@ size_t fft_series_bytes(const dxg2_plan* p, int L) {
     return std::max<size_t>(16, p->pix_idx.size() * (size_t)L * size);
 }
 
+// Sums of one bin in the FFT path's power buffer.
+int64_t fft_power_row(const FftShape& f) { return (int64_t)(f.G / 2 + 1) * f.H; }
+
 int ensure_fft_buffers(dxg2_plan* p, hipStream_t s) {
     if (p->d_power) return DXG2_OK;
     p->kb_work.clear();
@@ -740,7 +743,7 @@ int ensure_fft_buffers(dxg2_plan* p, hipStream_t s) {
          (dev_alloc(p->alloc, (void**)&kbw, p->kb_work.size() * sizeof(KbWork), s) != hipSuccess ||
           dev_alloc(p->alloc, (void**)&kbg, p->kb_gather.size() * sizeof(KbWork), s) !=
               hipSuccess)) ||
-        dev_alloc(p->alloc, (void**)&power, (size_t)std::max(p->n_bins, 1) * (L + 1) * sizeof(double), s) !=
+        dev_alloc(p->alloc, (void**)&power, (size_t)std::max(p->n_bins, 1) * fft_power_row(shape) * sizeof(double), s) !=
             hipSuccess) {
         for (void* b : {(void*)xs, (void*)tw, (void*)fnum, (void*)kbw, (void*)kbg, (void*)power,
                         (void*)pixf, (void*)qkb})
@@ -1330,7 +1333,7 @@ int dxg2_plan_footprint(const dxg2_plan* p, int32_t path, size_t* bytes) {
             for (const auto& bd : p->bins) nkb += bd.nkb;
             *bytes = common + fft_series_bytes(p, L) +
                      (2 * (size_t)shape.H + L + 1) * sizeof(float2) +
-                     (size_t)std::max(p->n_bins, 1) * ((L + 1) + p->N) * sizeof(double) +
+                     (size_t)std::max(p->n_bins, 1) * (fft_power_row(shape) + p->N) * sizeof(double) +
                      (2 * (size_t)nkb + (size_t)N_XCD * PM_XCD_GROUP) * sizeof(KbWork) +
                      (p->pix_idx.size() + (size_t)std::max(p->n_bins, 1)) * sizeof(int32_t);
             return DXG2_OK;
@@ -1976,7 +1979,7 @@ int dxg2_correlate_fft(dxg2_plan* p, const void* d_frames, double* d_num, int64_
     hipEvent_t* ev = nullptr;
     if (p->profiling && (rc = next_events(p, &ev))) return rc;
     if (ev) DXG2_HIP(hipEventRecord(ev[0], s));
-    launch_fill_i64(reinterpret_cast<int64_t*>(p->d_power), (int64_t)p->n_bins * (p->fft.L + 1), s);
+    launch_fill_i64(reinterpret_cast<int64_t*>(p->d_power), p->n_bins * fft_power_row(p->fft), s);
     const bool quads = reinterpret_cast<uintptr_t>(d_frames) % 4 == 0;
     launch_gather_pm((const uint8_t*)d_frames, p->dtype, (int64_t)p->H * p->W, p->N, p->fft,
                      p->d_pixfft, quads ? p->d_fftqkb : nullptr, p->d_bins, p->n_bins,
@@ -1985,7 +1988,7 @@ int dxg2_correlate_fft(dxg2_plan* p, const void* d_frames, double* d_num, int64_
     if (launch_fft_power(p->fft, p->dtype, p->d_xs, p->d_bins, p->d_kbwork,
                          (int)p->kb_work.size(), p->d_tw, p->d_power, s))
         return set_error(DXG2_EUNSUPPORTED, "no FFT kernel for length %d", p->fft.L);
-    launch_fft_inverse(p->d_power, p->fft.L, p->n_bins, p->N, p->d_fnum, s);
+    launch_fft_inverse(p->d_power, p->fft, p->n_bins, p->N, p->d_fnum, s);
     if (ev) DXG2_HIP(hipEventRecord(ev[2], s));
     launch_finalize_f64(sums, p->d_fnum, p->d_bins, p->n_bins, p->N, p->d_prefix, p->d_smax,
                         p->d_dpre, d_num, d_den, d_g2, p->dmf, s);

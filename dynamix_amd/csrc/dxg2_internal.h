@@ -250,12 +250,12 @@ void launch_gather_pm(const uint8_t* frames, int dtype, int64_t hw, int nframes,
                       const BinDev* bins, int n_bins, const KbWork* work, int n_work,
                       uint8_t* xs, int64_t* sums, hipStream_t s);
 // tw: exp(-2 pi i m / H), m < H; the same by (r, b) = r * H / last + b: exp(-2 pi i r b / H);
-// exp(-pi i m / L), m <= L.
+// exp(-pi i m / L), m <= L.  work: the k-blocks.  power: (G / 2 + 1) H sums of each bin, added to.
 int launch_fft_power(const FftShape& shape, int dtype, const uint8_t* xs, const BinDev* bins,
                      const KbWork* work, int n_work, const float2* tw, double* power,
                      hipStream_t s);
-void launch_fft_inverse(const double* power, int L, int n_bins, int nframes, double* num,
-                        hipStream_t s);
+void launch_fft_inverse(const double* power, const FftShape& shape, int n_bins, int nframes,
+                        double* num, hipStream_t s);
 void launch_excl_scan(const uint32_t* in, int64_t n, uint32_t* tot, uint32_t* out, hipStream_t s);
 void launch_events_window(int dtype, const uint32_t* offsets, const int32_t* times,
                           const void* data, int64_t npix, int t0, int t1, uint32_t* scratch,

@@ -503,15 +503,15 @@ enum FftClass {
     SINGLE       // classes between: one series each
 };
 
-// The transforms of one k-block (npair pairs from `rows`, nser series) and one class; the
-// sums of |Z[k]|^2 over them go to prow[f], f = G k + cls folded into [0, L].
+// The transforms of nser series (pairs from `rows`) and one class; the sums of |Z[k]|^2
+// over them are added to prow[k], k < H.
 template <typename E, typename Plan, int G, FftClass MODE>
 __device__ __forceinline__ void spectra_class(const uint8_t* __restrict__ rows, int nser, int cls,
                                               const float2* __restrict__ twl,
                                               const float2* __restrict__ uw,
                                               double* __restrict__ prow, c32* z, const c32* tab2,
                                               const c32* tab3) {
-    constexpr int H = Plan::L, T = Plan::T, L = H * (G / 2);
+    constexpr int H = Plan::L, T = Plan::T;
     constexpr int R1 = Plan::R1, R2 = Plan::R2, R3 = Plan::R3, RL = Plan::RL;
     constexpr int NB1 = H / R1, M1 = (NB1 + T - 1) / T;  // first pass
     constexpr int NBL = H / RL, ML = (NBL + T - 1) / T;  // last pass
@@ -624,33 +624,31 @@ __device__ __forceinline__ void spectra_class(const uint8_t* __restrict__ rows, 
         }
         __syncthreads();  // z is rewritten by the next transform
     }
-    // f and Nf - f are the same bin.  A pair class sees every bin but f = 0 and L twice.
 #pragma unroll
     for (int m = 0; m < ML; ++m) {
         const int b = tid + m * T;
-        if (b >= NBL) continue;
+        if (NBL % T != 0 && b >= NBL) continue;
 #pragma unroll
-        for (int q = 0; q < RL; ++q) {
-            const int f = G * (b + q * NBL) + cls;
-            const int g = f <= L ? f : 2 * L - f;
-            const double w = MODE == SINGLE || g == 0 || g == L ? 1.0 : 0.5;
-            if (acc[m][q] != 0.0) atomicAdd(prow + g, w * acc[m][q]);
-        }
+        for (int q = 0; q < RL; ++q)
+            if (acc[m][q] != 0.0) atomicAdd(prow + b + q * NBL, acc[m][q]);
     }
 }
 
 // G / 2 + 1 workgroups (classes) per k-block, the classes of a k-block 8 apart so that they
-// share an XCD's L2.  What bounds the kernel is VALU issue and, with the barriers of each
-// pass, the wavefronts a CU holds: at H = L / 2 twice the workgroups fit that one transform
-// of L points allowed.  Against such transforms with an unpacking step (and, above 16,384
-// frames, a scratch in HBM): 14.2 -> 13.7 ms at 479,980 series of 10,000 frames, 55 -> 15.1
-// ms at 262,144 of 20,000; error of g2 against 64 bits 7e-6 -> 8e-7 and 4e-6 -> 1.3e-6.
+// share an XCD's L2 (items of 2, 4 and 8 k-blocks, which flush fewer sums, were 1, 4 and 9 %
+// slower).  What bounds the kernel is VALU issue and, with two barriers a pass, the waves a
+// CU holds: at H = L / 2 twice the workgroups fit that a transform of L points allows, and
+// plans of 8 to 10 points a thread leave 20 waves a CU where radix-16 passes of 16 points
+// left 15 (10.6 against 13.7 ms at 479,980 series of 10,000 frames; 14.2 for whole
+// transforms with an unpacking step).  262,144 series of 20,000 frames: 14.0 ms, against
+// 55 for whole transforms through a scratch in HBM; folding those once more (G = 8, H =
+// 5,120) 16.  Error of g2 against 64 bits: 7e-6 -> 8e-7 and 4e-6 -> 1.3e-6.
 template <typename E, typename Plan, int G>
-__global__ __launch_bounds__(Plan::T, Plan::T > 512 ? 1 : 4) void fft_spectra_kernel(
+__global__ __launch_bounds__(Plan::T, Plan::T == 640 ? 5 : 4) void fft_spectra_kernel(
     const uint8_t* __restrict__ xs, const BinDev* __restrict__ bins,
     const KbWork* __restrict__ work, int n_work, const float2* __restrict__ tw,
     double* __restrict__ power) {
-    constexpr int H = Plan::L, T = Plan::T, L = H * (G / 2), NC = G / 2 + 1;
+    constexpr int H = Plan::L, T = Plan::T, NC = G / 2 + 1;
     __shared__ c32 z[H];
     __shared__ c32 tab2[Plan::P2];
     __shared__ c32 tab3[Plan::P3];
@@ -665,7 +663,7 @@ __global__ __launch_bounds__(Plan::T, Plan::T > 512 ? 1 : 4) void fft_spectra_ke
     const uint8_t* rows = xs + kb * (KB / 2) * ((int64_t)H * G * sizeof(E));
     const float2* twl = tw + H;
     const float2* uw = tw + 2 * H;
-    double* prow = power + (int64_t)w.bin * (L + 1);
+    double* prow = power + ((int64_t)w.bin * NC + cls) * H;
     for (int m = threadIdx.x; m < Plan::P2; m += T) tab2[m] = c_of(tw[m * (H / Plan::P2)]);
     if (Plan::NP == 4)
         for (int m = threadIdx.x; m < Plan::P3; m += T) tab3[m] = c_of(tw[m * (H / Plan::P3)]);
@@ -685,11 +683,28 @@ __global__ __launch_bounds__(Plan::T, Plan::T > 512 ? 1 : 4) void fft_spectra_ke
 // recurrences (k = k0 + 4 m + r, each turning by 4 theta, theta = 2 pi tau / Nf), so four
 // dependent chains overlap; each chain is re-anchored with sincospi at every chunk start
 // (512 rotations at most), and the four partial sums are joined in a fixed order.
+// The rows of `power` are the classes' sums [class c <= G/2][k < H]: bin f = G k + c, and
+// f = Nf - G k - c for the classes past G/2.  The pair classes hold every bin twice, as f
+// and Nf - f (but f = 0 and L once), each time the same |X_1|^2 + |X_2|^2 plus a term that
+// changes sign: P_f is their mean.
+__device__ __forceinline__ double power_of(const double* __restrict__ row, int G, int H, int f) {
+    int c = f % G, k = f / G;
+    if (2 * c > G) {  // the mirror of a class below G/2: Nf - f = G (H - 1 - k) + G - c
+        c = G - c;
+        k = H - 1 - k;
+    }
+    const double p = row[c * H + k];
+    if (c != 0 && 2 * c != G) return p;
+    const int m = c ? H - 1 - k : (k ? H - k : 0);
+    return 0.5 * (p + row[c * H + m]);
+}
 constexpr int INV_CH = 2048;
 constexpr int INV_G = 4;
 __global__ __launch_bounds__(256) void fft_inverse_kernel(const double* __restrict__ power,
-                                                          int L, int n_bins, int nframes,
+                                                          int G, int H, int n_bins, int nframes,
                                                           double* __restrict__ num) {
+    const int L = G / 2 * H;
+    const int64_t row = (int64_t)(G / 2 + 1) * H;  // doubles of a bin
     __shared__ double pk[INV_G][INV_CH];
     const int b0 = blockIdx.y * INV_G;
     const int ng = min(INV_G, n_bins - b0);
@@ -710,7 +725,7 @@ __global__ __launch_bounds__(256) void fft_inverse_kernel(const double* __restri
         __syncthreads();                     // the previous chunk has been read
         for (int i = threadIdx.x; i < INV_G * INV_CH; i += 256) {
             const int g = i / INV_CH, k = i % INV_CH;
-            pk[g][k] = (g < ng && k < n) ? power[(int64_t)(b0 + g) * (L + 1) + k0 + k] : 0.0;
+            pk[g][k] = (g < ng && k < n) ? power_of(power + (b0 + g) * row, G, H, k0 + k) : 0.0;
         }
         __syncthreads();
         double c[4], s[4];
@@ -733,8 +748,8 @@ __global__ __launch_bounds__(256) void fft_inverse_kernel(const double* __restri
 #pragma unroll
     for (int g = 0; g < INV_G; ++g) {
         if (g >= ng) break;
-        const double* ps = power + (int64_t)(b0 + g) * (L + 1);
-        const double last = (tau & 1) ? -ps[L] : ps[L];
+        const double* ps = power + (b0 + g) * row;
+        const double pl = power_of(ps, G, H, L), last = (tau & 1) ? -pl : pl;
         num[(int64_t)(b0 + g) * nframes + tau] =
             (ps[0] + last + 2.0 * ((acc[g][0] + acc[g][1]) + (acc[g][2] + acc[g][3]))) / nf;
     }
@@ -744,16 +759,16 @@ __global__ __launch_bounds__(256) void fft_inverse_kernel(const double* __restri
 // Plans: H points, threads, radices.
 using Plan512 = FftPlan<512, 64, 8, 8, 8, 1>;
 using Plan640 = FftPlan<640, 64, 10, 8, 8, 1>;
-using Plan1024 = FftPlan<1024, 64, 16, 16, 4, 1>;
-using Plan1280 = FftPlan<1280, 128, 16, 16, 5, 1>;
-using Plan2048 = FftPlan<2048, 128, 16, 16, 8, 1>;
+using Plan1024 = FftPlan<1024, 128, 16, 8, 8, 1>;
+using Plan1280 = FftPlan<1280, 128, 16, 8, 10, 1>;
+using Plan2048 = FftPlan<2048, 256, 8, 8, 8, 4>;
 using Plan2560 = FftPlan<2560, 256, 16, 4, 8, 5>;
 using Plan4096 = FftPlan<4096, 256, 16, 16, 16, 1>;
-using Plan5120 = FftPlan<5120, 320, 16, 16, 5, 4>;
-using Plan8192 = FftPlan<8192, 512, 16, 16, 8, 4>;
-using Plan10240 = FftPlan<10240, 640, 16, 16, 5, 8>;
-using Plan12800 = FftPlan<12800, 832, 16, 16, 10, 5>;
-using Plan16384 = FftPlan<16384, 1024, 16, 16, 4, 16>;
+using Plan5120 = FftPlan<5120, 640, 8, 8, 8, 10>;
+using Plan8192 = FftPlan<8192, 1024, 8, 8, 8, 16>;
+using Plan10240 = FftPlan<10240, 1024, 16, 10, 8, 8>;
+using Plan12800 = FftPlan<12800, 1024, 16, 10, 10, 8>;
+using Plan16384 = FftPlan<16384, 1024, 16, 8, 8, 16>;
 
 // Series lengths L = G H / 2 with their plan.  Each L is one of the lengths a series of N
 // frames may be padded to (the smallest with L >= N).
@@ -850,12 +865,12 @@ int launch_fft_power(const FftShape& shape, int dtype, const uint8_t* xs, const 
     return -1;
 }
 
-void launch_fft_inverse(const double* power, int L, int n_bins, int nframes, double* num,
-                        hipStream_t s) {
+void launch_fft_inverse(const double* power, const FftShape& shape, int n_bins, int nframes,
+                        double* num, hipStream_t s) {
     if (n_bins <= 0) return;
     fft_inverse_kernel<<<dim3((unsigned)((nframes + 255) / 256),
                               (unsigned)((n_bins + INV_G - 1) / INV_G)),
-                         256, 0, s>>>(power, L, n_bins, nframes, num);
+                         256, 0, s>>>(power, shape.G, shape.H, n_bins, nframes, num);
 }
 
 }  // namespace dxg2
