@@ -12,18 +12,31 @@
 //
 // Data movement: the slab is stored fragment-contiguous (slab_offset()): the 32 frames
 // x 32 bytes an MFMA operand takes from one k-block are one 1 KiB run in lane order.
-// Each wave (2 x 2 waves per tile, WM x WN blocks of 32 x 32 each) loads its operand
-// fragments straight from global memory into VGPRs with one global_load_dwordx4 per
-// fragment -- no LDS staging, no barriers in the loop.  Two register slots form a
-// software pipeline: the loads of k-block kb + 2 are issued right after the MFMAs of
-// kb have consumed the slot, so a full k-block of MFMAs (WM*WN*2 instructions) covers
-// every load's latency.  Two compiler behaviours must be kept out of the loop:
-//   * the machine scheduler sinks loads towards their first use (it would undo the
-//     pipeline), so sched_barrier fences pin the order MFMA group / load group;
-//   * the waitcnt pass takes the minimum over paths, so a conditionally issued load
-//     makes it wait for every load in flight: every path issues the same loads (the
-//     k-block index is clamped to the item's last k-block near the end).
-// Both operands of a wave are re-read by the wave beside it; those reads hit L1/L2.
+//
+// T = 256 (PanelTile): 2 x 2 waves of 4 x 4 blocks.  The runs of a tile's row and column
+// panels go to LDS by global->LDS DMA and each wave reads its eight fragments of a unit
+// (one K = 32 step) from there, so a run crosses the CU's vector-memory path once instead of
+// once for each of the two waves that use it (64 B/clk a CU, which the 128 x 128 blocks of
+// four waves would need in full at the MFMA rate).  Three buffers of GRAM_UNITS units form a
+// ring; everything is spread over the unit's 16 MFMAs, four at a time: two or three fragment
+// reads of the next unit and one DMA of the unit two stages ahead (DMAs issued in a burst
+// hold back the wave's MFMAs behind them: 17.0 ms against 13.3 for this order; 15.7 for
+// fragments loaded straight into registers, 480,000 pixels x 10,000 frames).  One barrier a
+// stage, ahead of its last unit: by then that unit's fragments are in registers, so the
+// buffer is free, and the next stage has landed (the wait leaves this stage's DMAs in
+// flight), so its first fragments are read under the last unit's MFMAs and no latency is
+// seen.  Two compiler behaviours shape the code:
+//   * sched_barrier fences pin the order, which the machine scheduler would undo;
+//   * the waitcnt pass waits for every DMA before an LDS read that may alias it: the buffers
+//     are separate __shared__ arrays and each stage names its own, with the loop unrolled
+//     over the ring and no branch inside (a merge of paths brings the wait back).
+// Units past the item's end read zeros for A, so a stage is always whole.
+//
+// T = 128 (GramTile): each wave loads its operand fragments straight from global memory into
+// VGPRs with one global_load_dwordx4 per fragment, two register slots deep: the loads of
+// k-block kb + 2 are issued right after the MFMAs of kb have consumed the slot.  Every path
+// issues the same loads (the k-block index is clamped to the item's last k-block near the
+// end), as the waitcnt pass takes the minimum over paths.
 //
 // Diagonal tiles (ti == tj): the wave below the diagonal has nothing to compute and
 // skips the loop; the other waves compute whole 32 x 32 blocks and the epilogue drops
@@ -43,6 +56,7 @@
 // T <= 256 tile collects at most 256 values, so sum(lo) < 2^24 and |sum(hi)| < 2^23
 // are exact, and the 64-bit total hi_sum * 2^16 + lo_sum is formed once per slot.
 #include <algorithm>
+#include <type_traits>
 
 #include "dxg2_internal.h"
 
@@ -84,6 +98,72 @@ struct GramShape {
     static constexpr int TN = 2 * WN * 32;
     static constexpr int NDIAG = TM + TN - 1;
 };
+
+// Frame sums of a diagonal tile's wave: rs[m] = this lane's share of row row + 32 m +
+// lane % 32 (lanes l and l + 32 hold the two 32-byte halves of the frame row).
+template <int WM>
+__device__ __forceinline__ void frame_sums(const int (&rs)[WM], int row, int lane, int nframes,
+                                           int64_t bias, int64_t* __restrict__ sums) {
+#pragma unroll
+    for (int m = 0; m < WM; ++m) {
+        const int v = rs[m] + __shfl_xor(rs[m], 32);
+        const int t = row + m * 32 + lane;
+        const int64_t s64 = (int64_t)v + bias;
+        if (lane < 32 && t < nframes && s64 != 0) gatomic_add(sums + t, s64);
+    }
+}
+
+// A wave's accumulators added to the tile's diagonal sums in LDS, and with STORE written to
+// `tile` (row-major).  32x32 i32 accumulator layout: lane holds column (lane & 31) and rows
+// 8*(v/4) + 4*(lane/32) + (v%4), v = 0..15.  Diagonal slot c - r + TM - 1.
+template <int WM, int WN, bool STORE>
+__device__ __forceinline__ void fold_tile(const v16i (&acc)[WM][WN], int wr, int wc, int lane,
+                                          unsigned int* sDiag, int* __restrict__ tile) {
+    using S = GramShape<WM, WN>;
+    // slot = lane part + (n - m) 32 - 8 (v / 4) - v % 4; the second part is a
+    // compile-time constant >= MINOFF, so every atomic is one base VGPR plus an
+    // immediate offset (no per-element address registers).
+    constexpr int MINOFF = -(WM - 1) * 32 - 15;
+    unsigned int* sd = sDiag + (wc * WN * 32 + (lane & 31)) - (wr * WM * 32 + 4 * (lane >> 5)) +
+                       S::TM - 1 + MINOFF;
+#pragma unroll
+    for (int m = 0; m < WM; ++m)
+#pragma unroll
+        for (int n = 0; n < WN; ++n) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const int k = (n - m) * 32 - 8 * (v >> 2) - (v & 3) - MINOFF;
+                const int val = acc[m][n][v];
+                atomicAdd(sd + k, (unsigned)(val & 0xFFFF));
+                atomicAdd(sd + S::NDIAG + k, (unsigned)(val >> 16));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    if (STORE) {
+        // Lanes 0-31 and 32-63 of one store write two 128-byte row segments.
+#pragma unroll
+        for (int m = 0; m < WM; ++m)
+#pragma unroll
+            for (int n = 0; n < WN; ++n) {
+                const int c = wc * WN * 32 + n * 32 + (lane & 31);
+                const int rbase = wr * WM * 32 + m * 32 + 4 * (lane >> 5);
+#pragma unroll
+                for (int v = 0; v < 16; ++v)
+                    tile[(rbase + 8 * (v >> 2) + (v & 3)) * S::TN + c] = acc[m][n][v];
+            }
+    }
+}
+
+// The tile's diagonal sums to the numerators: lag = shift + slot - (TM - 1).
+template <typename S>
+__device__ __forceinline__ void flush_diagonals(const unsigned int* sDiag, int tid, int shift,
+                                                int nframes, int64_t* __restrict__ out) {
+    for (int i = tid; i < S::NDIAG; i += 256) {
+        const long long v = (long long)(int)sDiag[S::NDIAG + i] * 65536 + (long long)sDiag[i];
+        const int tau = shift + i - (S::TM - 1);
+        if (v != 0 && tau >= 0 && tau < nframes) gatomic_add(out + tau, v);
+    }
+}
 
 template <int WM, int WN, bool DIAG, bool CROSS, bool STORE = false>
 struct GramTile {
@@ -184,62 +264,191 @@ struct GramTile {
             }
         }
 
-        if (DIAG && !STORE && wr == wc) {
-            // lanes l and l + 32 hold the two 32-byte halves of frame row (l & 31)
-            const int64_t bias = biased ? (int64_t)128 * (kb1 - kb0) * KB : 0;
+        if (DIAG && !STORE && wr == wc)
+            frame_sums<WM>(rs, row0 + wr * WM * 32, lane, nframes,
+                           biased ? (int64_t)128 * (kb1 - kb0) * KB : 0, sums);
+        __syncthreads();
+        if (!idle) fold_tile<WM, WN, STORE>(acc, wr, wc, lane, sDiag, tile);
+        __syncthreads();
+        flush_diagonals<S>(sDiag, tid, col0 - row0, nframes, out);
+    }
+};
+
+// One 256 x 256 tile through an LDS ring (see above).
+constexpr int GRAM_UNITS = 3;                      // K = 32 units per stage
+constexpr int GRAM_PANEL = 8 * 1024;               // one unit of a panel: 8 runs
+constexpr int GRAM_STAGE = GRAM_UNITS * 2 * GRAM_PANEL;
+typedef __attribute__((address_space(3))) void lds_void;
+
+__device__ const int8_t gram_zeros[4 * 2048] __attribute__((aligned(1024))) = {};
+
+// s_waitcnt immediates (vmcnt in bits 3:0 and 15:14, expcnt and lgkmcnt not waited for unless
+// said).
+constexpr int wait_vm(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
+constexpr int wait_vm_lgkm0(int n) { return 0x0070 | (n & 15) | ((n >> 4) << 14); }
+
+template <bool DIAG, bool CROSS, bool STORE>
+struct PanelTile {
+    using S = GramShape<4, 4>;
+    const int8_t* __restrict__ slab_bin;
+    int kb0, kb1, row0, col0, nframes, nrows;
+    int tid, lane, wr, wc;
+    int nkbp;  // CROSS: k-blocks per digit plane (B reads kb + nkbp or kb - nkbp)
+    unsigned int* sDiag;
+
+    v16i acc[4][4];
+    v4i fa[GRAM_UNITS][4], fb[GRAM_UNITS][4];
+    int rs[4];         // DIAG: partial frame sums of this lane's A rows
+
+    // This wave's source of unit u (its four runs are 2048 bytes apart): waves 0 and 1 copy
+    // the row panel, 2 and 3 the column panel.
+    __device__ __forceinline__ const int8_t* source(int u) const {
+        int kb = u >> 1;
+        const bool past = kb >= kb1;
+        kb = min(kb, kb1 - 1);
+        if (CROSS && wr) kb = kb < nkbp ? kb + nkbp : kb - nkbp;
+        const int group = ((wr ? col0 : row0) >> 5) + wc * 4;
+        const int8_t* p = slab_bin + ((int64_t)kb * (nrows >> 5) + group) * 2048 + (u & 1) * 1024;
+        return past && !wr ? gram_zeros : p;
+    }
+    __device__ __forceinline__ void dma(int8_t* buf, int un, const int8_t* src, int o) const {
+        __builtin_amdgcn_global_load_lds(
+            (const void*)(src + o * 2048 + lane * 16),
+            (lds_void*)(buf + (un * 2 + wr) * GRAM_PANEL + (wc * 4 + o) * 1024), 16, 0, 0);
+    }
+    __device__ __forceinline__ v4i frag_a(const int8_t* unit, int m) const {
+        return *reinterpret_cast<const v4i*>(unit + (wr * 4 + m) * 1024 + lane * 16);
+    }
+    __device__ __forceinline__ v4i frag_b(const int8_t* unit, int n) const {
+        return *reinterpret_cast<const v4i*>(unit + GRAM_PANEL + (wc * 4 + n) * 1024 + lane * 16);
+    }
+
+    // The units of stage `cur` (unit 0's fragments are in slot 0), with the first fragments of
+    // `next` and the copies of units u .. u + GRAM_UNITS - 1 into `rel`, the buffer of the
+    // stage before.
+    __device__ __forceinline__ void stage(const int8_t* cur, const int8_t* next, int8_t* rel,
+                                          int u) {
 #pragma unroll
-            for (int m = 0; m < WM; ++m) {
-                const int v = rs[m] + __shfl_xor(rs[m], 32);
-                const int t = row0 + wr * WM * 32 + m * 32 + lane;
-                const int64_t s64 = (int64_t)v + bias;
-                if (lane < 32 && t < nframes && s64 != 0) gatomic_add(sums + t, s64);
+        for (int un = 0; un < GRAM_UNITS; ++un) {
+            if (un == GRAM_UNITS - 1) {
+                __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0((GRAM_UNITS - 1) * 4));
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");  // the reads below stay below
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            const int8_t* src = source(u + un);
+            const int8_t* from = un + 1 < GRAM_UNITS ? cur + (un + 1) * 2 * GRAM_PANEL : next;
+            const int sl = (un + 1) % GRAM_UNITS;
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                if (m == 0) {
+                    fa[sl][0] = frag_a(from, 0);
+                    fb[sl][0] = frag_b(from, 0);
+                    fb[sl][1] = frag_b(from, 1);
+                } else if (m == 1) {
+                    fb[sl][2] = frag_b(from, 2);
+                    fb[sl][3] = frag_b(from, 3);
+                    fa[sl][1] = frag_a(from, 1);
+                } else if (m == 2) {
+                    fa[sl][2] = frag_a(from, 2);
+                    fa[sl][3] = frag_a(from, 3);
+                }
+                dma(rel, un, src, m);
+#pragma unroll
+                for (int n = 0; n < 4; ++n)
+                    acc[m][n] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[un][m], fb[un][n],
+                                                                      acc[m][n], 0, 0, 0);
+                if (DIAG) {
+                    const v4i x = fa[un][m];
+                    rs[m] = __builtin_amdgcn_sdot4(x.x, 0x01010101, rs[m], false);
+                    rs[m] = __builtin_amdgcn_sdot4(x.y, 0x01010101, rs[m], false);
+                    rs[m] = __builtin_amdgcn_sdot4(x.z, 0x01010101, rs[m], false);
+                    rs[m] = __builtin_amdgcn_sdot4(x.w, 0x01010101, rs[m], false);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    }
+    // The same for a wave with nothing to compute: its copies and the barrier.
+    __device__ __forceinline__ void idle_stage(int8_t* rel, int u) const {
+#pragma unroll
+        for (int un = 0; un < GRAM_UNITS; ++un) {
+            if (un == GRAM_UNITS - 1) {
+                __builtin_amdgcn_s_waitcnt(wait_vm((GRAM_UNITS - 1) * 4));
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+            }
+            const int8_t* src = source(u + un);
+#pragma unroll
+            for (int o = 0; o < 4; ++o) dma(rel, un, src, o);
+        }
+    }
+
+    __device__ __forceinline__ void run(int biased, int64_t* __restrict__ out,
+                                        int64_t* __restrict__ sums, int* __restrict__ tile,
+                                        int8_t* buf0, int8_t* buf1, int8_t* buf2) {
+        for (int i = tid; i < 2 * S::NDIAG; i += 256) sDiag[i] = 0u;
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            rs[m] = 0;
+#pragma unroll
+            for (int n = 0; n < 4; ++n)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[m][n][v] = 0;
+        }
+        // idle: every block of this wave is below the diagonal, or lies wholly in the
+        // padding frames past the last one (a STORE tile's readers skip both parts)
+        const bool idle = (DIAG && wr > wc) || row0 + wr * 128 >= nframes ||
+                          col0 + wc * 128 >= nframes;
+        const int u0 = 2 * kb0;
+        const int n_stage = (2 * (kb1 - kb0) + GRAM_UNITS - 1) / GRAM_UNITS;
+#pragma unroll
+        for (int un = 0; un < 2 * GRAM_UNITS; ++un) {
+            const int8_t* src = source(u0 + un);
+#pragma unroll
+            for (int o = 0; o < 4; ++o)
+                dma(un < GRAM_UNITS ? buf0 : buf1, un % GRAM_UNITS, src, o);
+        }
+        __builtin_amdgcn_s_waitcnt(wait_vm(GRAM_UNITS * 4));
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        constexpr int U = GRAM_UNITS;
+        int st = 0, u = u0 + 2 * U;  // u: first unit copied by stage st
+        if (idle) {
+            for (; st + 3 <= n_stage; st += 3, u += 3 * U) {
+                idle_stage(buf2, u);
+                idle_stage(buf0, u + U);
+                idle_stage(buf1, u + 2 * U);
+            }
+            if (st < n_stage) {
+                idle_stage(buf2, u);
+                if (st + 1 < n_stage) idle_stage(buf0, u + U);
+            }
+        } else {
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                fa[0][m] = frag_a(buf0, m);
+                fb[0][m] = frag_b(buf0, m);
+            }
+            for (; st + 3 <= n_stage; st += 3, u += 3 * U) {
+                stage(buf0, buf1, buf2, u);
+                stage(buf1, buf2, buf0, u + U);
+                stage(buf2, buf0, buf1, u + 2 * U);
+            }
+            if (st < n_stage) {
+                stage(buf0, buf1, buf2, u);
+                if (st + 1 < n_stage) stage(buf1, buf2, buf0, u + U);
             }
         }
 
-        // Epilogue.  32x32 i32 accumulator layout: lane holds column (lane & 31) and
-        // rows 8*(v/4) + 4*(lane/32) + (v%4), v = 0..15.  Diagonal slot c - r + TM - 1.
+        if (DIAG && !STORE && wr == wc)
+            frame_sums<4>(rs, row0 + wr * 128, lane, nframes,
+                          biased ? (int64_t)128 * (kb1 - kb0) * KB : 0, sums);
+        __builtin_amdgcn_s_waitcnt(wait_vm(0));  // no copy is in flight into a reused buffer
         __syncthreads();
-        if (!idle) {
-            // slot = lane part + (n - m) 32 - 8 (v / 4) - v % 4; the second part is a
-            // compile-time constant >= MINOFF, so every atomic is one base VGPR plus an
-            // immediate offset (no per-element address registers).
-            constexpr int MINOFF = -(WM - 1) * 32 - 15;
-            unsigned int* sd = sDiag + (wc * WN * 32 + (lane & 31)) -
-                               (wr * WM * 32 + 4 * (lane >> 5)) + S::TM - 1 + MINOFF;
-#pragma unroll
-            for (int m = 0; m < WM; ++m)
-#pragma unroll
-                for (int n = 0; n < WN; ++n) {
-#pragma unroll
-                    for (int v = 0; v < 16; ++v) {
-                        const int k = (n - m) * 32 - 8 * (v >> 2) - (v & 3) - MINOFF;
-                        const int val = acc[m][n][v];
-                        atomicAdd(sd + k, (unsigned)(val & 0xFFFF));
-                        atomicAdd(sd + S::NDIAG + k, (unsigned)(val >> 16));
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            if (STORE) {
-                // Lanes 0-31 and 32-63 of one store write two 128-byte row segments.
-#pragma unroll
-                for (int m = 0; m < WM; ++m)
-#pragma unroll
-                    for (int n = 0; n < WN; ++n) {
-                        const int c = wc * WN * 32 + n * 32 + (lane & 31);
-                        const int rbase = wr * WM * 32 + m * 32 + 4 * (lane >> 5);
-#pragma unroll
-                        for (int v = 0; v < 16; ++v)
-                            tile[(rbase + 8 * (v >> 2) + (v & 3)) * S::TN + c] = acc[m][n][v];
-                    }
-            }
-        }
+        if (!idle) fold_tile<4, 4, STORE>(acc, wr, wc, lane, sDiag, tile);
         __syncthreads();
-        for (int i = tid; i < S::NDIAG; i += 256) {
-            const long long v =
-                (long long)(int)sDiag[S::NDIAG + i] * 65536 + (long long)sDiag[i];
-            const int tau = col0 - row0 + i - (S::TM - 1);
-            if (v != 0 && tau >= 0 && tau < nframes) gatomic_add(out + tau, v);
-        }
+        flush_diagonals<S>(sDiag, tid, col0 - row0, nframes, out);
     }
 };
 
@@ -268,25 +477,42 @@ __device__ __forceinline__ ItemRange item_range(const GramWork& w, int nkb, cons
 
 // One work item: the tile of `w` in a bin whose slab starts at slab_bin, over k-blocks
 // [r.kb0, r.kb1) (a CROSS item's B operand r.nkbp k-blocks away).
+// LDS of one workgroup: the diagonal sums, and for T = 256 the ring's buffers, which stay
+// separate __shared__ arrays of the kernel (see the top of the file).
+#define DXG2_GRAM_LDS(WM)                                                                     \
+    constexpr int ring_bytes = WM == 4 ? GRAM_STAGE : 16;                                     \
+    __shared__ __attribute__((aligned(1024))) int8_t buf0[ring_bytes];                        \
+    __shared__ __attribute__((aligned(1024))) int8_t buf1[ring_bytes];                        \
+    __shared__ __attribute__((aligned(1024))) int8_t buf2[ring_bytes];                        \
+    __shared__ unsigned int sDiag[2 * GramShape<WM, WM>::NDIAG]
+
 template <int WM, int WN, bool CROSS, bool STORE>
 __device__ __forceinline__ void gram_item(const GramWork& w, ItemRange r, const int8_t* slab_bin,
                                           int nframes, int nrows, int biased,
                                           int64_t* __restrict__ out, int64_t* __restrict__ sums,
-                                          int* __restrict__ tile, unsigned int* sDiag) {
+                                          int* __restrict__ tile, unsigned int* sDiag,
+                                          int8_t* buf0, int8_t* buf1, int8_t* buf2) {
     using S = GramShape<WM, WN>;
     const int tid = threadIdx.x;
-    const int wave = tid >> 6;
-    if (!CROSS && w.ti == w.tj) {
-        GramTile<WM, WN, true, false, STORE> t{slab_bin, r.kb0, r.kb1, w.ti * S::TM,
-                                               w.tj * S::TN, nframes, nrows, tid, tid & 63,
-                                               wave >> 1, wave & 1, 0, sDiag};
-        t.run(biased, out, sums, tile);
-    } else {
-        GramTile<WM, WN, false, CROSS, STORE> t{slab_bin, r.kb0, r.kb1, w.ti * S::TM,
-                                                w.tj * S::TN, nframes, nrows, tid, tid & 63,
-                                                wave >> 1, wave & 1, r.nkbp, sDiag};
-        t.run(biased, out, sums, tile);
-    }
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    auto go = [&](auto diag) {
+        constexpr bool DIAG = decltype(diag)::value;
+        if constexpr (WM == 4) {
+            PanelTile<DIAG, CROSS, STORE> t{slab_bin, r.kb0, r.kb1, w.ti * S::TM, w.tj * S::TN,
+                                            nframes, nrows, tid, tid & 63, wave >> 1, wave & 1,
+                                            r.nkbp, sDiag};
+            t.run(biased, out, sums, tile, buf0, buf1, buf2);
+        } else {
+            GramTile<WM, WN, DIAG, CROSS, STORE> t{slab_bin, r.kb0, r.kb1, w.ti * S::TM,
+                                                   w.tj * S::TN, nframes, nrows, tid, tid & 63,
+                                                   wave >> 1, wave & 1, r.nkbp, sDiag};
+            t.run(biased, out, sums, tile);
+        }
+    };
+    if (!CROSS && w.ti == w.tj)
+        go(std::true_type{});
+    else
+        go(std::false_type{});
 }
 
 template <int WM, int WN, bool CROSS>
@@ -299,7 +525,7 @@ __global__ __launch_bounds__(256) void gram_i8_kernel(const int8_t* __restrict__
                                                       int64_t* __restrict__ sums) {
     using S = GramShape<WM, WN>;
     static_assert(S::TM == S::TN, "square tiles");
-    __shared__ unsigned int sDiag[2 * S::NDIAG];
+    DXG2_GRAM_LDS(WM);
     const GramWork w = work[blockIdx.x];
     if (w.bin < 0) return;  // padding item
     const BinDev bd = bins[w.bin];
@@ -307,7 +533,7 @@ __global__ __launch_bounds__(256) void gram_i8_kernel(const int8_t* __restrict__
     if (r.kb1 <= r.kb0) return;  // nothing of this item is left
     gram_item<WM, WN, CROSS, false>(w, r, slab + bd.slab_off, nframes, nrows, biased,
                                     ugram + (int64_t)w.out * nframes,
-                                    sums + (int64_t)w.out * nframes, nullptr, sDiag);
+                                    sums + (int64_t)w.out * nframes, nullptr, sDiag, buf0, buf1, buf2);
 }
 
 // XCD (accelerator complex die) this wave runs on: HW_REG_XCC_ID bits [3:0].
@@ -342,7 +568,7 @@ __global__ __launch_bounds__(256) void gram_i8_queue_kernel(
     int64_t* __restrict__ sums) {
     using S = GramShape<WM, WN>;
     static_assert(S::TM == S::TN, "square tiles");
-    __shared__ unsigned int sDiag[2 * S::NDIAG];
+    DXG2_GRAM_LDS(WM);
     __shared__ int s_item;
     const int home = xcc_id();
     for (;;) {
@@ -356,7 +582,7 @@ __global__ __launch_bounds__(256) void gram_i8_queue_kernel(
         if (r.kb1 > r.kb0)  // the same for every thread of the workgroup
             gram_item<WM, WN, CROSS, false>(w, r, slab + bd.slab_off, nframes, nrows, biased,
                                             ugram + (int64_t)w.out * nframes,
-                                            sums + (int64_t)w.out * nframes, nullptr, sDiag);
+                                            sums + (int64_t)w.out * nframes, nullptr, sDiag, buf0, buf1, buf2);
         __syncthreads();  // s_item and sDiag are reused by the next item
     }
 }
@@ -425,13 +651,14 @@ __global__ __launch_bounds__(256) void gram_i8_store_kernel(
     int64_t* __restrict__ ugram, int* __restrict__ tiles) {
     using S = GramShape<WM, WN>;
     static_assert(S::TM == S::TN, "square tiles");
-    __shared__ unsigned int sDiag[2 * S::NDIAG];
+    DXG2_GRAM_LDS(WM);
     const GramWork w = work[blockIdx.x];
     if (w.bin < 0) return;  // padding item
     const BinDev bd = bins[w.bin];
     gram_item<WM, WN, CROSS, true>(w, ItemRange{w.kb0, w.kb1, bd.nkb}, slab + bd.slab_off,
                                    nframes, nrows, biased, ugram + (int64_t)w.out * nframes,
-                                   nullptr, tiles + (int64_t)w.slot * S::TM * S::TN, sDiag);
+                                   nullptr, tiles + (int64_t)w.slot * S::TM * S::TN, sDiag,
+                                   buf0, buf1, buf2);
 }
 
 // Grouped launch over several plans (continuous batching of dense jobs): the same tile
@@ -441,7 +668,7 @@ __global__ __launch_bounds__(256) void gram_i8_jobs_kernel(const GramJob* __rest
                                                            const GramWork* __restrict__ work) {
     using S = GramShape<WM, WN>;
     static_assert(S::TM == S::TN, "square tiles");
-    __shared__ unsigned int sDiag[2 * S::NDIAG];
+    DXG2_GRAM_LDS(WM);
     const GramWork w = work[blockIdx.x];
     if (w.bin < 0) return;  // padding item
     const GramJob j = jobs[w.job];
@@ -449,7 +676,7 @@ __global__ __launch_bounds__(256) void gram_i8_jobs_kernel(const GramJob* __rest
     gram_item<WM, WN, CROSS, false>(w, ItemRange{w.kb0, w.kb1, bd.nkb}, j.slab + bd.slab_off,
                                     j.nframes, j.nrows, j.biased,
                                     j.ugram + (int64_t)w.out * j.nframes,
-                                    j.sums + (int64_t)w.out * j.nframes, nullptr, sDiag);
+                                    j.sums + (int64_t)w.out * j.nframes, nullptr, sDiag, buf0, buf1, buf2);
 }
 
 void launch_gram_i8_jobs(int tile, bool cross, const GramJob* jobs, const GramWork* work,
