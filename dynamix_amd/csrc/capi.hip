@@ -247,8 +247,10 @@ struct dxg2_plan {
     GramWork* d_qmwork = nullptr;
     GramWork* d_qxwork = nullptr;
     int* d_qoff = nullptr;
-    int* d_heads = nullptr;
+    int* d_heads = nullptr;        // 16 queue heads, then the route's four ints
     int8_t* d_slab = nullptr;
+    int8_t* d_slab4 = nullptr;     // narrow slab (k_narrow.hip), half the slab's bytes
+    int64_t* d_wsums = nullptr;    // its wide pixels' frame sums, n_bins rows
     int64_t* d_ugram = nullptr;
     int64_t* d_sums = nullptr;
     int64_t* d_psums = nullptr;   // digit planes: S_H, S_L, then S_Lw rows (n_bins each)
@@ -864,15 +866,59 @@ int ensure_event_buffers(dxg2_plan* p, int64_t nnz_coo, hipStream_t s) {
     return DXG2_OK;
 }
 
+// Plans whose plain dense calls may keep narrow pixels in FP4 (k_narrow.hip): 8-bit frames
+// through the band gather and the persistent launch of 256-frame tiles, with enough Gram work
+// (pixels x frames^2) that halving it pays for the launches of the narrow route
+// (DXG2_NARROW: 0 never, 2 whatever the work).
+constexpr double NARROW_MIN_WORK = 5e11;
+constexpr int HEAD_INTS = 20;
+bool narrow_applies(const dxg2_plan* p) {
+    if (p->dtype == DXG2_U16 || p->gband.empty() || !p->use_queue || p->gram_tile != 256)
+        return false;
+    const int opt = env_int("DXG2_NARROW", 1);
+    return opt == 2 ||
+           (opt && (double)p->pix_idx.size() * p->N * p->N >= NARROW_MIN_WORK);
+}
+size_t narrow_bytes(const dxg2_plan* p) {
+    if (!narrow_applies(p)) return 0;
+    return p->slab_bytes / 2 + (size_t)p->n_bins * p->N * sizeof(int64_t) + p->pix_idx.size() * 4 +
+           (size_t)p->H * p->W + 16 + (size_t)(2 * p->n_bins + 1) * sizeof(int);
+}
+
 // Slab of the dense path, allocated on the first dense call and cleared on its stream:
 // rows past the last frame stay zero for the life of the plan.
-int ensure_dense_buffers(dxg2_plan* p, hipStream_t s) {
+int ensure_dense_buffers(dxg2_plan* p, hipStream_t s, bool narrow = false) {
     if (!p->d_slab && p->slab_bytes) {
         if (dev_alloc(p->alloc, (void**)&p->d_slab, p->slab_bytes, s) != hipSuccess) {
             p->d_slab = nullptr;
             return set_error(DXG2_ENOMEM, "cannot allocate %zu bytes of slab", p->slab_bytes);
         }
         DXG2_HIP(hipMemsetAsync(p->d_slab, 0, p->slab_bytes, s));
+    }
+    if (narrow && !p->d_slab4 && narrow_applies(p)) {
+        // d_slab4 is set last: it marks the narrow workspace complete
+        int8_t* slab4 = nullptr;
+        int64_t* wsums = nullptr;
+        uint8_t* flag = nullptr;
+        int32_t* pixw = nullptr;
+        int* nwkb = nullptr;
+        if (dev_alloc(p->alloc, (void**)&slab4, p->slab_bytes / 2, s) != hipSuccess ||
+            dev_alloc(p->alloc, (void**)&wsums, (size_t)p->n_bins * p->N * sizeof(int64_t), s) !=
+                hipSuccess ||
+            dev_alloc(p->alloc, (void**)&flag, (size_t)p->H * p->W + 16, s) != hipSuccess ||
+            dev_alloc(p->alloc, (void**)&pixw, p->pix_idx.size() * 4, s) != hipSuccess ||
+            dev_alloc(p->alloc, (void**)&nwkb, (size_t)(2 * p->n_bins + 1) * sizeof(int), s) !=
+                hipSuccess) {
+            for (void* b : {(void*)slab4, (void*)wsums, (void*)flag, (void*)pixw, (void*)nwkb})
+                dev_free(p->alloc, b, s);
+            return set_error(DXG2_ENOMEM, "cannot allocate the narrow slab");
+        }
+        DXG2_HIP(hipMemsetAsync(slab4, 0, p->slab_bytes / 2, s));
+        p->d_wsums = wsums;
+        p->d_wflag = flag;
+        p->d_pixw = pixw;
+        p->d_nwkb = nwkb;
+        p->d_slab4 = slab4;
     }
     return DXG2_OK;
 }
@@ -883,16 +929,49 @@ int ensure_dense_buffers(dxg2_plan* p, hipStream_t s) {
 // wide_first (uint16 plans; the plain dense calls): the low plane in list order with the
 // wide pixels flagged in the same pass, then the wide pixels' own k-blocks (k_wide.hip),
 // for a Gram clipped to them (dense_gram and dense_finish with the same flag).
+//
+// Narrow calls (uint8/int8 plans; the plain dense calls, with the same frames throughout) fill
+// the narrow slab or the i8 slab, as decided on the device (k_narrow.hip).
+bool narrow_call(const dxg2_plan* p, const void* d_frames) {
+    return p->d_slab4 && narrow_applies(p) && reinterpret_cast<uintptr_t>(d_frames) % 16 == 0;
+}
 int64_t* dense_gather(dxg2_plan* p, const void* d_frames, int64_t* d_sums, hipStream_t s,
                       bool wide_first = false) {
     int64_t* sums = d_sums ? d_sums : p->d_sums;
     const bool wide = p->dtype == DXG2_U16;
     int64_t* gsums = wide ? p->d_psums : sums;
     const int64_t nbn = (int64_t)p->n_bins * p->N;
+    const int64_t hw = (int64_t)p->H * p->W;
+    int64_t max_npix = 0;
+    for (auto n : p->npix) max_npix = std::max(max_npix, n);
+    if (wide_first && narrow_call(p, d_frames)) {
+        const uint8_t* frames = (const uint8_t*)d_frames;
+        const int* route = p->d_heads + 16;
+        int64_t n_pix = 0;
+        for (auto n : p->npix) n_pix += n;
+        launch_clear_call(gsums, nbn, p->d_ugram, nbn, p->d_heads, HEAD_INTS, s, p->d_wflag, hw,
+                          p->d_wsums, nbn);
+        launch_fill_i32(p->d_nwkb + p->n_bins, p->n_bins + 1, s);
+        launch_narrow_sample(frames, p->dtype, hw, p->N, p->d_pix, (int64_t)p->pix_idx.size(),
+                             n_pix, p->d_heads + 16, s);
+        launch_gather_band_f4(frames, p->dtype, hw, p->W, p->N, p->nrows, p->gband_srow, p->d_pix,
+                              p->d_bins, p->d_gband, (int)p->gband.size(), p->d_gband_kb,
+                              p->d_gfall, (int)p->gfall.size(), p->d_slab4, p->d_wflag, route, s);
+        launch_gather_band(frames, p->dtype, hw, p->W, p->N, p->nrows, p->gband_srow, p->d_pix,
+                           p->d_bins, p->d_gband, (int)p->gband.size(), p->d_gband_kb, p->d_gfall,
+                           (int)p->gfall.size(), p->d_slab, s, route);
+        launch_wide_compact(p->d_pix, p->d_bins, p->n_bins, (int)max_npix, p->d_wflag, p->d_pixw,
+                            p->d_nwkb + p->n_bins + 1, s);
+        launch_narrow_clip(p->d_bins, p->n_bins, route, p->d_nwkb, s);
+        launch_narrow_mask(p->d_pix, p->d_bins, p->n_bins, (int)((max_npix + KB - 1) / KB),
+                           p->d_wflag, route, p->nrows, p->d_nwkb, p->d_slab4, s);
+        launch_wide_gather(frames, p->dtype, hw, p->N, p->nrows, p->d_pix, p->d_pixw, p->d_bins,
+                           p->n_bins, p->d_nwkb, p->d_slab, route, s);
+        return gsums;
+    }
     // the queue heads of the persistent Gram are cleared here too
     launch_clear_call(gsums, (wide ? 2 : 1) * nbn, p->d_ugram, (wide ? 3 : 1) * nbn, p->d_heads,
-                      16, s);
-    const int64_t hw = (int64_t)p->H * p->W;
+                      HEAD_INTS, s);
     uint32_t* flagw = wide && wide_first ? reinterpret_cast<uint32_t*>(p->d_wflag) : nullptr;
     if (flagw) launch_fill_u32(flagw, (hw + 3) / 4, s);
     if (!p->gband.empty() && reinterpret_cast<uintptr_t>(d_frames) % 16 == 0) {
@@ -905,12 +984,10 @@ int64_t* dense_gather(dxg2_plan* p, const void* d_frames, int64_t* d_sums, hipSt
                             p->gather_frames, p->d_slab, s, flagw);
     }
     if (flagw) {
-        int64_t max_npix = 0;
-        for (auto n : p->npix) max_npix = std::max(max_npix, n);
         launch_wide_partition(p->d_pix, p->d_bins, p->n_bins, (int)max_npix, p->d_wflag,
                               p->d_pixw, p->d_nwkb, s);
-        launch_wide_gather((const uint16_t*)d_frames, hw, p->N, p->nrows, p->d_pix, p->d_pixw,
-                           p->d_bins, p->n_bins, p->d_nwkb, p->d_slab, s);
+        launch_wide_gather((const uint8_t*)d_frames, p->dtype, hw, p->N, p->nrows, p->d_pix,
+                           p->d_pixw, p->d_bins, p->n_bins, p->d_nwkb, p->d_slab, nullptr, s);
         launch_wide_low_sums(p->d_slab, p->d_bins, p->d_nwkb, p->n_bins, p->N, p->nrows,
                              gsums + 2 * nbn, s);
     }
@@ -919,8 +996,17 @@ int64_t* dense_gather(dxg2_plan* p, const void* d_frames, int64_t* d_sums, hipSt
 
 // The Gram of every bin: the persistent launch over the per-XCD work queues (heads
 // cleared by dense_gather), or one workgroup per tile.
-void dense_gram(dxg2_plan* p, int64_t* gsums, hipStream_t s, bool wide_first = false) {
+void dense_gram(dxg2_plan* p, int64_t* gsums, hipStream_t s, bool wide_first = false,
+                bool narrow = false) {
     const int biased = p->dtype == DXG2_I8 ? 0 : 1;
+    if (narrow) {
+        launch_gram_f4_queue(p->d_slab4, p->d_bins, p->d_qmwork, (int)p->qm_work.size(), p->d_qoff,
+                             p->d_heads, p->N, p->nrows, p->d_heads + 16, p->d_ugram, gsums, s);
+        launch_gram_i8_queue(p->gram_tile, false, p->d_slab, p->d_bins, p->d_qmwork,
+                             (int)p->qm_work.size(), p->d_qoff, p->d_heads + 8, p->N, p->nrows,
+                             biased, p->d_nwkb, p->d_ugram, gsums, s, p->n_bins, p->d_wsums);
+        return;
+    }
     const int* nwkb = wide_first && p->dtype == DXG2_U16 ? p->d_nwkb : nullptr;
     if (p->use_queue) {
         launch_gram_i8_queue(p->gram_tile, false, p->d_slab, p->d_bins, p->d_qmwork,
@@ -941,13 +1027,14 @@ void dense_gram(dxg2_plan* p, int64_t* gsums, hipStream_t s, bool wide_first = f
 
 // Bias corrections, exact denominators and g2 after the Gram.
 void dense_finish(dxg2_plan* p, int64_t* gsums, int64_t* d_num, int64_t* d_sums, double* d_den,
-                  float* d_g2, hipStream_t s, bool wide_first = false) {
+                  float* d_g2, hipStream_t s, bool wide_first = false, bool narrow = false) {
     int64_t* sums = d_sums ? d_sums : p->d_sums;
     const bool wide = p->dtype == DXG2_U16;
-    const int mode = wide ? (wide_first ? 3 : 2) : (p->dtype == DXG2_U8 ? 1 : 0);
+    const int mode = wide ? (wide_first ? 3 : 2)
+                          : (p->dtype == DXG2_U8 ? (narrow ? 4 : 1) : 0);
     launch_finalize(gsums, sums, p->d_ugram, p->d_bins, p->n_bins, p->N, mode, p->d_prefix,
-                    p->d_smax, p->d_dpre, wide ? p->d_nwkb : nullptr, d_num, d_den, d_g2,
-                    p->dmf, s);
+                    p->d_smax, p->d_dpre, wide || mode == 4 ? p->d_nwkb : nullptr, d_num, d_den,
+                    d_g2, p->dmf, s, mode == 4 ? p->d_wsums : nullptr);
 }
 
 }  // namespace
@@ -1197,7 +1284,7 @@ int dxg2_plan_create(const dxg2_plan_desc* desc, dxg2_plan** out) {
     if (!rc)
         rc = upload((void**)&p->d_qxwork, p->qx_work.data(), p->qx_work.size() * sizeof(GramWork));
     if (!rc) rc = upload((void**)&p->d_qoff, p->q_off, sizeof(p->q_off));
-    if (!rc && dev_alloc(p->alloc, (void**)&p->d_heads, 16 * sizeof(int), s0) != hipSuccess)
+    if (!rc && dev_alloc(p->alloc, (void**)&p->d_heads, HEAD_INTS * sizeof(int), s0) != hipSuccess)
         rc = set_error(DXG2_ENOMEM, "cannot allocate work-queue heads");
     const size_t nb_n = (size_t)std::max(p->n_bins, 1) * p->N * sizeof(int64_t);
     const int planes = slab_planes(p->dtype);
@@ -1214,7 +1301,7 @@ int dxg2_plan_create(const dxg2_plan_desc* desc, dxg2_plan** out) {
                    s0) != hipSuccess))
         rc = set_error(DXG2_ENOMEM, "cannot allocate wide-pixel workspace");
     if (!rc && planes == 2) rc = upload((void**)&p->d_pixw, p->pix_idx.data(), p->pix_idx.size() * 4);
-    if (!rc && (dev_alloc(p->alloc, (void**)&p->d_prefix, (size_t)(planes == 2 ? 3 : 1) *
+    if (!rc && (dev_alloc(p->alloc, (void**)&p->d_prefix, (size_t)(planes == 2 ? 3 : 2) *
                                                      std::max(p->n_bins, 1) *
                                                      (p->N + 1) * sizeof(int64_t), s0) !=
                     hipSuccess ||
@@ -1267,7 +1354,7 @@ static void plan_release(dxg2_plan* p, hipStream_t s) {
                     p->d_etimes, p->d_edata, p->d_kbwork, p->d_kbgather, p->d_xs, p->d_tw,
                     p->d_pixfft, p->d_fftqkb,
                     p->d_power, p->d_fnum, p->d_qmwork, p->d_qxwork, p->d_qoff,
-                    p->d_heads, p->d_gband, p->d_gband_kb, p->d_gfall,
+                    p->d_slab4, p->d_wsums, p->d_heads, p->d_gband, p->d_gband_kb, p->d_gfall,
                     p->coo_sort.keys, p->coo_sort.vals0, p->coo_sort.vals1, p->coo_sort.tmp,
                     p->d_wflag, p->d_pixw, p->d_nwkb};
     drop_std(p, s);
@@ -1307,7 +1394,7 @@ int dxg2_plan_footprint(const dxg2_plan* p, int32_t path, size_t* bytes) {
     const int planes = slab_planes(p->dtype);
     size_t common = p->pix_idx.size() * 4 + p->bins.size() * sizeof(BinDev) +
                     (p->dmf.up > 0 ? den_mfma_bytes(p) : 0) + (planes == 2 ? 8 : 3) * nb_n +
-                    (size_t)std::max(p->n_bins, 1) * ((planes == 2 ? 3 : 1) * (p->N + 1) + 1) *
+                    (size_t)std::max(p->n_bins, 1) * ((planes == 2 ? 3 : 2) * (p->N + 1) + 1) *
                         sizeof(int64_t) +
                     (planes == 2 ? p->pix_idx.size() * 4 + (size_t)p->H * p->W +
                                        (size_t)std::max(p->n_bins, 1) * 4
@@ -1317,7 +1404,7 @@ int dxg2_plan_footprint(const dxg2_plan* p, int32_t path, size_t* bytes) {
             *bytes = common + p->slab_bytes + p->gather_work.size() * sizeof(GatherWork) +
                      p->gather_slots.size() * sizeof(KbWork) +
                      (p->gram_work.size() + p->gram_xwork.size() + p->qm_work.size() +
-                      p->qx_work.size()) * sizeof(GramWork) + sizeof(p->q_off) + 16 * sizeof(int);
+                      p->qx_work.size()) * sizeof(GramWork) + sizeof(p->q_off) + HEAD_INTS * sizeof(int) + narrow_bytes(p);
             return DXG2_OK;
         case 1: {
             int64_t mx = 0;
@@ -1390,17 +1477,18 @@ int dxg2_correlate_dense(dxg2_plan* p, const void* d_frames, int64_t* d_num, int
     if (!d_frames || !d_g2) return set_error(DXG2_EINVAL, "frames and g2 must be non-null");
     if (p->n_bins == 0) return DXG2_OK;
     hipStream_t s = (hipStream_t)stream;
-    int rc = ensure_dense_buffers(p, s);
+    int rc = ensure_dense_buffers(p, s, true);
     if (rc) return rc;
     (void)hipGetLastError();
     hipEvent_t* ev = nullptr;
     if (p->profiling && (rc = next_events(p, &ev))) return rc;
     if (ev) DXG2_HIP(hipEventRecord(ev[0], s));
+    const bool narrow = narrow_call(p, d_frames);
     int64_t* gsums = dense_gather(p, d_frames, d_sums, s, true);
     if (ev) DXG2_HIP(hipEventRecord(ev[1], s));
-    dense_gram(p, gsums, s, true);
+    dense_gram(p, gsums, s, true, narrow);
     if (ev) DXG2_HIP(hipEventRecord(ev[2], s));
-    dense_finish(p, gsums, d_num, d_sums, d_den, d_g2, s, true);
+    dense_finish(p, gsums, d_num, d_sums, d_den, d_g2, s, true, narrow);
     if (ev) DXG2_HIP(hipEventRecord(ev[3], s));
     DXG2_HIP(hipGetLastError());
     return DXG2_OK;
@@ -1511,7 +1599,7 @@ int dxg2_correlate_dense_graph(dxg2_plan* p, const void* d_frames, int64_t* d_nu
     if (!d_frames || !d_g2) return set_error(DXG2_EINVAL, "frames and g2 must be non-null");
     if (p->n_bins == 0) return DXG2_OK;
     hipStream_t s = (hipStream_t)stream;
-    int rc = ensure_dense_buffers(p, s);  // the one-time slab clear runs eagerly, on s
+    int rc = ensure_dense_buffers(p, s, true);  // the one-time slab clears run eagerly, on s
     if (rc) return rc;
     const std::array<const void*, 5> key{d_frames, d_num, d_sums, d_den, d_g2};
     if (!p->gexec || key != p->gkey) {
@@ -1522,8 +1610,9 @@ int dxg2_correlate_dense_graph(dxg2_plan* p, const void* d_frames, int64_t* d_nu
         (void)hipGetLastError();
         DXG2_HIP(hipStreamBeginCapture(p->cap_stream, hipStreamCaptureModeThreadLocal));
         int64_t* gsums = dense_gather(p, d_frames, d_sums, p->cap_stream, true);
-        dense_gram(p, gsums, p->cap_stream, true);
-        dense_finish(p, gsums, d_num, d_sums, d_den, d_g2, p->cap_stream, true);
+        const bool narrow = narrow_call(p, d_frames);
+        dense_gram(p, gsums, p->cap_stream, true, narrow);
+        dense_finish(p, gsums, d_num, d_sums, d_den, d_g2, p->cap_stream, true, narrow);
         hipGraph_t g = nullptr;
         const hipError_t e1 = hipStreamEndCapture(p->cap_stream, &g);
         const hipError_t e0 = hipGetLastError();

@@ -112,6 +112,19 @@ struct StdPart {         // one diagonal segment of one tile: count, mean, sum o
 // biased by -128 like uint8.  Numerators combine as 65536 HH + 256 (HL + LH) + LL.
 inline int slab_planes(int dtype) { return dtype == DXG2_U16 ? 2 : 1; }
 
+// Routes of a dense call whose plan has a narrow slab, decided on the device from a sample of
+// its frames (k_narrow.hip).
+enum { NARROW_F4 = 0, NARROW_OFF = 1 };
+// Largest count of a narrow pixel: the FP4 magnitudes 0, 0.5, .. 2 are codes 0 .. 4.
+constexpr int NARROW_MAX = 4;
+// Byte offset in a bin's narrow slab of the 16 bytes of frame t's codes of pixels 32 h .. + 31
+// of k-block kb: fragment-contiguous like slab_offset(), one run of 1 KiB per 32 frames.  Byte
+// 4 w + b of the 16 holds pixel 8 w + b in its low and 8 w + 4 + b in its high half; a code is
+// the count's magnitude with the sign in bit 3.
+__host__ __device__ inline int64_t narrow_offset(int kb, int t, int h, int nrows) {
+    return ((int64_t)kb * (nrows >> 5) + (t >> 5)) * 1024 + (h * 32 + (t & 31)) * 16;
+}
+
 struct EventWork {       // one workgroup of the event pair kernel (x dimension)
     int32_t bin;
     int32_t k0;          // range [k0, k1) of the bin's pixel list
@@ -141,21 +154,39 @@ struct KbWork {          // one k-block (64 pixels) of one bin
 // ------------------------------------------------------------------ launchers
 void launch_lds_atomic_rate(int mode, int blocks, int iters, uint32_t* out, hipStream_t s);
 void launch_fill_i64(int64_t* p, int64_t n, hipStream_t s);
-// a[0, na), b[0, nb) and c[0, nc) (nc <= 256) zeroed by one launch.
+// a[0, na), b[0, nb), c[0, nc), the bytes d[0, nd) rounded up to 8 and e[0, ne) zeroed by one
+// launch.
 void launch_clear_call(int64_t* a, int64_t na, int64_t* b, int64_t nb, int* c, int nc,
-                       hipStream_t s);
+                       hipStream_t s, uint8_t* d = nullptr, int64_t nd = 0, int64_t* e = nullptr,
+                       int64_t ne = 0);
 void launch_gather_slots(const uint8_t* frames, int dtype, int64_t hw, int nframes, int nrows,
                          const int32_t* pix_idx, const BinDev* bins, const KbWork* kbl,
                          int n_items, int tf, int8_t* slab, hipStream_t s, uint32_t* flagw);
-void launch_wide_gather(const uint16_t* frames, int64_t hw, int nframes, int nrows,
+void launch_wide_gather(const uint8_t* frames, int dtype, int64_t hw, int nframes, int nrows,
                         const int32_t* pix, const int32_t* pix_w, const BinDev* bins, int n_bins,
-                        const int* nwkb, int8_t* slab, hipStream_t s);
+                        const int* nwkb, int8_t* slab, const int* route, hipStream_t s);
 // Band gather of uint8/int8 frames: stage `rows` detector rows of 4 frames in LDS
 // (srow bytes per frame), write every k-block of the band from there.
 void launch_gather_band(const uint8_t* frames, int dtype, int64_t hw, int width, int nframes,
                         int nrows, int srow, const int32_t* pix_idx, const BinDev* bins,
                         const BandWork* bands, int n_bands, const int2* band_kb,
-                        const GatherWork* fall, int n_fall, int8_t* slab, hipStream_t s);
+                        const GatherWork* fall, int n_fall, int8_t* slab, hipStream_t s,
+                        const int* route = nullptr);
+// The same into the narrow slab, wide pixels flagged (k_narrow.hip).
+void launch_gather_band_f4(const uint8_t* frames, int dtype, int64_t hw, int width, int nframes,
+                           int nrows, int srow, const int32_t* pix_idx, const BinDev* bins,
+                           const BandWork* bands, int n_bands, const int2* band_kb,
+                           const GatherWork* fall, int n_fall, int8_t* slab4, uint8_t* flag,
+                           const int* route, hipStream_t s);
+// The route of a dense call with a narrow slab into ctl[0] (four zeroed ints).
+void launch_narrow_sample(const uint8_t* frames, int dtype, int64_t hw, int nframes,
+                          const int32_t* pix, int64_t n_entries, int64_t n_pix, int* ctl,
+                          hipStream_t s);
+void launch_narrow_clip(const BinDev* bins, int n_bins, const int* route, int* nwkb,
+                        hipStream_t s);
+void launch_narrow_mask(const int32_t* pix, const BinDev* bins, int n_bins, int max_nkb,
+                        const uint8_t* flag, const int* route, int nrows, const int* nwkb,
+                        int8_t* slab4, hipStream_t s);
 // cross: the work items are cross-plane ([H|L] [L|H]^T) items of uint16 frames.
 // nwkb (uint16 slabs with the wide pixels apart, else null): per bin, the k-blocks the
 // HH and cross items are clipped to (item_range in k_gram.hip).
@@ -164,15 +195,26 @@ void launch_gram_i8(int tile, bool cross, const int8_t* slab, const BinDev* bins
                     const int* nwkb, int64_t* ugram, int64_t* sums, hipStream_t s);
 // Persistent launch over per-XCD work queues: queue x is items [qoff[x], qoff[x+1]) of
 // `work`; heads (8 ints) must be zero.
+// Items of plans with a narrow slab (route: see above).
+void launch_gram_f4_queue(const int8_t* slab4, const BinDev* bins, const GramWork* work,
+                          int n_work, const int* qoff, int* heads, int nframes, int nrows,
+                          const int* route, int64_t* ugram, int64_t* sums, hipStream_t s);
+// wsums (with nwkb; may be null): the frame sums of the clipped items go there too, and a call
+// without wide pixels (nwkb[n_bins] = 0) returns at once.
 void launch_gram_i8_queue(int tile, bool cross, const int8_t* slab, const BinDev* bins,
                           const GramWork* work, int n_work, const int* qoff, int* heads,
                           int nframes, int nrows, int biased, const int* nwkb, int64_t* ugram,
-                          int64_t* sums, hipStream_t s);
+                          int64_t* sums, hipStream_t s, int n_bins = 0,
+                          int64_t* wsums = nullptr);
 // uint16 wide pixels apart (k_wide.hip): from the flags of the pixels with a count > 255
 // in some frame, each bin's wide pixels listed in pix_w, their count and clip = nwkb per
 // bin (nwkb[n_bins] the largest clip, nwkb[n_bins + 1 + b] the counts).
 void launch_wide_partition(const int32_t* pix, const BinDev* bins, int n_bins, int max_npix,
                            const uint8_t* flag, int32_t* pix_w, int* nwkb, hipStream_t s);
+// The first half of it: the wide pixels of each bin listed in pix_w and counted in
+// count[n_bins] (zeroed beforehand).
+void launch_wide_compact(const int32_t* pix, const BinDev* bins, int n_bins, int max_npix,
+                         const uint8_t* flag, int32_t* pix_w, int* count, hipStream_t s);
 // Low-byte frame sums over the nwkb k-blocks each bin's cross term reads them from.
 void launch_wide_low_sums(const int8_t* slab, const BinDev* bins, const int* nwkb, int n_bins,
                           int nframes, int nrows, int64_t* lsums, hipStream_t s);
@@ -203,7 +245,8 @@ void launch_den_mfma(const int64_t* sums, int n_bins, int nframes, const int64_t
 void launch_finalize(const int64_t* plane_sums, int64_t* sums, const int64_t* ugram,
                      const BinDev* bins, int n_bins, int nframes, int mode, int64_t* prefix,
                      int64_t* smax, double* dpre, const int* nwkb, int64_t* num, double* den,
-                     float* g2, const DenMfma& dm, hipStream_t s);
+                     float* g2, const DenMfma& dm, hipStream_t s,
+                     const int64_t* wsums = nullptr);
 void launch_plain_bin(const uint8_t* frames, int dtype, int64_t hw, int nframes,
                       const int32_t* pix, int npix, float* a, float* gram, float* means,
                       float* g2_row, hipStream_t s);

@@ -384,14 +384,14 @@ __device__ __forceinline__ int64_t edge_sums(const int64_t* P, int nframes, int 
 
 // The numerator of entry o from the raw Gram diagonals: n as stored in `num`, nd its FP64
 // value.  `stride` separates the rows of the digit products; pairs = padded pixel pairs on
-// the diagonal, pairs_w the same of the wide k-blocks (mode 3); edges(p) the edge sums of
+// the diagonal, pairs_w the same of the wide k-blocks (modes 3, 4); edges(p) the edge sums of
 // plane p.  Modes as in finalize_kernel.
 template <typename NumT, typename Edges>
 __device__ __forceinline__ void complete_numerator(const NumT* __restrict__ ugram, int64_t o,
                                                    int64_t stride, int mode, int64_t pairs,
                                                    int64_t pairs_w, Edges edges, NumT& n,
                                                    double& nd) {
-    if (mode >= 2) {
+    if (mode == 2 || mode == 3) {
         // biased digit products: (h-128)(h'-128) etc.; padding entries are -128 too
         const int64_t eh = edges(0), el = edges(1);
         const int64_t elx = mode == 3 ? edges(2) : el;
@@ -405,6 +405,7 @@ __device__ __forceinline__ void complete_numerator(const NumT* __restrict__ ugra
     } else {
         n = ugram[o];
         if (mode == 1) n += (NumT)(128 * edges(0) - 16384 * pairs);
+        if (mode == 4) n += (NumT)(128 * edges(1) - 16384 * pairs_w);
         nd = (double)n;
     }
 }
@@ -460,7 +461,7 @@ __global__ __launch_bounds__(FIN_THREADS) void finalize_kernel(
         NumT n;
         complete_numerator<NumT>(
             ugram, o, (int64_t)nb * nframes, mode, pairs,
-            mode == 3 ? (int64_t)nwkb[b] * KB * (nframes - tau) : 0,
+            mode >= 3 ? (int64_t)nwkb[b] * KB * (nframes - tau) : 0,
             [&](int p) {
                 return edge_sums(prefix + ((int64_t)p * nb + b) * (nframes + 1), nframes, tau);
             },
@@ -493,13 +494,13 @@ constexpr int FS_LEN = FINISH_SMALL + FS_LAGS + 8;   // frames staged, zeros pas
 __device__ __forceinline__ int fs_pad(int i) { return i + (i >> 2); }
 
 // PLANES as in sums_prep_kernel: 1 (S = plane_sums), 2 or 3 (uint16 digit planes; the
-// combined S goes to `sums`).  mode, nwkb, num, den, g2 as in finalize_kernel.
+// combined S goes to `sums`); mode 4 (wsums not null): 2, S = plane_sums and wsums.  mode, nwkb, num, den, g2 as in finalize_kernel.
 template <typename NumT, int PLANES>
 __global__ __launch_bounds__(256) void finish_small_kernel(
     const int64_t* __restrict__ plane_sums, int64_t* __restrict__ sums,
-    const NumT* __restrict__ ugram, const BinDev* __restrict__ bins, int nframes, int mode,
-    const int* __restrict__ nwkb, NumT* __restrict__ num, double* __restrict__ den,
-    float* __restrict__ g2) {
+    const int64_t* __restrict__ wsums, const NumT* __restrict__ ugram,
+    const BinDev* __restrict__ bins, int nframes, int mode, const int* __restrict__ nwkb,
+    NumT* __restrict__ num, double* __restrict__ den, float* __restrict__ g2) {
     __shared__ double sS[FS_LEN + FS_LEN / 4];
     __shared__ __attribute__((aligned(16))) unsigned char sred[4 * FS_LAGS * 8];
     __shared__ int64_t sP[3][257];   // sums of the chunks before chunk i of each plane
@@ -509,7 +510,8 @@ __global__ __launch_bounds__(256) void finish_small_kernel(
     const int tau0 = blockIdx.x * FS_LAGS;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t* X[3] = {plane_sums + (int64_t)b * nframes,
-                           plane_sums + (int64_t)(nb + b) * nframes,
+                           (wsums ? wsums - (int64_t)nb * nframes : plane_sums) +
+                               (int64_t)(nb + b) * nframes,
                            plane_sums + (int64_t)(2 * nb + b) * nframes};
     // S into LDS, its largest magnitude
     long long mx = 0;
@@ -518,7 +520,7 @@ __global__ __launch_bounds__(256) void finish_small_kernel(
         int64_t v = 0;
         if (t < nframes) {
             v = X[0][t];
-            if (PLANES >= 2) {
+            if (PLANES >= 2 && !wsums) {
                 v = 256 * v + X[1][t];
                 if (blockIdx.x == 0) sums[(int64_t)b * nframes + t] = v;
             }
@@ -626,7 +628,7 @@ __global__ __launch_bounds__(256) void finish_small_kernel(
     NumT n;
     complete_numerator<NumT>(ugram, o, (int64_t)nb * nframes, mode,
                              (int64_t)bd.nkb * KB * (nframes - tau),
-                             mode == 3 ? (int64_t)nwkb[b] * KB * (nframes - tau) : 0,
+                             mode >= 3 ? (int64_t)nwkb[b] * KB * (nframes - tau) : 0,
                              [&](int p) { return edges(PLANES > p ? p : 0); }, n, nd);
     if (num) num[o] = n;
     if (den) den[o] = d;
@@ -638,20 +640,24 @@ static bool finish_is_small(int n_bins, int nframes) {
 }
 
 template <typename NumT>
-static void launch_finish_small(const int64_t* plane_sums, int64_t* sums, const NumT* ugram,
+static void launch_finish_small(const int64_t* plane_sums, int64_t* sums, const int64_t* wsums,
+                                const NumT* ugram,
                                 const BinDev* bins, int n_bins, int nframes, int mode,
                                 const int* nwkb, NumT* num, double* den, float* g2,
                                 hipStream_t s) {
     const dim3 grid((unsigned)((nframes + FS_LAGS - 1) / FS_LAGS), (unsigned)n_bins);
     if (mode == 3)
-        finish_small_kernel<NumT, 3><<<grid, 256, 0, s>>>(plane_sums, sums, ugram, bins, nframes,
+        finish_small_kernel<NumT, 3><<<grid, 256, 0, s>>>(plane_sums, sums, nullptr, ugram, bins, nframes,
                                                           mode, nwkb, num, den, g2);
     else if (mode == 2)
-        finish_small_kernel<NumT, 2><<<grid, 256, 0, s>>>(plane_sums, sums, ugram, bins, nframes,
+        finish_small_kernel<NumT, 2><<<grid, 256, 0, s>>>(plane_sums, sums, nullptr, ugram, bins, nframes,
+                                                          mode, nwkb, num, den, g2);
+    else if (mode == 4)
+        finish_small_kernel<NumT, 2><<<grid, 256, 0, s>>>(sums, sums, wsums, ugram, bins, nframes,
                                                           mode, nwkb, num, den, g2);
     else
-        finish_small_kernel<NumT, 1><<<grid, 256, 0, s>>>(sums, sums, ugram, bins, nframes, mode,
-                                                          nwkb, num, den, g2);
+        finish_small_kernel<NumT, 1><<<grid, 256, 0, s>>>(sums, sums, nullptr, ugram, bins, nframes,
+                                                          mode, nwkb, num, den, g2);
 }
 
 // Den for every bin with N M^2 < 2^52: i8 MFMA for the bins whose |S| fits two digits
@@ -679,10 +685,10 @@ static void launch_den_fp64(const int64_t* sums, int n_bins, int nframes, const 
 void launch_finalize(const int64_t* plane_sums, int64_t* sums, const int64_t* ugram,
                      const BinDev* bins, int n_bins, int nframes, int mode, int64_t* prefix,
                      int64_t* smax, double* dpre, const int* nwkb, int64_t* num, double* den,
-                     float* g2, const DenMfma& dm, hipStream_t s) {
+                     float* g2, const DenMfma& dm, hipStream_t s, const int64_t* wsums) {
     if (n_bins <= 0 || nframes <= 0) return;
     if (finish_is_small(n_bins, nframes)) {
-        launch_finish_small<int64_t>(plane_sums, sums, ugram, bins, n_bins, nframes, mode, nwkb,
+        launch_finish_small<int64_t>(plane_sums, sums, wsums, ugram, bins, n_bins, nframes, mode, nwkb,
                                      num, den, g2, s);
         return;
     }
@@ -694,7 +700,10 @@ void launch_finalize(const int64_t* plane_sums, int64_t* sums, const int64_t* ug
         launch_sums_prep<2>(plane_sums, sums, n_bins, nframes, prefix, smax, s);
     else
         launch_sums_prep<1>(sums, sums, n_bins, nframes, prefix, smax, s);
-    launch_den_fp64(sums, n_bins, nframes, smax, prefix, mode >= 2 ? 2 : 1, dm, dpre, s);
+    if (mode == 4)  // prefixes of the wide pixels' sums (at most S: smax stays)
+        launch_sums_prep<1>(wsums, nullptr, n_bins, nframes,
+                            prefix + (int64_t)n_bins * (nframes + 1), smax, s);
+    launch_den_fp64(sums, n_bins, nframes, smax, prefix, mode == 2 || mode == 3 ? 2 : 1, dm, dpre, s);
     dim3 grid((unsigned)((nframes + FIN_SPAN - 1) / FIN_SPAN), (unsigned)n_bins);
     finalize_kernel<int64_t><<<grid, dim3(FIN_THREADS), 0, s>>>(
         sums, ugram, bins, nframes, mode, prefix, smax, dpre, nwkb, num, den, g2);
@@ -705,7 +714,7 @@ void launch_finalize_f64(const int64_t* sums, const double* fnum, const BinDev* 
                          double* den, float* g2, const DenMfma& dm, hipStream_t s) {
     if (n_bins <= 0 || nframes <= 0) return;
     if (finish_is_small(n_bins, nframes)) {
-        launch_finish_small<double>(sums, const_cast<int64_t*>(sums), fnum, bins, n_bins, nframes,
+        launch_finish_small<double>(sums, const_cast<int64_t*>(sums), nullptr, fnum, bins, n_bins, nframes,
                                     0, nullptr, num, den, g2, s);
         return;
     }

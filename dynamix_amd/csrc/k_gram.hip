@@ -13,7 +13,7 @@
 // Data movement: the slab is stored fragment-contiguous (slab_offset()): the 32 frames
 // x 32 bytes an MFMA operand takes from one k-block are one 1 KiB run in lane order.
 //
-// T = 256 (PanelTile): 2 x 2 waves of 4 x 4 blocks.  The runs of a tile's row and column
+// T = 256 (PanelLoop): 2 x 2 waves of 4 x 4 blocks.  The runs of a tile's row and column
 // panels go to LDS by global->LDS DMA and each wave reads its eight fragments of a unit
 // (one K = 32 step) from there, so a run crosses the CU's vector-memory path once instead of
 // once for each of the two waves that use it (64 B/clk a CU, which the 128 x 128 blocks of
@@ -116,8 +116,12 @@ __device__ __forceinline__ void frame_sums(const int (&rs)[WM], int row, int lan
 // A wave's accumulators added to the tile's diagonal sums in LDS, and with STORE written to
 // `tile` (row-major).  32x32 i32 accumulator layout: lane holds column (lane & 31) and rows
 // 8*(v/4) + 4*(lane/32) + (v%4), v = 0..15.  Diagonal slot c - r + TM - 1.
-template <int WM, int WN, bool STORE>
-__device__ __forceinline__ void fold_tile(const v16i (&acc)[WM][WN], int wr, int wc, int lane,
+// (FP4 accumulators hold quarters.)
+__device__ __forceinline__ int exact_value(int v) { return v; }
+__device__ __forceinline__ int exact_value(float v) { return (int)(4.f * v); }
+
+template <int WM, int WN, bool STORE, typename Acc>
+__device__ __forceinline__ void fold_tile(const Acc (&acc)[WM][WN], int wr, int wc, int lane,
                                           unsigned int* sDiag, int* __restrict__ tile) {
     using S = GramShape<WM, WN>;
     // slot = lane part + (n - m) 32 - 8 (v / 4) - v % 4; the second part is a
@@ -133,7 +137,7 @@ __device__ __forceinline__ void fold_tile(const v16i (&acc)[WM][WN], int wr, int
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 const int k = (n - m) * 32 - 8 * (v >> 2) - (v & 3) - MINOFF;
-                const int val = acc[m][n][v];
+                const int val = exact_value(acc[m][n][v]);
                 atomicAdd(sd + k, (unsigned)(val & 0xFFFF));
                 atomicAdd(sd + S::NDIAG + k, (unsigned)(val >> 16));
             }
@@ -149,7 +153,7 @@ __device__ __forceinline__ void fold_tile(const v16i (&acc)[WM][WN], int wr, int
                 const int rbase = wr * WM * 32 + m * 32 + 4 * (lane >> 5);
 #pragma unroll
                 for (int v = 0; v < 16; ++v)
-                    tile[(rbase + 8 * (v >> 2) + (v & 3)) * S::TN + c] = acc[m][n][v];
+                    tile[(rbase + 8 * (v >> 2) + (v & 3)) * S::TN + c] = exact_value(acc[m][n][v]);
             }
     }
 }
@@ -275,10 +279,12 @@ struct GramTile {
 };
 
 // One 256 x 256 tile through an LDS ring (see above).
-constexpr int GRAM_UNITS = 3;                      // K = 32 units per stage
+constexpr int GRAM_UNITS = 3;                      // units per stage
 constexpr int GRAM_PANEL = 8 * 1024;               // one unit of a panel: 8 runs
 constexpr int GRAM_STAGE = GRAM_UNITS * 2 * GRAM_PANEL;
 typedef __attribute__((address_space(3))) void lds_void;
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef int v8i __attribute__((ext_vector_type(8)));
 
 __device__ const int8_t gram_zeros[4 * 2048] __attribute__((aligned(1024))) = {};
 
@@ -287,33 +293,88 @@ __device__ const int8_t gram_zeros[4 * 2048] __attribute__((aligned(1024))) = {}
 constexpr int wait_vm(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
 constexpr int wait_vm_lgkm0(int n) { return 0x0070 | (n & 15) | ((n >> 4) << 14); }
 
-template <bool DIAG, bool CROSS, bool STORE>
-struct PanelTile {
-    using S = GramShape<4, 4>;
+// Operand formats.  I8: a unit is half a k-block (K = 32), one run is 32 frames x 32 bytes.
+// F4 (narrow pixels, see k_narrow.hip): a unit is a whole k-block (K = 64) of FP4 codes, one
+// run is 32 frames x 64 codes; a code c is the FP4 value c / 2, so sums of products come out
+// in quarters, exactly (multiples of 1/4 below 2^22).
+enum GramFormat { I8, F4 };
+template <GramFormat FMT>
+struct GramOps;
+template <>
+struct GramOps<I8> {
+    typedef v16i Acc;
+    static constexpr int PER_KB = 2;       // units per k-block
+    static constexpr int RUN_STRIDE = 2048;  // bytes between neighbouring frame groups
+    __device__ __forceinline__ static v16i mma(v4i a, v4i b, v16i c) {
+        return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
+    }
+    __device__ __forceinline__ static int sum(v4i x, int s) {  // + the 16 bytes
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s = __builtin_amdgcn_sdot4(x[i], 0x01010101, s, false);
+        return s;
+    }
+};
+template <>
+struct GramOps<F4> {
+    typedef v16f Acc;
+    static constexpr int PER_KB = 1;
+    static constexpr int RUN_STRIDE = 1024;
+    __device__ __forceinline__ static v16f mma(v4i a, v4i b, v16f c) {
+        const v8i x = __builtin_shufflevector(a, a, 0, 1, 2, 3, -1, -1, -1, -1);
+        const v8i y = __builtin_shufflevector(b, b, 0, 1, 2, 3, -1, -1, -1, -1);
+        return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(x, y, c, 4, 4, 0, 0, 0, 0);
+    }
+    __device__ __forceinline__ static int sum(v4i x, int s) {  // + the 32 codes' counts
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t mag = (uint32_t)x[i] & 0x77777777u;
+            const uint32_t neg = ((uint32_t)x[i] >> 3) & 0x11111111u;
+            s = (int)__builtin_amdgcn_udot8(mag, 0x11111111u, (uint32_t)s, false);
+            s -= 2 * (int)__builtin_amdgcn_udot8(mag, neg, 0u, false);
+        }
+        return s;
+    }
+};
+
+// One k-range of a tile in one format: acc += panel x panel^T.
+template <GramFormat FMT, bool DIAG, bool CROSS>
+struct PanelLoop {
+    using Ops = GramOps<FMT>;
+    static constexpr int U = GRAM_UNITS;
     const int8_t* __restrict__ slab_bin;
-    int kb0, kb1, row0, col0, nframes, nrows;
-    int tid, lane, wr, wc;
+    int kb0, kb1, row0, col0, nrows;
+    int lane, wr, wc;
     int nkbp;  // CROSS: k-blocks per digit plane (B reads kb + nkbp or kb - nkbp)
-    unsigned int* sDiag;
 
-    v16i acc[4][4];
-    v4i fa[GRAM_UNITS][4], fb[GRAM_UNITS][4];
-    int rs[4];         // DIAG: partial frame sums of this lane's A rows
+    typename Ops::Acc acc[4][4];
+    v4i fa[U][4], fb[U][4];
+    int rs[4];     // DIAG: partial frame sums of this lane's A rows
 
-    // This wave's source of unit u (its four runs are 2048 bytes apart): waves 0 and 1 copy
-    // the row panel, 2 and 3 the column panel.
+    __device__ __forceinline__ void clear() {
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            rs[m] = 0;
+#pragma unroll
+            for (int n = 0; n < 4; ++n)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[m][n][v] = 0;
+        }
+    }
+    // This wave's source of unit u (its four runs are RUN_STRIDE bytes apart): waves 0 and 1
+    // copy the row panel, 2 and 3 the column panel.
     __device__ __forceinline__ const int8_t* source(int u) const {
-        int kb = u >> 1;
+        int kb = u / Ops::PER_KB;
         const bool past = kb >= kb1;
         kb = min(kb, kb1 - 1);
         if (CROSS && wr) kb = kb < nkbp ? kb + nkbp : kb - nkbp;
         const int group = ((wr ? col0 : row0) >> 5) + wc * 4;
-        const int8_t* p = slab_bin + ((int64_t)kb * (nrows >> 5) + group) * 2048 + (u & 1) * 1024;
+        const int8_t* p = slab_bin + ((int64_t)kb * (nrows >> 5) + group) * Ops::RUN_STRIDE +
+                          (u % Ops::PER_KB) * 1024;
         return past && !wr ? gram_zeros : p;
     }
     __device__ __forceinline__ void dma(int8_t* buf, int un, const int8_t* src, int o) const {
         __builtin_amdgcn_global_load_lds(
-            (const void*)(src + o * 2048 + lane * 16),
+            (const void*)(src + o * Ops::RUN_STRIDE + lane * 16),
             (lds_void*)(buf + (un * 2 + wr) * GRAM_PANEL + (wc * 4 + o) * 1024), 16, 0, 0);
     }
     __device__ __forceinline__ v4i frag_a(const int8_t* unit, int m) const {
@@ -324,21 +385,20 @@ struct PanelTile {
     }
 
     // The units of stage `cur` (unit 0's fragments are in slot 0), with the first fragments of
-    // `next` and the copies of units u .. u + GRAM_UNITS - 1 into `rel`, the buffer of the
-    // stage before.
+    // `next` and the copies of units u .. u + U - 1 into `rel`, the buffer of the stage before.
     __device__ __forceinline__ void stage(const int8_t* cur, const int8_t* next, int8_t* rel,
                                           int u) {
 #pragma unroll
-        for (int un = 0; un < GRAM_UNITS; ++un) {
-            if (un == GRAM_UNITS - 1) {
-                __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0((GRAM_UNITS - 1) * 4));
+        for (int un = 0; un < U; ++un) {
+            if (un == U - 1) {
+                __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0((U - 1) * 4));
                 __builtin_amdgcn_s_barrier();
                 asm volatile("" ::: "memory");  // the reads below stay below
                 __builtin_amdgcn_sched_barrier(0);
             }
             const int8_t* src = source(u + un);
-            const int8_t* from = un + 1 < GRAM_UNITS ? cur + (un + 1) * 2 * GRAM_PANEL : next;
-            const int sl = (un + 1) % GRAM_UNITS;
+            const int8_t* from = un + 1 < U ? cur + (un + 1) * 2 * GRAM_PANEL : next;
+            const int sl = (un + 1) % U;
 #pragma unroll
             for (int m = 0; m < 4; ++m) {
                 if (m == 0) {
@@ -354,17 +414,10 @@ struct PanelTile {
                     fa[sl][3] = frag_a(from, 3);
                 }
                 dma(rel, un, src, m);
+                const v4i x = fa[un][m];
 #pragma unroll
-                for (int n = 0; n < 4; ++n)
-                    acc[m][n] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[un][m], fb[un][n],
-                                                                      acc[m][n], 0, 0, 0);
-                if (DIAG) {
-                    const v4i x = fa[un][m];
-                    rs[m] = __builtin_amdgcn_sdot4(x.x, 0x01010101, rs[m], false);
-                    rs[m] = __builtin_amdgcn_sdot4(x.y, 0x01010101, rs[m], false);
-                    rs[m] = __builtin_amdgcn_sdot4(x.z, 0x01010101, rs[m], false);
-                    rs[m] = __builtin_amdgcn_sdot4(x.w, 0x01010101, rs[m], false);
-                }
+                for (int n = 0; n < 4; ++n) acc[m][n] = Ops::mma(x, fb[un][n], acc[m][n]);
+                if (DIAG) rs[m] = Ops::sum(x, rs[m]);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
@@ -372,9 +425,9 @@ struct PanelTile {
     // The same for a wave with nothing to compute: its copies and the barrier.
     __device__ __forceinline__ void idle_stage(int8_t* rel, int u) const {
 #pragma unroll
-        for (int un = 0; un < GRAM_UNITS; ++un) {
-            if (un == GRAM_UNITS - 1) {
-                __builtin_amdgcn_s_waitcnt(wait_vm((GRAM_UNITS - 1) * 4));
+        for (int un = 0; un < U; ++un) {
+            if (un == U - 1) {
+                __builtin_amdgcn_s_waitcnt(wait_vm((U - 1) * 4));
                 __builtin_amdgcn_s_barrier();
                 asm volatile("" ::: "memory");
             }
@@ -383,36 +436,19 @@ struct PanelTile {
             for (int o = 0; o < 4; ++o) dma(rel, un, src, o);
         }
     }
-
-    __device__ __forceinline__ void run(int biased, int64_t* __restrict__ out,
-                                        int64_t* __restrict__ sums, int* __restrict__ tile,
-                                        int8_t* buf0, int8_t* buf1, int8_t* buf2) {
-        for (int i = tid; i < 2 * S::NDIAG; i += 256) sDiag[i] = 0u;
+    // kb0 < kb1.  Ends with no copy in flight and no wave of the workgroup past its reads.
+    __device__ __forceinline__ void run(bool idle, int8_t* buf0, int8_t* buf1, int8_t* buf2) {
+        const int u0 = Ops::PER_KB * kb0;
+        const int n_stage = (Ops::PER_KB * (kb1 - kb0) + U - 1) / U;
 #pragma unroll
-        for (int m = 0; m < 4; ++m) {
-            rs[m] = 0;
-#pragma unroll
-            for (int n = 0; n < 4; ++n)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) acc[m][n][v] = 0;
-        }
-        // idle: every block of this wave is below the diagonal, or lies wholly in the
-        // padding frames past the last one (a STORE tile's readers skip both parts)
-        const bool idle = (DIAG && wr > wc) || row0 + wr * 128 >= nframes ||
-                          col0 + wc * 128 >= nframes;
-        const int u0 = 2 * kb0;
-        const int n_stage = (2 * (kb1 - kb0) + GRAM_UNITS - 1) / GRAM_UNITS;
-#pragma unroll
-        for (int un = 0; un < 2 * GRAM_UNITS; ++un) {
+        for (int un = 0; un < 2 * U; ++un) {
             const int8_t* src = source(u0 + un);
 #pragma unroll
-            for (int o = 0; o < 4; ++o)
-                dma(un < GRAM_UNITS ? buf0 : buf1, un % GRAM_UNITS, src, o);
+            for (int o = 0; o < 4; ++o) dma(un < U ? buf0 : buf1, un % U, src, o);
         }
-        __builtin_amdgcn_s_waitcnt(wait_vm(GRAM_UNITS * 4));
+        __builtin_amdgcn_s_waitcnt(wait_vm(U * 4));
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        constexpr int U = GRAM_UNITS;
         int st = 0, u = u0 + 2 * U;  // u: first unit copied by stage st
         if (idle) {
             for (; st + 3 <= n_stage; st += 3, u += 3 * U) {
@@ -440,17 +476,39 @@ struct PanelTile {
                 if (st + 1 < n_stage) stage(buf1, buf2, buf0, u + U);
             }
         }
-
-        if (DIAG && !STORE && wr == wc)
-            frame_sums<4>(rs, row0 + wr * 128, lane, nframes,
-                          biased ? (int64_t)128 * (kb1 - kb0) * KB : 0, sums);
-        __builtin_amdgcn_s_waitcnt(wait_vm(0));  // no copy is in flight into a reused buffer
+        __builtin_amdgcn_s_waitcnt(wait_vm(0));
         __syncthreads();
-        if (!idle) fold_tile<4, 4, STORE>(acc, wr, wc, lane, sDiag, tile);
-        __syncthreads();
-        flush_diagonals<S>(sDiag, tid, col0 - row0, nframes, out);
     }
 };
+
+// A tile over k-blocks [kb0, kb1) of a slab in format FMT.  Its frame sums go to sums, and to
+// wsums when that is not null.
+template <GramFormat FMT, bool DIAG, bool CROSS, bool STORE>
+__device__ __forceinline__ void panel_tile(const int8_t* __restrict__ slab_bin, int kb0, int kb1,
+                                           int row0, int col0, int nframes, int nrows, int tid,
+                                           int wr, int wc, int nkbp, int biased,
+                                           int64_t* __restrict__ out, int64_t* __restrict__ sums,
+                                           int64_t* __restrict__ wsums, int* __restrict__ tile,
+                                           unsigned int* sDiag, int8_t* buf0, int8_t* buf1,
+                                           int8_t* buf2) {
+    using S = GramShape<4, 4>;
+    const int lane = tid & 63;
+    for (int i = tid; i < 2 * S::NDIAG; i += 256) sDiag[i] = 0u;
+    // idle: every block of this wave is below the diagonal, or lies wholly in the padding
+    // frames past the last one (a STORE tile's readers skip both parts)
+    const bool idle = (DIAG && wr > wc) || row0 + wr * 128 >= nframes || col0 + wc * 128 >= nframes;
+    PanelLoop<FMT, DIAG, CROSS> t{slab_bin, kb0, kb1, row0, col0, nrows, lane, wr, wc, nkbp};
+    t.clear();
+    t.run(idle, buf0, buf1, buf2);
+    if (DIAG && !STORE && wr == wc) {
+        const int64_t bias = biased ? (int64_t)128 * (kb1 - kb0) * KB : 0;
+        frame_sums<4>(t.rs, row0 + wr * 128, lane, nframes, bias, sums);
+        if (wsums) frame_sums<4>(t.rs, row0 + wr * 128, lane, nframes, bias, wsums);
+    }
+    if (!idle) fold_tile<4, 4, STORE>(t.acc, wr, wc, lane, sDiag, tile);
+    __syncthreads();
+    flush_diagonals<S>(sDiag, tid, col0 - row0, nframes, out);
+}
 
 // K-range of item `w` and the CROSS kernel's plane distance.  nwkb (uint16 plans whose
 // wide pixels -- those with a count above 255 -- have k-blocks of their own; null: every
@@ -491,17 +549,18 @@ __device__ __forceinline__ void gram_item(const GramWork& w, ItemRange r, const 
                                           int nframes, int nrows, int biased,
                                           int64_t* __restrict__ out, int64_t* __restrict__ sums,
                                           int* __restrict__ tile, unsigned int* sDiag,
-                                          int8_t* buf0, int8_t* buf1, int8_t* buf2) {
+                                          int8_t* buf0, int8_t* buf1, int8_t* buf2,
+                                          int64_t* __restrict__ wsums = nullptr) {
     using S = GramShape<WM, WN>;
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     auto go = [&](auto diag) {
         constexpr bool DIAG = decltype(diag)::value;
         if constexpr (WM == 4) {
-            PanelTile<DIAG, CROSS, STORE> t{slab_bin, r.kb0, r.kb1, w.ti * S::TM, w.tj * S::TN,
-                                            nframes, nrows, tid, tid & 63, wave >> 1, wave & 1,
-                                            r.nkbp, sDiag};
-            t.run(biased, out, sums, tile, buf0, buf1, buf2);
+            panel_tile<I8, DIAG, CROSS, STORE>(slab_bin, r.kb0, r.kb1, w.ti * S::TM,
+                                               w.tj * S::TN, nframes, nrows, tid, wave >> 1,
+                                               wave & 1, r.nkbp, biased, out, sums, wsums, tile,
+                                               sDiag, buf0, buf1, buf2);
         } else {
             GramTile<WM, WN, DIAG, CROSS, STORE> t{slab_bin, r.kb0, r.kb1, w.ti * S::TM,
                                                    w.tj * S::TN, nframes, nrows, tid, tid & 63,
@@ -564,12 +623,13 @@ template <int WM, int WN, bool CROSS>
 __global__ __launch_bounds__(256) void gram_i8_queue_kernel(
     const int8_t* __restrict__ slab, const BinDev* __restrict__ bins,
     const GramWork* __restrict__ work, const int* __restrict__ qoff, int* heads, int nframes,
-    int nrows, int biased, const int* __restrict__ nwkb, int64_t* __restrict__ ugram,
-    int64_t* __restrict__ sums) {
+    int nrows, int biased, const int* __restrict__ nwkb, int n_bins, int64_t* __restrict__ ugram,
+    int64_t* __restrict__ sums, int64_t* __restrict__ wsums) {
     using S = GramShape<WM, WN>;
     static_assert(S::TM == S::TN, "square tiles");
     DXG2_GRAM_LDS(WM);
     __shared__ int s_item;
+    if (wsums && nwkb[n_bins] == 0) return;  // no wide pixel in any bin
     const int home = xcc_id();
     for (;;) {
         if (threadIdx.x == 0) s_item = next_item(home, qoff, heads);
@@ -582,7 +642,44 @@ __global__ __launch_bounds__(256) void gram_i8_queue_kernel(
         if (r.kb1 > r.kb0)  // the same for every thread of the workgroup
             gram_item<WM, WN, CROSS, false>(w, r, slab + bd.slab_off, nframes, nrows, biased,
                                             ugram + (int64_t)w.out * nframes,
-                                            sums + (int64_t)w.out * nframes, nullptr, sDiag, buf0, buf1, buf2);
+                                            sums + (int64_t)w.out * nframes, nullptr, sDiag, buf0,
+                                            buf1, buf2,
+                                            wsums ? wsums + (int64_t)w.out * nframes : nullptr);
+        __syncthreads();  // s_item and sDiag are reused by the next item
+    }
+}
+
+// The narrow pixels' Gram of a plan with an FP4 slab (k_narrow.hip), when the call took that
+// route.  The wide pixels' follows through gram_i8_queue_kernel, with nwkb and wsums.
+__global__ __launch_bounds__(256) void gram_f4_queue_kernel(
+    const int8_t* __restrict__ slab4, const BinDev* __restrict__ bins,
+    const GramWork* __restrict__ work, const int* __restrict__ qoff, int* heads, int nframes,
+    int nrows, const int* __restrict__ route, int64_t* __restrict__ ugram,
+    int64_t* __restrict__ sums) {
+    DXG2_GRAM_LDS(4);
+    __shared__ int s_item;
+    if (route[0] != NARROW_F4) return;
+    const int home = xcc_id();
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    for (;;) {
+        if (tid == 0) s_item = next_item(home, qoff, heads);
+        __syncthreads();
+        const int it = s_item;
+        if (it < 0) break;
+        const GramWork w = work[it];
+        const int8_t* s4 = slab4 + bins[w.bin].slab_off / 2;
+        const int64_t o = (int64_t)w.bin * nframes;
+        if (w.ti == w.tj)
+            panel_tile<F4, true, false, false>(s4, w.kb0, w.kb1, w.ti * 256, w.tj * 256, nframes,
+                                               nrows, tid, wave >> 1, wave & 1, 0, 0, ugram + o,
+                                               sums + o, nullptr, nullptr, sDiag, buf0, buf1,
+                                               buf2);
+        else
+            panel_tile<F4, false, false, false>(s4, w.kb0, w.kb1, w.ti * 256, w.tj * 256, nframes,
+                                                nrows, tid, wave >> 1, wave & 1, 0, 0, ugram + o,
+                                                sums + o, nullptr, nullptr, sDiag, buf0, buf1,
+                                                buf2);
         __syncthreads();  // s_item and sDiag are reused by the next item
     }
 }
@@ -606,6 +703,15 @@ int queue_grid() {
     return grid[dev];
 }
 
+void launch_gram_f4_queue(const int8_t* slab4, const BinDev* bins, const GramWork* work,
+                          int n_work, const int* qoff, int* heads, int nframes, int nrows,
+                          const int* route, int64_t* ugram, int64_t* sums, hipStream_t s) {
+    if (n_work <= 0) return;
+    gram_f4_queue_kernel<<<dim3((unsigned)std::min(n_work, queue_grid<4, 4, false>())), 256, 0,
+                           s>>>(slab4, bins, work, qoff, heads, nframes, nrows, route, ugram,
+                                sums);
+}
+
 void gram_queue_prepare(int tile) {
     if (tile == 128) {
         (void)queue_grid<2, 2, false>();
@@ -619,13 +725,14 @@ void gram_queue_prepare(int tile) {
 void launch_gram_i8_queue(int tile, bool cross, const int8_t* slab, const BinDev* bins,
                           const GramWork* work, int n_work, const int* qoff, int* heads,
                           int nframes, int nrows, int biased, const int* nwkb, int64_t* ugram,
-                          int64_t* sums, hipStream_t s) {
+                          int64_t* sums, hipStream_t s, int n_bins, int64_t* wsums) {
     if (n_work <= 0) return;
     const dim3 block(256);
 #define DXG2_QUEUE_LAUNCH(WM, CR)                                                             \
     gram_i8_queue_kernel<WM, WM, CR><<<dim3((unsigned)std::min(n_work, queue_grid<WM, WM, CR>())), \
                                        block, 0, s>>>(slab, bins, work, qoff, heads, nframes,    \
-                                                      nrows, biased, nwkb, ugram, sums)
+                                                      nrows, biased, nwkb, n_bins, ugram, sums,  \
+                                                      wsums)
     if (tile == 128) {
         if (cross)
             DXG2_QUEUE_LAUNCH(2, true);

@@ -89,14 +89,19 @@ __global__ __launch_bounds__(256) void wide_low_sums_kernel(const int8_t* __rest
     lsums[(int64_t)b * nframes + t] = total + (int64_t)128 * KB * nw;
 }
 
+void launch_wide_compact(const int32_t* pix, const BinDev* bins, int n_bins, int max_npix,
+                         const uint8_t* flag, int32_t* pix_w, int* count, hipStream_t s) {
+    if (n_bins > 0 && max_npix > 0)
+        wide_compact_kernel<<<dim3((unsigned)((max_npix + 255) / 256), (unsigned)n_bins), 256, 0,
+                              s>>>(pix, bins, flag, pix_w, count);
+}
+
 void launch_wide_partition(const int32_t* pix, const BinDev* bins, int n_bins, int max_npix,
                            const uint8_t* flag, int32_t* pix_w, int* nwkb, hipStream_t s) {
     if (n_bins <= 0) return;
     int* count = nwkb + n_bins + 1;
     launch_fill_i32(nwkb + n_bins, n_bins + 1, s);  // the maximum and the counts
-    if (max_npix > 0)
-        wide_compact_kernel<<<dim3((unsigned)((max_npix + 255) / 256), (unsigned)n_bins), 256, 0,
-                              s>>>(pix, bins, flag, pix_w, count);
+    launch_wide_compact(pix, bins, n_bins, max_npix, flag, pix_w, count, s);
     wide_clip_kernel<<<1, 256, 0, s>>>(bins, n_bins, count, nwkb);
 }
 
