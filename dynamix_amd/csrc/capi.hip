@@ -247,7 +247,7 @@ struct dxg2_plan {
     GramWork* d_qmwork = nullptr;
     GramWork* d_qxwork = nullptr;
     int* d_qoff = nullptr;
-    int* d_heads = nullptr;        // 16 queue heads, then the route's four ints
+    int* d_heads = nullptr;        // 16 queue heads, then the route's ints (k_narrow.hip)
     int8_t* d_slab = nullptr;
     int8_t* d_slab4 = nullptr;     // narrow slab (k_narrow.hip), half the slab's bytes
     int64_t* d_wsums = nullptr;    // its wide pixels' frame sums, n_bins rows
@@ -871,7 +871,7 @@ int ensure_event_buffers(dxg2_plan* p, int64_t nnz_coo, hipStream_t s) {
 // (pixels x frames^2) that halving it pays for the launches of the narrow route
 // (DXG2_NARROW: 0 never, 2 whatever the work).
 constexpr double NARROW_MIN_WORK = 5e11;
-constexpr int HEAD_INTS = 20;
+constexpr int HEAD_INTS = 24;
 bool narrow_applies(const dxg2_plan* p) {
     if (p->dtype == DXG2_U16 || p->gband.empty() || !p->use_queue || p->gram_tile != 256)
         return false;
@@ -947,13 +947,11 @@ int64_t* dense_gather(dxg2_plan* p, const void* d_frames, int64_t* d_sums, hipSt
     if (wide_first && narrow_call(p, d_frames)) {
         const uint8_t* frames = (const uint8_t*)d_frames;
         const int* route = p->d_heads + 16;
-        int64_t n_pix = 0;
-        for (auto n : p->npix) n_pix += n;
         launch_clear_call(gsums, nbn, p->d_ugram, nbn, p->d_heads, HEAD_INTS, s, p->d_wflag, hw,
                           p->d_wsums, nbn);
         launch_fill_i32(p->d_nwkb + p->n_bins, p->n_bins + 1, s);
         launch_narrow_sample(frames, p->dtype, hw, p->N, p->d_pix, (int64_t)p->pix_idx.size(),
-                             n_pix, p->d_heads + 16, s);
+                             p->d_heads + 16, s);
         launch_gather_band_f4(frames, p->dtype, hw, p->W, p->N, p->nrows, p->gband_srow, p->d_pix,
                               p->d_bins, p->d_gband, (int)p->gband.size(), p->d_gband_kb,
                               p->d_gfall, (int)p->gfall.size(), p->d_slab4, p->d_wflag, route, s);

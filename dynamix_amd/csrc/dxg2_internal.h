@@ -178,10 +178,9 @@ void launch_gather_band_f4(const uint8_t* frames, int dtype, int64_t hw, int wid
                            const BandWork* bands, int n_bands, const int2* band_kb,
                            const GatherWork* fall, int n_fall, int8_t* slab4, uint8_t* flag,
                            const int* route, hipStream_t s);
-// The route of a dense call with a narrow slab into ctl[0] (four zeroed ints).
+// The route of a dense call with a narrow slab into ctl[0] (five zeroed ints).
 void launch_narrow_sample(const uint8_t* frames, int dtype, int64_t hw, int nframes,
-                          const int32_t* pix, int64_t n_entries, int64_t n_pix, int* ctl,
-                          hipStream_t s);
+                          const int32_t* pix, int64_t n_entries, int* ctl, hipStream_t s);
 void launch_narrow_clip(const BinDev* bins, int n_bins, const int* route, int* nwkb,
                         hipStream_t s);
 void launch_narrow_mask(const int32_t* pix, const BinDev* bins, int n_bins, int max_nkb,

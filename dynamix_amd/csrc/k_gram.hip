@@ -54,7 +54,8 @@
 // LDS diagonal sums stay in 32-bit words: every int32 value v is split as
 // v = hi * 2^16 + lo with lo in [0, 2^16) and hi in [-2^15, 2^15); a diagonal of a
 // T <= 256 tile collects at most 256 values, so sum(lo) < 2^24 and |sum(hi)| < 2^23
-// are exact, and the 64-bit total hi_sum * 2^16 + lo_sum is formed once per slot.
+// are exact, and the 64-bit total hi_sum * 2^16 + lo_sum is formed once per slot.  Values
+// below 2^23 (short k-ranges, FP4) are added whole.
 #include <algorithm>
 #include <type_traits>
 
@@ -113,16 +114,20 @@ __device__ __forceinline__ void frame_sums(const int (&rs)[WM], int row, int lan
     }
 }
 
-// A wave's accumulators added to the tile's diagonal sums in LDS, and with STORE written to
-// `tile` (row-major).  32x32 i32 accumulator layout: lane holds column (lane & 31) and rows
-// 8*(v/4) + 4*(lane/32) + (v%4), v = 0..15.  Diagonal slot c - r + TM - 1.
 // (FP4 accumulators hold quarters.)
 __device__ __forceinline__ int exact_value(int v) { return v; }
 __device__ __forceinline__ int exact_value(float v) { return (int)(4.f * v); }
 
+// A wave's accumulators added to the tile's diagonal sums in LDS, and with STORE written to
+// `tile` (row-major).  32x32 accumulator layout: lane holds column (lane & 31) and rows
+// 8*(v/4) + 4*(lane/32) + (v%4), v = 0..15.  Diagonal slot c - r + TM - 1: the blocks of one
+// n - m fall on the same slots and are added in registers first, since the LDS takes about
+// 11 atomics a clock (a tile's 512 a lane were 5 us).
+// small: every |value| < 2^23, so a diagonal's up to 256 values need no splitting.
 template <int WM, int WN, bool STORE, typename Acc>
 __device__ __forceinline__ void fold_tile(const Acc (&acc)[WM][WN], int wr, int wc, int lane,
-                                          unsigned int* sDiag, int* __restrict__ tile) {
+                                          bool small, unsigned int* sDiag,
+                                          int* __restrict__ tile) {
     using S = GramShape<WM, WN>;
     // slot = lane part + (n - m) 32 - 8 (v / 4) - v % 4; the second part is a
     // compile-time constant >= MINOFF, so every atomic is one base VGPR plus an
@@ -130,19 +135,30 @@ __device__ __forceinline__ void fold_tile(const Acc (&acc)[WM][WN], int wr, int 
     constexpr int MINOFF = -(WM - 1) * 32 - 15;
     unsigned int* sd = sDiag + (wc * WN * 32 + (lane & 31)) - (wr * WM * 32 + 4 * (lane >> 5)) +
                        S::TM - 1 + MINOFF;
+    auto fold = [&](auto split) {
 #pragma unroll
-    for (int m = 0; m < WM; ++m)
-#pragma unroll
-        for (int n = 0; n < WN; ++n) {
+        for (int d = -(WM - 1); d < WN; ++d) {  // d = n - m
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
-                const int k = (n - m) * 32 - 8 * (v >> 2) - (v & 3) - MINOFF;
-                const int val = exact_value(acc[m][n][v]);
-                atomicAdd(sd + k, (unsigned)(val & 0xFFFF));
-                atomicAdd(sd + S::NDIAG + k, (unsigned)(val >> 16));
+                const int k = d * 32 - 8 * (v >> 2) - (v & 3) - MINOFF;
+                unsigned lo = 0u, hi = 0u;
+#pragma unroll
+                for (int m = 0; m < WM; ++m) {
+                    if (m + d < 0 || m + d >= WN) continue;
+                    const int val = exact_value(acc[m][m + d][v]);
+                    lo += decltype(split)::value ? (unsigned)(val & 0xFFFF) : (unsigned)val;
+                    hi += (unsigned)(val >> 16);
+                }
+                atomicAdd(sd + k, lo);
+                if (decltype(split)::value) atomicAdd(sd + S::NDIAG + k, hi);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
+    };
+    if (small)
+        fold(std::false_type{});
+    else
+        fold(std::true_type{});
     if (STORE) {
         // Lanes 0-31 and 32-63 of one store write two 128-byte row segments.
 #pragma unroll
@@ -160,10 +176,13 @@ __device__ __forceinline__ void fold_tile(const Acc (&acc)[WM][WN], int wr, int 
 
 // The tile's diagonal sums to the numerators: lag = shift + slot - (TM - 1).
 template <typename S>
-__device__ __forceinline__ void flush_diagonals(const unsigned int* sDiag, int tid, int shift,
-                                                int nframes, int64_t* __restrict__ out) {
+__device__ __forceinline__ void flush_diagonals(const unsigned int* sDiag, bool small, int tid,
+                                                int shift, int nframes,
+                                                int64_t* __restrict__ out) {
     for (int i = tid; i < S::NDIAG; i += 256) {
-        const long long v = (long long)(int)sDiag[S::NDIAG + i] * 65536 + (long long)sDiag[i];
+        const long long v = small ? (long long)(int)sDiag[i]
+                                  : (long long)(int)sDiag[S::NDIAG + i] * 65536 +
+                                        (long long)sDiag[i];
         const int tau = shift + i - (S::TM - 1);
         if (v != 0 && tau >= 0 && tau < nframes) gatomic_add(out + tau, v);
     }
@@ -272,9 +291,9 @@ struct GramTile {
             frame_sums<WM>(rs, row0 + wr * WM * 32, lane, nframes,
                            biased ? (int64_t)128 * (kb1 - kb0) * KB : 0, sums);
         __syncthreads();
-        if (!idle) fold_tile<WM, WN, STORE>(acc, wr, wc, lane, sDiag, tile);
+        if (!idle) fold_tile<WM, WN, STORE>(acc, wr, wc, lane, false, sDiag, tile);
         __syncthreads();
-        flush_diagonals<S>(sDiag, tid, col0 - row0, nframes, out);
+        flush_diagonals<S>(sDiag, false, tid, col0 - row0, nframes, out);
     }
 };
 
@@ -505,9 +524,11 @@ __device__ __forceinline__ void panel_tile(const int8_t* __restrict__ slab_bin, 
         frame_sums<4>(t.rs, row0 + wr * 128, lane, nframes, bias, sums);
         if (wsums) frame_sums<4>(t.rs, row0 + wr * 128, lane, nframes, bias, wsums);
     }
-    if (!idle) fold_tile<4, 4, STORE>(t.acc, wr, wc, lane, sDiag, tile);
+    // |value| <= 64 x 16384 a k-block (i8), 64 x 16 (FP4, at most 2047 k-blocks)
+    const bool small = FMT == F4 || kb1 - kb0 < 8;
+    if (!idle) fold_tile<4, 4, STORE>(t.acc, wr, wc, lane, small, sDiag, tile);
     __syncthreads();
-    flush_diagonals<S>(sDiag, tid, col0 - row0, nframes, out);
+    flush_diagonals<S>(sDiag, small, tid, col0 - row0, nframes, out);
 }
 
 // K-range of item `w` and the CROSS kernel's plane distance.  nwkb (uint16 plans whose

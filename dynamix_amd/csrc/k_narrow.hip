@@ -21,11 +21,13 @@
 
 namespace dxg2 {
 
-constexpr int NARROW_SAMPLES = 64;
+constexpr int NARROW_SAMPLES = 64;           // frames
+constexpr int NARROW_SAMPLE_KB = 1024;       // k-blocks (at the line of 30 % of 65,536 pixels
+                                             // about 20,000 turn wide over the stack)
 
-// One thread per list entry: wide in the first half of the sampled frames (ctl[1]), in any of
-// them (ctl[2]); the last block decides (ctl[0] is the route, ctl[3] counts blocks; all zeroed
-// beforehand).  Pixels that turn wide go on appearing at the rate of the second half at most
+// One thread per list entry of every `stride`-th k-block: wide in the first half of the sampled frames (ctl[1]), in any of
+// them (ctl[2]), of ctl[4] pixels; the last block decides (ctl[0] is the route, ctl[3] counts
+// blocks; all zeroed beforehand).  Pixels that turn wide go on appearing at the rate of the second half at most
 // (hot pixels are all seen in the first frames, and the rest saturate), so
 //   wide <= ctl[2] + (ctl[2] - ctl[1]) (N - n) / (n / 2).
 // The line is at 30 % of the pixels: a wide pixel costs its share of the i8 Gram, of the time
@@ -33,9 +35,10 @@ constexpr int NARROW_SAMPLES = 64;
 template <bool SGN>
 __global__ __launch_bounds__(256) void narrow_sample_kernel(
     const uint8_t* __restrict__ frames, int64_t hw, int nframes,
-    const int32_t* __restrict__ pix, int64_t n_entries, int64_t n_pix, int* __restrict__ ctl) {
+    const int32_t* __restrict__ pix, int64_t n_entries, int stride, int* __restrict__ ctl) {
     const int n = min(nframes, NARROW_SAMPLES);
-    const int64_t k = blockIdx.x * 256 + (int64_t)threadIdx.x;
+    const int64_t i0 = blockIdx.x * 256 + (int64_t)threadIdx.x;
+    const int64_t k = i0 / KB * stride * KB + i0 % KB;
     const int p = k < n_entries ? pix[k] : -1;
     bool first = false, any = false;
     if (p >= 0) {
@@ -50,9 +53,11 @@ __global__ __launch_bounds__(256) void narrow_sample_kernel(
         }
     }
     const int nf = __popcll(__ballot(first)), na = __popcll(__ballot(any));
+    const int np = __popcll(__ballot(p >= 0));
     if ((threadIdx.x & 63) == 0) {
         if (nf) atomicAdd(ctl + 1, nf);
         if (na) atomicAdd(ctl + 2, na);
+        if (np) atomicAdd(ctl + 4, np);
     }
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -62,7 +67,7 @@ __global__ __launch_bounds__(256) void narrow_sample_kernel(
             const double half = (n + 1) / 2;  // frames with 2 i < n
             const double grow = n > 1 ? (a - f) / (n - half) : 0.0;
             const double wide = a + grow * (double)(nframes - n);
-            ctl[0] = wide <= 0.3 * (double)n_pix ? NARROW_F4 : NARROW_OFF;
+            ctl[0] = wide <= 0.3 * (double)atomicAdd(ctl + 4, 0) ? NARROW_F4 : NARROW_OFF;
         }
     }
 }
@@ -124,15 +129,16 @@ __global__ __launch_bounds__(256) void narrow_mask_kernel(const int32_t* __restr
 }
 
 void launch_narrow_sample(const uint8_t* frames, int dtype, int64_t hw, int nframes,
-                          const int32_t* pix, int64_t n_entries, int64_t n_pix, int* ctl,
-                          hipStream_t s) {
-    const dim3 grid((unsigned)((n_entries + 255) / 256));
+                          const int32_t* pix, int64_t n_entries, int* ctl, hipStream_t s) {
+    const int64_t nkb = n_entries / KB;  // the lists are padded to whole k-blocks
+    const int stride = (int)((nkb + NARROW_SAMPLE_KB - 1) / NARROW_SAMPLE_KB);
+    const dim3 grid((unsigned)((nkb + stride - 1) / stride * KB + 255) / 256);
     if (dtype == DXG2_I8)
-        narrow_sample_kernel<true><<<grid, 256, 0, s>>>(frames, hw, nframes, pix, n_entries, n_pix,
+        narrow_sample_kernel<true><<<grid, 256, 0, s>>>(frames, hw, nframes, pix, n_entries, stride,
                                                         ctl);
     else
         narrow_sample_kernel<false><<<grid, 256, 0, s>>>(frames, hw, nframes, pix, n_entries,
-                                                         n_pix, ctl);
+                                                         stride, ctl);
 }
 
 void launch_narrow_clip(const BinDev* bins, int n_bins, const int* route, int* nwkb,
