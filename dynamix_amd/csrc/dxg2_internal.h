@@ -323,7 +323,7 @@ void launch_synth(void* frames, int dtype, int nframes, int64_t hw, const float*
 // frame sums from the slab, per-tile diagonal segments of the ratios, and dev.
 void launch_gram_i8_store(int tile, bool cross, const int8_t* slab, const BinDev* bins,
                           const GramWork* work, int n_work, int nframes, int nrows, int biased,
-                          int64_t* ugram, int* tiles, hipStream_t s);
+                          int64_t* ugram, int64_t* sums, int* tiles, hipStream_t s);
 void launch_slab_sums(const int8_t* slab, int dtype, const BinDev* bins, const GatherWork* work,
                       int n_work, int n_bins, int nframes, int nrows, int64_t* sums,
                       hipStream_t s);

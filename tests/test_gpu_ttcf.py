@@ -102,3 +102,25 @@ def test_two_time_from_events_equals_dense_and_oracle(dtype):
     assert np.isnan(ce.two_time(t, d, o, 2)).all()
     with pytest.raises(ValueError):
         ce.two_time(t, d, o, 5)
+
+
+@pytest.mark.parametrize("dtype,tile,chunks", [(np.uint8, 256, 1), (np.int8, 128, 1),
+                                               (np.uint16, 256, 1), (np.uint8, 256, 4)])
+def test_two_time_of_a_large_and_a_small_bin(monkeypatch, dtype, tile, chunks):
+    """A bin of more than half the detector (every bin is gathered) and small ones (gathered
+    alone), in turn on one correlator with new frames each time, then g2 of all of them."""
+    from dynamix_amd.correlator.dense import MatMulCorrelator
+    _announce("ttcf large / small bin %s tile=%d chunks=%d" % (np.dtype(dtype), tile, chunks))
+    if chunks > 1:
+        monkeypatch.setenv("DXG2_STD_SCRATCH_MB", "1")
+    rng = np.random.default_rng(31)
+    shape, n = (13, 21), 700 if chunks > 1 else 257
+    q = np.ones(shape, np.int32)
+    q[rng.random(shape) < 0.3] = 2
+    q.flat[:2] = 3
+    c = MatMulCorrelator(shape, n, q, extra_options={"tile": tile})
+    for b in (1, 2, 3, 1):
+        f = rng.poisson(1.5, size=(n,) + shape).astype(dtype)
+        _check(c.two_time(f, b), og.two_time_fp64(f, q, b))
+    c.correlate(f)
+    assert np.array_equal(c.last_numerators.cpu().numpy(), og.dense_g2(f, q)["num"])
