@@ -207,7 +207,8 @@ struct dxg2_plan {
     int tune_band = 4;    // tile rows per raster band of the Gram work list
     int tune_group = 32;  // consecutive items per XCD chunk (0: no XCD permutation)
     int tune_kchunk = MAX_KBLOCKS_PER_ITEM;
-    int gather_frames = 64;  // frames per workgroup of the general gather (a multiple of 8)
+    int gather_frames = 0;   // frames per workgroup of the general gather (a multiple of 8;
+                             // 0: gather_tile())
     // graph replay of the dense chain (dxg2_correlate_dense_graph)
     hipStream_t cap_stream = nullptr;
     hipGraphExec_t gexec = nullptr;
@@ -226,6 +227,7 @@ struct dxg2_plan {
     std::vector<GatherWork> gfall;
     int64_t gfall_kb = 0;  // k-blocks on the fallback
     int gband_srow = 0;
+    int gband_frames = BAND_FRAMES;  // frames per workgroup
     BandWork* d_gband = nullptr;
     int2* d_gband_kb = nullptr;
     GatherWork* d_gfall = nullptr;
@@ -413,9 +415,21 @@ void build_band_work(dxg2_plan* p, const std::vector<std::vector<int32_t>>& list
         }
         if (fall0 >= 0) flush(nkb);
     }
-    // one work item per band and run of at most BAND_ITEM_KMAX k-blocks (the band kernel
-    // keeps BAND_KMAX k-blocks per wave in registers)
-    const int kmax = BAND_ITEM_KMAX;
+    // One work item per band and run of at most kmax k-blocks (the band kernel keeps BAND_KMAX
+    // k-blocks per wave in registers), gband_frames frames a workgroup: the most of both, which
+    // stages rows and sets registers up the least, unless that leaves the chip's 512 slots
+    // (two workgroups a CU) part empty.  96 x 96 x 500: 4 workgroups, 104 us; 567 of 8
+    // frames and at most 16 k-blocks, 14 us.
+    int kmax = BAND_ITEM_KMAX;
+    auto units = [&]() {
+        int64_t n = (int64_t)p->gfall.size();
+        for (const auto& v : per) n += ((int64_t)v.size() + kmax - 1) / kmax;
+        return n * ((p->N + p->gband_frames - 1) / p->gband_frames);
+    };
+    p->gband_frames = BAND_FRAMES;
+    while (units() < 512 && p->gband_frames > 16) p->gband_frames /= 2;
+    while (units() < 512 && kmax > 16) kmax = kmax > 64 ? 64 : kmax / 2;
+    if (units() < 512) p->gband_frames = BAND_STAGE;
     for (int band = 0; band < nbands; ++band) {
         const int y0 = band * RB;
         for (size_t k = 0; k < per[band].size(); k += kmax) {
@@ -437,6 +451,45 @@ void build_band_work(dxg2_plan* p, const std::vector<std::vector<int32_t>>& list
     }
 }
 
+// Frames per workgroup of a general gather of `items` items: 64, or fewer where that leaves
+// the chip part empty (four workgroups a CU).
+int gather_tile(const dxg2_plan* p, size_t items) {
+    if (p->gather_frames) return p->gather_frames;
+    int tf = 64;
+    while (tf > 8 && items * (size_t)((p->N + tf - 1) / tf) < 1024) tf /= 2;
+    return tf;
+}
+
+// K-blocks per item of the plain Gram launch, at most tune_kchunk: all of a bin's, unless the
+// items are then too few or too uneven for the chip's CUs and shorter ones end sooner.  An item
+// costs about 0.5 us a k-block and 10 us for itself (first copies, fold, flush, next item) in a
+// 256-frame tile, a quarter of the former in a 128-frame tile; n items on 256 CUs end after
+// their mean load and half the longest item, and not before the longest.  96 x 96 x 500, 5
+// bins (15 whole items of 29 k-blocks): 45 us, in items of 4 and more 16 us.
+int gram_kchunk(const dxg2_plan* p) {
+    const int nT = (p->N + p->gram_tile - 1) / p->gram_tile;
+    const double tiles = (double)nT * (nT + 1) / 2 * (slab_planes(p->dtype) == 2 ? 2 : 1);
+    const double a = p->gram_tile == 256 ? 0.5 : 0.125, c = 10.0;
+    int most = 0;
+    for (const BinDev& b : p->bins) most = std::max(most, b.nkb);
+    int best = p->tune_kchunk;
+    double best_t = 0.0;
+    for (int parts = 1; parts <= 64; parts = parts < 4 ? parts + 1 : parts + parts / 2) {
+        const int k = std::min(p->tune_kchunk, (most + parts - 1) / parts);
+        if (parts > 1 && k < 4) break;
+        double total = 0.0;
+        for (const BinDev& b : p->bins)
+            total += tiles * (a * b.nkb + c * ((b.nkb + k - 1) / std::max(k, 1)));
+        const double longest = a * k + c;
+        const double t = std::max(longest, total / 256 + 0.5 * longest);
+        if (parts == 1 || t < 0.95 * best_t) {
+            best_t = t;
+            best = parts == 1 ? p->tune_kchunk : k;
+        }
+    }
+    return best;
+}
+
 // Tile order of the grouped Gram launch.  Within a bin (largest bins first) the
 // upper-triangle tiles are walked in bands of `band` tile rows, column by column, so
 // consecutive items share row and column frame panels; the list is then dealt to the
@@ -446,8 +499,7 @@ void build_gram_work(dxg2_plan* p) {
     const int T = p->gram_tile;
     const int nT = (p->N + T - 1) / T;
     const int band = p->tune_band;
-    const int group = p->tune_group;
-    const int kchunk = p->tune_kchunk;
+    const int kchunk = gram_kchunk(p);
     std::vector<int> order(p->n_bins);
     for (int b = 0; b < p->n_bins; ++b) order[b] = b;
     // Largest bins first so their long tiles start early (LPT).
@@ -482,6 +534,8 @@ void build_gram_work(dxg2_plan* p) {
         }
     }
     GramWork pad{-1, 0, 0, 0, 0, 0, 0, 0, 0, 0};  // job 0
+    // every XCD has a share of a short list
+    const int group = std::min<int>(p->tune_group, std::max<size_t>(1, raster.size() / N_XCD));
     p->gram_work = group > 0 ? remap_for_xcds(raster, group, pad) : raster;
     p->gram_xwork = group > 0 ? remap_for_xcds(xraster, group, pad) : xraster;
     p->qm_work = split_for_xcds(raster, group > 0 ? group : 1, p->q_off);
@@ -970,12 +1024,13 @@ int64_t* dense_gather(dxg2_plan* p, const void* d_frames, int64_t* d_sums, hipSt
         launch_fill_i32(p->d_nwkb + p->n_bins, p->n_bins + 1, s);
         launch_narrow_sample(frames, p->dtype, hw, p->N, p->d_pix, (int64_t)p->pix_idx.size(),
                              p->d_heads + 16, s);
-        launch_gather_band_f4(frames, p->dtype, hw, p->W, p->N, p->nrows, p->gband_srow, p->d_pix,
-                              p->d_bins, p->d_gband, (int)p->gband.size(), p->d_gband_kb,
-                              p->d_gfall, (int)p->gfall.size(), p->d_slab4, p->d_wflag, route, s);
-        launch_gather_band(frames, p->dtype, hw, p->W, p->N, p->nrows, p->gband_srow, p->d_pix,
-                           p->d_bins, p->d_gband, (int)p->gband.size(), p->d_gband_kb, p->d_gfall,
-                           (int)p->gfall.size(), p->d_slab, s, route);
+        launch_gather_band_f4(frames, p->dtype, hw, p->W, p->N, p->nrows, p->gband_srow,
+                              p->gband_frames, p->d_pix, p->d_bins, p->d_gband,
+                              (int)p->gband.size(), p->d_gband_kb, p->d_gfall,
+                              (int)p->gfall.size(), p->d_slab4, p->d_wflag, route, s);
+        launch_gather_band(frames, p->dtype, hw, p->W, p->N, p->nrows, p->gband_srow,
+                           p->gband_frames, p->d_pix, p->d_bins, p->d_gband, (int)p->gband.size(),
+                           p->d_gband_kb, p->d_gfall, (int)p->gfall.size(), p->d_slab, s, route);
         launch_wide_compact(p->d_pix, p->d_bins, p->n_bins, (int)max_npix, p->d_wflag, p->d_pixw,
                             p->d_nwkb + p->n_bins + 1, s);
         launch_narrow_clip(p->d_bins, p->n_bins, route, p->d_nwkb, s);
@@ -993,15 +1048,16 @@ int64_t* dense_gather(dxg2_plan* p, const void* d_frames, int64_t* d_sums, hipSt
     if (one && !one->gslots.empty()) {
         launch_gather_slots((const uint8_t*)d_frames, p->dtype, hw, p->N, p->nrows, p->d_pix,
                             p->d_bins, one->d_gslots, (int)(one->gslots.size() / 16),
-                            p->gather_frames, p->d_slab, s, nullptr);
+                            gather_tile(p, one->gslots.size() / 16), p->d_slab, s, nullptr);
     } else if (!p->gband.empty() && reinterpret_cast<uintptr_t>(d_frames) % 16 == 0) {
         launch_gather_band((const uint8_t*)d_frames, p->dtype, hw, p->W, p->N, p->nrows,
-                           p->gband_srow, p->d_pix, p->d_bins, p->d_gband, (int)p->gband.size(),
-                           p->d_gband_kb, p->d_gfall, (int)p->gfall.size(), p->d_slab, s);
+                           p->gband_srow, p->gband_frames, p->d_pix, p->d_bins, p->d_gband,
+                           (int)p->gband.size(), p->d_gband_kb, p->d_gfall, (int)p->gfall.size(),
+                           p->d_slab, s);
     } else {
         launch_gather_slots((const uint8_t*)d_frames, p->dtype, hw, p->N, p->nrows, p->d_pix,
                             p->d_bins, p->d_gslots, (int)(p->gather_slots.size() / 16),
-                            p->gather_frames, p->d_slab, s, flagw);
+                            gather_tile(p, p->gather_slots.size() / 16), p->d_slab, s, flagw);
     }
     if (flagw) {
         launch_wide_partition(p->d_pix, p->d_bins, p->n_bins, (int)max_npix, p->d_wflag,
@@ -1127,7 +1183,8 @@ dxg2_plan* build_plan_host(const dxg2_plan_desc* desc, int* rc) {
     // dxg2_plan_set_tuning replaces them.
     p->tune_band = std::max(1, env_int("DXG2_GRAM_BAND", 4));
     p->tune_group = std::max(0, env_int("DXG2_GRAM_GROUP", 32));
-    p->gather_frames = std::max(8, env_int("DXG2_GATHER_FRAMES", 64) / 8 * 8);
+    const int gf = env_int("DXG2_GATHER_FRAMES", 0);
+    p->gather_frames = gf > 0 ? std::max(8, gf / 8 * 8) : 0;
     p->tune_kchunk = std::min(MAX_KBLOCKS_PER_ITEM,
                               std::max(1, env_int("DXG2_GRAM_KCHUNK", default_kchunk(p->dtype))));
     p->use_queue = env_int("DXG2_GRAM_QUEUE", 1) != 0 && !(desc->flags & DXG2_FLAG_NO_QUEUE);

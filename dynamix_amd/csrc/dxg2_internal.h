@@ -56,6 +56,7 @@ constexpr int PM_XCD_GROUP = 128;
 constexpr int PM_KPB = 2;  // k-blocks per workgroup of the pixel-major gather
 constexpr int BAND_ROW_BYTES = 9728;
 constexpr int BAND_KMAX = 36;
+constexpr int BAND_FRAMES = 128;  // most frames of a workgroup (a multiple of BAND_STAGE)
 constexpr int BAND_ITEM_KMAX = 4 * BAND_KMAX;
 constexpr int GFX950_LDS_BYTES = 160 * 1024;  // LDS per CU
 
@@ -168,13 +169,13 @@ void launch_wide_gather(const uint8_t* frames, int dtype, int64_t hw, int nframe
 // Band gather of uint8/int8 frames: stage `rows` detector rows of 4 frames in LDS
 // (srow bytes per frame), write every k-block of the band from there.
 void launch_gather_band(const uint8_t* frames, int dtype, int64_t hw, int width, int nframes,
-                        int nrows, int srow, const int32_t* pix_idx, const BinDev* bins,
+                        int nrows, int srow, int bf, const int32_t* pix_idx, const BinDev* bins,
                         const BandWork* bands, int n_bands, const int2* band_kb,
                         const GatherWork* fall, int n_fall, int8_t* slab, hipStream_t s,
                         const int* route = nullptr);
 // The same into the narrow slab, wide pixels flagged (k_narrow.hip).
 void launch_gather_band_f4(const uint8_t* frames, int dtype, int64_t hw, int width, int nframes,
-                           int nrows, int srow, const int32_t* pix_idx, const BinDev* bins,
+                           int nrows, int srow, int bf, const int32_t* pix_idx, const BinDev* bins,
                            const BandWork* bands, int n_bands, const int2* band_kb,
                            const GatherWork* fall, int n_fall, int8_t* slab4, uint8_t* flag,
                            const int* route, hipStream_t s);

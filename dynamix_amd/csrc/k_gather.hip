@@ -358,7 +358,9 @@ void launch_gather_slots(const uint8_t* frames, int dtype, int64_t hw, int nfram
 }
 
 // Band gather (uint8 / int8 frames).  A workgroup takes one band of detector rows and up
-// to BAND_ITEM_KMAX full k-blocks whose pixels lie in those rows, for BAND_FRAMES frames.
+// to BAND_ITEM_KMAX full k-blocks whose pixels lie in those rows, for `bf` frames (at most
+// BAND_FRAMES; fewer k-blocks and frames where the launch would not fill the chip, see
+// build_band_work() in capi.hip).
 // Each wave loads its k-blocks' pixel quads (16-bit offsets into the band) and slab
 // addresses (in 4-byte units) once, into registers.  Then, BAND_STAGE frames at a time,
 // the workgroup copies the band's rows of each frame -- one contiguous byte range, from
@@ -372,9 +374,8 @@ void launch_gather_slots(const uint8_t* frames, int dtype, int64_t hw, int nfram
 // staged below the band, so k-blocks spanning two rows are covered; the others, and
 // every bin's partial last k-block, go to the general gather.  Two workgroups share a CU:
 // one copies while the other assembles.
-constexpr int BAND_FRAMES = 128;    // frames per workgroup (a multiple of BAND_STAGE)
 constexpr int BAND_GROUP = 4;       // k-blocks whose LDS reads are issued together
-static_assert(BAND_FRAMES % BAND_STAGE == 0 && BAND_STAGE == 8, "band stage");
+static_assert(BAND_STAGE == 8, "band stage");
 
 // Frames [t0, t0 + BAND_STAGE) of a band (`span` bytes of each frame from band0) into LDS,
 // frame f at stage + f srow, its first byte shift[f] further; all 256 threads, between
@@ -421,7 +422,7 @@ __device__ __forceinline__ void stage_band(const uint8_t* __restrict__ frames, i
 template <bool BIAS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gather_band_kernel(
     const uint8_t* __restrict__ frames, int64_t hw, int width, int nframes, int nrows, int srow,
-    const int32_t* __restrict__ pix_idx, const BinDev* __restrict__ bins,
+    int bf, const int32_t* __restrict__ pix_idx, const BinDev* __restrict__ bins,
     const BandWork* __restrict__ bands, int n_bands, const int2* __restrict__ band_kb,
     const GatherWork* __restrict__ fall, int8_t* __restrict__ slab,
     const int* __restrict__ route) {
@@ -429,10 +430,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     __shared__ int shift[BAND_STAGE];
     if (route && route[0] != NARROW_OFF) return;
     if ((int)blockIdx.x >= n_bands) {  // a k-block run the bands do not cover
-        const int t0 = blockIdx.y * BAND_FRAMES;
+        const int t0 = blockIdx.y * bf;
         gather_general<uint8_t, BIAS>(frames, hw, nframes, nrows, pix_idx, bins,
                                       fall[blockIdx.x - n_bands], t0,
-                                      min(nframes, t0 + BAND_FRAMES), slab);
+                                      min(nframes, t0 + bf), slab);
         return;
     }
     const BandWork bw = bands[blockIdx.x];
@@ -467,8 +468,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
     }
 
-    const int tb = blockIdx.y * BAND_FRAMES;
-    const int te = min(nframes, tb + BAND_FRAMES);
+    const int tb = blockIdx.y * bf;
+    const int te = min(nframes, tb + bf);
     for (int t0 = tb; t0 < te; t0 += BAND_STAGE) {
         stage_band(frames, hw, nframes, t0, band0, span, srow, stage, shift, wave, lane);
         const int t = t0 + i;
@@ -589,15 +590,15 @@ __device__ __forceinline__ void gather_general_f4(const uint8_t* __restrict__ fr
 template <bool SGN>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gather_band_f4_kernel(
     const uint8_t* __restrict__ frames, int64_t hw, int width, int nframes, int nrows, int srow,
-    const int32_t* __restrict__ pix_idx, const BinDev* __restrict__ bins,
+    int bf, const int32_t* __restrict__ pix_idx, const BinDev* __restrict__ bins,
     const BandWork* __restrict__ bands, int n_bands, const int2* __restrict__ band_kb,
     const GatherWork* __restrict__ fall, int8_t* __restrict__ slab4, uint8_t* __restrict__ flag,
     const int* __restrict__ route) {
     extern __shared__ __attribute__((aligned(16))) uint8_t stage[];  // BAND_STAGE x srow
     __shared__ int shift[BAND_STAGE];
     if (route[0] != NARROW_F4) return;
-    const int tb = blockIdx.y * BAND_FRAMES;
-    const int te = min(nframes, tb + BAND_FRAMES);
+    const int tb = blockIdx.y * bf;
+    const int te = min(nframes, tb + bf);
     if ((int)blockIdx.x >= n_bands) {  // a k-block run the bands do not cover
         gather_general_f4<SGN>(frames, hw, nframes, nrows, pix_idx, bins,
                                fall[blockIdx.x - n_bands], tb, te, slab4, flag);
@@ -678,40 +679,40 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 }
 
 void launch_gather_band_f4(const uint8_t* frames, int dtype, int64_t hw, int width, int nframes,
-                           int nrows, int srow, const int32_t* pix_idx, const BinDev* bins,
+                           int nrows, int srow, int bf, const int32_t* pix_idx, const BinDev* bins,
                            const BandWork* bands, int n_bands, const int2* band_kb,
                            const GatherWork* fall, int n_fall, int8_t* slab4, uint8_t* flag,
                            const int* route, hipStream_t s) {
     if (n_bands + n_fall <= 0 || nframes <= 0) return;
     const dim3 grid((unsigned)(n_bands + n_fall),
-                    (unsigned)((nframes + BAND_FRAMES - 1) / BAND_FRAMES));
+                    (unsigned)((nframes + bf - 1) / bf));
     const size_t lds = (size_t)BAND_STAGE * srow;
     if (dtype == DXG2_U8)
         gather_band_f4_kernel<false><<<grid, dim3(256), lds, s>>>(
-            frames, hw, width, nframes, nrows, srow, pix_idx, bins, bands, n_bands, band_kb, fall,
+            frames, hw, width, nframes, nrows, srow, bf, pix_idx, bins, bands, n_bands, band_kb, fall,
             slab4, flag, route);
     else
         gather_band_f4_kernel<true><<<grid, dim3(256), lds, s>>>(
-            frames, hw, width, nframes, nrows, srow, pix_idx, bins, bands, n_bands, band_kb, fall,
+            frames, hw, width, nframes, nrows, srow, bf, pix_idx, bins, bands, n_bands, band_kb, fall,
             slab4, flag, route);
 }
 
 void launch_gather_band(const uint8_t* frames, int dtype, int64_t hw, int width, int nframes,
-                        int nrows, int srow, const int32_t* pix_idx, const BinDev* bins,
+                        int nrows, int srow, int bf, const int32_t* pix_idx, const BinDev* bins,
                         const BandWork* bands, int n_bands, const int2* band_kb,
                         const GatherWork* fall, int n_fall, int8_t* slab, hipStream_t s,
                         const int* route) {
     if (n_bands + n_fall <= 0 || nframes <= 0) return;
     const dim3 grid((unsigned)(n_bands + n_fall),
-                    (unsigned)((nframes + BAND_FRAMES - 1) / BAND_FRAMES));
+                    (unsigned)((nframes + bf - 1) / bf));
     const size_t lds = (size_t)BAND_STAGE * srow;
     if (dtype == DXG2_U8)
         gather_band_kernel<true><<<grid, dim3(256), lds, s>>>(frames, hw, width, nframes, nrows,
-                                                              srow, pix_idx, bins, bands, n_bands,
+                                                              srow, bf, pix_idx, bins, bands, n_bands,
                                                               band_kb, fall, slab, route);
     else
         gather_band_kernel<false><<<grid, dim3(256), lds, s>>>(frames, hw, width, nframes, nrows,
-                                                               srow, pix_idx, bins, bands, n_bands,
+                                                               srow, bf, pix_idx, bins, bands, n_bands,
                                                                band_kb, fall, slab, route);
 }
 

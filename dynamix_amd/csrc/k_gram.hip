@@ -625,13 +625,29 @@ __device__ __forceinline__ int xcc_id() {
 // (once that is drained) the other XCDs' queues in turn.  Queue x holds items
 // [qoff[x], qoff[x+1]) of the work list; heads[x] counts the items taken from it.
 __device__ __forceinline__ int next_item(int home, const int* __restrict__ qoff, int* heads) {
-    for (int k = 0; k < 8; ++k) {
-        const int x = (home + k) & 7;
+    auto pop = [&](int x) {
         const int n = qoff[x + 1] - qoff[x];
-        if (__hip_atomic_load(heads + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= n)
-            continue;
         const int i = atomicAdd(heads + x, 1);
-        if (i < n) return qoff[x] + i;
+        return i < n ? qoff[x] + i : -1;
+    };
+    const int n0 = qoff[home + 1] - qoff[home];
+    if (__hip_atomic_load(heads + home, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < n0) {
+        const int i = pop(home);
+        if (i >= 0) return i;
+    }
+    // the other heads are read together: one after the other, the last look at the drained
+    // queues alone was several microseconds of every launch
+    int seen[8];
+#pragma unroll
+    for (int k = 1; k < 8; ++k)
+        seen[k] = __hip_atomic_load(heads + ((home + k) & 7), __ATOMIC_RELAXED,
+                                    __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+    for (int k = 1; k < 8; ++k) {
+        const int x = (home + k) & 7;
+        if (seen[k] >= qoff[x + 1] - qoff[x]) continue;
+        const int i = pop(x);
+        if (i >= 0) return i;
     }
     return -1;
 }
@@ -651,7 +667,7 @@ __global__ __launch_bounds__(256) void gram_i8_queue_kernel(
     DXG2_GRAM_LDS(WM);
     __shared__ int s_item;
     if (wsums && nwkb[n_bins] == 0) return;  // no wide pixel in any bin
-    const int home = xcc_id();
+    const int home = xcc_id() & 7;
     for (;;) {
         if (threadIdx.x == 0) s_item = next_item(home, qoff, heads);
         __syncthreads();
@@ -680,7 +696,7 @@ __global__ __launch_bounds__(256) void gram_f4_queue_kernel(
     DXG2_GRAM_LDS(4);
     __shared__ int s_item;
     if (route[0] != NARROW_F4) return;
-    const int home = xcc_id();
+    const int home = xcc_id() & 7;
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     for (;;) {

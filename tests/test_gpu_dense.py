@@ -343,3 +343,22 @@ def test_device_speckle_generator_statistics():
         assert abs(g2[tau] - (1 + np.exp(-2 * tau / 20.0))) < 0.08, (tau, g2[tau])
     ref = og.dense_g2(f.cpu().numpy(), None)
     np.testing.assert_array_equal(c.last_numerators.cpu().numpy(), ref["num"])
+
+
+@pytest.mark.parametrize("shape,n,nbins,dtype", [
+    ((7, 9), 1, 1, np.uint8), ((96, 96), 129, 5, np.uint8), ((64, 200), 257, 2, np.int8),
+    ((40, 41), 1031, 3, np.uint16), ((3, 700), 40, 1, np.uint8)])
+def test_few_tiles_split_into_short_items(shape, n, nbins, dtype):
+    """Calls too small for the chip: short k-ranges, few frames and k-blocks a workgroup."""
+    from dynamix_amd.correlator.dense import MatMulCorrelator
+    rng = np.random.default_rng(n)
+    f = rng.poisson(1.0, size=(n,) + shape).astype(dtype)
+    if dtype == np.uint16:
+        f[:, 1, 1] += 700
+    yy, xx = np.indices(shape)
+    q = ((yy + 2 * xx) * nbins // (shape[0] + 2 * shape[1]) + 1).astype(np.int32)
+    c = MatMulCorrelator(shape, n, q)
+    c.correlate(f)
+    ref = og.dense_g2(f, q)
+    assert np.array_equal(c.last_numerators.cpu().numpy(), ref["num"])
+    assert np.array_equal(c.last_sums.cpu().numpy(), ref["sums"])
