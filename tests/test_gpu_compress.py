@@ -93,3 +93,39 @@ def test_streaming_overflow_raises():
         fc.process_frame(x)
     with pytest.raises(IndexError):
         fc.get_compacted_events()
+
+
+@pytest.mark.parametrize("shape,n,dtype,density", [
+    ((363, 365), 70, np.uint8, 0.05),    # odd frame size, last word and tile partial
+    ((364, 364), 129, np.int8, 0.05),    # aligned
+    ((257, 259), 131, np.uint16, 0.05),  # odd number of 2-byte samples
+    ((363, 365), 300, np.uint8, 0.3),    # runs past the LDS
+    ((256, 258), 150, np.uint16, 0.9),
+])
+def test_compress_large_detectors(shape, n, dtype, density):
+    """Detectors of 512 tiles and more, whose runs are assembled in LDS, against the oracle;
+    the stack at an odd byte too."""
+    import torch
+    from dynamix_amd.correlator.event import FramesCompressor
+    _announce("compress tiles %s n=%d %s" % (shape, n, np.dtype(dtype).name))
+    rng = np.random.default_rng(n)
+    f = (rng.random((n,) + shape) < density) * rng.integers(1, 100, size=(n,) + shape)
+    f = (f * (rng.integers(0, 2, size=f.shape) * 2 - 1) if dtype == np.int8 else f).astype(dtype)
+    f.flat[-1] = 7
+    ref = ev.compress_all_stack(f)
+    for a, b in zip(FramesCompressor.compress_all_stack(f), ref):
+        np.testing.assert_array_equal(a, b)
+    if dtype == np.uint8:
+        flat = torch.zeros(f.size + 1, dtype=torch.uint8, device="cuda")
+        flat[1:] = torch.from_numpy(f).cuda().flatten()
+        for a, b in zip(FramesCompressor.compress_all_stack(flat[1:].view(f.shape)), ref):
+            np.testing.assert_array_equal(a.cpu().numpy().astype(b.dtype), b)
+
+
+@pytest.mark.parametrize("shape,dtype", [((1, 1), np.uint8), ((1, 3), np.int8), ((1, 1), np.uint16),
+                                         ((1, 2), np.uint16), ((5, 1), np.uint8)])
+def test_compress_frames_of_a_word_and_less(shape, dtype):
+    from dynamix_amd.correlator.event import FramesCompressor
+    f = np.random.default_rng(3).integers(0, 3, size=(300,) + shape).astype(dtype)
+    for a, b in zip(FramesCompressor.compress_all_stack(f), ev.compress_all_stack(f)):
+        np.testing.assert_array_equal(a, b)
