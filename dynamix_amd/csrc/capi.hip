@@ -858,7 +858,7 @@ void build_event_work(dxg2_plan* p) {
     const int64_t want_items = std::max<int64_t>(1, (512 + windows - 1) / windows);
     int item = EVENT_ITEM_PIXELS;
     while (item < 8 * EVENT_ITEM_PIXELS && total / (2 * item) >= want_items) item *= 2;
-    item = std::max(64, env_int("DXG2_EVENT_ITEM_PIXELS", item));
+    item = std::min(EVENT_ITEM_MAX, std::max(64, env_int("DXG2_EVENT_ITEM_PIXELS", item)));
     for (int b = 0; b < p->n_bins; ++b)
         for (int k0 = 0; k0 < p->bins[b].npix; k0 += item)
             p->event_work.push_back(

@@ -133,6 +133,8 @@ struct EventWork {       // one workgroup of the event pair kernel (x dimension)
     int32_t pad;         // job of a grouped launch (0 otherwise)
 };
 
+constexpr int EVENT_ITEM_MAX = 1 << 15;  // most pixels of one event work item
+
 struct EventJob {        // one job of a grouped event launch
     const int32_t* times;
     const void* data;

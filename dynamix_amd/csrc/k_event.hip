@@ -13,7 +13,8 @@
 //    partner j > i whose lag t_j - t_i reaches the window, and the pairs up to the
 //    window's end go to an LDS lag histogram (EvHist below), flushed once per work
 //    item with one global 64-bit atomic per non-zero lag;
-//  * S_b(t) and the self pairs (lag 0, d_i^2) are added in the first window;
+//  * the self pairs (lag 0, d_i^2) are added in the first window; S_b(t) comes from a launch of
+//    its own (event_sums_item);
 //  * the input is validated on the device (frames in [0, N), strictly increasing per
 //    pixel, as compress_all_stack produces, event.py:267-284); a violation sets a
 //    flag the host turns into an error instead of reading out of bounds.
@@ -90,7 +91,7 @@ __device__ __forceinline__ void event_pairs_item(
     const int32_t* __restrict__ times, const T* __restrict__ data,
     const uint32_t* __restrict__ offsets, const int32_t* __restrict__ pix_idx,
     const BinDev* __restrict__ bins, const EventWork w, int nframes, int64_t nnz,
-    int64_t* __restrict__ num, int64_t* __restrict__ sums, int* __restrict__ err,
+    int64_t* __restrict__ num, int* __restrict__ err,
     typename EvHist<T>::type* __restrict__ hist, int (*__restrict__ st)[NW][ECAP]) {
     int (*const st_t)[ECAP] = st[0];
     int (*const st_d)[ECAP] = st[1];
@@ -107,7 +108,6 @@ __device__ __forceinline__ void event_pairs_item(
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     for (int k = threadIdx.x; k < EW; k += NT) hist[k] = 0;
     __syncthreads();
-    int64_t* srow = sums + (int64_t)w.bin * nframes;
     unsigned long long* nwin = reinterpret_cast<unsigned long long*>(num + (int64_t)w.bin * nframes + w0);
     long long used = 0;  // this wave's sum of d^2 added to the histogram (BOUNDED)
 
@@ -203,8 +203,7 @@ __device__ __forceinline__ void event_pairs_item(
                 if constexpr (S) return (C)st_d[wave][k];
                 else return (C)as_count<T>(data[beg + k]);
             };
-            // Validation, in the first lag window (the one that also writes the frame
-            // sums): frames in [0, N) and strictly increasing.  An invalid pixel is
+            // Validation, in the first lag window: frames in [0, N) and strictly increasing.  An invalid pixel is
             // skipped there and flagged, and the call reports the error; the other
             // windows do not repeat the check, and their lag test below keeps every
             // write inside the window whatever the input.
@@ -324,14 +323,6 @@ __device__ __forceinline__ void event_pairs_item(
                 const int ti1 = has1 ? time_of(i1) : 0;
                 const C d0 = count_of(i0);
                 const C d1 = has1 ? count_of(i1) : (C)0;
-                if (w0 == 0) {
-                    if (d0 != 0)
-                        atomicAdd(reinterpret_cast<unsigned long long*>(srow + ti0),
-                                  (unsigned long long)(long long)d0);
-                    if (d1 != 0)
-                        atomicAdd(reinterpret_cast<unsigned long long*>(srow + ti1),
-                                  (unsigned long long)(long long)d1);
-                }
                 // first partner: i + 1 in the first window (times strictly increase),
                 // else one past the last p >= i with t_p < t_i + w0, by a descent over
                 // power-of-two steps (a monotone test; reads clamped inside the list)
@@ -373,11 +364,11 @@ __global__ __launch_bounds__(64 * NW) void event_pairs_kernel(
     const int32_t* __restrict__ times, const T* __restrict__ data,
     const uint32_t* __restrict__ offsets, const int32_t* __restrict__ pix_idx,
     const BinDev* __restrict__ bins, const EventWork* __restrict__ work, int nframes,
-    int64_t nnz, int64_t* __restrict__ num, int64_t* __restrict__ sums, int* __restrict__ err) {
+    int64_t nnz, int64_t* __restrict__ num, int* __restrict__ err) {
     __shared__ typename EvHist<T>::type hist[EvHist<T>::lags_per_wave * NW];
     __shared__ __attribute__((aligned(16))) int st[2][NW][ECAP];
     event_pairs_item<T, NW>(times, data, offsets, pix_idx, bins, work[blockIdx.x], nframes, nnz,
-                            num, sums, err, hist, st);
+                            num, err, hist, st);
 }
 
 // A pointer read from a job table, marked as global memory (a generic pointer would
@@ -400,9 +391,105 @@ __global__ __launch_bounds__(64 * NW) void event_pairs_jobs_kernel(
     const EventJob j = jobs[w.pad];
     event_pairs_item<T, NW>(global_ptr(j.times), global_ptr(reinterpret_cast<const T*>(j.data)),
                             global_ptr(j.offsets), global_ptr(j.pix), global_ptr(j.bins), w,
-                            j.nframes, j.nnz, global_ptr(j.num), global_ptr(j.sums),
-                            global_ptr(j.err), hist, st);
+                            j.nframes, j.nnz, global_ptr(j.num), global_ptr(j.err), hist, st);
 }
+
+// Frame sums S_b(t) of a work item's pixels (densecorrelator.cl:65-150 has them dense,
+// evtcorrelator.cl:40 adds each event to global memory), in LDS counters of the frames [t0, t0 +
+// window) and from there to `sums`.  One 64-bit global atomic an event, as the pair kernel had
+// them, held a call at 17-23e9 events/s whatever its pairs.  A wave loads the ranges of 64
+// pixels and streams each stretch of them that is one run of the event list (neighbours in a
+// row are).  32-bit counters: an item has at most EVENT_ITEM_MAX pixels, each with one event a
+// frame.  Ranges and frames that the pair kernel reports as invalid are left out.
+constexpr int SUMS_WINDOW = 40000;  // frames: 160,000 bytes
+template <typename T>
+__device__ __forceinline__ void event_sums_item(const int32_t* __restrict__ times,
+                                                const T* __restrict__ data,
+                                                const uint32_t* __restrict__ offsets,
+                                                const int32_t* __restrict__ pix_idx,
+                                                const BinDev* __restrict__ bins, const EventWork w,
+                                                int nframes, int64_t nnz, int window,
+                                                int64_t* __restrict__ sums, uint32_t* hist) {
+    const int t0 = blockIdx.y * window;
+    if (t0 >= nframes) return;
+    const unsigned len = (unsigned)min(window, nframes - t0);
+    for (unsigned i = threadIdx.x; i < len; i += blockDim.x) hist[i] = 0u;
+    __syncthreads();
+    const int lane = threadIdx.x & 63;
+    const int32_t* list = pix_idx + bins[w.bin].idx_off;
+    const int step = (int)blockDim.x;
+    for (int r = w.k0 + (int)(threadIdx.x - lane); r < w.k1; r += step) {
+        const int p = r + lane < w.k1 ? list[r + lane] : -1;
+        uint32_t b = 0u, e = 0u;
+        if (p >= 0) {
+            b = offsets[p];
+            e = offsets[p + 1];
+            if (e < b || (int64_t)e > nnz) e = b = 0u;
+        }
+        const uint32_t before = (uint32_t)__shfl_up((int)e, 1);
+        uint64_t runs = __ballot(lane == 0 || b != before);
+        while (runs) {
+            const int first = __builtin_ctzll(runs);
+            runs &= runs - 1;
+            const int last = (runs ? __builtin_ctzll(runs) : 64) - 1;
+            const uint32_t x1 = (uint32_t)__builtin_amdgcn_readlane((int)e, last);
+            for (uint32_t x = (uint32_t)__builtin_amdgcn_readlane((int)b, first) + lane;
+                 x - lane < x1; x += 512) {
+                int t[8], d[8];
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    const bool in = x + 64 * q < x1 && x + 64 * q >= x;
+                    t[q] = in ? times[x + 64 * q] : -1;
+                    d[q] = in ? (int)data[x + 64 * q] : 0;
+                }
+#pragma unroll
+                for (int q = 0; q < 8; ++q)
+                    if ((unsigned)(t[q] - t0) < len && t[q] >= 0)
+                        atomicAdd(&hist[t[q] - t0], (uint32_t)d[q]);
+                if (x1 - (x - lane) <= 512u) break;  // (no wrap at 2^32)
+            }
+        }
+    }
+    __syncthreads();
+    int64_t* row = sums + (int64_t)w.bin * nframes + t0;
+    for (unsigned i = threadIdx.x; i < len; i += blockDim.x) {
+        const uint32_t v = hist[i];
+        if (v)
+            atomicAdd(reinterpret_cast<unsigned long long*>(row + i),
+                      std::is_signed<T>::value ? (unsigned long long)(long long)(int32_t)v
+                                               : (unsigned long long)v);
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(1024) void event_sums_kernel(
+    const int32_t* __restrict__ times, const T* __restrict__ data,
+    const uint32_t* __restrict__ offsets, const int32_t* __restrict__ pix_idx,
+    const BinDev* __restrict__ bins, const EventWork* __restrict__ work, int nframes, int64_t nnz,
+    int window, int64_t* __restrict__ sums) {
+    extern __shared__ uint32_t sums_hist[];
+    event_sums_item<T>(times, data, offsets, pix_idx, bins, work[blockIdx.x], nframes, nnz, window,
+                       sums, sums_hist);
+}
+template <typename T>
+__global__ __launch_bounds__(1024) void event_sums_jobs_kernel(const EventJob* __restrict__ jobs,
+                                                               const EventWork* __restrict__ work,
+                                                               int window) {
+    extern __shared__ uint32_t sums_hist[];
+    const EventWork w = work[blockIdx.x];
+    if (w.bin < 0) return;
+    const EventJob j = jobs[w.pad];
+    event_sums_item<T>(global_ptr(j.times), global_ptr(reinterpret_cast<const T*>(j.data)),
+                       global_ptr(j.offsets), global_ptr(j.pix), global_ptr(j.bins), w, j.nframes,
+                       j.nnz, window, global_ptr(j.sums), sums_hist);
+}
+// Frames per window: as even as SUMS_WINDOW allows.
+static int sums_window(int nframes) {
+    const int n = (nframes + SUMS_WINDOW - 1) / SUMS_WINDOW;
+    return (nframes + n - 1) / n;
+}
+// Threads: two workgroups share a CU's threads where their counters leave room for it.
+static int sums_threads(int window) { return window > SUMS_WINDOW / 2 ? 1024 : 512; }
 
 // Waves per workgroup of the pair kernels: 16 (one workgroup per CU, 32,768 counters and
 // windows of 32,704 lags for 8-bit counts: the fewest windows, so the least per-window
@@ -428,6 +515,9 @@ template <typename T, int NW>
 void pairs_jobs_launch(const EventJob* jobs, const EventWork* work, int n_work, int max_frames,
                        hipStream_t s) {
     constexpr int WS = EvHist<T>::window(NW);
+    const int win = sums_window(max_frames);
+    event_sums_jobs_kernel<T><<<dim3((unsigned)n_work, (unsigned)((max_frames + win - 1) / win)),
+                                sums_threads(win), 4 * win, s>>>(jobs, work, win);
     event_pairs_jobs_kernel<T, NW><<<dim3((unsigned)n_work, (unsigned)((max_frames + WS - 1) / WS)),
                                      64 * NW, 0, s>>>(jobs, work);
 }
@@ -459,9 +549,13 @@ void pairs_launch(const int32_t* times, const void* data, const uint32_t* offset
                   const int32_t* pix_idx, const BinDev* bins, const EventWork* work, int n_work,
                   int nframes, int64_t nnz, int64_t* num, int64_t* sums, int* err, hipStream_t s) {
     constexpr int WS = EvHist<T>::window(NW);
+    const int win = sums_window(nframes);
+    event_sums_kernel<T><<<dim3((unsigned)n_work, (unsigned)((nframes + win - 1) / win)),
+                           sums_threads(win), 4 * win, s>>>(times, (const T*)data, offsets, pix_idx,
+                                                            bins, work, nframes, nnz, win, sums);
     event_pairs_kernel<T, NW><<<dim3((unsigned)n_work, (unsigned)((nframes + WS - 1) / WS)),
                                 64 * NW, 0, s>>>(times, (const T*)data, offsets, pix_idx, bins,
-                                                 work, nframes, nnz, num, sums, err);
+                                                 work, nframes, nnz, num, err);
 }
 
 template <typename T>
