@@ -716,9 +716,6 @@ int next_events(dxg2_plan* p, hipEvent_t** out) {
     return DXG2_OK;
 }
 
-// Pixels of one bin's list handled by one event work item.
-constexpr int EVENT_ITEM_PIXELS = 1024;
-
 // Bytes of the FFT path's series: L elements per entry of the (padded) pixel lists.
 size_t fft_series_bytes(const dxg2_plan* p, int L) {
     const size_t size = p->dtype == DXG2_U16 ? 2 : 1;
@@ -847,17 +844,18 @@ int ensure_fft_buffers(dxg2_plan* p, hipStream_t s) {
     return DXG2_OK;
 }
 
-// Larger items flush fewer lag histograms and repeat less per-item work; the size is
-// the largest power of two from EVENT_ITEM_PIXELS up to 8 times that for which the
-// items still give about 512 workgroups over the series' lag windows (two per CU).
-// DXG2_EVENT_ITEM_PIXELS fixes it instead.
+// Work items of the event launches (DXG2_EVENT_ITEM_PIXELS: pixels an item).
 void build_event_work(dxg2_plan* p) {
     int64_t total = 0;
     for (const auto& n : p->npix) total += n;
-    const int windows = (p->N + event_lag_window(p->dtype) - 1) / event_lag_window(p->dtype);
-    const int64_t want_items = std::max<int64_t>(1, (512 + windows - 1) / windows);
-    int item = EVENT_ITEM_PIXELS;
-    while (item < 8 * EVENT_ITEM_PIXELS && total / (2 * item) >= want_items) item *= 2;
+    // At most 1,024 items where their counters are few (two workgroups a CU, twice), else 384
+    // a lag window, and at most 8,192 pixels each: an item clears and flushes as many counters
+    // whatever it holds.  514 x 1030 x 20,000: 0.75 ms a call with 940 items, 0.63 with 240 to
+    // 470; 1030 x 1065 x 100,000, 4 windows: 5.7, 5.5, 5.6 ms with 1,072, 360, 260 a window;
+    // x 2,000: 1.56 ms with 1,024, 1.66 with 540.
+    const int lags = std::min(event_lag_window(p->dtype, p->N), p->N);
+    const int64_t items = lags <= 8192 ? 1024 : 384;
+    int item = (int)std::min<int64_t>(8192, (total / items + 63) / 64 * 64);
     item = std::min(EVENT_ITEM_MAX, std::max(64, env_int("DXG2_EVENT_ITEM_PIXELS", item)));
     for (int b = 0; b < p->n_bins; ++b)
         for (int k0 = 0; k0 < p->bins[b].npix; k0 += item)

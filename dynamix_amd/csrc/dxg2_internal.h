@@ -253,7 +253,7 @@ void launch_plain_bin(const uint8_t* frames, int dtype, int64_t hw, int nframes,
                       const int32_t* pix, int npix, float* a, float* gram, float* means,
                       float* g2_row, hipStream_t s);
 // Lags per workgroup of the event pair kernel (its lag window) for a count type.
-int event_lag_window(int dtype);
+int event_lag_window(int dtype, int nframes);
 void launch_event_pairs_jobs(int dtype, const EventJob* jobs, const EventWork* work, int n_work,
                              int max_frames, hipStream_t s);
 void launch_event_pairs(int dtype, const int32_t* times, const void* data,

@@ -6,13 +6,15 @@
 // res[bin][t_i - t_j] += d_i d_j, plus sums[bin][t_i] += d_i.
 //
 // Here:
-//  * work items are (bin, range of the bin's pixel list) x (lag window);
-//    a wave takes one pixel at a time (the next pixel's events load into registers
-//    meanwhile), stages its events in LDS, and each lane takes
-//    events i = lane + 128 r and i + 64 together; a binary search finds the first
-//    partner j > i whose lag t_j - t_i reaches the window, and the pairs up to the
-//    window's end go to an LDS lag histogram (EvHist below), flushed once per work
-//    item with one global 64-bit atomic per non-zero lag;
+//  * work items are (bin, range of the bin's pixel list) x (lag window), and pairs go to an LDS
+//    lag histogram (EvHist below) flushed once per work item with one global 64-bit atomic per
+//    non-zero lag;
+//  * 8-bit counts: a wave stages the events of several pixels in LDS and a lane takes an event
+//    (event_flat_item);
+//  * 16-bit counts and the longest series: a wave takes one pixel at a time (the next pixel's
+//    events load into registers meanwhile), stages its events in LDS, and each lane takes
+//    events i = lane + 128 r and i + 64 together; a binary search finds the first partner j > i
+//    whose lag t_j - t_i reaches the window (event_pairs_item);
 //  * the self pairs (lag 0, d_i^2) are added in the first window; S_b(t) comes from a launch of
 //    its own (event_sums_item);
 //  * the input is validated on the device (frames in [0, N), strictly increasing per
@@ -24,6 +26,8 @@
 // index needs), so each pixel's events keep the input's frame order; the offsets are
 // the lower bounds of every pixel in the sorted keys, and the packed words are split
 // into times and counts.
+#include <algorithm>
+
 #include "dxg2_internal.h"
 
 namespace dxg2 {
@@ -82,6 +86,135 @@ struct EvPixel {
     int n;  // events to correlate: 0 for an empty, unbinned or invalid range
 };
 
+// One pixel's pairs by a wave, lags [w0, w1), its n > 0 events at `beg`: staged by the wave (S; pt,
+// pd: frames and counts, sq: this lane's share of the sum of d^2) or read from memory.  used: see
+// EvHist.
+template <typename T, int NW, bool S>
+__device__ __forceinline__ void event_pixel(const int32_t* __restrict__ times,
+                                            const T* __restrict__ data, uint32_t beg, int n,
+                                            int lane, int w0, int w1, int nframes, const int* pt,
+                                            const int* pd,
+                                            typename EvHist<T>::type* __restrict__ hist,
+                                            unsigned long long* __restrict__ nwin, long long& used,
+                                            long long sq, int* __restrict__ err) {
+    using H = typename EvHist<T>::type;
+    constexpr bool BOUNDED = sizeof(H) == 4;
+    auto time_of = [&](int k) -> int {
+        if constexpr (S) return pt[k];
+        else return times[beg + k];
+    };
+    // 8-bit counts multiply in 32 bits (|d_i d_j| <= 255^2), 16-bit in 64
+    using C = typename std::conditional<sizeof(T) == 1, int, long long>::type;
+    auto count_of = [&](int k) -> C {
+        if constexpr (S) return (C)pd[k];
+        else return (C)as_count<T>(data[beg + k]);
+    };
+    // Validation, in the first lag window: frames in [0, N) and strictly increasing.  An invalid pixel is
+    // skipped there and flagged, and the call reports the error; the other
+    // windows do not repeat the check, and their lag test below keeps every
+    // write inside the window whatever the input.
+    if (w0 == 0) {
+        int bad = 0;
+        for (int k = lane; k < n; k += 64) {
+            const int t = time_of(k);
+            if (t < 0 || t >= nframes) bad = 1;
+            if (k + 1 < n && time_of(k + 1) <= t) bad = 1;
+        }
+        if (bad) atomicOr(err, 1);
+        if (__any(bad)) return;
+    }
+    long long sq_lane = sq;
+    if constexpr (!S)
+        for (int k = lane; k < n; k += 64) {
+            const long long d = count_of(k);
+            sq_lane += d * d;
+        }
+    const long long sqw = wave_sum64(sq_lane);  // sum of d^2: the lag-0 term
+    bool to_lds = true;
+    if constexpr (BOUNDED) {
+        to_lds = used + sqw < EvHist<T>::budget(NW);
+        if (to_lds) used += sqw;
+    }
+    if (w0 == 0 && lane == 0 && sqw != 0) {  // lag 0
+        if (to_lds)
+            atomicAdd(&hist[0], (H)sqw);
+        else
+            atomicAdd(nwin, (unsigned long long)sqw);
+    }
+    const unsigned span = (unsigned)(w1 - w0);
+    // the rest in one of two instantiations: LDS counters, or (past the budget)
+    // the global 64-bit numerators, so the pair loop carries no branch on it
+    auto events = [&](auto lds_tag) {
+    constexpr bool LDS = decltype(lds_tag)::value;
+    auto add = [&](int lag, C prod) {  // lag in [0, w1 - w0)
+        if constexpr (LDS)
+            atomicAdd(&hist[lag], (H)prod);
+        else
+            atomicAdd(nwin + lag, (unsigned long long)(long long)prod);
+    };
+    // pairs (i, j), j > i, with lag t_j - t_i in [max(w0, 1), w1): partners from
+    // the first j with t_j >= t_i + max(w0, 1) while t_j < t_i + w1, four per
+    // step so that their reads and atomics overlap.  The lag test is one unsigned
+    // compare, which also rejects a negative lag.
+    auto partners = [&](int ti, C di, int j) {
+        const int base = ti + w0;
+        for (; j < n; j += 4) {
+            int tj[4];
+            C dj[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const bool in = j + u < n;
+                const int jj = in ? j + u : n - 1;
+                const int t = time_of(jj);
+                const C d = count_of(jj);
+                tj[u] = in ? t : base + (int)span;
+                dj[u] = in ? d : (C)0;
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const unsigned lag = (unsigned)(tj[u] - base);
+                const C prod = di * dj[u];
+                if (lag < span && prod != 0) add((int)lag, prod);
+            }
+            if (tj[3] - base >= (int)span) break;  // times increase: the rest are later
+        }
+    };
+    // wave-uniform steps of the first-partner search: powers of two from the
+    // largest not above n
+    const int top = 1 << (31 - __builtin_clz(n));
+    // Each lane takes events i and i + 64 together, so that their two searches
+    // for the first partner overlap.
+    for (int i0 = lane; i0 < n; i0 += 128) {
+        const int i1 = i0 + 64;
+        const bool has1 = i1 < n;
+        const int ti0 = time_of(i0);
+        const int ti1 = has1 ? time_of(i1) : 0;
+        const C d0 = count_of(i0);
+        const C d1 = has1 ? count_of(i1) : (C)0;
+        // first partner: i + 1 in the first window (times strictly increase),
+        // else one past the last p >= i with t_p < t_i + w0, by a descent over
+        // power-of-two steps (a monotone test; reads clamped inside the list)
+        int p0 = i0, p1 = has1 ? i1 : n - 1;
+        if (w0 > 0) {
+            const int g0 = ti0 + w0, g1 = ti1 + w0;
+            for (int step = top; step > 0; step >>= 1) {
+                const int q0 = p0 + step, q1 = p1 + step;
+                const int t0 = time_of(min(q0, n - 1));
+                const int t1 = time_of(min(q1, n - 1));
+                if (q0 < n && t0 < g0) p0 = q0;
+                if (q1 < n && t1 < g1) p1 = q1;
+            }
+        }
+        partners(ti0, d0, p0 + 1);
+        if (has1) partners(ti1, d1, p1 + 1);
+    }
+    };
+    if (to_lds)
+        events(std::true_type{});
+    else
+        events(std::false_type{});
+}
+
 // The pairs of one work item (a run of one bin's pixels) in lag window blockIdx.y, with
 // the workgroup's LDS: the lag histogram and each wave's staged events (uint8, int8 and
 // uint16 counts fit 32 bits), times and counts in one array st[2][NW][ECAP] so that the
@@ -99,7 +232,6 @@ __device__ __forceinline__ void event_pairs_item(
     constexpr int EW = EvHist<T>::lags_per_wave * NW;  // counters
     constexpr int WS = EvHist<T>::window(NW);          // lags of a window
     constexpr int NT = 64 * NW;
-    constexpr bool BOUNDED = sizeof(H) == 4;
     const BinDev bd = bins[w.bin];
     const int w0 = blockIdx.y * WS;
     if (w0 >= nframes) return;
@@ -189,167 +321,12 @@ __device__ __forceinline__ void event_pairs_item(
         if (n == 0) continue;
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): staged values visible to the wave
         __builtin_amdgcn_wave_barrier();
-        // The pixel's pairs, with its events read from LDS (staged) or from HBM; the two
-        // are separate instantiations so that each reads through its own address space.
-        auto pixel = [&](auto staged_tag) {
-            constexpr bool S = decltype(staged_tag)::value;
-            auto time_of = [&](int k) -> int {
-                if constexpr (S) return st_t[wave][k];
-                else return times[beg + k];
-            };
-            // 8-bit counts multiply in 32 bits (|d_i d_j| <= 255^2), 16-bit in 64
-            using C = typename std::conditional<sizeof(T) == 1, int, long long>::type;
-            auto count_of = [&](int k) -> C {
-                if constexpr (S) return (C)st_d[wave][k];
-                else return (C)as_count<T>(data[beg + k]);
-            };
-            // Validation, in the first lag window: frames in [0, N) and strictly increasing.  An invalid pixel is
-            // skipped there and flagged, and the call reports the error; the other
-            // windows do not repeat the check, and their lag test below keeps every
-            // write inside the window whatever the input.
-            if (w0 == 0) {
-                int bad = 0;
-                for (int k = lane; k < n; k += 64) {
-                    const int t = time_of(k);
-                    if (t < 0 || t >= nframes) bad = 1;
-                    if (k + 1 < n && time_of(k + 1) <= t) bad = 1;
-                }
-                if (bad) atomicOr(err, 1);
-                if (__any(bad)) return;
-            }
-            long long sq_lane = sq;
-            if constexpr (!S)
-                for (int k = lane; k < n; k += 64) {
-                    const long long d = count_of(k);
-                    sq_lane += d * d;
-                }
-            const long long sqw = wave_sum64(sq_lane);  // sum of d^2: the lag-0 term
-            bool to_lds = true;
-            if constexpr (BOUNDED) {
-                to_lds = used + sqw < EvHist<T>::budget(NW);
-                if (to_lds) used += sqw;
-            }
-            if (w0 == 0 && lane == 0 && sqw != 0) {  // lag 0
-                if (to_lds)
-                    atomicAdd(&hist[0], (H)sqw);
-                else
-                    atomicAdd(nwin, (unsigned long long)sqw);
-            }
-            const unsigned span = (unsigned)(w1 - w0);
-            // the rest in one of two instantiations: LDS counters, or (past the budget)
-            // the global 64-bit numerators, so the pair loop carries no branch on it
-            auto events = [&](auto lds_tag) {
-            constexpr bool LDS = decltype(lds_tag)::value;
-            auto add = [&](int lag, C prod) {  // lag in [0, w1 - w0)
-                if constexpr (LDS)
-                    atomicAdd(&hist[lag], (H)prod);
-                else
-                    atomicAdd(nwin + lag, (unsigned long long)(long long)prod);
-            };
-            // pairs (i, j), j > i, with lag t_j - t_i in [max(w0, 1), w1): partners from
-            // the first j with t_j >= t_i + max(w0, 1) while t_j < t_i + w1, four per
-            // step so that their reads and atomics overlap.  The lag test is one unsigned
-            // compare, which also rejects a negative lag.
-            auto partners = [&](int ti, C di, int j) {
-                const int base = ti + w0;
-                if constexpr (S && LDS && sizeof(T) == 1) {
-                    // Staged 8-bit counts into the LDS histogram: the four partners of a
-                    // step come from one aligned 16-byte read of each staged array, from
-                    // j & ~3 (j <= n <= EMAX, so the reads stay inside the wave's n + 4
-                    // staged entries, the sentinels included, and a step that reaches
-                    // them ends the loop: no test of j against n).  With lo = max(w0, 1), a partner has t - (t_i + lo) in
-                    // [0, span1); everything else lies outside as an unsigned value:
-                    // entries before j lie below t_i + lo (times strictly increase; in the
-                    // first window entry i itself sits at lag 0 < lo), and the entries
-                    // from n on hold the staging's sentinel time INT_MAX.  The counter
-                    // index min(t - (t_i + lo), span1 + lane) sends every non-partner to
-                    // a counter past the window (the 64 that no window covers), so every
-                    // slot adds without a test or a branch.  Products of two 8-bit counts
-                    // fit 24 bits.
-                    const int lo = w0 > 0 ? w0 : 1;
-                    const int base1 = ti + lo;
-                    const unsigned span1 = span - (unsigned)(lo - w0);
-                    const unsigned park = span1 + (unsigned)lane;
-                    H* const h1 = hist + (lo - w0);
-                    const int4* t4p = reinterpret_cast<const int4*>(st_t[wave]);
-                    const int4* d4p = reinterpret_cast<const int4*>(st_d[wave]);
-                    for (int j4 = j & ~3;; j4 += 4) {
-                        const int4 t4 = t4p[j4 >> 2];
-                        const int4 d4 = d4p[j4 >> 2];
-                        const int tt[4] = {t4.x, t4.y, t4.z, t4.w};
-                        const int dd[4] = {d4.x, d4.y, d4.z, d4.w};
-#pragma unroll
-                        for (int u = 0; u < 4; ++u) {
-                            const unsigned lag = min((unsigned)(tt[u] - base1), park);
-                            const int prod = std::is_signed<T>::value
-                                                 ? __mul24((int)di, dd[u])
-                                                 : (int)__umul24((unsigned)di, (unsigned)dd[u]);
-                            atomicAdd(&h1[lag], (H)prod);
-                        }
-                        if (tt[3] - base1 >= (int)span1) break;  // INT_MAX past n
-                    }
-                    return;
-                }
-                for (; j < n; j += 4) {
-                    int tj[4];
-                    C dj[4];
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        const bool in = j + u < n;
-                        const int jj = in ? j + u : n - 1;
-                        const int t = time_of(jj);
-                        const C d = count_of(jj);
-                        tj[u] = in ? t : base + (int)span;
-                        dj[u] = in ? d : (C)0;
-                    }
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        const unsigned lag = (unsigned)(tj[u] - base);
-                        const C prod = di * dj[u];
-                        if (lag < span && prod != 0) add((int)lag, prod);
-                    }
-                    if (tj[3] - base >= (int)span) break;  // times increase: the rest are later
-                }
-            };
-            // wave-uniform steps of the first-partner search: powers of two from the
-            // largest not above n
-            const int top = 1 << (31 - __builtin_clz(n));
-            // Each lane takes events i and i + 64 together, so that their two searches
-            // for the first partner overlap.
-            for (int i0 = lane; i0 < n; i0 += 128) {
-                const int i1 = i0 + 64;
-                const bool has1 = i1 < n;
-                const int ti0 = time_of(i0);
-                const int ti1 = has1 ? time_of(i1) : 0;
-                const C d0 = count_of(i0);
-                const C d1 = has1 ? count_of(i1) : (C)0;
-                // first partner: i + 1 in the first window (times strictly increase),
-                // else one past the last p >= i with t_p < t_i + w0, by a descent over
-                // power-of-two steps (a monotone test; reads clamped inside the list)
-                int p0 = i0, p1 = has1 ? i1 : n - 1;
-                if (w0 > 0) {
-                    const int g0 = ti0 + w0, g1 = ti1 + w0;
-                    for (int step = top; step > 0; step >>= 1) {
-                        const int q0 = p0 + step, q1 = p1 + step;
-                        const int t0 = time_of(min(q0, n - 1));
-                        const int t1 = time_of(min(q1, n - 1));
-                        if (q0 < n && t0 < g0) p0 = q0;
-                        if (q1 < n && t1 < g1) p1 = q1;
-                    }
-                }
-                partners(ti0, d0, p0 + 1);
-                if (has1) partners(ti1, d1, p1 + 1);
-            }
-            };
-            if (to_lds)
-                events(std::true_type{});
-            else
-                events(std::false_type{});
-        };
         if (staged)
-            pixel(std::true_type{});
+            event_pixel<T, NW, true>(times, data, beg, n, lane, w0, w1, nframes, st_t[wave],
+                                     st_d[wave], hist, nwin, used, sq, err);
         else
-            pixel(std::false_type{});
+            event_pixel<T, NW, false>(times, data, beg, n, lane, w0, w1, nframes, nullptr, nullptr,
+                                      hist, nwin, used, 0, err);
         __builtin_amdgcn_wave_barrier();
     }
     __syncthreads();
@@ -491,12 +468,274 @@ static int sums_window(int nframes) {
 // Threads: two workgroups share a CU's threads where their counters leave room for it.
 static int sums_threads(int window) { return window > SUMS_WINDOW / 2 ? 1024 : 512; }
 
-// Waves per workgroup of the pair kernels: 16 (one workgroup per CU, 32,768 counters and
-// windows of 32,704 lags for 8-bit counts: the fewest windows, so the least per-window
-// work per pixel), or DXG2_EVENT_WAVES = 8 (two per CU, 16,384 counters) or 4 (four per
-// CU, 8,192 counters).
-// Measured on the events workload (1030x1065 x 100,000 frames): pairs 8.4 ms at 16
-// waves, 9.8 ms at 8, 13.2 ms at 4 (largest work items each).
+// ---------------------------------------------------------------- 8-bit counts
+//
+// The pair kernel of 8-bit counts, N <= FLAT_FRAMES (others: event_pairs_item()).  A wave takes up to 64 neighbouring pixels
+// of a bin at a time and their events in batches of up to FLAT_EVENTS, end to end in LDS as
+// (frame << 10 | count), and a lane takes an event, whatever its pixel: few events a pixel (0.3
+// to 120 in use) leave no lane idle, and no pixel costs a wave's steps for itself.
+//  * ONE (one lag window, N <= 32,704): event i of a pixel's n pairs with the (n - 1) / 2 events
+//    after it in the circle of the pixel's events, and for even n the first half with the one
+//    opposite too: each pair once, the same number of steps for every lane of a pixel.  The
+//    first n / 2 events are staged again behind the last, so a lane's partners lie in a row.
+//  * otherwise event i's partners run from the first with a lag in the window, found by a
+//    search, to the first past it, and what lies outside goes to one of 64 counters behind it.
+// Partners go four a step; the last step adds zeros for those past the lane's count, so every
+// atomic falls on a counter whatever the input.  A step is 16 VALU instructions, four LDS atomics
+// and two LDS reads.  Events out of range are staged as frame 0, and out of order can only
+// misplace counts: both are flagged.  Pixels of more events than a batch go through
+// event_pixel().  Bound by VALU issue and LDS atomics.
+// Pairs, against a wave a pixel: 1030 x 1065 x 2,000 (4.4e7 events, 8.8e8 pairs) 1.31 -> 0.45 ms;
+// 514 x 1030 x 20,000 (1.1e7) 0.36 -> 0.15; x 100,000 (1.1e8, 5.6e9 pairs, four windows) 5.36 ->
+// 4.43; 60 x 80 x 1,000 0.110 -> 0.005.
+constexpr int FLAT_EVENTS = 256;
+constexpr int FLAT_STAGE = 512;  // words a wave: 3 / 2 FLAT_EVENTS, 4 past them, 64 of marks
+constexpr int FLAT_WAVES = 16;
+constexpr int FLAT_WINDOW = 32704;       // lags; 64 more counters take what lies outside
+constexpr int FLAT_FRAMES = 1 << 21;     // frame + lag below 2^22
+
+// Inclusive scans over a wave (0 is the identity).
+template <typename Op>
+__device__ __forceinline__ int wave_scan(int v, Op op) {
+    v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false));  // row_shr:1
+    v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false));
+    v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false));
+    v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false));
+    v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false));  // row_bcast:15
+    v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false));  // row_bcast:31
+    return v;
+}
+
+// LDS written by this wave's lanes is read by its others after this.
+__device__ __forceinline__ void wave_lds() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    __builtin_amdgcn_wave_barrier();
+    asm volatile("" ::: "memory");
+}
+
+template <typename T, bool ONE>
+__device__ __forceinline__ void event_flat_item(
+    const int32_t* __restrict__ times, const T* __restrict__ data,
+    const uint32_t* __restrict__ offsets, const int32_t* __restrict__ pix_idx,
+    const BinDev* __restrict__ bins, const EventWork w, int nframes, int64_t nnz,
+    int64_t* __restrict__ num, int* __restrict__ err, uint32_t* __restrict__ hist,
+    uint32_t* __restrict__ stages) {
+    constexpr int R = FLAT_EVENTS / 64;
+    const int w0 = ONE ? 0 : (int)blockIdx.y * FLAT_WINDOW;
+    if (w0 >= nframes) return;
+    const int span = min(FLAT_WINDOW, nframes - w0);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (int k = threadIdx.x; k < span + 64; k += 64 * FLAT_WAVES) hist[k] = 0u;
+    __syncthreads();
+    const int32_t* list = pix_idx + bins[w.bin].idx_off;
+    unsigned long long* nwin =
+        reinterpret_cast<unsigned long long*>(num + (int64_t)w.bin * nframes + w0);
+    uint32_t* st = stages + wave * FLAT_STAGE;
+    uint8_t* marks = reinterpret_cast<uint8_t*>(st + FLAT_STAGE - FLAT_EVENTS / 4);
+    long long used = 0;  // this wave's sum of d^2 in the histogram (EvHist)
+    const auto sum = [](int a, int b) { return a + b; };
+    const auto most = [](int a, int b) { return a > b ? a : b; };
+    const auto from = [](int v, int l) { return __builtin_amdgcn_ds_bpermute(4 * l, v); };
+    const auto count = [](uint32_t word) -> int {
+        return std::is_signed<T>::value ? (int)(int8_t)word : (int)(word & 0xFFu);
+    };
+
+    // a short item is spread over its waves
+    const int chunk = min(64, (w.k1 - w.k0 + FLAT_WAVES - 1) / FLAT_WAVES);
+    for (int r0 = w.k0 + wave * chunk; r0 < w.k1; r0 += FLAT_WAVES * chunk) {
+        const int p = lane < chunk && r0 + lane < w.k1 ? list[r0 + lane] : -1;
+        uint32_t beg = 0u;
+        int n = 0;
+        if (p >= 0) {
+            beg = offsets[p];
+            const uint32_t end = offsets[p + 1];
+            if (end < beg || (int64_t)end > nnz)
+                atomicOr(err, 2);
+            else
+                n = (int)min(end - beg, 0x7fffffffu);
+        }
+        for (uint64_t longs = __ballot(n > FLAT_EVENTS); longs; longs &= longs - 1) {
+            const int l = __builtin_ctzll(longs);
+            event_pixel<T, FLAT_WAVES, false>(times, data,
+                                              (uint32_t)__builtin_amdgcn_readlane((int)beg, l),
+                                              __builtin_amdgcn_readlane(n, l), lane, w0, w0 + span,
+                                              nframes, nullptr, nullptr, hist, nwin, used, 0, err);
+        }
+        if (n > FLAT_EVENTS) n = 0;
+        // events and staged words of the lanes up to and with this one
+        const int own = n | (ONE ? n + n / 2 : n) << 16;
+        const int upto = wave_scan(own, sum);
+        const int total = __builtin_amdgcn_readlane(upto, 63) & 0xFFFF;
+        int done = 0, first = 0;  // events and lanes of earlier batches (done: as upto)
+        while ((done & 0xFFFF) < total) {
+            const int end = __popcll(__ballot((upto & 0xFFFF) - (done & 0xFFFF) <= FLAT_EVENTS));
+            const int all = __builtin_amdgcn_readlane(upto, end - 1) - done;
+            const int E = all & 0xFFFF;
+            const int at = upto - own - done;  // this pixel's first event and staged word
+            // each event's pixel: its first event is marked, the largest mark so far is its own
+            reinterpret_cast<uint32_t*>(marks)[lane] = 0u;
+            wave_lds();
+            if (lane >= first && lane < end && n > 0) marks[at & 0xFFFF] = (uint8_t)(lane + 1);
+            wave_lds();
+            int carry = 0, i_[R], n_[R], s_[R];
+            uint32_t x_[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int x = lane + 64 * r;
+                const int m = most(wave_scan((int)marks[x], most), carry);
+                carry = __builtin_amdgcn_readlane(m, 63);
+                const int l = m > 0 ? m - 1 : 0;
+                const int a = from(at, l), size = from(n, l);  // (by all lanes, for all lanes)
+                n_[r] = x < E ? size : 0;
+                i_[r] = x - (a & 0xFFFF);
+                s_[r] = a >> 16;
+                x_[r] = (uint32_t)from((int)beg, l) + (uint32_t)i_[r];
+            }
+            int t_[R], d_[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                t_[r] = n_[r] ? times[x_[r]] : 0;
+                d_[r] = n_[r] ? (int)data[x_[r]] : 0;
+            }
+            int bad = 0;
+            uint32_t sq = 0u;  // below 2^24 over the batch
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                if ((unsigned)t_[r] >= (unsigned)nframes) {
+                    bad = 1;
+                    t_[r] = 0;
+                }
+                const uint32_t word = (uint32_t)t_[r] << 10 | ((uint32_t)d_[r] & 0xFFu);
+                if (n_[r]) {
+                    st[s_[r] + i_[r]] = word;
+                    if (ONE && i_[r] < n_[r] / 2) st[s_[r] + n_[r] + i_[r]] = word;
+                }
+                sq += (uint32_t)(d_[r] * d_[r]);
+            }
+            if (lane < 4) st[(all >> 16) + lane] = 0u;  // read by last steps, counted as zeros
+            wave_lds();
+            if (w0 == 0) {
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+                    if (i_[r] + 1 < n_[r] && (int)(st[s_[r] + i_[r] + 1] >> 10) <= t_[r]) bad = 1;
+                if (bad) atomicOr(err, 1);
+            }
+            const int sqw = __builtin_amdgcn_readlane(wave_scan((int)sq, sum), 63);
+            const bool to_lds = used + sqw < EvHist<T>::budget(FLAT_WAVES);
+            if (to_lds) used += sqw;
+            if (w0 == 0 && lane == 0 && sqw) {  // lag 0
+                if (to_lds)
+                    atomicAdd(&hist[0], (uint32_t)sqw);
+                else
+                    atomicAdd(nwin, (unsigned long long)sqw);
+            }
+            // partners of each event: `m` staged words from `a` on (with several windows, those
+            // of them up to the window's end), lags from t0
+            auto pairs = [&](auto lds_tag) {
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    int a = s_[r] + i_[r] + 1, m;
+                    if (ONE) {
+                        m = n_[r] ? (n_[r] - 1) / 2 + (n_[r] % 2 == 0 && i_[r] < n_[r] / 2) : 0;
+                    } else {
+                        const int end = s_[r] + n_[r];
+                        if (w0 > 0) {  // past the events below the window's first lag
+                            const uint32_t k0 = (uint32_t)(t_[r] + w0) << 10;
+                            int at = a - 1;
+#pragma unroll
+                            for (int step = FLAT_EVENTS / 2; step > 0; step >>= 1) {
+                                const int q = at + step;
+                                if (st[min(q, FLAT_EVENTS)] < k0 && q < end) at = q;
+                            }
+                            a = at + 1;
+                        }
+                        m = n_[r] ? end - a : 0;
+                    }
+                    const uint32_t t0 = (uint32_t)(t_[r] + w0) << 10;
+                    // a word is frame << 10 | count: a difference >> 8 is the counter's byte
+                    auto add = [&](uint32_t word, int d) {
+                        uint32_t at;
+                        if (ONE) {
+                            uint32_t diff;
+                            asm("v_sad_u32 %0, %1, %2, 0" : "=v"(diff) : "v"(word & ~0x3FFu), "v"(t0));
+                            at = diff >> 8;
+                        } else {
+                            at = min((word - t0) >> 8, 4u * (uint32_t)(span + lane));
+                        }
+                        const int prod = std::is_signed<T>::value
+                                             ? __mul24(d, count(word))
+                                             : (int)__umul24((unsigned)d, (unsigned)count(word));
+                        if constexpr (decltype(lds_tag)::value) {
+                            atomicAdd(reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(hist) +
+                                                                  at),
+                                      (uint32_t)prod);
+                        } else {
+                            if (prod && (at >> 2) < (uint32_t)span)
+                                atomicAdd(nwin + (at >> 2), (unsigned long long)(long long)prod);
+                        }
+                    };
+                    const uint32_t* q = st + a;
+                    bool more = true;
+                    for (; m >= 4 && more; m -= 4, q += 4) {
+                        const uint32_t y[4] = {q[0], q[1], q[2], q[3]};
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) add(y[u], d_[r]);
+                        if (!ONE) more = (int)(y[3] - t0) < span << 10;
+                    }
+                    if (m > 0 && more) {
+                        const uint32_t y[3] = {q[0], q[1], q[2]};
+#pragma unroll
+                        for (int u = 0; u < 3; ++u) add(y[u], u < m ? d_[r] : 0);
+                    }
+                }
+            };
+            if (to_lds)
+                pairs(std::true_type{});
+            else
+                pairs(std::false_type{});
+            wave_lds();  // the next batch overwrites the stage
+            done += all;
+            first = end;
+        }
+    }
+    __syncthreads();
+    for (int k = threadIdx.x; k < span; k += 64 * FLAT_WAVES) {
+        const uint32_t v = hist[k];
+        if (v != 0) atomicAdd(nwin + k, EvHist<T>::widen(v));
+    }
+}
+
+template <typename T, bool ONE>
+__global__ __launch_bounds__(64 * FLAT_WAVES) void event_flat_kernel(
+    const int32_t* __restrict__ times, const T* __restrict__ data,
+    const uint32_t* __restrict__ offsets, const int32_t* __restrict__ pix_idx,
+    const BinDev* __restrict__ bins, const EventWork* __restrict__ work, int nframes, int64_t nnz,
+    int64_t* __restrict__ num, int* __restrict__ err) {
+    extern __shared__ uint32_t flat_lds[];
+    event_flat_item<T, ONE>(times, data, offsets, pix_idx, bins, work[blockIdx.x], nframes, nnz, num,
+                            err, flat_lds + FLAT_WAVES * FLAT_STAGE, flat_lds);
+}
+template <typename T, bool ONE>
+__global__ __launch_bounds__(64 * FLAT_WAVES) void event_flat_jobs_kernel(
+    const EventJob* __restrict__ jobs, const EventWork* __restrict__ work) {
+    extern __shared__ uint32_t flat_lds[];
+    const EventWork w = work[blockIdx.x];
+    if (w.bin < 0) return;
+    const EventJob j = jobs[w.pad];
+    event_flat_item<T, ONE>(global_ptr(j.times), global_ptr(reinterpret_cast<const T*>(j.data)),
+                            global_ptr(j.offsets), global_ptr(j.pix), global_ptr(j.bins), w,
+                            j.nframes, j.nnz, global_ptr(j.num), global_ptr(j.err),
+                            flat_lds + FLAT_WAVES * FLAT_STAGE, flat_lds);
+}
+static size_t flat_lds_bytes(int nframes) {
+    return 4 * ((size_t)FLAT_WAVES * FLAT_STAGE + std::min(nframes, FLAT_WINDOW) + 64);
+}
+
+// Waves per workgroup of event_pairs_kernel: 16 (one workgroup per CU, the most counters, so the
+// fewest windows and the least per-window work per pixel), or DXG2_EVENT_WAVES = 8 (two per CU)
+// or 4 (four per CU).
 int event_waves() {
     static const int nw = [] {
         const char* v = getenv("DXG2_EVENT_WAVES");
@@ -506,9 +745,9 @@ int event_waves() {
     return nw;
 }
 
-int event_lag_window(int dtype) {
-    return dtype == DXG2_U16 ? EvHist<uint16_t>::window(event_waves())
-                             : EvHist<uint8_t>::window(event_waves());
+int event_lag_window(int dtype, int nframes) {
+    if (dtype == DXG2_U16) return EvHist<uint16_t>::window(event_waves());
+    return nframes <= FLAT_FRAMES ? FLAT_WINDOW : EvHist<uint8_t>::window(event_waves());
 }
 
 template <typename T, int NW>
@@ -518,6 +757,17 @@ void pairs_jobs_launch(const EventJob* jobs, const EventWork* work, int n_work, 
     const int win = sums_window(max_frames);
     event_sums_jobs_kernel<T><<<dim3((unsigned)n_work, (unsigned)((max_frames + win - 1) / win)),
                                 sums_threads(win), 4 * win, s>>>(jobs, work, win);
+    if constexpr (sizeof(T) == 1) {
+        if (max_frames <= FLAT_FRAMES) {
+            const dim3 grid((unsigned)n_work, (unsigned)((max_frames + FLAT_WINDOW - 1) / FLAT_WINDOW));
+            const size_t lds = flat_lds_bytes(max_frames);
+            if (grid.y == 1)
+                event_flat_jobs_kernel<T, true><<<grid, 64 * FLAT_WAVES, lds, s>>>(jobs, work);
+            else
+                event_flat_jobs_kernel<T, false><<<grid, 64 * FLAT_WAVES, lds, s>>>(jobs, work);
+            return;
+        }
+    }
     event_pairs_jobs_kernel<T, NW><<<dim3((unsigned)n_work, (unsigned)((max_frames + WS - 1) / WS)),
                                      64 * NW, 0, s>>>(jobs, work);
 }
@@ -553,6 +803,19 @@ void pairs_launch(const int32_t* times, const void* data, const uint32_t* offset
     event_sums_kernel<T><<<dim3((unsigned)n_work, (unsigned)((nframes + win - 1) / win)),
                            sums_threads(win), 4 * win, s>>>(times, (const T*)data, offsets, pix_idx,
                                                             bins, work, nframes, nnz, win, sums);
+    if constexpr (sizeof(T) == 1) {
+        if (nframes <= FLAT_FRAMES) {
+            const dim3 grid((unsigned)n_work, (unsigned)((nframes + FLAT_WINDOW - 1) / FLAT_WINDOW));
+            const size_t lds = flat_lds_bytes(nframes);
+            if (grid.y == 1)
+                event_flat_kernel<T, true><<<grid, 64 * FLAT_WAVES, lds, s>>>(
+                    times, (const T*)data, offsets, pix_idx, bins, work, nframes, nnz, num, err);
+            else
+                event_flat_kernel<T, false><<<grid, 64 * FLAT_WAVES, lds, s>>>(
+                    times, (const T*)data, offsets, pix_idx, bins, work, nframes, nnz, num, err);
+            return;
+        }
+    }
     event_pairs_kernel<T, NW><<<dim3((unsigned)n_work, (unsigned)((nframes + WS - 1) / WS)),
                                 64 * NW, 0, s>>>(times, (const T*)data, offsets, pix_idx, bins,
                                                  work, nframes, nnz, num, err);

@@ -262,3 +262,53 @@ def test_events_lags_at_window_edges(dtype):
     num, sums = ev.event_brute_force(times, data, offsets, q, n)
     np.testing.assert_array_equal(c.last_numerators.cpu().numpy(), num.astype(np.int64))
     np.testing.assert_array_equal(c.last_sums.cpu().numpy(), sums.astype(np.int64))
+
+
+@pytest.mark.parametrize("n,dtype", [(300, np.uint8), (1000, np.int8), (32704, np.uint8),
+                                     (32705, np.int8), (70000, np.uint8), (5000, np.uint16)])
+def test_pixels_of_every_event_count(n, dtype):
+    """Pixels of 0, 1, 2, .. events next to one another, around the batches' 256 events, events
+    at the first and last frame, over one and several lag windows."""
+    from dynamix_amd.correlator.event import EventCorrelator
+    _announce("events counts n=%d %s" % (n, np.dtype(dtype).name))
+    rng = np.random.default_rng(n)
+    counts = np.array([0, 0, 1, 2, 3, 4, 5, 0, 6, 7, 63, 64, 65, 1, 0, 127, 128, 129, 2, 255,
+                       256, 257, 2, 290, 3, 254] + [1, 0, 2] * 60 + [12] * 50)
+    counts = np.concatenate([counts, rng.poisson(0.7, 1000 - counts.size)])
+    shape = (25, 40)
+    times, data = [], []
+    for k in counts:
+        t = np.sort(rng.choice(n, size=k, replace=False)).astype(np.int32)
+        if k > 1:
+            t[0], t[-1] = 0, n - 1
+        times.append(t)
+        hi = 128 if dtype == np.int8 else 256 if dtype == np.uint8 else 65536
+        data.append(rng.integers(1, hi, size=k).astype(dtype))
+    times, data = np.concatenate(times), np.concatenate(data)
+    offsets = np.concatenate([[0], np.cumsum(counts)]).astype(np.uint32)
+    q = np.ones(shape, np.int32)
+    q[:, 30:] = 2
+    q[3, 3:9] = 0
+    c = EventCorrelator(shape, n, 300, qmask=q, dtype=dtype)
+    c.correlate(times, data, offsets)
+    s, num = ev.event_sums_numerators_fast(times, data, offsets, q, n, [1, 2])
+    np.testing.assert_array_equal(c.last_numerators.cpu().numpy(), num)
+    np.testing.assert_array_equal(c.last_sums.cpu().numpy(), s)
+
+
+def test_more_frames_than_a_packed_word_holds():
+    """Series past 2^21 frames: event by event, as for 16-bit counts."""
+    from dynamix_amd.correlator.event import EventCorrelator
+    _announce("events 2^21 + 9 frames")
+    n = (1 << 21) + 9
+    rng = np.random.default_rng(8)
+    counts = [5, 0, 300, 1]
+    times = np.concatenate([np.sort(rng.choice(n, size=k, replace=False)) for k in counts])
+    data = rng.integers(1, 256, size=times.size).astype(np.uint8)
+    offsets = np.concatenate([[0], np.cumsum(counts)]).astype(np.uint32)
+    q = np.ones((2, 2), np.int32)
+    c = EventCorrelator((2, 2), n, 300, qmask=q, dtype=np.uint8)
+    c.correlate(times.astype(np.int32), data, offsets)
+    s, num = ev.event_sums_numerators_fast(times, data, offsets, q, n, [1])
+    np.testing.assert_array_equal(c.last_numerators.cpu().numpy(), num)
+    np.testing.assert_array_equal(c.last_sums.cpu().numpy(), s)
