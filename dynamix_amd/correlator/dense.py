@@ -241,7 +241,8 @@ def fft_length(nframes):
     """Nf = 2 L for the smallest L of FFT_HALF_LENGTHS with L >= nframes, or above 16384
     the smallest product L1 L2 >= nframes of FFT_ROW_LENGTHS x FFT_COL_LENGTHS: Nf >= 2 N - 1
     is all the linear autocorrelation needs (the reference uses get_next_power(2N),
-    utils.py:50-60, another smooth length of the same kind).  0 when N > 131072."""
+    utils.py:50-60, another smooth length of the same kind).  A plan may transform at a
+    shorter length that is enough too.  0 when N > 131072."""
     for L in FFT_HALF_LENGTHS:
         if L >= nframes:
             return 2 * L

@@ -197,3 +197,20 @@ def test_fft_long_series_every_length(n, L, dtype):
     q[0, :4] = 2
     c = FFTCorrelator(shape, n, q)
     _check(c, c.correlate(f), f, q, _sparse_ref(f, q))
+
+
+@pytest.mark.parametrize("n", [1, 2, 256, 512, 513, 640, 641, 1281, 1600, 2561, 3200, 5121, 6400,
+                               10241, 12800])
+@pytest.mark.parametrize("dtype", [np.uint8, np.uint16])
+def test_fft_at_the_ends_of_the_lengths(n, dtype):
+    """The longest and shortest series of the lengths between the powers of two, odd frame
+    sizes (byte loads) included."""
+    from dynamix_amd.correlator.dense import FFTCorrelator
+    _announce("fft lengths n=%d %s" % (n, np.dtype(dtype).name))
+    shape = (9, 15)
+    rng = np.random.default_rng(n)
+    f = rng.poisson(0.5, size=(n,) + shape).astype(dtype)
+    f[0, 0, 0] += 1
+    q = _qmask(n, shape, 2)
+    c = FFTCorrelator(shape, n, q)
+    _check(c, c.correlate(f), f, q)
