@@ -313,6 +313,7 @@ struct dxg2_plan {
     float2* d_tw = nullptr;        // twiddles (launch_fft_power)
     double* d_power = nullptr;     // n_bins rows of fft_power_row doubles
     double* d_fnum = nullptr;      // (n_bins, N)
+    double2* d_finv = nullptr;     // n_bins rows of fft_inverse_elems
     FftShape fft{};
 
     // Profiling: each correlate call records 4 events on its stream (no host sync);
@@ -797,6 +798,7 @@ int ensure_fft_buffers(dxg2_plan* p, hipStream_t s) {
     uint8_t* xs = nullptr;
     float2* tw = nullptr;
     double *power = nullptr, *fnum = nullptr;
+    double2* finv = nullptr;
     KbWork* kbw = nullptr;
     KbWork* kbg = nullptr;
     int32_t* pixf = nullptr;
@@ -809,6 +811,9 @@ int ensure_fft_buffers(dxg2_plan* p, hipStream_t s) {
         dev_alloc(p->alloc, (void**)&tw, p->twiddles.size() * sizeof(float2), s) != hipSuccess ||
         dev_alloc(p->alloc, (void**)&fnum, (size_t)std::max(p->n_bins, 1) * p->N * sizeof(double), s) !=
             hipSuccess ||
+        dev_alloc(p->alloc, (void**)&finv,
+                  std::max(p->n_bins, 1) * fft_inverse_elems(shape) * sizeof(double2), s) !=
+            hipSuccess ||
         (!p->kb_work.empty() &&
          (dev_alloc(p->alloc, (void**)&kbw, p->kb_work.size() * sizeof(KbWork), s) != hipSuccess ||
           dev_alloc(p->alloc, (void**)&kbg, p->kb_gather.size() * sizeof(KbWork), s) !=
@@ -816,7 +821,7 @@ int ensure_fft_buffers(dxg2_plan* p, hipStream_t s) {
         dev_alloc(p->alloc, (void**)&power, (size_t)std::max(p->n_bins, 1) * fft_power_row(shape) * sizeof(double), s) !=
             hipSuccess) {
         for (void* b : {(void*)xs, (void*)tw, (void*)fnum, (void*)kbw, (void*)kbg, (void*)power,
-                        (void*)pixf, (void*)qkb})
+                        (void*)pixf, (void*)qkb, (void*)finv})
             dev_free(p->alloc, b, s);
         return set_error(DXG2_ENOMEM, "cannot allocate FFT workspace");
     }
@@ -825,6 +830,7 @@ int ensure_fft_buffers(dxg2_plan* p, hipStream_t s) {
     p->d_xs = xs;
     p->d_tw = tw;
     p->d_fnum = fnum;
+    p->d_finv = finv;
     p->d_kbwork = kbw;
     p->d_kbgather = kbg;
     p->d_power = power;
@@ -1428,7 +1434,7 @@ static void plan_release(dxg2_plan* p, hipStream_t s) {
                     p->d_ework, p->d_err,  p->d_cnt,   p->d_scan,  p->d_off,
                     p->d_etimes, p->d_edata, p->d_kbwork, p->d_kbgather, p->d_xs, p->d_tw,
                     p->d_pixfft, p->d_fftqkb,
-                    p->d_power, p->d_fnum, p->d_qmwork, p->d_qxwork, p->d_qoff,
+                    p->d_power, p->d_fnum, p->d_finv, p->d_qmwork, p->d_qxwork, p->d_qoff,
                     p->d_slab4, p->d_wsums, p->d_heads, p->d_gband, p->d_gband_kb, p->d_gfall,
                     p->coo_sort.keys, p->coo_sort.vals0, p->coo_sort.vals1, p->coo_sort.tmp,
                     p->d_wflag, p->d_pixw, p->d_nwkb};
@@ -1495,7 +1501,9 @@ int dxg2_plan_footprint(const dxg2_plan* p, int32_t path, size_t* bytes) {
             for (const auto& bd : p->bins) nkb += bd.nkb;
             *bytes = common + fft_series_bytes(p, L) +
                      (2 * (size_t)shape.H + L + 1) * sizeof(float2) +
-                     (size_t)std::max(p->n_bins, 1) * (fft_power_row(shape) + p->N) * sizeof(double) +
+                     (size_t)std::max(p->n_bins, 1) *
+                         ((fft_power_row(shape) + p->N) * sizeof(double) +
+                          fft_inverse_elems(shape) * sizeof(double2)) +
                      (2 * (size_t)nkb + (size_t)N_XCD * PM_XCD_GROUP) * sizeof(KbWork) +
                      (p->pix_idx.size() + (size_t)std::max(p->n_bins, 1)) * sizeof(int32_t);
             return DXG2_OK;
@@ -2160,7 +2168,7 @@ int dxg2_correlate_fft(dxg2_plan* p, const void* d_frames, double* d_num, int64_
     if (launch_fft_power(p->fft, p->dtype, p->d_xs, p->d_bins, p->d_kbwork,
                          (int)p->kb_work.size(), p->d_tw, p->d_power, s))
         return set_error(DXG2_EUNSUPPORTED, "no FFT kernel for length %d", p->fft.L);
-    launch_fft_inverse(p->d_power, p->fft, p->n_bins, p->N, p->d_fnum, s);
+    launch_fft_inverse(p->d_power, p->fft, p->n_bins, p->N, p->d_finv, p->d_fnum, s);
     if (ev) DXG2_HIP(hipEventRecord(ev[2], s));
     launch_finalize_f64(sums, p->d_fnum, p->d_bins, p->n_bins, p->N, p->d_prefix, p->d_smax,
                         p->d_dpre, d_num, d_den, d_g2, p->dmf, s);

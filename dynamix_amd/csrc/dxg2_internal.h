@@ -299,8 +299,10 @@ void launch_gather_pm(const uint8_t* frames, int dtype, int64_t hw, int nframes,
 int launch_fft_power(const FftShape& shape, int dtype, const uint8_t* xs, const BinDev* bins,
                      const KbWork* work, int n_work, const float2* tw, double* power,
                      hipStream_t s);
+// work: fft_inverse_elems(shape) elements a bin.
+size_t fft_inverse_elems(const FftShape& shape);
 void launch_fft_inverse(const double* power, const FftShape& shape, int n_bins, int nframes,
-                        double* num, hipStream_t s);
+                        double2* work, double* num, hipStream_t s);
 void launch_excl_scan(const uint32_t* in, int64_t n, uint32_t* tot, uint32_t* out, hipStream_t s);
 void launch_events_window(int dtype, const uint32_t* offsets, const int32_t* times,
                           const void* data, int64_t npix, int t0, int t1, uint32_t* scratch,
