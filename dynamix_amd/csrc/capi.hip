@@ -469,14 +469,17 @@ int gather_tile(const dxg2_plan* p, size_t items) {
 // items are then too few or too uneven for the chip's CUs and shorter ones end sooner.  An item
 // costs about 0.5 us a k-block and 10 us for itself (first copies, fold, flush, next item) in a
 // 256-frame tile, a quarter of the former in a 128-frame tile; n items on 256 CUs end after
-// their mean load and half the longest item, and not before the longest.  96 x 96 x 500, 5
+// their mean load and half the longest item, and not before the longest (`only`: the tiles of
+// that bin alone).  96 x 96 x 500, 5
 // bins (15 whole items of 29 k-blocks): 45 us, in items of 4 and more 16 us.
-int gram_kchunk(const dxg2_plan* p) {
+int gram_kchunk(const dxg2_plan* p, int only = -1, double item_us = 10.0) {
     const int nT = (p->N + p->gram_tile - 1) / p->gram_tile;
     const double tiles = (double)nT * (nT + 1) / 2 * (slab_planes(p->dtype) == 2 ? 2 : 1);
-    const double a = p->gram_tile == 256 ? 0.5 : 0.125, c = 10.0;
+    const double a = p->gram_tile == 256 ? 0.5 : 0.125, c = item_us;
     int most = 0;
-    for (const BinDev& b : p->bins) most = std::max(most, b.nkb);
+    auto mine = [&](const BinDev& b) { return only < 0 || &b == &p->bins[only]; };
+    for (const BinDev& b : p->bins)
+        if (mine(b)) most = std::max(most, b.nkb);
     int best = p->tune_kchunk;
     double best_t = 0.0;
     for (int parts = 1; parts <= 64; parts = parts < 4 ? parts + 1 : parts + parts / 2) {
@@ -484,7 +487,7 @@ int gram_kchunk(const dxg2_plan* p) {
         if (parts > 1 && k < 4) break;
         double total = 0.0;
         for (const BinDev& b : p->bins)
-            total += tiles * (a * b.nkb + c * ((b.nkb + k - 1) / std::max(k, 1)));
+            if (mine(b)) total += tiles * (a * b.nkb + c * ((b.nkb + k - 1) / std::max(k, 1)));
         const double longest = a * k + c;
         const double t = std::max(longest, total / 256 + 0.5 * longest);
         if (parts == 1 || t < 0.95 * best_t) {
@@ -558,7 +561,10 @@ void build_tile_work(const dxg2_plan* p, int only, size_t cap_bytes, TileWork& t
     const int64_t ntri = (int64_t)nT * (nT + 1) / 2;
     const int band = p->tune_band;
     const int group = p->tune_group;
-    const int kchunk = p->tune_kchunk;
+    // one bin's few tiles are cut like the plain launch's (an item also stores its tile); all
+    // bins' are not, as std_tile_kernel is fastest with one item a tile.  One ring of 4, 300 x 400
+    // x 1,000 (10 tiles): Gram 377 -> 45 us, the call 574 -> 137 us.
+    const int kchunk = only >= 0 ? gram_kchunk(p, only, 20.0) : p->tune_kchunk;
     const bool wide = slab_planes(p->dtype) == 2;
     const size_t tile_bytes = (size_t)T * T * 4;
     int max_items = 0;
@@ -673,7 +679,7 @@ int ensure_std_buffers(dxg2_plan* p, hipStream_t s) {
 // most half the detector is gathered alone, by the general gather (4.0 ms a 480,000 pixels x
 // 10,000 frames, in proportion to the pixels); the band gather reads every row whatever the
 // bin holds (1.2 ms of staging and 2.25 ms with every pixel of that size).  One ring of 20,
-// 514 x 1030 x 5,000: gather and sums 1,640 -> 421 us, the call 2.21 -> 1.04 ms.
+// 514 x 1030 x 5,000: gather and sums 1,640 -> 223 us.
 int ensure_ttcf_buffers(dxg2_plan* p, int b, hipStream_t s) {
     if (p->ttcf_bin == b) return DXG2_OK;
     drop_tile_work(p->alloc, p->ttw, s);

@@ -245,9 +245,11 @@ void launch_std_tiles(int tile, const StdTile* tiles, int n_tiles, const BinDev*
 
 // Two-time correlation of one bin (event_y.py:137-157): trc(t, u) = n_b G(t, u) /
 // (S(t) S(u)) for u > t, mirrored to (u, t); NaN where S(t) S(u) = 0.  One workgroup per
-// tile, a band of BR rows at a time: the row-major upper entries are written straight
+// tile and TTCF_ROWS rows (a tile's rows one after the other left most of the chip idle:
+// 229 -> 127 us at 5,000 frames, one item a tile): the row-major upper entries are written straight
 // from the lanes (consecutive u), the mirrored ones from an LDS transpose, 32 lanes per
 // output row (128-byte runs).
+constexpr int TTCF_ROWS = 32;
 template <int T>
 __global__ __launch_bounds__(256) void ttcf_tile_kernel(const StdTile* __restrict__ tiles,
                                                         const BinDev* __restrict__ bins,
@@ -255,7 +257,7 @@ __global__ __launch_bounds__(256) void ttcf_tile_kernel(const StdTile* __restric
                                                         const int64_t* __restrict__ sums,
                                                         int mode, int n_bins, int nframes,
                                                         float* __restrict__ trc) {
-    constexpr int BR = 32;
+    constexpr int BR = TTCF_ROWS;
     constexpr int RPP = 256 / T;
     __shared__ float x[BR][T + 1];
 
@@ -277,39 +279,39 @@ __global__ __launch_bounds__(256) void ttcf_tile_kernel(const StdTile* __restric
     const int64_t TT = (int64_t)T * T;
     const int* base = scratch + (int64_t)tl.slot0 * TT;
 
-    for (int r0 = 0; r0 < T && t0 + r0 < nframes; r0 += BR) {
-        __syncthreads();
-        for (int rr = rsub; rr < BR; rr += RPP) {
-            const int r = r0 + rr;
-            const int t = t0 + r;
-            float val = 0.0f;
-            // the last diagonal entry keeps the pairs within frame N-1: G(t, t) - S(t)
-            const bool corner = t == nframes - 1 && u == t;
-            if (t < nframes && u < nframes && (u > t || corner)) {
-                int64_t S_t, c_t;
-                frame_terms(sums, mode, n_bins, nframes, tl.bin, t, S_t, c_t);
-                if (S_t != 0 && S_u != 0) {
-                    const int* e = base + (int64_t)r * T + c;
-                    int64_t g = c_t + c_u - Kc;
-                    int k = 0;
-                    for (; k < tl.n_hh; ++k) g += (int64_t)w_hh * e[k * TT];
-                    for (; k < tl.n_hh + tl.n_ll; ++k) g += e[k * TT];
-                    for (; k < tl.n_hh + tl.n_ll + tl.n_x; ++k) g += (int64_t)256 * e[k * TT];
-                    if (corner) g -= S_t;
-                    val = (float)(npix * (double)g / ((double)S_t * (double)S_u));
-                } else {
-                    val = __builtin_nanf("");
-                }
-                trc[(int64_t)t * N + u] = val;
+    const int r0 = blockIdx.y * BR;
+    if (t0 + r0 >= nframes) return;
+    for (int rr = rsub; rr < BR; rr += RPP) {
+        const int r = r0 + rr;
+        const int t = t0 + r;
+        float val = 0.0f;
+        // the last diagonal entry keeps the pairs within frame N-1: G(t, t) - S(t)
+        const bool corner = t == nframes - 1 && u == t;
+        if (t < nframes && u < nframes && (u > t || corner)) {
+            int64_t S_t, c_t;
+            frame_terms(sums, mode, n_bins, nframes, tl.bin, t, S_t, c_t);
+            if (S_t != 0 && S_u != 0) {
+                const int* e = base + (int64_t)r * T + c;
+                int64_t g = c_t + c_u - Kc;
+                int k = 0;
+#pragma unroll 4
+                for (; k < tl.n_hh; ++k) g += (int64_t)w_hh * e[k * TT];
+                for (; k < tl.n_hh + tl.n_ll; ++k) g += e[k * TT];
+                for (; k < tl.n_hh + tl.n_ll + tl.n_x; ++k) g += (int64_t)256 * e[k * TT];
+                if (corner) g -= S_t;
+                val = (float)(npix * (double)g / ((double)S_t * (double)S_u));
+            } else {
+                val = __builtin_nanf("");
             }
-            x[rr][c] = val;
+            trc[(int64_t)t * N + u] = val;
         }
-        __syncthreads();
-        for (int k = tid; k < T * BR; k += 256) {
-            const int cu = k / BR, rr = k % BR;
-            const int uu = u0 + cu, t = t0 + r0 + rr;
-            if (t < nframes && uu < nframes && uu > t) trc[(int64_t)uu * N + t] = x[rr][cu];
-        }
+        x[rr][c] = val;
+    }
+    __syncthreads();
+    for (int k = tid; k < T * BR; k += 256) {
+        const int cu = k / BR, rr = k % BR;
+        const int uu = u0 + cu, t = t0 + r0 + rr;
+        if (t < nframes && uu < nframes && uu > t) trc[(int64_t)uu * N + t] = x[rr][cu];
     }
 }
 
@@ -357,10 +359,10 @@ void launch_ttcf_tiles(int tile, const StdTile* tiles, int n_tiles, const BinDev
                        int nframes, float* trc, hipStream_t s) {
     if (n_tiles <= 0) return;
     if (tile == 128)
-        ttcf_tile_kernel<128><<<dim3((unsigned)n_tiles), dim3(256), 0, s>>>(
+        ttcf_tile_kernel<128><<<dim3((unsigned)n_tiles, 128 / TTCF_ROWS), dim3(256), 0, s>>>(
             tiles, bins, scratch, sums, mode, n_bins, nframes, trc);
     else
-        ttcf_tile_kernel<256><<<dim3((unsigned)n_tiles), dim3(256), 0, s>>>(
+        ttcf_tile_kernel<256><<<dim3((unsigned)n_tiles, 256 / TTCF_ROWS), dim3(256), 0, s>>>(
             tiles, bins, scratch, sums, mode, n_bins, nframes, trc);
 }
 
