@@ -347,7 +347,7 @@ def bench_events(seed):
                            "executed_ops": den_exec_ops, "useful_ops": den_useful_ops,
                            "note": "the kernel's time is in the kernel trace (rocprofv3); the "
                                    "stage time above adds the prefix sums and the finaliser"},
-            "pairs_kernel": {"kernel": "event_pairs_kernel", "pairs_per_s": pairs / (pairs_ms * 1e-3),
+            "pairs_kernel": {"kernel": "event_flat_kernel", "pairs_per_s": pairs / (pairs_ms * 1e-3),
                              "lds_atomic_ceiling_per_s": lds_rate.value,
                              "frac_of_lds_atomic_ceiling": pairs / (pairs_ms * 1e-3) / lds_rate.value,
                              "note": "one LDS atomic add per pair at least; the ceiling is "
