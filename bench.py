@@ -1,20 +1,21 @@
-"""Benchmark: g2 pixel*frames/s of the dense batched i8-MFMA path on one MI355X.
+"""Benchmark: g2 pixel*frames/s of the dense batched MFMA path on one MI355X.
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload headline]
 
 A step is one dense correlate of the whole workload: qmask gather of every bin into
-i8 slabs, one grouped i8-MFMA Gram launch over all bins with the fused tau
-reduction, exact denominators and g2.  Frames are generated on the GPU (seeded AR(1)
+slabs, grouped MFMA Gram launches over all bins with the fused tau reduction (FP4 codes
+for the pixels whose counts stay within 4, which is exact, i8 for the others; i8 for
+every pixel when many are wide), exact denominators and g2.  Frames are generated on the GPU (seeded AR(1)
 speckle) before the timed region, so inputs are resident in HBM; g2, the int64
 numerators, sums and FP64 denominators stay in HBM.
 
 Printed as one JSON line.  Besides the metric it reports
-  roofline      the Gram kernel's achieved int8 ops/s (algorithmic ops: the upper
-                triangle with the diagonal, 2 * sum_b n_b * N (N+1)/2, per launch)
+  roofline      the Gram stage's achieved ops/s (algorithmic ops: the upper
+                triangle with the diagonal, 2 * sum_b n_b * N (N+1)/2, per call)
                 over its average duration from HIP events recorded around each
-                launch inside the timed region, against the 5.0 POP/s dense int8 peak
-                (the persistent launch over per-XCD work queues, with the fill kernel
-                that clears the queue heads);
+                launch inside the timed region, against what the executed formats
+                allow: 5.0 POP/s dense int8; with narrow pixels 10 POP/s FP4 for every
+                pixel and the wide ones again at the int8 peak;
   calc_std      the dense path with calc_std=True (dev(tau)) on the same stack;
   compress      the on-device frames -> events compaction of the same stack;
   ttcf          the two-time matrix of one bin of the same stack;
@@ -51,6 +52,8 @@ sys.path.insert(0, ROOT)
 METRIC = ("g2 pixel·frames/s at 514×1030×10k uint8, 20 bins; "
           "p50/p99 mixed-job latency")
 INT8_PEAK_TOPS = 5000.0   # MI355X dense int8 MFMA, 5.0 POP/s
+FP4_PEAK_TOPS = 10000.0   # dense FP4 MFMA
+NARROW_MIN_WORK, NARROW_MAX, NARROW_WIDE = 5e11, 4, 0.3  # the library's narrow route
 HBM_PEAK_GBS = 8000.0
 
 
@@ -98,17 +101,36 @@ def cpu_baseline(frames_dev, qmask, target_s=15.0):
                       % (", ".join(done), n, spent, cores)}
 
 
-def gather_roofline(qmask, shape, n, gather_ms):
-    """HBM roofline of the gather stage: every frame byte read once, and one byte per
-    binned pixel (rounded up to whole 64-pixel k-blocks) per frame written to the slab."""
+def gather_roofline(qmask, shape, n, gather_ms, narrow):
+    """HBM roofline of the gather stage: every frame byte read once, and one byte (half a
+    byte on the narrow route) per binned pixel (rounded up to whole 64-pixel k-blocks) per
+    frame written to the slab."""
     import numpy as np
     counts = np.bincount(qmask.ravel())[1:]
     read = float(n) * shape[0] * shape[1]
-    write = float(n) * int((64 * np.ceil(counts / 64.0)).sum())
+    write = float(n) * int((64 * np.ceil(counts / 64.0)).sum()) * (0.5 if narrow else 1.0)
     gbps = (read + write) / (gather_ms * 1e-3) / 1e9
     return {"ms": gather_ms, "bytes_read": read, "bytes_written": write, "GBps": gbps,
             "peak_GBps": HBM_PEAK_GBS, "frac_of_hbm": gbps / HBM_PEAK_GBS,
-            "kernel": "gather_band_kernel"}
+            "kernel": "gather_band_f4_kernel" if narrow else "gather_band_kernel"}
+
+
+def gram_peak(frames, qmask, n):
+    """Peak TOP/s of the Gram of these 8-bit frames and the share of wide pixels (None: every
+    pixel in i8): FP4 for all pixels and i8 for the wide ones on the narrow route."""
+    import torch
+    inside = torch.from_numpy(qmask.ravel() > 0).to(frames.device)
+    npix = int(inside.sum())
+    if frames.element_size() != 1 or npix * n * n < NARROW_MIN_WORK:
+        return INT8_PEAK_TOPS, None
+    top, low = frames.amax(0).ravel(), frames.amin(0).ravel()
+    wide = top > NARROW_MAX
+    if frames.dtype == torch.int8:
+        wide |= low < -NARROW_MAX
+    share = float((wide & inside).sum()) / npix
+    if share > NARROW_WIDE:
+        return INT8_PEAK_TOPS, None
+    return 1.0 / (1.0 / FP4_PEAK_TOPS + share / INT8_PEAK_TOPS), share
 
 
 def cpu_baseline_fft(frames_dev, qmask, target_s=8.0, chunk=4096):
@@ -546,6 +568,7 @@ def main():
     # sanity: g2 finite where denominators are positive
     assert torch.isfinite(g2[den > 0]).all().item()
 
+    peak, wide_share = gram_peak(frames, q, n)
     out = {
         "metric": METRIC,
         "value": pf / (ms * 1e-3),
@@ -561,17 +584,23 @@ def main():
         "data": "synthetic",
         "config": {"workload": "%s: %dx%d x %d frames %s, %d annular bins, %d binned px"
                                % (args.workload, shape[0], shape[1], n, wl["dtype"], nb, npix),
-                   "path": "dense batched i8-MFMA Gram (gather + gram + finalise)",
+                   "path": "dense batched MFMA Gram, exact integer sums: %s (gather + gram + finalise)"
+                           % ("i8" if wide_share is None else
+                              "FP4 codes for counts up to %d, i8 for the %.1f %% wide pixels"
+                              % (NARROW_MAX, 100 * wide_share)),
                    "stage_ms": {"gather": gather_ms, "gram": gram_ms, "finalise": fin_ms},
                    "gram_tuning": plan.get_tuning(),
                    "autotune": None if tuning is None else {
                        "gram_ms": tuning["gram_ms"], "default_gram_ms": tuning["default_ms"],
                        "candidates": len(tuning["trials"])}},
-        "gather": gather_roofline(q, shape, n, gather_ms),
-        "roofline": {"bound": "mfma", "achieved": achieved, "peak": INT8_PEAK_TOPS,
-                     "unit": "TOP/s", "frac": achieved / INT8_PEAK_TOPS,
-                     "traffic": read_traffic("gram_i8_%s_traffic.txt" % args.workload),
-                     "kernel": ("gram_i8_queue_kernel" if plan.get_tuning()["queue"]
+        "gather": gather_roofline(q, shape, n, gather_ms, wide_share is not None),
+        "roofline": {"bound": "mfma", "achieved": achieved, "peak": peak,
+                     "unit": "TOP/s", "frac": achieved / peak,
+                     "traffic": (read_traffic("gram_i8_%s_traffic.txt" % args.workload)
+                                 if wide_share is None else None),
+                     "kernel": ("gram_f4_queue_kernel + gram_i8_queue_kernel"
+                                if wide_share is not None and plan.get_tuning()["queue"] else
+                                "gram_i8_queue_kernel" if plan.get_tuning()["queue"]
                                 else "gram_i8_kernel"), "ops_per_launch": ops},
     }
 
