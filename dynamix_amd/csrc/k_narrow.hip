@@ -25,10 +25,11 @@ constexpr int NARROW_SAMPLES = 64;           // frames
 constexpr int NARROW_SAMPLE_KB = 1024;       // k-blocks (at the line of 30 % of 65,536 pixels
                                              // about 20,000 turn wide over the stack)
 
-// One thread per list entry of every `stride`-th k-block: wide in the first half of the sampled frames (ctl[1]), in any of
-// them (ctl[2]), of ctl[4] pixels; the last block decides (ctl[0] is the route, ctl[3] counts
-// blocks; all zeroed beforehand).  Pixels that turn wide go on appearing at the rate of the second half at most
-// (hot pixels are all seen in the first frames, and the rest saturate), so
+// One thread per list entry of every `stride`-th k-block: wide in the first half of the sampled
+// frames (ctl[1]), in any of them (ctl[2]), of ctl[4] pixels; the last block decides (ctl[0] is
+// the route, ctl[3] counts blocks; all zeroed beforehand).  Pixels that turn wide go on
+// appearing at the rate of the second half at most (hot pixels are all seen in the first
+// frames, and the rest saturate), so
 //   wide <= ctl[2] + (ctl[2] - ctl[1]) (N - n) / (n / 2).
 // The line is at 30 % of the pixels: a wide pixel costs its share of the i8 Gram, of the time
 // of which the FP4 Gram of every pixel takes about half.
