@@ -869,9 +869,26 @@ void build_event_work(dxg2_plan* p) {
     // whatever it holds.  514 x 1030 x 20,000: 0.75 ms a call with 940 items, 0.63 with 240 to
     // 470; 1030 x 1065 x 100,000, 4 windows: 5.7, 5.5, 5.6 ms with 1,072, 360, 260 a window;
     // x 2,000: 1.56 ms with 1,024, 1.66 with 540.
-    const int lags = std::min(event_lag_window(p->dtype, p->N), p->N);
+    const int window = event_lag_window(p->dtype, p->N), lags = std::min(window, p->N);
     const int64_t items = lags <= 8192 ? 1024 : 384;
     int item = (int)std::min<int64_t>(8192, (total / items + 63) / 64 * 64);
+    // Several windows repeat that for each of them, and small detectors are soon cut too fine:
+    // the power of two with the least cost, where an item costs as much as 512 pixels for itself
+    // and n items on 256 CUs end after their mean load and half an item.  Pairs and sums, total /
+    // 384 pixels -> these: 128 x 128, 1.6e6 events, 4 windows 306 -> 208 us (128 to 512 pixels:
+    // 219, 163, 208), 31 windows 1,690 -> 478 (512 to 2,048: 513, 478, 531); 512 x 512, 5.2e6
+    // events, 7 windows 703 -> 456; 1030 x 1065, 1.1e8 events, 4 windows 4.91 -> 4.83 ms.
+    const int64_t windows = (p->N + window - 1) / window;
+    double best = 0.0;
+    for (int px = 64; windows > 1 && px <= 8192; px *= 2) {
+        double n = 0.0;
+        for (const auto& k : p->npix) n += (double)((k + px - 1) / px);
+        const double cost = 512.0 + px, t = n * (double)windows * cost / 256 + 0.5 * cost;
+        if (px == 64 || t < best) {
+            best = t;
+            item = px;
+        }
+    }
     item = std::min(EVENT_ITEM_MAX, std::max(64, env_int("DXG2_EVENT_ITEM_PIXELS", item)));
     for (int b = 0; b < p->n_bins; ++b)
         for (int k0 = 0; k0 < p->bins[b].npix; k0 += item)
