@@ -2024,8 +2024,11 @@ int dxg2_batch_correlate_events(dxg2_batch* b, int32_t n, dxg2_plan* const* plan
     std::vector<EventJob> jobs(n);
     std::vector<EventWork> work;
     int max_frames = 0;
+    int64_t counters = 0, events = 0;
     for (int i = 0; i < n; ++i) {
         dxg2_plan* p = plans[i];
+        counters += (int64_t)p->event_work.size() * p->N;
+        events += nnz[i];
         const int64_t nbn = (int64_t)p->n_bins * p->N;
         int64_t* sums = d_sums && d_sums[i] ? d_sums[i] : p->d_sums;
         launch_clear_call(sums, nbn, p->d_ugram, nbn, p->d_err, 1, s);
@@ -2049,7 +2052,8 @@ int dxg2_batch_correlate_events(dxg2_batch* b, int32_t n, dxg2_plan* const* plan
         DXG2_HIP(hipMemcpyAsync(b->d_ework, b->h_ework, work.size() * sizeof(EventWork),
                                 hipMemcpyHostToDevice, s));
     DXG2_HIP(hipEventRecord(b->staged, s));
-    launch_event_pairs_jobs(dtype, b->d_ejobs, b->d_ework, (int)work.size(), max_frames, s);
+    launch_event_pairs_jobs(dtype, b->d_ejobs, b->d_ework, (int)work.size(), max_frames, counters,
+                            events, s);
     for (int i = 0; i < n; ++i) {
         dxg2_plan* p = plans[i];
         if (p->n_bins == 0) continue;

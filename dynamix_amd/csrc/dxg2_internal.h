@@ -254,8 +254,9 @@ void launch_plain_bin(const uint8_t* frames, int dtype, int64_t hw, int nframes,
                       float* g2_row, hipStream_t s);
 // Lags per workgroup of the event pair kernel (its lag window) for a count type.
 int event_lag_window(int dtype, int nframes);
+// counters: frames of every item together; nnz: events of every job.
 void launch_event_pairs_jobs(int dtype, const EventJob* jobs, const EventWork* work, int n_work,
-                             int max_frames, hipStream_t s);
+                             int max_frames, int64_t counters, int64_t nnz, hipStream_t s);
 void launch_event_pairs(int dtype, const int32_t* times, const void* data,
                         const uint32_t* offsets, const int32_t* pix_idx, const BinDev* bins,
                         const EventWork* work, int n_work, int nframes, int64_t nnz,

@@ -16,7 +16,7 @@
 //    events i = lane + 128 r and i + 64 together; a binary search finds the first partner j > i
 //    whose lag t_j - t_i reaches the window (event_pairs_item);
 //  * the self pairs (lag 0, d_i^2) are added in the first window; S_b(t) comes from a launch of
-//    its own (event_sums_item);
+//    its own (event_sums_item), or from the first window's launch where events are few;
 //  * the input is validated on the device (frames in [0, N), strictly increasing per
 //    pixel, as compress_all_stack produces, event.py:267-284); a violation sets a
 //    flag the host turns into an error instead of reading out of bounds.
@@ -86,9 +86,14 @@ struct EvPixel {
     int n;  // events to correlate: 0 for an empty, unbinned or invalid range
 };
 
+// One event's count to its frame's sum (few events: see event_sums_item()).
+__device__ __forceinline__ void add_sum(int64_t* sum, long long d) {
+    if (d) atomicAdd(reinterpret_cast<unsigned long long*>(sum), (unsigned long long)d);
+}
+
 // One pixel's pairs by a wave, lags [w0, w1), its n > 0 events at `beg`: staged by the wave (S; pt,
 // pd: frames and counts, sq: this lane's share of the sum of d^2) or read from memory.  used: see
-// EvHist.
+// EvHist.  srow: the bin's frame sums where this launch forms them, else null.
 template <typename T, int NW, bool S>
 __device__ __forceinline__ void event_pixel(const int32_t* __restrict__ times,
                                             const T* __restrict__ data, uint32_t beg, int n,
@@ -96,7 +101,8 @@ __device__ __forceinline__ void event_pixel(const int32_t* __restrict__ times,
                                             const int* pd,
                                             typename EvHist<T>::type* __restrict__ hist,
                                             unsigned long long* __restrict__ nwin, long long& used,
-                                            long long sq, int* __restrict__ err) {
+                                            long long sq, int64_t* __restrict__ srow,
+                                            int* __restrict__ err) {
     using H = typename EvHist<T>::type;
     constexpr bool BOUNDED = sizeof(H) == 4;
     auto time_of = [&](int k) -> int {
@@ -118,6 +124,7 @@ __device__ __forceinline__ void event_pixel(const int32_t* __restrict__ times,
         for (int k = lane; k < n; k += 64) {
             const int t = time_of(k);
             if (t < 0 || t >= nframes) bad = 1;
+            else if (srow) add_sum(srow + t, (long long)count_of(k));
             if (k + 1 < n && time_of(k + 1) <= t) bad = 1;
         }
         if (bad) atomicOr(err, 1);
@@ -224,7 +231,7 @@ __device__ __forceinline__ void event_pairs_item(
     const int32_t* __restrict__ times, const T* __restrict__ data,
     const uint32_t* __restrict__ offsets, const int32_t* __restrict__ pix_idx,
     const BinDev* __restrict__ bins, const EventWork w, int nframes, int64_t nnz,
-    int64_t* __restrict__ num, int* __restrict__ err,
+    int64_t* __restrict__ num, int64_t* __restrict__ sums, int* __restrict__ err,
     typename EvHist<T>::type* __restrict__ hist, int (*__restrict__ st)[NW][ECAP]) {
     int (*const st_t)[ECAP] = st[0];
     int (*const st_d)[ECAP] = st[1];
@@ -241,6 +248,7 @@ __device__ __forceinline__ void event_pairs_item(
     for (int k = threadIdx.x; k < EW; k += NT) hist[k] = 0;
     __syncthreads();
     unsigned long long* nwin = reinterpret_cast<unsigned long long*>(num + (int64_t)w.bin * nframes + w0);
+    int64_t* srow = sums ? sums + (int64_t)w.bin * nframes : nullptr;
     long long used = 0;  // this wave's sum of d^2 added to the histogram (BOUNDED)
 
     // The wave takes pixels w.k0 + wave + NW r, r < nr.  Their list entries and offsets are
@@ -323,10 +331,10 @@ __device__ __forceinline__ void event_pairs_item(
         __builtin_amdgcn_wave_barrier();
         if (staged)
             event_pixel<T, NW, true>(times, data, beg, n, lane, w0, w1, nframes, st_t[wave],
-                                     st_d[wave], hist, nwin, used, sq, err);
+                                     st_d[wave], hist, nwin, used, sq, srow, err);
         else
             event_pixel<T, NW, false>(times, data, beg, n, lane, w0, w1, nframes, nullptr, nullptr,
-                                      hist, nwin, used, 0, err);
+                                      hist, nwin, used, 0, srow, err);
         __builtin_amdgcn_wave_barrier();
     }
     __syncthreads();
@@ -341,11 +349,11 @@ __global__ __launch_bounds__(64 * NW) void event_pairs_kernel(
     const int32_t* __restrict__ times, const T* __restrict__ data,
     const uint32_t* __restrict__ offsets, const int32_t* __restrict__ pix_idx,
     const BinDev* __restrict__ bins, const EventWork* __restrict__ work, int nframes,
-    int64_t nnz, int64_t* __restrict__ num, int* __restrict__ err) {
+    int64_t nnz, int64_t* __restrict__ num, int64_t* __restrict__ sums, int* __restrict__ err) {
     __shared__ typename EvHist<T>::type hist[EvHist<T>::lags_per_wave * NW];
     __shared__ __attribute__((aligned(16))) int st[2][NW][ECAP];
     event_pairs_item<T, NW>(times, data, offsets, pix_idx, bins, work[blockIdx.x], nframes, nnz,
-                            num, err, hist, st);
+                            num, sums, err, hist, st);
 }
 
 // A pointer read from a job table, marked as global memory (a generic pointer would
@@ -360,7 +368,7 @@ __device__ __forceinline__ P* global_ptr(P* p) {
 // lag windows past a job's frame count return at once.
 template <typename T, int NW>
 __global__ __launch_bounds__(64 * NW) void event_pairs_jobs_kernel(
-    const EventJob* __restrict__ jobs, const EventWork* __restrict__ work) {
+    const EventJob* __restrict__ jobs, const EventWork* __restrict__ work, bool with_sums) {
     __shared__ typename EvHist<T>::type hist[EvHist<T>::lags_per_wave * NW];
     __shared__ __attribute__((aligned(16))) int st[2][NW][ECAP];
     const EventWork w = work[blockIdx.x];
@@ -368,16 +376,18 @@ __global__ __launch_bounds__(64 * NW) void event_pairs_jobs_kernel(
     const EventJob j = jobs[w.pad];
     event_pairs_item<T, NW>(global_ptr(j.times), global_ptr(reinterpret_cast<const T*>(j.data)),
                             global_ptr(j.offsets), global_ptr(j.pix), global_ptr(j.bins), w,
-                            j.nframes, j.nnz, global_ptr(j.num), global_ptr(j.err), hist, st);
+                            j.nframes, j.nnz, global_ptr(j.num),
+                            with_sums ? global_ptr(j.sums) : nullptr, global_ptr(j.err), hist, st);
 }
 
 // Frame sums S_b(t) of a work item's pixels (densecorrelator.cl:65-150 has them dense,
 // evtcorrelator.cl:40 adds each event to global memory), in LDS counters of the frames [t0, t0 +
-// window) and from there to `sums`.  One 64-bit global atomic an event, as the pair kernel had
-// them, held a call at 17-23e9 events/s whatever its pairs.  A wave loads the ranges of 64
-// pixels and streams each stretch of them that is one run of the event list (neighbours in a
-// row are).  32-bit counters: an item has at most EVENT_ITEM_MAX pixels, each with one event a
-// frame.  Ranges and frames that the pair kernel reports as invalid are left out.
+// window) and from there to `sums`.  One 64-bit global atomic an event holds a call at 17-23e9
+// events/s whatever its pairs, and is left to calls of few events (sums_with_pairs()).  A wave
+// loads the ranges of 64 pixels and streams each stretch of them that is one run of the event
+// list (neighbours in a row are).  32-bit counters: an item has at most EVENT_ITEM_MAX pixels,
+// each with one event a frame.  Ranges and frames that the pair kernel reports as invalid are
+// left out.
 constexpr int SUMS_WINDOW = 40000;  // frames: 160,000 bytes
 template <typename T>
 __device__ __forceinline__ void event_sums_item(const int32_t* __restrict__ times,
@@ -465,6 +475,18 @@ static int sums_window(int nframes) {
     const int n = (nframes + SUMS_WINDOW - 1) / SUMS_WINDOW;
     return (nframes + n - 1) / n;
 }
+// Whether the pair kernel adds each event to its frame's sum by a global atomic (add_sum) and
+// event_sums_item()'s launch is left out.  So few events that their atomics, at about 21e9/s
+// beside the pairs, take less than that launch, and that LDS counters (`counters`: frames of every
+// item) would join none of them.  Pairs and sums with the launch -> without: 8-bit, 128 x 128 x
+// 400,000 (1.6e6 events, 13 windows) 264 -> 233 us, 514 x 1030 x 40,000 (2.1e6, 2 windows) 167 ->
+// 166, 300 x 300 x 40,000 (3.6e6) 165 -> 191; 16-bit, whose pairs take longer, 512 x 512 x 100,000
+// (5.2e6) 1,327 -> 1,234, 300 x 300 x 30,000 (2.7e6) 286 -> 264, 514 x 1030 x 5,000 (1.3e7)
+// 692 -> 720.
+template <typename T>
+static bool sums_with_pairs(int64_t counters, int64_t nnz) {
+    return nnz <= std::min<int64_t>(counters, sizeof(T) == 1 ? 2000000 : 7000000);
+}
 // Threads: two workgroups share a CU's threads where their counters leave room for it.
 static int sums_threads(int window) { return window > SUMS_WINDOW / 2 ? 1024 : 512; }
 
@@ -519,8 +541,8 @@ __device__ __forceinline__ void event_flat_item(
     const int32_t* __restrict__ times, const T* __restrict__ data,
     const uint32_t* __restrict__ offsets, const int32_t* __restrict__ pix_idx,
     const BinDev* __restrict__ bins, const EventWork w, int nframes, int64_t nnz,
-    int64_t* __restrict__ num, int* __restrict__ err, uint32_t* __restrict__ hist,
-    uint32_t* __restrict__ stages) {
+    int64_t* __restrict__ num, int64_t* __restrict__ sums, int* __restrict__ err,
+    uint32_t* __restrict__ hist, uint32_t* __restrict__ stages) {
     constexpr int R = FLAT_EVENTS / 64;
     const int w0 = ONE ? 0 : (int)blockIdx.y * FLAT_WINDOW;
     if (w0 >= nframes) return;
@@ -532,6 +554,7 @@ __device__ __forceinline__ void event_flat_item(
     const int32_t* list = pix_idx + bins[w.bin].idx_off;
     unsigned long long* nwin =
         reinterpret_cast<unsigned long long*>(num + (int64_t)w.bin * nframes + w0);
+    int64_t* srow = sums && w0 == 0 ? sums + (int64_t)w.bin * nframes : nullptr;
     uint32_t* st = stages + wave * FLAT_STAGE;
     uint8_t* marks = reinterpret_cast<uint8_t*>(st + FLAT_STAGE - FLAT_EVENTS / 4);
     long long used = 0;  // this wave's sum of d^2 in the histogram (EvHist)
@@ -561,7 +584,8 @@ __device__ __forceinline__ void event_flat_item(
             event_pixel<T, FLAT_WAVES, false>(times, data,
                                               (uint32_t)__builtin_amdgcn_readlane((int)beg, l),
                                               __builtin_amdgcn_readlane(n, l), lane, w0, w0 + span,
-                                              nframes, nullptr, nullptr, hist, nwin, used, 0, err);
+                                              nframes, nullptr, nullptr, hist, nwin, used, 0, srow,
+                                              err);
         }
         if (n > FLAT_EVENTS) n = 0;
         // events and staged words of the lanes up to and with this one
@@ -606,6 +630,8 @@ __device__ __forceinline__ void event_flat_item(
                 if ((unsigned)t_[r] >= (unsigned)nframes) {
                     bad = 1;
                     t_[r] = 0;
+                } else if (srow) {
+                    add_sum(srow + t_[r], d_[r]);
                 }
                 const uint32_t word = (uint32_t)t_[r] << 10 | ((uint32_t)d_[r] & 0xFFu);
                 if (n_[r]) {
@@ -712,21 +738,22 @@ __global__ __launch_bounds__(64 * FLAT_WAVES) void event_flat_kernel(
     const int32_t* __restrict__ times, const T* __restrict__ data,
     const uint32_t* __restrict__ offsets, const int32_t* __restrict__ pix_idx,
     const BinDev* __restrict__ bins, const EventWork* __restrict__ work, int nframes, int64_t nnz,
-    int64_t* __restrict__ num, int* __restrict__ err) {
+    int64_t* __restrict__ num, int64_t* __restrict__ sums, int* __restrict__ err) {
     extern __shared__ uint32_t flat_lds[];
     event_flat_item<T, ONE>(times, data, offsets, pix_idx, bins, work[blockIdx.x], nframes, nnz, num,
-                            err, flat_lds + FLAT_WAVES * FLAT_STAGE, flat_lds);
+                            sums, err, flat_lds + FLAT_WAVES * FLAT_STAGE, flat_lds);
 }
 template <typename T, bool ONE>
 __global__ __launch_bounds__(64 * FLAT_WAVES) void event_flat_jobs_kernel(
-    const EventJob* __restrict__ jobs, const EventWork* __restrict__ work) {
+    const EventJob* __restrict__ jobs, const EventWork* __restrict__ work, bool with_sums) {
     extern __shared__ uint32_t flat_lds[];
     const EventWork w = work[blockIdx.x];
     if (w.bin < 0) return;
     const EventJob j = jobs[w.pad];
     event_flat_item<T, ONE>(global_ptr(j.times), global_ptr(reinterpret_cast<const T*>(j.data)),
                             global_ptr(j.offsets), global_ptr(j.pix), global_ptr(j.bins), w,
-                            j.nframes, j.nnz, global_ptr(j.num), global_ptr(j.err),
+                            j.nframes, j.nnz, global_ptr(j.num),
+                            with_sums ? global_ptr(j.sums) : nullptr, global_ptr(j.err),
                             flat_lds + FLAT_WAVES * FLAT_STAGE, flat_lds);
 }
 static size_t flat_lds_bytes(int nframes) {
@@ -752,46 +779,50 @@ int event_lag_window(int dtype, int nframes) {
 
 template <typename T, int NW>
 void pairs_jobs_launch(const EventJob* jobs, const EventWork* work, int n_work, int max_frames,
-                       hipStream_t s) {
+                       int64_t counters, int64_t nnz, hipStream_t s) {
     constexpr int WS = EvHist<T>::window(NW);
+    const bool with_sums = sums_with_pairs<T>(counters, nnz);
     const int win = sums_window(max_frames);
-    event_sums_jobs_kernel<T><<<dim3((unsigned)n_work, (unsigned)((max_frames + win - 1) / win)),
-                                sums_threads(win), 4 * win, s>>>(jobs, work, win);
+    if (!with_sums)
+        event_sums_jobs_kernel<T><<<dim3((unsigned)n_work, (unsigned)((max_frames + win - 1) / win)),
+                                    sums_threads(win), 4 * win, s>>>(jobs, work, win);
     if constexpr (sizeof(T) == 1) {
         if (max_frames <= FLAT_FRAMES) {
             const dim3 grid((unsigned)n_work, (unsigned)((max_frames + FLAT_WINDOW - 1) / FLAT_WINDOW));
             const size_t lds = flat_lds_bytes(max_frames);
             if (grid.y == 1)
-                event_flat_jobs_kernel<T, true><<<grid, 64 * FLAT_WAVES, lds, s>>>(jobs, work);
+                event_flat_jobs_kernel<T, true><<<grid, 64 * FLAT_WAVES, lds, s>>>(jobs, work,
+                                                                                   with_sums);
             else
-                event_flat_jobs_kernel<T, false><<<grid, 64 * FLAT_WAVES, lds, s>>>(jobs, work);
+                event_flat_jobs_kernel<T, false><<<grid, 64 * FLAT_WAVES, lds, s>>>(jobs, work,
+                                                                                    with_sums);
             return;
         }
     }
     event_pairs_jobs_kernel<T, NW><<<dim3((unsigned)n_work, (unsigned)((max_frames + WS - 1) / WS)),
-                                     64 * NW, 0, s>>>(jobs, work);
+                                     64 * NW, 0, s>>>(jobs, work, with_sums);
 }
 
 template <typename T>
 void pairs_jobs_typed(const EventJob* jobs, const EventWork* work, int n_work, int max_frames,
-                      hipStream_t s) {
+                      int64_t counters, int64_t nnz, hipStream_t s) {
     if (event_waves() == 4)
-        pairs_jobs_launch<T, 4>(jobs, work, n_work, max_frames, s);
+        pairs_jobs_launch<T, 4>(jobs, work, n_work, max_frames, counters, nnz, s);
     else if (event_waves() == 16)
-        pairs_jobs_launch<T, 16>(jobs, work, n_work, max_frames, s);
+        pairs_jobs_launch<T, 16>(jobs, work, n_work, max_frames, counters, nnz, s);
     else
-        pairs_jobs_launch<T, 8>(jobs, work, n_work, max_frames, s);
+        pairs_jobs_launch<T, 8>(jobs, work, n_work, max_frames, counters, nnz, s);
 }
 
 void launch_event_pairs_jobs(int dtype, const EventJob* jobs, const EventWork* work, int n_work,
-                             int max_frames, hipStream_t s) {
+                             int max_frames, int64_t counters, int64_t nnz, hipStream_t s) {
     if (n_work <= 0 || max_frames <= 0) return;
     if (dtype == DXG2_U16)
-        pairs_jobs_typed<uint16_t>(jobs, work, n_work, max_frames, s);
+        pairs_jobs_typed<uint16_t>(jobs, work, n_work, max_frames, counters, nnz, s);
     else if (dtype == DXG2_I8)
-        pairs_jobs_typed<int8_t>(jobs, work, n_work, max_frames, s);
+        pairs_jobs_typed<int8_t>(jobs, work, n_work, max_frames, counters, nnz, s);
     else
-        pairs_jobs_typed<uint8_t>(jobs, work, n_work, max_frames, s);
+        pairs_jobs_typed<uint8_t>(jobs, work, n_work, max_frames, counters, nnz, s);
 }
 
 template <typename T, int NW>
@@ -799,26 +830,33 @@ void pairs_launch(const int32_t* times, const void* data, const uint32_t* offset
                   const int32_t* pix_idx, const BinDev* bins, const EventWork* work, int n_work,
                   int nframes, int64_t nnz, int64_t* num, int64_t* sums, int* err, hipStream_t s) {
     constexpr int WS = EvHist<T>::window(NW);
-    const int win = sums_window(nframes);
-    event_sums_kernel<T><<<dim3((unsigned)n_work, (unsigned)((nframes + win - 1) / win)),
-                           sums_threads(win), 4 * win, s>>>(times, (const T*)data, offsets, pix_idx,
-                                                            bins, work, nframes, nnz, win, sums);
+    int64_t* psums = nullptr;  // frame sums of the pair kernel
+    if (sums_with_pairs<T>((int64_t)n_work * nframes, nnz)) {
+        psums = sums;
+    } else {
+        const int win = sums_window(nframes);
+        event_sums_kernel<T><<<dim3((unsigned)n_work, (unsigned)((nframes + win - 1) / win)),
+                               sums_threads(win), 4 * win, s>>>(
+            times, (const T*)data, offsets, pix_idx, bins, work, nframes, nnz, win, sums);
+    }
     if constexpr (sizeof(T) == 1) {
         if (nframes <= FLAT_FRAMES) {
             const dim3 grid((unsigned)n_work, (unsigned)((nframes + FLAT_WINDOW - 1) / FLAT_WINDOW));
             const size_t lds = flat_lds_bytes(nframes);
             if (grid.y == 1)
                 event_flat_kernel<T, true><<<grid, 64 * FLAT_WAVES, lds, s>>>(
-                    times, (const T*)data, offsets, pix_idx, bins, work, nframes, nnz, num, err);
+                    times, (const T*)data, offsets, pix_idx, bins, work, nframes, nnz, num, psums,
+                    err);
             else
                 event_flat_kernel<T, false><<<grid, 64 * FLAT_WAVES, lds, s>>>(
-                    times, (const T*)data, offsets, pix_idx, bins, work, nframes, nnz, num, err);
+                    times, (const T*)data, offsets, pix_idx, bins, work, nframes, nnz, num, psums,
+                    err);
             return;
         }
     }
     event_pairs_kernel<T, NW><<<dim3((unsigned)n_work, (unsigned)((nframes + WS - 1) / WS)),
                                 64 * NW, 0, s>>>(times, (const T*)data, offsets, pix_idx, bins,
-                                                 work, nframes, nnz, num, err);
+                                                 work, nframes, nnz, num, psums, err);
 }
 
 template <typename T>

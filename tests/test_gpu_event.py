@@ -312,3 +312,32 @@ def test_more_frames_than_a_packed_word_holds():
     s, num = ev.event_sums_numerators_fast(times, data, offsets, q, n, [1])
     np.testing.assert_array_equal(c.last_numerators.cpu().numpy(), num)
     np.testing.assert_array_equal(c.last_sums.cpu().numpy(), s)
+
+
+@pytest.mark.parametrize("n,shape,p,dtype", [(20, (40, 64), 0.5, np.uint8),
+                                             (20, (40, 64), 0.5, np.int8),
+                                             (300, (33, 35), 0.3, np.uint16),
+                                             (90000, (8, 8), 0.02, np.uint8),
+                                             (90000, (8, 8), 0.02, np.uint16)])
+def test_frame_sums_of_many_events_a_frame(n, shape, p, dtype):
+    """More events than the items have frames in all, so that the frame sums come from LDS
+    counters (the other tests' few events add to them one by one): one and several windows of
+    frames, pixels of more events than a stage holds."""
+    from dynamix_amd.correlator.event import EventCorrelator
+    _announce("event sums n=%d %s" % (n, np.dtype(dtype).name))
+    rng = np.random.default_rng(n + shape[1])
+    npix = shape[0] * shape[1]
+    lo, hi = np.iinfo(dtype).min, np.iinfo(dtype).max
+    seen = rng.random((npix, n)) < p
+    counts = seen.sum(1)
+    times = np.nonzero(seen)[1].astype(np.int32)
+    data = rng.integers(lo, hi + 1, size=times.size).astype(dtype)
+    data[data == 0] = 1
+    offsets = np.concatenate([[0], np.cumsum(counts)]).astype(np.uint32)
+    q = np.ones(shape, np.int32)
+    q[0, ::3] = 0
+    c = EventCorrelator(shape, n, int(counts.max()), qmask=q, dtype=dtype)
+    c.correlate(times, data, offsets)
+    s, num = ev.event_sums_numerators_fast(times, data, offsets, q, n, [1])
+    np.testing.assert_array_equal(c.last_numerators.cpu().numpy(), num)
+    np.testing.assert_array_equal(c.last_sums.cpu().numpy(), s)
