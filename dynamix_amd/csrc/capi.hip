@@ -262,6 +262,7 @@ struct dxg2_plan {
     int* d_heads = nullptr;        // 16 queue heads, then the route's ints (k_narrow.hip)
     int8_t* d_slab = nullptr;
     int8_t* d_slab4 = nullptr;     // narrow slab (k_narrow.hip), half the slab's bytes
+    bool narrow_refused = false;   // its memory could not be had
     int64_t* d_wsums = nullptr;    // its wide pixels' frame sums, n_bins rows
     int64_t* d_ugram = nullptr;
     int64_t* d_sums = nullptr;
@@ -988,7 +989,8 @@ size_t narrow_bytes(const dxg2_plan* p) {
 }
 
 // Slab of the dense path, allocated on the first dense call and cleared on its stream:
-// rows past the last frame stay zero for the life of the plan.
+// rows past the last frame stay zero for the life of the plan.  The narrow slab beside it is an
+// option: a plan that is refused the memory once keeps every pixel in the i8 slab.
 int ensure_dense_buffers(dxg2_plan* p, hipStream_t s, bool narrow = false) {
     if (!p->d_slab && p->slab_bytes) {
         if (dev_alloc(p->alloc, (void**)&p->d_slab, p->slab_bytes, s) != hipSuccess) {
@@ -997,7 +999,7 @@ int ensure_dense_buffers(dxg2_plan* p, hipStream_t s, bool narrow = false) {
         }
         DXG2_HIP(hipMemsetAsync(p->d_slab, 0, p->slab_bytes, s));
     }
-    if (narrow && !p->d_slab4 && narrow_applies(p)) {
+    if (narrow && !p->d_slab4 && !p->narrow_refused && narrow_applies(p)) {
         // d_slab4 is set last: it marks the narrow workspace complete
         int8_t* slab4 = nullptr;
         int64_t* wsums = nullptr;
@@ -1013,7 +1015,9 @@ int ensure_dense_buffers(dxg2_plan* p, hipStream_t s, bool narrow = false) {
                 hipSuccess) {
             for (void* b : {(void*)slab4, (void*)wsums, (void*)flag, (void*)pixw, (void*)nwkb})
                 dev_free(p->alloc, b, s);
-            return set_error(DXG2_ENOMEM, "cannot allocate the narrow slab");
+            (void)hipGetLastError();
+            p->narrow_refused = true;
+            return DXG2_OK;
         }
         DXG2_HIP(hipMemsetAsync(slab4, 0, p->slab_bytes / 2, s));
         p->d_wsums = wsums;

@@ -1,0 +1,106 @@
+"""The narrow slab (FP4) is an option of the dense call: where it cannot be had, or would not
+be used, the call takes the i8 slab alone and gives the same integers."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from oracle import g2 as og
+
+pytestmark = pytest.mark.gpu
+
+SHAPE, N = (40, 48), 520
+
+
+class _Allocator(object):
+    """Device memory from torch's allocator, but for the size `refuse`; every size asked for."""
+
+    def __init__(self, refuse=0):
+        import torch
+        from dynamix_amd import _lib
+        self.refuse, self.sizes, self.live = refuse, [], 0
+        dev = torch.cuda.current_device()
+
+        def alloc(nbytes, stream, ctx):
+            self.sizes.append(int(nbytes))
+            if nbytes == self.refuse:
+                return None
+            self.live += 1
+            return torch.cuda.caching_allocator_alloc(int(nbytes), dev, int(stream or 0))
+
+        def free(ptr, stream, ctx):
+            self.live -= 1
+            torch.cuda.caching_allocator_delete(int(ptr))
+
+        self.lib = _lib.load()
+        self._alloc, self._free = _lib.ALLOC_FN(alloc), _lib.FREE_FN(free)
+
+    def plan(self, q, dtype):
+        """A plan that keeps this allocator."""
+        from dynamix_amd import _lib
+        from dynamix_amd.correlator.common import Plan
+        _lib.check(self.lib.dxg2_set_allocator(self._alloc, self._free, None))
+        try:
+            return Plan(SHAPE, N, q, dtype)
+        finally:
+            _lib.check(self.lib.dxg2_set_allocator(_lib.ALLOC_FN(), _lib.FREE_FN(), None))
+
+
+def _inputs(dtype=np.uint8):
+    rng = np.random.default_rng(5)
+    q = rng.integers(0, 4, size=SHAPE).astype(np.int32)
+    f = np.where(rng.random((N,) + SHAPE) < 0.1, rng.integers(1, 6, size=(N,) + SHAPE), 0)
+    return q, f.astype(dtype)
+
+
+def _slab4(q):
+    """Bytes of the narrow slab: half a byte an entry of the lists padded to 64 pixels, 768
+    rows (520 frames in steps of 256)."""
+    n = np.bincount(q.ravel(), minlength=4)[1:]
+    return int(((n + 63) // 64 * 64).sum()) * 768 // 2
+
+
+def _outs(nb):
+    import torch
+    return (torch.zeros((nb, N), dtype=torch.int64, device="cuda"),
+            torch.zeros((nb, N), dtype=torch.int64, device="cuda"),
+            torch.zeros((nb, N), dtype=torch.float64, device="cuda"),
+            torch.zeros((nb, N), dtype=torch.float32, device="cuda"))
+
+
+def _call(plan, frames, outs):
+    import torch
+    from dynamix_amd import _lib
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    _lib.check(plan.lib.dxg2_correlate_dense(plan.handle, _lib.ptr(frames),
+                                             *[_lib.ptr(x) for x in outs], st))
+
+
+def _check(outs, ref):
+    np.testing.assert_array_equal(outs[0].cpu().numpy(), ref["num"])
+    np.testing.assert_array_equal(outs[1].cpu().numpy(), ref["sums"])
+    np.testing.assert_array_equal(outs[2].cpu().numpy(), np.asarray(ref["den"], np.float64))
+
+
+@pytest.mark.parametrize("which", ["slab", "lists"])
+def test_refused_workspace_leaves_the_i8_route(which, monkeypatch):
+    """The narrow slab, or its wide pixels' list, is refused: the call succeeds on the i8 slab,
+    keeps nothing of the workspace and does not ask again."""
+    import torch
+    print("[case] narrow workspace refused: %s" % which, flush=True)
+    monkeypatch.setenv("DXG2_NARROW", "2")
+    q, f = _inputs()
+    slab4 = _slab4(q)
+    refuse = slab4 if which == "slab" else SHAPE[0] * SHAPE[1] + 16   # the flags of the pixels
+    a = _Allocator(refuse)
+    plan = a.plan(q, np.uint8)
+    outs, ref = _outs(3), og.dense_g2(f, q)
+    d = torch.from_numpy(f).cuda()
+    before = a.live
+    for _ in range(2):
+        _call(plan, d, outs)
+        _check(outs, ref)
+    assert a.sizes.count(refuse) == 1 and a.sizes.count(slab4) == 1
+    assert a.live == before + 1           # the i8 slab
+    plan.close()
+    assert a.live == 0
