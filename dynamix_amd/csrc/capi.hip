@@ -982,6 +982,10 @@ bool narrow_applies(const dxg2_plan* p) {
     return opt == 2 ||
            (opt && (double)p->pix_idx.size() * p->N * p->N >= NARROW_MIN_WORK);
 }
+// Narrow calls read the frames as the band gather does, 16 bytes at a time.
+bool narrow_frames(const void* d_frames) {
+    return reinterpret_cast<uintptr_t>(d_frames) % 16 == 0;
+}
 size_t narrow_bytes(const dxg2_plan* p) {
     if (!narrow_applies(p)) return 0;
     return p->slab_bytes / 2 + (size_t)p->n_bins * p->N * sizeof(int64_t) + p->pix_idx.size() * 4 +
@@ -1039,7 +1043,7 @@ int ensure_dense_buffers(dxg2_plan* p, hipStream_t s, bool narrow = false) {
 // Narrow calls (uint8/int8 plans; the plain dense calls, with the same frames throughout) fill
 // the narrow slab or the i8 slab, as decided on the device (k_narrow.hip).
 bool narrow_call(const dxg2_plan* p, const void* d_frames) {
-    return p->d_slab4 && narrow_applies(p) && reinterpret_cast<uintptr_t>(d_frames) % 16 == 0;
+    return p->d_slab4 && narrow_applies(p) && narrow_frames(d_frames);
 }
 // one (not with wide_first; may be null): gather only the bin whose slots it has.
 int64_t* dense_gather(dxg2_plan* p, const void* d_frames, int64_t* d_sums, hipStream_t s,
@@ -1591,7 +1595,7 @@ int dxg2_correlate_dense(dxg2_plan* p, const void* d_frames, int64_t* d_num, int
     if (!d_frames || !d_g2) return set_error(DXG2_EINVAL, "frames and g2 must be non-null");
     if (p->n_bins == 0) return DXG2_OK;
     hipStream_t s = (hipStream_t)stream;
-    int rc = ensure_dense_buffers(p, s, true);
+    int rc = ensure_dense_buffers(p, s, narrow_frames(d_frames));
     if (rc) return rc;
     (void)hipGetLastError();
     hipEvent_t* ev = nullptr;
@@ -1713,7 +1717,8 @@ int dxg2_correlate_dense_graph(dxg2_plan* p, const void* d_frames, int64_t* d_nu
     if (!d_frames || !d_g2) return set_error(DXG2_EINVAL, "frames and g2 must be non-null");
     if (p->n_bins == 0) return DXG2_OK;
     hipStream_t s = (hipStream_t)stream;
-    int rc = ensure_dense_buffers(p, s, true);  // the one-time slab clears run eagerly, on s
+    // the one-time slab clears run eagerly, on s
+    int rc = ensure_dense_buffers(p, s, narrow_frames(d_frames));
     if (rc) return rc;
     const std::array<const void*, 5> key{d_frames, d_num, d_sums, d_den, d_g2};
     if (!p->gexec || key != p->gkey) {

@@ -104,3 +104,24 @@ def test_refused_workspace_leaves_the_i8_route(which, monkeypatch):
     assert a.live == before + 1           # the i8 slab
     plan.close()
     assert a.live == 0
+
+
+def test_frames_that_cannot_use_it_do_not_make_it(monkeypatch):
+    """Frames at an odd address take the general gather: no narrow slab is allocated for them."""
+    import torch
+    print("[case] narrow workspace, frames at an odd address", flush=True)
+    monkeypatch.setenv("DXG2_NARROW", "2")
+    q, f = _inputs()
+    a = _Allocator()
+    plan = a.plan(q, np.uint8)
+    outs, ref = _outs(3), og.dense_g2(f, q)
+    buf = torch.empty(f.size + 16, dtype=torch.uint8, device="cuda")
+    odd = buf[1:1 + f.size].view(f.shape)
+    odd.copy_(torch.from_numpy(f))
+    _call(plan, odd, outs)
+    _check(outs, ref)
+    assert _slab4(q) not in a.sizes
+    _call(plan, torch.from_numpy(f).cuda(), outs)
+    _check(outs, ref)
+    assert a.sizes.count(_slab4(q)) == 1
+    plan.close()
