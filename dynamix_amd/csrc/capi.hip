@@ -992,9 +992,19 @@ size_t narrow_bytes(const dxg2_plan* p) {
            (size_t)p->H * p->W + 16 + (size_t)(2 * p->n_bins + 1) * sizeof(int);
 }
 
+// Whether the caller records s into a graph, or that cannot be told (the null stream while
+// another one records).
+bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+
 // Slab of the dense path, allocated on the first dense call and cleared on its stream:
 // rows past the last frame stay zero for the life of the plan.  The narrow slab beside it is an
-// option: a plan that is refused the memory once keeps every pixel in the i8 slab.
+// option: a plan that is refused the memory once keeps every pixel in the i8 slab, and a call
+// recorded into a caller's graph neither allocates nor clears it.
 int ensure_dense_buffers(dxg2_plan* p, hipStream_t s, bool narrow = false) {
     if (!p->d_slab && p->slab_bytes) {
         if (dev_alloc(p->alloc, (void**)&p->d_slab, p->slab_bytes, s) != hipSuccess) {
@@ -1003,7 +1013,7 @@ int ensure_dense_buffers(dxg2_plan* p, hipStream_t s, bool narrow = false) {
         }
         DXG2_HIP(hipMemsetAsync(p->d_slab, 0, p->slab_bytes, s));
     }
-    if (narrow && !p->d_slab4 && !p->narrow_refused && narrow_applies(p)) {
+    if (narrow && !p->d_slab4 && !p->narrow_refused && narrow_applies(p) && !capturing(s)) {
         // d_slab4 is set last: it marks the narrow workspace complete
         int8_t* slab4 = nullptr;
         int64_t* wsums = nullptr;

@@ -125,3 +125,38 @@ def test_frames_that_cannot_use_it_do_not_make_it(monkeypatch):
     _check(outs, ref)
     assert a.sizes.count(_slab4(q)) == 1
     plan.close()
+
+
+def test_capture_after_another_dense_call(monkeypatch):
+    """A plan that has its i8 slab (from a calc_std call) and is then captured by its user's
+    graph: the plain call allocates and clears nothing under the capture.  Several replays,
+    each against the oracle."""
+    import torch
+    from dynamix_amd import _lib
+    from dynamix_amd.correlator.common import Plan
+    print("[case] plain dense call first made under capture", flush=True)
+    monkeypatch.setenv("DXG2_NARROW", "2")
+    q, f = _inputs()
+    other = (f[::-1] % 5).copy()
+    refs = [og.dense_g2(f, q), og.dense_g2(other, q)]
+    plan = Plan(SHAPE, N, q, np.uint8)
+    outs = _outs(3)
+    d = torch.from_numpy(f).cuda()
+    dev = torch.zeros((3, N), dtype=torch.float32, device="cuda")
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    _lib.check(plan.lib.dxg2_correlate_dense_std(plan.handle, _lib.ptr(d),
+                                                 *[_lib.ptr(x) for x in outs], _lib.ptr(dev), st))
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        _call(plan, d, outs)
+    for k in range(4):
+        d.copy_(torch.from_numpy(other if k % 2 else f))
+        for x in outs:
+            x.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        _check(outs, refs[k % 2])
+        (torch.randn(1 << 16, device="cuda") * 2).sum().item()
+    _call(plan, d, outs)                  # the same plan, eagerly, may take the narrow route
+    _check(outs, refs[1])
