@@ -262,6 +262,7 @@ struct dxg2_plan {
     int* d_heads = nullptr;        // 16 queue heads, then the route's ints (k_narrow.hip)
     int8_t* d_slab = nullptr;
     int8_t* d_slab4 = nullptr;     // narrow slab (k_narrow.hip), half the slab's bytes
+    int narrow_opt = 1;            // narrow_applies()
     bool narrow_refused = false;   // its memory could not be had
     int64_t* d_wsums = nullptr;    // its wide pixels' frame sums, n_bins rows
     int64_t* d_ugram = nullptr;
@@ -972,15 +973,14 @@ int ensure_event_buffers(dxg2_plan* p, int64_t nnz_coo, hipStream_t s) {
 // Plans whose plain dense calls may keep narrow pixels in FP4 (k_narrow.hip): 8-bit frames
 // through the band gather and the persistent launch of 256-frame tiles, with enough Gram work
 // (pixels x frames^2) that halving it pays for the launches of the narrow route
-// (DXG2_NARROW: 0 never, 2 whatever the work).
+// (DXG2_NARROW, read when the plan is created: 0 never, 2 whatever the work).
 constexpr double NARROW_MIN_WORK = 5e11;
 constexpr int HEAD_INTS = 24;
 bool narrow_applies(const dxg2_plan* p) {
     if (p->dtype == DXG2_U16 || p->gband.empty() || !p->use_queue || p->gram_tile != 256)
         return false;
-    const int opt = env_int("DXG2_NARROW", 1);
-    return opt == 2 ||
-           (opt && (double)p->pix_idx.size() * p->N * p->N >= NARROW_MIN_WORK);
+    return p->narrow_opt == 2 ||
+           (p->narrow_opt && (double)p->pix_idx.size() * p->N * p->N >= NARROW_MIN_WORK);
 }
 // Narrow calls read the frames as the band gather does, 16 bytes at a time.
 bool narrow_frames(const void* d_frames) {
@@ -1237,6 +1237,7 @@ dxg2_plan* build_plan_host(const dxg2_plan_desc* desc, int* rc) {
     p->tune_kchunk = std::min(MAX_KBLOCKS_PER_ITEM,
                               std::max(1, env_int("DXG2_GRAM_KCHUNK", default_kchunk(p->dtype))));
     p->use_queue = env_int("DXG2_GRAM_QUEUE", 1) != 0 && !(desc->flags & DXG2_FLAG_NO_QUEUE);
+    p->narrow_opt = env_int("DXG2_NARROW", 1);
     // i8-MFMA denominators for the bins whose frame sums fit two digits; DXG2_DEN_MFMA=0
     // leaves every bin to the VALU kernels
     p->dmf.up = env_int("DXG2_DEN_MFMA", 1) ? den_mfma_columns(p->N) : 0;

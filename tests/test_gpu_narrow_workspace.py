@@ -160,3 +160,25 @@ def test_capture_after_another_dense_call(monkeypatch):
         (torch.randn(1 << 16, device="cuda") * 2).sum().item()
     _call(plan, d, outs)                  # the same plan, eagerly, may take the narrow route
     _check(outs, refs[1])
+
+
+def test_settings_are_read_when_the_plan_is_created(monkeypatch):
+    """DXG2_NARROW is a setting of the plan: a change after its creation moves neither its
+    footprint nor its route."""
+    import torch
+    print("[case] DXG2_NARROW changed after the plan's creation", flush=True)
+    q, f = _inputs()
+    ref, outs, d = og.dense_g2(f, q), _outs(3), torch.from_numpy(f).cuda()
+    size = {}
+    for made, later in (("2", "0"), ("0", "2")):
+        monkeypatch.setenv("DXG2_NARROW", made)
+        a = _Allocator()
+        plan = a.plan(q, np.uint8)
+        size[made] = plan.footprint(0)
+        monkeypatch.setenv("DXG2_NARROW", later)
+        assert plan.footprint(0) == size[made]
+        _call(plan, d, outs)
+        _check(outs, ref)
+        assert (_slab4(q) in a.sizes) == (made == "2")
+        plan.close()
+    assert size["2"] > size["0"] + _slab4(q)
