@@ -53,7 +53,7 @@ METRIC = ("g2 pixel·frames/s at 514×1030×10k uint8, 20 bins; "
           "p50/p99 mixed-job latency")
 INT8_PEAK_TOPS = 5000.0   # MI355X dense int8 MFMA, 5.0 POP/s
 FP4_PEAK_TOPS = 10000.0   # dense FP4 MFMA
-NARROW_MIN_WORK, NARROW_MAX, NARROW_WIDE = 5e11, 4, 0.3  # the library's narrow route
+NARROW_MAX = 4           # largest count of a pixel in FP4
 HBM_PEAK_GBS = 8000.0
 
 
@@ -115,22 +115,13 @@ def gather_roofline(qmask, shape, n, gather_ms, narrow):
             "kernel": "gather_band_f4_kernel" if narrow else "gather_band_kernel"}
 
 
-def gram_peak(frames, qmask, n):
-    """Peak TOP/s of the Gram of these 8-bit frames and the share of wide pixels (None: every
-    pixel in i8): FP4 for all pixels and i8 for the wide ones on the narrow route."""
-    import torch
-    inside = torch.from_numpy(qmask.ravel() > 0).to(frames.device)
-    npix = int(inside.sum())
-    if frames.element_size() != 1 or npix * n * n < NARROW_MIN_WORK:
+def gram_peak(plan, npix):
+    """Peak TOP/s of the Gram of the plan's last dense call and the share of wide pixels (None:
+    every pixel in i8): FP4 for all pixels and i8 for the wide ones on the narrow route."""
+    fp4, wide = plan.dense_route()
+    if not fp4:
         return INT8_PEAK_TOPS, None
-    top, low = frames.amax(0).ravel(), frames.amin(0).ravel()
-    wide = top > NARROW_MAX
-    if frames.dtype == torch.int8:
-        wide |= low < -NARROW_MAX
-    share = float((wide & inside).sum()) / npix
-    if share > NARROW_WIDE:
-        return INT8_PEAK_TOPS, None
-    return 1.0 / (1.0 / FP4_PEAK_TOPS + share / INT8_PEAK_TOPS), share
+    return 1.0 / (1.0 / FP4_PEAK_TOPS + wide / npix / INT8_PEAK_TOPS), wide / npix
 
 
 def cpu_baseline_fft(frames_dev, qmask, target_s=8.0, chunk=4096):
@@ -568,7 +559,7 @@ def main():
     # sanity: g2 finite where denominators are positive
     assert torch.isfinite(g2[den > 0]).all().item()
 
-    peak, wide_share = gram_peak(frames, q, n)
+    peak, wide_share = gram_peak(plan, npix)
     out = {
         "metric": METRIC,
         "value": pf / (ms * 1e-3),

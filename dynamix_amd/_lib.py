@@ -84,6 +84,8 @@ _SIGNATURES = {
     "dxg2_plan_event_status": (c_int, [c_void_p, ctypes.POINTER(c_int), c_void_p]),
     "dxg2_plan_set_profiling": (c_int, [c_void_p, c_int]),
     "dxg2_plan_stage_times": (c_int, [c_void_p, c_void_p, c_int]),
+    "dxg2_plan_dense_route": (c_int, [c_void_p, ctypes.POINTER(c_int), ctypes.POINTER(c_i64),
+                                      c_void_p]),
     "dxg2_synth_speckle": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_double,
                                    c_u64, c_void_p]),
     "dxg2_synth_events": (c_int, [c_void_p, c_int, c_int, c_int, c_double, c_u64, c_int,

@@ -164,6 +164,13 @@ class Plan(object):
         _lib.check(self.lib.dxg2_plan_stage_times(self.handle, t, 5))
         return list(t)
 
+    def dense_route(self):
+        """The last dense call's Gram: (narrow pixels in FP4?, wide pixels beside them)."""
+        fp4, wide = ctypes.c_int32(), ctypes.c_int64()
+        _lib.check(self.lib.dxg2_plan_dense_route(self.handle, ctypes.byref(fp4),
+                                                  ctypes.byref(wide), current_stream(_torch())))
+        return bool(fp4.value), wide.value
+
     def close(self):
         """Release the plan (waits for the device)."""
         if getattr(self, "handle", None):

@@ -263,6 +263,8 @@ struct dxg2_plan {
     int8_t* d_slab = nullptr;
     int8_t* d_slab4 = nullptr;     // narrow slab (k_narrow.hip), half the slab's bytes
     int narrow_opt = 1;            // narrow_applies()
+    bool last_narrow = false;      // the last dense call was a narrow call
+    bool graph_narrow = false;     // the captured one is
     bool narrow_refused = false;   // its memory could not be had
     int64_t* d_wsums = nullptr;    // its wide pixels' frame sums, n_bins rows
     int64_t* d_ugram = nullptr;
@@ -1065,7 +1067,8 @@ int64_t* dense_gather(dxg2_plan* p, const void* d_frames, int64_t* d_sums, hipSt
     const int64_t hw = (int64_t)p->H * p->W;
     int64_t max_npix = 0;
     for (auto n : p->npix) max_npix = std::max(max_npix, n);
-    if (wide_first && narrow_call(p, d_frames)) {
+    p->last_narrow = wide_first && narrow_call(p, d_frames);
+    if (p->last_narrow) {
         const uint8_t* frames = (const uint8_t*)d_frames;
         const int* route = p->d_heads + 16;
         launch_clear_call(gsums, nbn, p->d_ugram, nbn, p->d_heads, HEAD_INTS, s, p->d_wflag, hw,
@@ -1623,6 +1626,25 @@ int dxg2_correlate_dense(dxg2_plan* p, const void* d_frames, int64_t* d_num, int
     return DXG2_OK;
 }
 
+int dxg2_plan_dense_route(dxg2_plan* p, int32_t* fp4, int64_t* wide_pixels, void* stream) {
+    if (!p || !fp4) return set_error(DXG2_EINVAL, "null argument");
+    *fp4 = 0;
+    if (wide_pixels) *wide_pixels = 0;
+    if (!p->last_narrow) return DXG2_OK;
+    hipStream_t s = (hipStream_t)stream;
+    int route = NARROW_OFF;
+    std::vector<int> wide(p->n_bins);
+    DXG2_HIP(hipMemcpyAsync(&route, p->d_heads + 16, sizeof(int), hipMemcpyDeviceToHost, s));
+    DXG2_HIP(hipMemcpyAsync(wide.data(), p->d_nwkb + p->n_bins + 1, wide.size() * sizeof(int),
+                            hipMemcpyDeviceToHost, s));
+    DXG2_HIP(hipStreamSynchronize(s));
+    if (route != NARROW_F4) return DXG2_OK;
+    *fp4 = 1;
+    for (int w : wide)
+        if (wide_pixels) *wide_pixels += w;
+    return DXG2_OK;
+}
+
 int dxg2_plan_get_tuning(const dxg2_plan* p, dxg2_tuning* t) {
     if (!p || !t) return set_error(DXG2_EINVAL, "null argument");
     t->tile = p->gram_tile;
@@ -1740,7 +1762,7 @@ int dxg2_correlate_dense_graph(dxg2_plan* p, const void* d_frames, int64_t* d_nu
         (void)hipGetLastError();
         DXG2_HIP(hipStreamBeginCapture(p->cap_stream, hipStreamCaptureModeThreadLocal));
         int64_t* gsums = dense_gather(p, d_frames, d_sums, p->cap_stream, true);
-        const bool narrow = narrow_call(p, d_frames);
+        const bool narrow = p->graph_narrow = narrow_call(p, d_frames);
         dense_gram(p, gsums, p->cap_stream, true, narrow);
         dense_finish(p, gsums, d_num, d_sums, d_den, d_g2, p->cap_stream, true, narrow);
         hipGraph_t g = nullptr;
@@ -1760,6 +1782,7 @@ int dxg2_correlate_dense_graph(dxg2_plan* p, const void* d_frames, int64_t* d_nu
         p->gkey = key;
     }
     DXG2_HIP(hipGraphLaunch(p->gexec, s));
+    p->last_narrow = p->graph_narrow;
     return DXG2_OK;
 }
 

@@ -259,6 +259,13 @@ int dxg2_plan_event_status(dxg2_plan* plan, int32_t* flags, void* stream);
 int dxg2_plan_set_profiling(dxg2_plan* plan, int32_t on);
 int dxg2_plan_stage_times(dxg2_plan* plan, float* times, int32_t n);
 
+/* Waits for `stream` and tells how the plan's last dense call formed its Gram: *fp4 = 1 with
+ * narrow pixels (counts of at most 4 in magnitude) as FP4 codes and *wide_pixels binned pixels
+ * beside them in i8, *fp4 = 0 with every pixel in i8 (wide_pixels 0; it may be null).  Which of
+ * the two is decided on the device from the frames; the results are the same integers.  No
+ * reference counterpart. */
+int dxg2_plan_dense_route(dxg2_plan* plan, int32_t* fp4, int64_t* wide_pixels, void* stream);
+
 /* LDS atomic-add throughput of this GPU (32-bit adds per second, summed over the
  * chip), measured with workgroups of the event pair kernel's LDS footprint: mode 0
  * random counters, mode 1 lane-consecutive counters, `iters` adds per lane.  The

@@ -82,3 +82,36 @@ def test_narrow_by_work_equals_i8(n, shape, mean, monkeypatch):
                                               c.last_denominators)])
     for a, b in zip(*out):
         np.testing.assert_array_equal(a, b)
+
+
+def _route(c):
+    return next(iter(c._plans.values())).dense_route()
+
+
+@pytest.mark.parametrize("dtype", [np.uint8, np.int8])
+@pytest.mark.parametrize("kind,fp4", [("none", True), ("edges", True), ("all", False)])
+def test_narrow_route_taken(kind, fp4, dtype, monkeypatch):
+    """The integers are those of either route: which one ran, and with which wide pixels, is
+    what the plan says.  Then a call of another kind, a plan without the option, and a replay."""
+    import torch
+    from dynamix_amd.correlator.dense import MatMulCorrelator
+    print("[case] narrow route %s %s" % (kind, np.dtype(dtype).name), flush=True)
+    monkeypatch.setenv("DXG2_NARROW", "2")
+    n, shape = 257, (33, 37)
+    q = np.ones(shape, np.int32)
+    q[2, 3] = 0                               # one of the three wide pixels of "edges" is masked
+    f = _frames(n, shape, dtype, kind)
+    wide = int(((np.abs(f.astype(np.int32)) > 4).any(0) & (q > 0)).sum())
+    c, g2 = _correlate(f, q)
+    _check(c, g2, og.dense_g2(f, q))
+    assert _route(c) == (fp4, wide if fp4 else 0)
+    c.correlate(torch.from_numpy(f).cuda(), calc_std=True)
+    assert _route(c) == (False, 0)
+    graph = MatMulCorrelator(shape, n, q, extra_options={"graph": True})
+    d = torch.from_numpy(f).cuda()
+    for _ in range(3):
+        _check(graph, graph.correlate(d), og.dense_g2(f, q))
+    assert _route(graph) == (fp4, wide if fp4 else 0)
+    monkeypatch.setenv("DXG2_NARROW", "0")
+    c, g2 = _correlate(f, q)
+    assert _route(c) == (False, 0)
