@@ -61,6 +61,8 @@ _SIGNATURES = {
                                          ctypes.POINTER(ctypes.c_double), c_void_p]),
     "dxg2_plan_dry_run": (c_int, [ctypes.POINTER(PlanDesc), ctypes.POINTER(ctypes.c_int64),
                                   ctypes.c_int32]),
+    "dxg2_batch_dry_run": (c_int, [ctypes.POINTER(PlanDesc), ctypes.c_int32,
+                                   ctypes.POINTER(ctypes.c_int64), ctypes.c_int32]),
     "dxg2_plan_destroy": (c_int, [c_void_p]),
     "dxg2_plan_destroy_async": (c_int, [c_void_p, c_void_p]),
     "dxg2_plan_query": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p]),

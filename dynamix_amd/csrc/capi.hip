@@ -241,7 +241,7 @@ struct dxg2_plan {
     std::vector<GramWork> gram_raster, gram_xraster;  // the same before the XCD permutation
     std::vector<float2> twiddles;                     // FFT twiddle table (upload source)
     DevAllocator alloc;                               // allocator of every device buffer
-    int gram_group = 0;
+    int gram_k = 0;                                   // k-blocks per item of the lists above
     size_t slab_bytes = 0;
 
     // device (owned)
@@ -469,55 +469,61 @@ int gather_tile(const dxg2_plan* p, size_t items) {
     return tf;
 }
 
-// K-blocks per item of the plain Gram launch, at most tune_kchunk: all of a bin's, unless the
-// items are then too few or too uneven for the chip's CUs and shorter ones end sooner.  An item
-// costs about 0.5 us a k-block and 10 us for itself (first copies, fold, flush, next item) in a
-// 256-frame tile, a quarter of the former in a 128-frame tile; n items on 256 CUs end after
-// their mean load and half the longest item, and not before the longest (`only`: the tiles of
-// that bin alone).  96 x 96 x 500, 5
-// bins (15 whole items of 29 k-blocks): 45 us, in items of 4 and more 16 us.
-int gram_kchunk(const dxg2_plan* p, int only = -1, double item_us = 10.0) {
-    const int nT = (p->N + p->gram_tile - 1) / p->gram_tile;
-    const double tiles = (double)nT * (nT + 1) / 2 * (slab_planes(p->dtype) == 2 ? 2 : 1);
-    const double a = p->gram_tile == 256 ? 0.5 : 0.125, c = item_us;
+// K-blocks per item of a plain Gram launch over these plans' bins, at most each plan's
+// tune_kchunk: all of a bin's, unless the items are then too few or too uneven for the chip's CUs
+// and shorter ones end sooner.  An item costs about 0.5 us a k-block and 10 us for itself (first
+// copies, fold, flush, next item) in a 256-frame tile, a quarter of the former in a 128-frame
+// tile; n items on 256 CUs end after their mean load and half the longest item, and not before
+// the longest (`only`: the tiles of that bin alone).  96 x 96 x 500, 5 bins (15 whole items of 29
+// k-blocks): 45 us, in items of 4 and more 16 us; 16 such jobs in one launch fill the chip with
+// whole items: 45 us, 77 in items of 4.
+int gram_kchunk(const std::vector<const dxg2_plan*>& plans, int only = -1,
+                double item_us = 10.0) {
     int most = 0;
-    auto mine = [&](const BinDev& b) { return only < 0 || &b == &p->bins[only]; };
-    for (const BinDev& b : p->bins)
-        if (mine(b)) most = std::max(most, b.nkb);
-    int best = p->tune_kchunk;
+    auto each_bin = [&](auto f) {
+        for (const dxg2_plan* p : plans)
+            for (int b = 0; b < p->n_bins; ++b)
+                if (only < 0 || b == only) f(*p, p->bins[b].nkb);
+    };
+    each_bin([&](const dxg2_plan& p, int nkb) {
+        most = std::max(most, std::min(p.tune_kchunk, nkb));
+    });
+    int best = MAX_KBLOCKS_PER_ITEM;
     double best_t = 0.0;
     for (int parts = 1; parts <= 64; parts = parts < 4 ? parts + 1 : parts + parts / 2) {
-        const int k = std::min(p->tune_kchunk, (most + parts - 1) / parts);
+        const int k = std::max(1, (most + parts - 1) / parts);
         if (parts > 1 && k < 4) break;
-        double total = 0.0;
-        for (const BinDev& b : p->bins)
-            if (mine(b)) total += tiles * (a * b.nkb + c * ((b.nkb + k - 1) / std::max(k, 1)));
-        const double longest = a * k + c;
+        double total = 0.0, longest = 0.0;
+        each_bin([&](const dxg2_plan& p, int nkb) {
+            const int nT = (p.N + p.gram_tile - 1) / p.gram_tile, kk = std::min(p.tune_kchunk, k);
+            const double tiles = (double)nT * (nT + 1) / 2 * (slab_planes(p.dtype) == 2 ? 2 : 1);
+            const double a = p.gram_tile == 256 ? 0.5 : 0.125;
+            total += tiles * (a * nkb + item_us * ((nkb + kk - 1) / kk));
+            longest = std::max(longest, a * std::min(kk, nkb) + item_us);
+        });
         const double t = std::max(longest, total / 256 + 0.5 * longest);
         if (parts == 1 || t < 0.95 * best_t) {
             best_t = t;
-            best = parts == 1 ? p->tune_kchunk : k;
+            best = parts == 1 ? MAX_KBLOCKS_PER_ITEM : k;
         }
     }
     return best;
 }
 
-// Tile order of the grouped Gram launch.  Within a bin (largest bins first) the
-// upper-triangle tiles are walked in bands of `band` tile rows, column by column, so
-// consecutive items share row and column frame panels; the list is then dealt to the
-// XCDs in chunks of `group` items (0: no XCD remap).  Both are tuning parameters
-// (environment DXG2_GRAM_BAND, DXG2_GRAM_GROUP).
-void build_gram_work(dxg2_plan* p) {
+// Gram items of a plan in their tile order, at most kchunk k-blocks each: plain ones and the
+// cross-plane ones of uint16 plans.  Within a bin (largest bins first) the upper-triangle tiles
+// are walked in bands of tune_band tile rows, column by column, so consecutive items share row
+// and column frame panels.
+void gram_items(const dxg2_plan* p, int kchunk, std::vector<GramWork>& raster,
+                std::vector<GramWork>& xraster) {
     const int T = p->gram_tile;
     const int nT = (p->N + T - 1) / T;
     const int band = p->tune_band;
-    const int kchunk = gram_kchunk(p);
     std::vector<int> order(p->n_bins);
     for (int b = 0; b < p->n_bins; ++b) order[b] = b;
     // Largest bins first so their long tiles start early (LPT).
     std::stable_sort(order.begin(), order.end(),
                      [&](int a, int b) { return p->bins[a].nkb > p->bins[b].nkb; });
-    std::vector<GramWork> raster, xraster;
     // One pass of upper-triangle tiles over k-blocks [ka, kend) of bin b, adding into
     // output row `out`.
     auto triangle = [&](int b, int ka, int kend, int out, int cross) {
@@ -545,16 +551,53 @@ void build_gram_work(dxg2_plan* p) {
             triangle(b, nkb, 2 * nkb, 2 * nb + b, 1);
         }
     }
+}
+
+// Items per XCD chunk of a list: tune_group, or fewer so that every XCD has a share of a short one.
+int gram_group(const dxg2_plan* p, size_t items) {
+    return std::min<int>(p->tune_group, (int)std::max<size_t>(1, items / N_XCD));
+}
+
+// The plan's own Gram lists.  Band and XCD chunk are tuning parameters (environment
+// DXG2_GRAM_BAND, DXG2_GRAM_GROUP).
+void build_gram_work(dxg2_plan* p) {
+    std::vector<GramWork> raster, xraster;
+    p->gram_k = std::min(p->tune_kchunk, gram_kchunk({p}));
+    gram_items(p, p->gram_k, raster, xraster);
     GramWork pad{-1, 0, 0, 0, 0, 0, 0, 0, 0, 0};  // job 0
-    // every XCD has a share of a short list
-    const int group = std::min<int>(p->tune_group, std::max<size_t>(1, raster.size() / N_XCD));
+    const int group = gram_group(p, raster.size());
     p->gram_work = group > 0 ? remap_for_xcds(raster, group, pad) : raster;
     p->gram_xwork = group > 0 ? remap_for_xcds(xraster, group, pad) : xraster;
     p->qm_work = split_for_xcds(raster, group > 0 ? group : 1, p->q_off);
     p->qx_work = split_for_xcds(xraster, group > 0 ? group : 1, p->q_off + 9);
     p->gram_raster = std::move(raster);
     p->gram_xraster = std::move(xraster);
-    p->gram_group = group;
+}
+
+// One list over the items of several plans (job i: plans[i]), cut for the lot (what a plan alone
+// cuts to fill the chip is whole beside others), the longest items first whatever their job: a
+// workgroup takes one item, and an XCD the chunks that it is dealt.
+void batch_gram_work(const std::vector<const dxg2_plan*>& plans, std::vector<GramWork>& plain,
+                     std::vector<GramWork>& cross) {
+    const int kchunk = gram_kchunk(plans);
+    for (int i = 0; i < (int)plans.size(); ++i) {
+        const dxg2_plan* p = plans[i];
+        const int k = std::min(p->tune_kchunk, kchunk);
+        std::vector<GramWork> own, xown;
+        if (k != p->gram_k) gram_items(p, k, own, xown);
+        for (GramWork w : k != p->gram_k ? own : p->gram_raster) {
+            w.job = i;
+            plain.push_back(w);
+        }
+        for (GramWork w : k != p->gram_k ? xown : p->gram_xraster) {
+            w.job = i;
+            cross.push_back(w);
+        }
+    }
+    for (auto* list : {&plain, &cross})
+        std::stable_sort(list->begin(), list->end(), [](const GramWork& x, const GramWork& y) {
+            return x.kb1 - x.kb0 > y.kb1 - y.kb0;
+        });
 }
 
 // Tile work (see TileWork) for every bin, or for bin `only` (0-based) alone.  Tiles
@@ -568,7 +611,8 @@ void build_tile_work(const dxg2_plan* p, int only, size_t cap_bytes, TileWork& t
     // one bin's few tiles are cut like the plain launch's (an item also stores its tile); all
     // bins' are not, as std_tile_kernel is fastest with one item a tile.  One ring of 4, 300 x 400
     // x 1,000 (10 tiles): Gram 377 -> 45 us, the call 574 -> 137 us.
-    const int kchunk = only >= 0 ? gram_kchunk(p, only, 20.0) : p->tune_kchunk;
+    const int kchunk = only >= 0 ? std::min(p->tune_kchunk, gram_kchunk({p}, only, 20.0))
+                                 : p->tune_kchunk;
     const bool wide = slab_planes(p->dtype) == 2;
     const size_t tile_bytes = (size_t)T * T * 4;
     int max_items = 0;
@@ -1332,6 +1376,27 @@ int dxg2_plan_dry_run(const dxg2_plan_desc* desc, int64_t* summary, int32_t n) {
     return DXG2_OK;
 }
 
+int dxg2_batch_dry_run(const dxg2_plan_desc* descs, int32_t n, int64_t* summary, int32_t m) {
+    if (n < 0 || (n > 0 && !descs) || (m > 0 && !summary))
+        return set_error(DXG2_EINVAL, "null argument");
+    std::vector<std::unique_ptr<dxg2_plan>> own;
+    std::vector<const dxg2_plan*> plans;
+    for (int32_t i = 0; i < n; ++i) {
+        int rc = DXG2_OK;
+        own.emplace_back(build_plan_host(descs + i, &rc));
+        if (!own.back()) return rc;
+        plans.push_back(own.back().get());
+    }
+    std::vector<GramWork> plain, cross;
+    batch_gram_work(plans, plain, cross);
+    int64_t longest = 0;
+    for (const auto* list : {&plain, &cross})
+        for (const GramWork& w : *list) longest = std::max<int64_t>(longest, w.kb1 - w.kb0);
+    const int64_t v[] = {(int64_t)plain.size(), (int64_t)cross.size(), longest};
+    for (int32_t i = 0; i < m && i < (int32_t)(sizeof(v) / sizeof(v[0])); ++i) summary[i] = v[i];
+    return DXG2_OK;
+}
+
 int dxg2_plan_create(const dxg2_plan_desc* desc, dxg2_plan** out) {
     if (!desc || !out) return set_error(DXG2_EINVAL, "null argument");
     *out = nullptr;
@@ -1671,12 +1736,12 @@ int dxg2_plan_set_tuning(dxg2_plan* p, const dxg2_tuning* t) {
         bool queue;
         std::vector<GramWork> mwork, xwork, raster, xraster, qm, qx;
         int q_off[18];
-        int gram_group;
+        int gram_k;
     };
     auto save = [&]() {
         TuningState st{p->gram_tile, p->tune_band, p->tune_group, p->tune_kchunk, p->use_queue,
                        p->gram_work, p->gram_xwork, p->gram_raster, p->gram_xraster,
-                       p->qm_work, p->qx_work, {}, p->gram_group};
+                       p->qm_work, p->qx_work, {}, p->gram_k};
         memcpy(st.q_off, p->q_off, sizeof(p->q_off));
         return st;
     };
@@ -1693,7 +1758,7 @@ int dxg2_plan_set_tuning(dxg2_plan* p, const dxg2_tuning* t) {
         p->qm_work.swap(st.qm);
         p->qx_work.swap(st.qx);
         memcpy(p->q_off, st.q_off, sizeof(p->q_off));
-        p->gram_group = st.gram_group;
+        p->gram_k = st.gram_k;
     };
     TuningState old = save();
     p->gram_tile = t->tile;
@@ -1922,32 +1987,11 @@ int dxg2_batch_correlate_dense(dxg2_batch* b, int32_t n, dxg2_plan* const* plans
     }
     hipStream_t s = (hipStream_t)stream;
     (void)hipGetLastError();
-    // Work list: every job's items, largest jobs first, one XCD permutation over the lot.
-    std::vector<int> order(n);
-    for (int i = 0; i < n; ++i) order[i] = i;
-    auto ops = [&](int i) {
-        double w = 0;
-        for (const auto& it : plans[i]->gram_raster) w += it.kb1 - it.kb0;
-        for (const auto& it : plans[i]->gram_xraster) w += it.kb1 - it.kb0;
-        return w;
-    };
-    std::vector<double> wk(n);
-    for (int i = 0; i < n; ++i) wk[i] = ops(i);
-    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return wk[x] > wk[y]; });
+    // Work list: every job's items, one XCD permutation over the lot (with the first plan's chunk).
     std::vector<GramWork> plain, cross;
     std::vector<GramJob> jobs(n);
-    for (int i : order) {
-        dxg2_plan* p = plans[i];
-        for (GramWork w : p->gram_raster) {
-            w.job = i;
-            plain.push_back(w);
-        }
-        for (GramWork w : p->gram_xraster) {
-            w.job = i;
-            cross.push_back(w);
-        }
-    }
-    const int group = plans[0]->gram_group;
+    batch_gram_work({plans, plans + n}, plain, cross);
+    const int group = gram_group(plans[0], plain.size());
     GramWork pad{-1, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     if (group > 0) {
         plain = remap_for_xcds(plain, group, pad);

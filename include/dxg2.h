@@ -89,6 +89,10 @@ int dxg2_plan_create(const dxg2_plan_desc* desc, dxg2_plan** out);
  * For checking the plan builder off the GPU (sanitizers, fuzzing).  No reference
  * counterpart. */
 int dxg2_plan_dry_run(const dxg2_plan_desc* desc, int64_t* summary, int32_t n);
+/* The same for the joined Gram list of a grouped launch over n such plans
+ * (dxg2_batch_correlate_dense): up to m of plain items, cross-plane items, k-blocks of the
+ * longest item.  No reference counterpart. */
+int dxg2_batch_dry_run(const dxg2_plan_desc* descs, int32_t n, int64_t* summary, int32_t m);
 /* Waits for the device, then releases the plan. */
 int dxg2_plan_destroy(dxg2_plan* plan);
 /* Releases the plan without waiting for the device: its buffers go to the plan's

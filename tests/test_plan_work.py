@@ -8,12 +8,16 @@ import pytest
 from dynamix_amd import _lib
 from dynamix_amd.synth import annular_qmask
 
-EVENT_ITEMS = 9      # index of the summary
+GRAM_ITEMS, EVENT_ITEMS = 8, 9      # indexes of the summary
+
+
+def _desc(shape, nframes, q, dtype=_lib.DXG2_U8, flags=0):
+    return _lib.PlanDesc(shape[0], shape[1], nframes, dtype, q.ctypes.data, None, 0, flags)
 
 
 def _dry_run(shape, nframes, q, dtype=_lib.DXG2_U8, flags=0):
     q = np.ascontiguousarray(q, dtype=np.int32)
-    d = _lib.PlanDesc(shape[0], shape[1], nframes, dtype, q.ctypes.data, None, 0, flags)
+    d = _desc(shape, nframes, q, dtype, flags)
     s = (ctypes.c_int64 * 12)()
     _lib.check(_lib.load().dxg2_plan_dry_run(ctypes.byref(d), s, 12))
     return list(s)
@@ -32,3 +36,48 @@ def test_event_items_of_several_lag_windows(shape, nframes, bins):
     items = _dry_run(shape, nframes, q)[EVENT_ITEMS]
     assert items <= max(2 * 256 / windows, pixels / 1024) + bins
     assert items >= pixels / 8192
+
+
+def _batch(jobs, dtype=_lib.DXG2_U8):
+    masks = [np.ascontiguousarray(annular_qmask(s, b), dtype=np.int32) for s, _, b in jobs]
+    d = (_lib.PlanDesc * len(jobs))(*[_desc(s, n, q, dtype) for (s, n, _), q in zip(jobs, masks)])
+    out = (ctypes.c_int64 * 3)()
+    _lib.check(_lib.load().dxg2_batch_dry_run(d, len(jobs), out, 3))
+    return list(out), masks
+
+
+def _whole(jobs, masks):
+    """(items, k-blocks of the longest) with a bin's k-blocks in one item: a tile pair and bin each."""
+    items = longest = 0
+    for (_, n, _), q in zip(jobs, masks):
+        nt = math.ceil(n / 256)
+        kb = np.ceil(np.bincount(q.ravel())[1:] / 64)
+        items += nt * (nt + 1) // 2 * int((kb > 0).sum())
+        longest = max(longest, int(kb.max()))
+    return items, longest
+
+
+def test_grouped_items_are_cut_for_the_joined_list():
+    """A small plan cuts its few tiles along k to fill the chip alone; sixteen of them in one
+    launch fill it with whole items, and their order among bigger jobs does not matter."""
+    small, large = ((96, 96), 500, 5), ((256, 256), 3000, 8)
+    alone, masks = _batch([small])
+    assert alone[0] > _whole([small], masks)[0]
+    assert alone[0] == _dry_run(small[0], small[1], masks[0])[GRAM_ITEMS]
+    for jobs in ([small] * 16, [large] * 4 + [small], [small] + [large] * 4):
+        got, masks = _batch(jobs)
+        assert (got[0], got[2]) == _whole(jobs, masks)
+
+
+def test_grouped_items_of_uint16_plans_and_empty_masks():
+    """HH and LL of every tile pair in the plain list, both halves of the cross product in the
+    other; a plan without bins adds none."""
+    small = ((96, 96), 500, 5)
+    jobs = [small] * 16
+    got, masks = _batch(jobs, _lib.DXG2_U16)
+    assert got[0] == got[1] == 2 * _whole(jobs, masks)[0]
+    q = np.zeros((8, 8), np.int32)
+    d = (_lib.PlanDesc * 1)(_desc((8, 8), 10, q))
+    out = (ctypes.c_int64 * 3)()
+    _lib.check(_lib.load().dxg2_batch_dry_run(d, 1, out, 3))
+    assert list(out) == [0, 0, 0]
