@@ -1359,6 +1359,9 @@ int dxg2_plan_dry_run(const dxg2_plan_desc* desc, int64_t* summary, int32_t n) {
     build_tile_work(p, -1, std_scratch_cap(), tw);
     int64_t items = 0;
     for (const auto& c : tw.chunks) items += (c.m1 - c.m0) + (c.x1 - c.x0);
+    size_t dense_bytes = 0, event_bytes = 0;
+    (void)dxg2_plan_footprint(p, 0, &dense_bytes);
+    (void)dxg2_plan_footprint(p, 3, &event_bytes);
     const int64_t v[] = {p->n_bins,
                          (int64_t)p->pix_idx.size(),
                          (int64_t)p->slab_bytes,
@@ -1370,7 +1373,9 @@ int dxg2_plan_dry_run(const dxg2_plan_desc* desc, int64_t* summary, int32_t n) {
                          (int64_t)(p->qm_work.size() + p->qx_work.size()),
                          (int64_t)p->event_work.size(),
                          (int64_t)tw.tiles.size(),
-                         items};
+                         items,
+                         (int64_t)dense_bytes,
+                         (int64_t)event_bytes};
     for (int32_t i = 0; i < n && i < (int32_t)(sizeof(v) / sizeof(v[0])); ++i) summary[i] = v[i];
     delete p;
     return DXG2_OK;

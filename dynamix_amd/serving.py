@@ -50,6 +50,7 @@ from .correlator.common import Plan
 SERVE_SHAPES = ((256, 256), (514, 1030), (1030, 1065))
 DENSE_MEAN = 0.02     # counts per pixel per frame of dense jobs
 EVENT_MEAN = 1e-3     # counts per pixel per frame of event jobs
+NARROW_MIN_WORK = 5e11   # list entries x frames^2 from which a plan may have a narrow slab
 
 
 @dataclass
@@ -518,20 +519,31 @@ class GpuExecutor(object):
         """Device bytes a job may hold, bounded before its plan exists (the scheduler
         reserves them when the job's input is staged): the input (dense frames; event
         CSR lists at 1.25 times the expected number of events, as a pixel-frame holds an
-        event with probability below EVENT_MEAN), the outputs and per-bin frame rows, the
-        pixel lists, for dense jobs the slab (every pixel binned, each bin padded to whole
-        64-pixel k-blocks, slab rows padded by up to 256) and the Gram work lists (one
-        item per 256-frame tile pair per bin and k-chunk, in two lists)."""
+        event with probability below EVENT_MEAN), the outputs and per-bin frame rows
+        (numerators, sums, denominators, two prefix sums and the denominator's two digit
+        planes), the pixel lists, and for dense jobs the slab (every pixel binned, each bin
+        padded to whole 64-pixel k-blocks, slab rows padded by up to 256), from
+        NARROW_MIN_WORK on the narrow slab of half its size with its lists, flags and sums,
+        and the Gram work lists.  An item costs 10 us and a k-block of it 0.5, and a plan's
+        items are cut along k only where that ends the launch sooner: beyond one item per
+        256-frame tile pair, bin and 2,047 k-blocks, no more of them than cost 256 CUs what
+        the longest bin's tile costs one."""
         h, w = spec.shape
         hw, n, nb = h * w, spec.nframes, max(int(spec.n_bins), 1)
-        rows = nb * (n + 2) * 8 * 4 + nb * n * (8 + 8 + 8 + 4) + hw * 4 + (1 << 16)
+        entries = hw + 64 * nb
+        rows = nb * (5 * (n + 2) * 8 + 2 * (n + 64 * 208) + 32) + nb * n * 28 + 4 * entries + \
+            (1 << 16)
         if spec.layout == "dense":
-            nkb = hw // 64 + nb
+            nkb = entries // 64
             nt = (n + 255) // 256
-            items = nt * (nt + 1) // 2 * (nb + nkb // 2047 + 1)
-            lists = 2 * 40 * items + 32 * nkb
-            return n * hw + (hw + 64 * nb) * (n + 256) + rows + lists
-        return int(1.25 * EVENT_MEAN * n * hw) * 5 + 4 * (hw + 1) * 4 + rows + hw
+            items = nt * (nt + 1) // 2 * (nb + nkb // 2047 + 1) + 256 * (1 + nkb // 20) + 512
+            lists = 2 * 40 * items + 10 * nkb + (1 << 14)
+            slab = entries * (n + 256)
+            # a plan has no narrow slab where the band gather cannot address the i8 slab
+            if float(entries) * n * n >= NARROW_MIN_WORK and hw * n < 1 << 34:
+                slab += slab // 2 + nb * n * 8 + 4 * entries + hw + 16 + 4 * (2 * nb + 1)
+            return n * hw + slab + rows + lists
+        return int(1.25 * EVENT_MEAN * n * hw) * 5 + 4 * (hw + 1) * 3 + hw // 128 + 16 * 1100 + rows
 
     def prepare(self, spec, staged=None):
         """Plan and footprint of a job; its input comes from stage() (waited for if it

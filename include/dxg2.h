@@ -85,7 +85,8 @@ int dxg2_plan_create(const dxg2_plan_desc* desc, dxg2_plan** out);
  * every work list) with no device call, and writes up to n of: n_bins, padded pixel
  * count, slab bytes, gather items, band items, band k-blocks, k-blocks on the band
  * gather's fallback, Gram items, Gram items of the queue schedule, event items, calc_std
- * tiles, calc_std chunk items.  Returns the error dxg2_plan_create would return for the description.
+ * tiles, calc_std chunk items, footprint of the dense path, of the event path (bytes, as
+ * dxg2_plan_footprint tells them of a new plan).  Returns the error dxg2_plan_create would return for the description.
  * For checking the plan builder off the GPU (sanitizers, fuzzing).  No reference
  * counterpart. */
 int dxg2_plan_dry_run(const dxg2_plan_desc* desc, int64_t* summary, int32_t n);

@@ -8,7 +8,7 @@ import pytest
 from dynamix_amd import _lib
 from dynamix_amd.synth import annular_qmask
 
-GRAM_ITEMS, EVENT_ITEMS = 8, 9      # indexes of the summary
+GRAM_ITEMS, EVENT_ITEMS, DENSE_BYTES, EVENT_BYTES = 8, 9, 12, 13   # indexes of the summary
 
 
 def _desc(shape, nframes, q, dtype=_lib.DXG2_U8, flags=0):
@@ -18,8 +18,8 @@ def _desc(shape, nframes, q, dtype=_lib.DXG2_U8, flags=0):
 def _dry_run(shape, nframes, q, dtype=_lib.DXG2_U8, flags=0):
     q = np.ascontiguousarray(q, dtype=np.int32)
     d = _desc(shape, nframes, q, dtype, flags)
-    s = (ctypes.c_int64 * 12)()
-    _lib.check(_lib.load().dxg2_plan_dry_run(ctypes.byref(d), s, 12))
+    s = (ctypes.c_int64 * 14)()
+    _lib.check(_lib.load().dxg2_plan_dry_run(ctypes.byref(d), s, 14))
     return list(s)
 
 
@@ -81,3 +81,32 @@ def test_grouped_items_of_uint16_plans_and_empty_masks():
     out = (ctypes.c_int64 * 3)()
     _lib.check(_lib.load().dxg2_batch_dry_run(d, 1, out, 3))
     assert list(out) == [0, 0, 0]
+
+
+@pytest.mark.parametrize("flags", [0, _lib.DXG2_FLAG_NO_QUEUE])
+def test_serving_reserves_at_least_what_a_job_takes(flags):
+    """GpuExecutor.footprint_bound() against the footprint of the plan it stands for, outputs and
+    input included, on both sides of the line from which a plan has a narrow slab."""
+    from dynamix_amd import serving
+    specs = serving.make_jobs(14, 10.0, 17)
+    specs += serving.make_jobs(20, 10.0, 18, shapes=((64, 48), (96, 96), (131, 77)),
+                               nframes=(100, 3000), bins=(1, 12))
+    specs += serving.make_jobs(10, 10.0, 19, shapes=((256, 256),), nframes=(2400, 3400))
+    seen = set()
+    for spec in specs:
+        h, w = spec.shape
+        n, q = spec.nframes, serving.job_qmask(spec)
+        nb = int(q.max())
+        s = _dry_run(spec.shape, n, q, flags=flags)
+        out = nb * n * 28
+        bound = serving.GpuExecutor.footprint_bound(None, spec)
+        if spec.layout == "dense":
+            need = s[DENSE_BYTES] + out + n * h * w
+            seen.add(s[DENSE_BYTES] > 1.3 * s[2])     # a narrow slab beside the i8 slab
+            if min(spec.shape) >= 256:
+                assert bound <= 1.25 * need or flags
+        else:
+            events = int(1.25 * serving.EVENT_MEAN * n * h * w)
+            need = s[EVENT_BYTES] + out + 5 * events + 4 * (h * w + 1)
+        assert need <= bound, spec
+    assert seen == ({False} if flags else {True, False})
