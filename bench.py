@@ -196,10 +196,12 @@ def bench_fft(plan, frames, nb, n, pf):
     ms = _timed(step, 2, torch)
     t = plan.stage_times()
     plan.set_profiling(False)
-    from dynamix_amd.correlator.dense import fft_length
-    L = fft_length(n) // 2
+    from dynamix_amd.correlator.dense import plan_fft_length
+    L = plan_fft_length(n) // 2
     npix = int(plan.pixel_counts[:nb].sum())
-    flop = npix * 5.0 * L * math.log2(L)   # one complex FFT of L points per pixel
+    # nominal: one complex FFT of L points per pixel (the classes' transforms of half that
+    # length are two per pixel)
+    flop = npix * 5.0 * L * math.log2(L)
     return {"ms": ms, "value": pf / (ms * 1e-3), "unit": "pixel*frames/s",
             "stage_ms": {"gather_and_sums": t[0], "spectra_and_inverse": t[1], "finalise": t[2]},
             "fft_length": 2 * L, "spectra_gflops": flop / (t[1] * 1e-3) / 1e9}

@@ -79,6 +79,7 @@ _SIGNATURES = {
     "dxg2_batch_correlate_dense": (c_int, [c_void_p, c_int] + [c_void_p] * 7),
     "dxg2_batch_correlate_events": (c_int, [c_void_p, c_int] + [c_void_p] * 9),
     "dxg2_correlate_fft": (c_int, [c_void_p] * 7),
+    "dxg2_fft_length": (c_int, [c_int, ctypes.POINTER(c_i64)]),
     "dxg2_correlate_events_csr": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_i64,
                                           c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     "dxg2_correlate_events_coo": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_i64,

@@ -27,6 +27,7 @@ Num and Den and one FP64 division, i.e. within float32 rounding of the FP64 valu
 After each call `last_numerators`, `last_sums`, `last_denominators` (torch tensors on
 the GPU, int64/int64/float64) hold the exact intermediate results.
 """
+import ctypes
 from collections import namedtuple
 
 import numpy as np
@@ -228,26 +229,24 @@ class PlainMatMulCorrelator(_DenseHIP):
         return g2.cpu().numpy()
 
 
-# Half-lengths L up to 16384 frames: 2^a 5^b, 1024 <= L <= 16384.
-FFT_HALF_LENGTHS = (1024, 1280, 2048, 2560, 4096, 5120, 8192, 10240, 16384)
+def plan_fft_length(nframes):
+    """Nf of the transforms that a series of nframes takes: the library's smallest length >= 2
+    nframes, padded from at most 131,072 frames (0 above), of the smooth lengths it has; Nf >=
+    2 N - 1 is all the linear autocorrelation needs (the reference uses get_next_power(2N),
+    utils.py:50-60, another smooth length of the same kind)."""
+    nf = ctypes.c_int64()
+    _lib.check(_lib.load().dxg2_fft_length(int(nframes), ctypes.byref(nf)), "dxg2_fft_length")
+    return nf.value
 
 
-# Long series (N > 16384): L = L1 L2, a row length L1 and a column count L2.
-FFT_ROW_LENGTHS = (8192, 5120, 4096, 2560, 2048, 1280, 1024)
-FFT_COL_LENGTHS = (2, 4, 5, 8, 16)
+_COARSE_LENGTHS = (1024, 1280, 2048, 2560, 4096, 5120, 8192, 10240, 16384, 20480, 25600, 32768,
+                   40960, 65536, 81920, 131072)
 
 
 def fft_length(nframes):
-    """Nf = 2 L for the smallest L of FFT_HALF_LENGTHS with L >= nframes, or above 16384
-    the smallest product L1 L2 >= nframes of FFT_ROW_LENGTHS x FFT_COL_LENGTHS: Nf >= 2 N - 1
-    is all the linear autocorrelation needs (the reference uses get_next_power(2N),
-    utils.py:50-60, another smooth length of the same kind).  A plan may transform at a
-    shorter length that is enough too.  0 when N > 131072."""
-    for L in FFT_HALF_LENGTHS:
-        if L >= nframes:
-            return 2 * L
-    long = [a * b for a in FFT_ROW_LENGTHS for b in FFT_COL_LENGTHS if a * b >= nframes]
-    return 2 * min(long) if long else 0
+    """2 L for the smallest L >= nframes of a coarse set (0 when nframes > 131072): never shorter
+    than plan_fft_length(), the length that is used."""
+    return 2 * next((L for L in _COARSE_LENGTHS if L >= nframes), 0)
 
 
 class FFTCorrelator(_DenseHIP):
@@ -269,8 +268,12 @@ class FFTCorrelator(_DenseHIP):
         super()._set_parameters(shape, nframes, qmask, scale_factor, extra_options)
         self._init_dense()
         self.precompute_fft_plans = precompute_fft_plans
-        self.Nf = fft_length(self.nframes)
         self.n_pix = {int(b): int(n) for b, n in zip(self.bins, self.pixel_counts)}
+
+    @property
+    def Nf(self):
+        """Length of the transforms."""
+        return plan_fft_length(self.nframes)
 
     def correlate(self, frames):
         torch = _torch()

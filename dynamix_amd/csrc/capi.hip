@@ -2269,6 +2269,13 @@ int dxg2_correlate_events_coo(dxg2_plan* p, const uint32_t* d_pixel, const uint3
                            d_g2, s, ev);
 }
 
+int dxg2_fft_length(int32_t nframes, int64_t* nf) {
+    if (!nf) return set_error(DXG2_EINVAL, "null argument");
+    FftShape shape{};
+    *nf = fft_shape(std::max(nframes, 1), &shape) ? 2 * (int64_t)shape.L : 0;
+    return DXG2_OK;
+}
+
 int dxg2_correlate_fft(dxg2_plan* p, const void* d_frames, double* d_num, int64_t* d_sums,
                        double* d_den, float* d_g2, void* stream) {
     if (!p) return set_error(DXG2_EINVAL, "null plan");

@@ -212,15 +212,18 @@ int dxg2_batch_correlate_events(dxg2_batch* batch, int32_t n, dxg2_plan* const* 
 int dxg2_correlate_dense_plain(dxg2_plan* plan, const void* d_frames, float* d_g2,
                                void* stream);
 
-/* FFT path for uint8 frames: per bin, the power spectra of every pixel's time series
- * (FP32 Stockham FFT of length Nf = 2L, L = smallest power of two >= max(N, 1024),
- * L <= 16384) summed in FP64, one FP64 inverse per bin, exact integer denominators.
+/* FFT path: per bin, the power spectra of every pixel's time series (FP32, of length Nf
+ * as dxg2_fft_length tells it, up to 131,072 frames) summed in FP64, one FP64 inverse per bin, exact integer denominators.
  * d_num receives the FP64 numerators (n_bins, N) (may be NULL); other outputs as for
  * the dense path.  Numerators carry FP32 FFT rounding: see the documented tolerance.
  * Replaces FFTWCorrelator.correlate / _correlate_fft (correlator/dense.py:314-369) and
  * CUFFTCorrelator (correlator/cuda.py:129-219). */
 int dxg2_correlate_fft(dxg2_plan* plan, const void* d_frames, double* d_num, int64_t* d_sums,
                        double* d_den, float* d_g2, void* stream);
+/* Nf of the transforms that a series of nframes takes: twice the library's smallest length
+ * >= nframes, 0 above 131,072 frames.  No reference counterpart: get_next_power(2N)
+ * (utils.py:50-60) is its rule. */
+int dxg2_fft_length(int32_t nframes, int64_t* nf);
 
 /* Event (sparse) path, pixel-major CSR exactly as the reference's EventCorrelator takes
  * it: d_times int32[nnz] frame indices, strictly increasing within a pixel; d_data

@@ -108,3 +108,14 @@ def test_reference_gpu_class_names_importable():
     assert issubclass(cuda.CublasMatMulCorrelator, dense.MatMulCorrelator)
     assert issubclass(cuda.CUFFTCorrelator, dense.FFTCorrelator)
     assert dense.FFTWCorrelator is dense.FFTCorrelator
+
+
+@pytest.mark.parametrize("n,nf", [(1, 1024), (100, 1024), (513, 1280), (600, 1280), (6000, 12800),
+                                  (12000, 25600), (16384, 32768), (16385, 40960),
+                                  (131072, 262144), (131073, 0)])
+def test_fft_correlator_reports_the_length_it_transforms_at(n, nf):
+    """Nf is the library's own, not a second table."""
+    from dynamix_amd.correlator.dense import FFTCorrelator, fft_length, plan_fft_length
+    assert plan_fft_length(n) == nf
+    assert FFTCorrelator((6, 7), n).Nf == nf
+    assert nf == 0 or 2 * n <= nf <= fft_length(n)
