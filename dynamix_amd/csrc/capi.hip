@@ -310,6 +310,10 @@ struct dxg2_plan {
     KbWork* d_kbwork = nullptr;
     std::vector<KbWork> kb_gather; // the same in gather order (kb -1: padding)
     KbWork* d_kbgather = nullptr;
+    struct FftPart {               // k-blocks [k0, k1) of kb_work, items [g0, g1) of kb_gather
+        int k0, k1, g0, g1;
+    };
+    std::vector<FftPart> fft_parts;
     // the FFT path's pixel order within each bin (its sums do not depend on it): aligned
     // quads of detector pixels 4a .. 4a + 3 that lie wholly in the bin first, then the
     // rest, in raster order; fft_qkb[b] leading k-blocks of bin b are all such quads
@@ -776,9 +780,45 @@ int next_events(dxg2_plan* p, hipEvent_t** out) {
 }
 
 // Bytes of the FFT path's series: L elements per entry of the (padded) pixel lists.
-size_t fft_series_bytes(const dxg2_plan* p, int L) {
+size_t fft_series_bytes(const dxg2_plan* p, int L, size_t entries) {
     const size_t size = p->dtype == DXG2_U16 ? 2 : 1;
-    return std::max<size_t>(16, p->pix_idx.size() * (size_t)L * size);
+    return std::max<size_t>(16, entries * (size_t)L * size);
+}
+size_t fft_series_bytes(const dxg2_plan* p, int L) {
+    return fft_series_bytes(p, L, p->pix_idx.size());
+}
+
+// The k-blocks of the FFT path in `n` parts, each with its gather items: PM_KPB k-blocks
+// consecutive in detector order (kb -1 past the end), dealt to the XCDs as units.
+void fft_partition(dxg2_plan* p, int n) {
+    using Item = std::array<KbWork, PM_KPB>;
+    Item pad;
+    pad.fill(KbWork{0, -1});
+    p->kb_gather.clear();
+    p->fft_parts.clear();
+    const int total = (int)p->kb_work.size(), each = (total + n - 1) / n;
+    for (int k0 = 0; k0 < total; k0 += each) {
+        const int k1 = std::min(total, k0 + each);
+        std::vector<std::pair<int64_t, KbWork>> order;
+        for (int k = k0; k < k1; ++k) {
+            const KbWork w = p->kb_work[k];
+            order.push_back({(int64_t)p->pix_fft[p->bins[w.bin].idx_off + (int64_t)w.kb * KB], w});
+        }
+        std::stable_sort(order.begin(), order.end(),
+                         [](const std::pair<int64_t, KbWork>& a,
+                            const std::pair<int64_t, KbWork>& b) { return a.first < b.first; });
+        std::vector<Item> items;
+        for (size_t i = 0; i < order.size(); i += PM_KPB) {
+            Item it;
+            for (int j = 0; j < PM_KPB; ++j)
+                it[j] = i + j < order.size() ? order[i + j].second : KbWork{0, -1};
+            items.push_back(it);
+        }
+        items = remap_for_xcds(items, PM_XCD_GROUP / PM_KPB, pad);
+        const int g0 = (int)(p->kb_gather.size() / PM_KPB);
+        for (const Item& it : items) p->kb_gather.insert(p->kb_gather.end(), it.begin(), it.end());
+        p->fft_parts.push_back({k0, k1, g0, (int)(p->kb_gather.size() / PM_KPB)});
+    }
 }
 
 // Sums of one bin in the FFT path's power buffer.
@@ -817,29 +857,6 @@ int ensure_fft_buffers(dxg2_plan* p, hipStream_t s) {
         std::copy(rest.begin(), rest.end(), out + quad.size());
         p->fft_qkb[b] = (int32_t)(quad.size() / KB);
     }
-    // gather items: PM_KPB k-blocks consecutive in detector order (kb -1 past the end),
-    // dealt to the XCDs as units
-    {
-        std::vector<std::pair<int64_t, KbWork>> order;
-        for (const KbWork& w : p->kb_work)
-            order.push_back({(int64_t)p->pix_fft[p->bins[w.bin].idx_off + (int64_t)w.kb * KB], w});
-        std::stable_sort(order.begin(), order.end(),
-                         [](const std::pair<int64_t, KbWork>& a,
-                            const std::pair<int64_t, KbWork>& b) { return a.first < b.first; });
-        using Item = std::array<KbWork, PM_KPB>;
-        std::vector<Item> items;
-        for (size_t i = 0; i < order.size(); i += PM_KPB) {
-            Item it;
-            for (int j = 0; j < PM_KPB; ++j)
-                it[j] = i + j < order.size() ? order[i + j].second : KbWork{0, -1};
-            items.push_back(it);
-        }
-        Item pad;
-        pad.fill(KbWork{0, -1});
-        items = remap_for_xcds(items, PM_XCD_GROUP / PM_KPB, pad);
-        p->kb_gather.clear();
-        for (const Item& it : items) p->kb_gather.insert(p->kb_gather.end(), it.begin(), it.end());
-    }
     p->twiddles.resize(2 * (size_t)H + L + 1);
     auto root = [](int64_t m, int64_t n) {  // exp(-2 pi i m / n)
         const double a = -2.0 * M_PI * (double)m / (double)n;
@@ -851,8 +868,10 @@ int ensure_fft_buffers(dxg2_plan* p, hipStream_t s) {
         for (int b = 0; b < stride; ++b)
             p->twiddles[H + r * stride + b] = root((int64_t)r * b, H);
     for (int m = 0; m <= L; ++m) p->twiddles[2 * H + m] = root(m, 2 * (int64_t)L);
-    // d_power is allocated last: it marks the workspace complete.  A failure releases
-    // what this call allocated, so a later call starts again from nothing.
+    // The series of every k-block at once, or where that memory cannot be had (a series takes up to
+    // 1.6 times its frames' bytes) of half of them, a quarter and so on, one part after the other.
+    // A failure releases what was allocated, so a later call starts again from nothing.
+    // d_power is set last: it marks the workspace complete.
     uint8_t* xs = nullptr;
     float2* tw = nullptr;
     double *power = nullptr, *fnum = nullptr;
@@ -861,27 +880,33 @@ int ensure_fft_buffers(dxg2_plan* p, hipStream_t s) {
     KbWork* kbg = nullptr;
     int32_t* pixf = nullptr;
     int32_t* qkb = nullptr;
-    if ((!p->pix_fft.empty() &&
-         dev_alloc(p->alloc, (void**)&pixf, p->pix_fft.size() * sizeof(int32_t), s) !=
-             hipSuccess) ||
-        dev_alloc(p->alloc, (void**)&qkb, p->fft_qkb.size() * sizeof(int32_t), s) != hipSuccess ||
-        dev_alloc(p->alloc, (void**)&xs, fft_series_bytes(p, L), s) != hipSuccess ||
-        dev_alloc(p->alloc, (void**)&tw, p->twiddles.size() * sizeof(float2), s) != hipSuccess ||
-        dev_alloc(p->alloc, (void**)&fnum, (size_t)std::max(p->n_bins, 1) * p->N * sizeof(double), s) !=
-            hipSuccess ||
-        dev_alloc(p->alloc, (void**)&finv,
-                  std::max(p->n_bins, 1) * fft_inverse_elems(shape) * sizeof(double2), s) !=
-            hipSuccess ||
-        (!p->kb_work.empty() &&
-         (dev_alloc(p->alloc, (void**)&kbw, p->kb_work.size() * sizeof(KbWork), s) != hipSuccess ||
-          dev_alloc(p->alloc, (void**)&kbg, p->kb_gather.size() * sizeof(KbWork), s) !=
-              hipSuccess)) ||
-        dev_alloc(p->alloc, (void**)&power, (size_t)std::max(p->n_bins, 1) * fft_power_row(shape) * sizeof(double), s) !=
-            hipSuccess) {
-        for (void* b : {(void*)xs, (void*)tw, (void*)fnum, (void*)kbw, (void*)kbg, (void*)power,
-                        (void*)pixf, (void*)qkb, (void*)finv})
-            dev_free(p->alloc, b, s);
-        return set_error(DXG2_ENOMEM, "cannot allocate FFT workspace");
+    const size_t nb = (size_t)std::max(p->n_bins, 1);
+    const int total = (int)p->kb_work.size();
+    for (int parts = 1;; parts *= 2) {
+        fft_partition(p, parts);
+        const size_t entries = (size_t)((total + parts - 1) / parts) * KB;
+        auto have = [&](auto** ptr, size_t bytes) {
+            return bytes == 0 || dev_alloc(p->alloc, (void**)ptr, bytes, s) == hipSuccess;
+        };
+        if (have(&xs, fft_series_bytes(p, L, entries)) &&
+            have(&pixf, p->pix_fft.size() * sizeof(int32_t)) &&
+            have(&qkb, p->fft_qkb.size() * sizeof(int32_t)) &&
+            have(&tw, p->twiddles.size() * sizeof(float2)) &&
+            have(&fnum, nb * p->N * sizeof(double)) &&
+            have(&finv, nb * fft_inverse_elems(shape) * sizeof(double2)) &&
+            have(&kbw, p->kb_work.size() * sizeof(KbWork)) &&
+            have(&kbg, p->kb_gather.size() * sizeof(KbWork)) &&
+            have(&power, nb * fft_power_row(shape) * sizeof(double)))
+            break;
+        auto drop = [&](auto*& ptr) {
+            dev_free(p->alloc, ptr, s);
+            ptr = nullptr;
+        };
+        drop(xs), drop(pixf), drop(qkb), drop(tw), drop(fnum), drop(finv), drop(kbw), drop(kbg);
+        power = nullptr;  // the last one asked for
+        (void)hipGetLastError();
+        if (2 * parts > std::min(total, 64))
+            return set_error(DXG2_ENOMEM, "cannot allocate FFT workspace");
     }
     p->d_pixfft = pixf;
     p->d_fftqkb = qkb;
@@ -2291,13 +2316,21 @@ int dxg2_correlate_fft(dxg2_plan* p, const void* d_frames, double* d_num, int64_
     if (ev) DXG2_HIP(hipEventRecord(ev[0], s));
     launch_fill_i64(reinterpret_cast<int64_t*>(p->d_power), p->n_bins * fft_power_row(p->fft), s);
     const bool quads = reinterpret_cast<uintptr_t>(d_frames) % 4 == 0;
-    launch_gather_pm((const uint8_t*)d_frames, p->dtype, (int64_t)p->H * p->W, p->N, p->fft,
-                     p->d_pixfft, quads ? p->d_fftqkb : nullptr, p->d_bins, p->n_bins,
-                     p->d_kbgather, (int)(p->kb_gather.size() / PM_KPB), p->d_xs, sums, s);
-    if (ev) DXG2_HIP(hipEventRecord(ev[1], s));
-    if (launch_fft_power(p->fft, p->dtype, p->d_xs, p->d_bins, p->d_kbwork,
-                         (int)p->kb_work.size(), p->d_tw, p->d_power, s))
-        return set_error(DXG2_EUNSUPPORTED, "no FFT kernel for length %d", p->fft.L);
+    launch_fill_i64(sums, (int64_t)p->n_bins * p->N, s);
+    for (const auto& part : p->fft_parts) {
+        // the kernels address a k-block's series by its place among all of them
+        uint8_t* xs = reinterpret_cast<uint8_t*>(
+            reinterpret_cast<uintptr_t>(p->d_xs) -
+            (part.k0 ? fft_series_bytes(p, p->fft.L, (size_t)part.k0 * KB) : 0));
+        launch_gather_pm((const uint8_t*)d_frames, p->dtype, (int64_t)p->H * p->W, p->N, p->fft,
+                         p->d_pixfft, quads ? p->d_fftqkb : nullptr, p->d_bins, p->n_bins,
+                         p->d_kbgather + (size_t)part.g0 * PM_KPB, part.g1 - part.g0, xs, sums, s);
+        if (ev && part.k0 == 0) DXG2_HIP(hipEventRecord(ev[1], s));
+        if (launch_fft_power(p->fft, p->dtype, xs, p->d_bins, p->d_kbwork + part.k0,
+                             part.k1 - part.k0, p->d_tw, p->d_power, s))
+            return set_error(DXG2_EUNSUPPORTED, "no FFT kernel for length %d", p->fft.L);
+    }
+    if (ev && p->fft_parts.empty()) DXG2_HIP(hipEventRecord(ev[1], s));
     launch_fft_inverse(p->d_power, p->fft, p->n_bins, p->N, p->d_finv, p->d_fnum, s);
     if (ev) DXG2_HIP(hipEventRecord(ev[2], s));
     launch_finalize_f64(sums, p->d_fnum, p->d_bins, p->n_bins, p->N, p->d_prefix, p->d_smax,

@@ -288,7 +288,7 @@ struct FftShape {
 // The shape of the smallest L >= n; false above 131072.
 bool fft_shape(int n, FftShape* out);
 // Series of every bin in pairs (pairs of pix_idx's entries; H G elements a pair) and the
-// exact frame sums (sums[b][t] for t < nframes, zeroed here first).  work: n_work items of
+// exact frame sums (added to sums[b][t], t < nframes).  work: n_work items of
 // PM_KPB k-blocks (kb -1: none).  quad_kb (8-bit frames; may be null): per bin, the leading
 // k-blocks whose entries are 16 aligned pixel quads.
 void launch_gather_pm(const uint8_t* frames, int dtype, int64_t hw, int nframes,

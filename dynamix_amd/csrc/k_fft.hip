@@ -273,7 +273,7 @@ struct RawPoint {
 // load is a byte, 1.27 -> 1.06 ms a call).  The tile's frames are G / 2 runs,
 // run m at frames H m + n0 .., so it holds every element of SEG points of the pairs: a
 // thread reads the G words (series, run) of a few points of one pair, transposes them in
-// registers and stores 4 G contiguous bytes.  The frame sums S_b(t) (zeroed first)
+// registers and stores 4 G contiguous bytes.  The frame sums S_b(t) (zeroed by the caller)
 // come from the same tile: a thread adds one word (4 frames of 8-bit values in 16-bit
 // halves, or 2 of 16-bit values in 32-bit registers) down 16 or 32 pixel rows, the row
 // groups meet in LDS, and each frame's total over the 64 pixels (below 2^31) goes to
@@ -868,9 +868,7 @@ void launch_gather_pm(const uint8_t* frames, int dtype, int64_t hw, int nframes,
                       const FftShape& shape, const int32_t* pix_idx, const int32_t* quad_kb,
                       const BinDev* bins, int n_bins, const KbWork* work, int n_work,
                       uint8_t* xs, int64_t* sums, hipStream_t s) {
-    if (n_bins <= 0) return;
-    launch_fill_i64(sums, (int64_t)n_bins * nframes, s);
-    if (n_work <= 0) return;
+    if (n_bins <= 0 || n_work <= 0) return;
     // aligned quad loads need 4 | hw and a 4-aligned frame pointer
     if (hw % 4 != 0 || reinterpret_cast<uintptr_t>(frames) % 4 != 0) quad_kb = nullptr;
     if (shape.G == 4)

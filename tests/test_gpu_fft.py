@@ -214,3 +214,72 @@ def test_fft_at_the_ends_of_the_lengths(n, dtype):
     q = _qmask(n, shape, 2)
     c = FFTCorrelator(shape, n, q)
     _check(c, c.correlate(f), f, q)
+
+
+@pytest.mark.parametrize("dtype,nbins", [(np.uint8, 3), (np.int8, 1), (np.uint16, 5)])
+def test_fft_series_in_parts_where_memory_is_short(dtype, nbins):
+    """The series of every pixel do not fit: they are formed and transformed part by part (up to
+    four, across bins and partial k-blocks), with the same sums and, within the FFT's
+    tolerance, numerators; a later failure still leaves nothing behind."""
+    import ctypes
+
+    import torch
+    from dynamix_amd import _lib
+    from dynamix_amd.correlator.common import Plan
+    from dynamix_amd.correlator.dense import plan_fft_length
+    _announce("fft in parts %s" % np.dtype(dtype).name)
+    n, shape = 700, (20, 28)
+    rng = np.random.default_rng(nbins)
+    info = np.iinfo(dtype)
+    f = (rng.random((n,) + shape) < 0.3) * rng.integers(info.min, info.max + 1, size=(n,) + shape)
+    f = f.astype(dtype)
+    q = _qmask(n, shape, nbins)
+    counts = np.bincount(q.ravel(), minlength=nbins + 1)[1:]
+    kblocks = int(((counts + 63) // 64).sum())
+    series = plan_fft_length(n) // 2 * 64 * np.dtype(dtype).itemsize     # bytes a k-block
+    state = {"most": series * ((kblocks + 1) // 2) - 1, "live": 0, "sizes": []}
+    dev = torch.cuda.current_device()
+
+    def alloc(nbytes, stream, ctx):
+        state["sizes"].append(int(nbytes))
+        if nbytes > state["most"]:
+            return None
+        state["live"] += 1
+        return torch.cuda.caching_allocator_alloc(int(nbytes), dev, int(stream or 0))
+
+    def free(ptr, stream, ctx):
+        state["live"] -= 1
+        torch.cuda.caching_allocator_delete(int(ptr))
+
+    cb_a, cb_f, lib = _lib.ALLOC_FN(alloc), _lib.FREE_FN(free), _lib.load()
+    _lib.check(lib.dxg2_set_allocator(cb_a, cb_f, None))
+    try:
+        plan = Plan(shape, n, q, dtype)
+    finally:
+        _lib.check(lib.dxg2_set_allocator(_lib.ALLOC_FN(), _lib.FREE_FN(), None))
+    num = torch.zeros((nbins, n), dtype=torch.float64, device="cuda")
+    sums = torch.zeros((nbins, n), dtype=torch.int64, device="cuda")
+    den, g2 = torch.zeros_like(num), torch.zeros((nbins, n), dtype=torch.float32, device="cuda")
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    d = torch.from_numpy(f.view(np.int16) if dtype == np.uint16 else f).cuda()
+
+    def call():
+        _lib.check(lib.dxg2_correlate_fft(plan.handle, _lib.ptr(d), _lib.ptr(num), _lib.ptr(sums),
+                                          _lib.ptr(den), _lib.ptr(g2), st))
+
+    before, most = state["live"], state["most"]
+    state["most"] = series - 1
+    with pytest.raises(MemoryError):
+        call()
+    assert state["live"] == before
+    state["most"] = most
+    for _ in range(2):
+        call()
+    assert series * ((kblocks + 3) // 4) in state["sizes"]
+    ref = og.dense_g2(f, q)
+    np.testing.assert_array_equal(sums.cpu().numpy(), ref["sums"])
+    np.testing.assert_array_equal(den.cpu().numpy(), np.asarray(ref["den"], np.float64))
+    num0 = np.maximum(np.abs(ref["num"][:, :1]).astype(np.float64), 1.0)
+    assert (np.abs(num.cpu().numpy() - ref["num"]) / num0).max() <= NUM_TOL
+    plan.close()
+    assert state["live"] == 0
