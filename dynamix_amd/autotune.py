@@ -2,13 +2,15 @@
 
 The Gram's speed depends on the tile size (128 or 256 frames), on the raster band and
 XCD chunk of its work list, on the launch form (persistent workgroups over per-XCD
-work queues, or one workgroup per tile) and on the k-chunk (k-blocks per work item:
-shorter items let the tiles that run together share a chunk of frame panel in L2).  The best choice depends on the number of
-frames and on how the binned pixels split into bins, so results are cached under a key
-built from (frame dtype, nframes, histogram of bin sizes in power-of-two k-block
-buckets).  `autotune()` times candidates on real frames with the library's own HIP event
-stage timers, keeps the fastest, applies it to the plan and records it; `apply_cached()`
-applies a recorded result to a new plan of the same key.
+work queues, or one workgroup per tile) and on the k-chunk (most k-blocks per work item:
+shorter items let the tiles that run together share a chunk of frame panel in L2; where
+the library itself takes fewer to fill the chip, larger k-chunks are the same list and
+time alike).  The best choice depends on the number of frames and on how the binned pixels
+split into bins, so results are cached under a key built from (frame dtype, nframes,
+histogram of bin sizes in power-of-two k-block buckets).  `autotune()` times candidates on
+real frames with the library's own HIP event stage timers, keeps the fastest, applies it to
+the plan and records it; `apply_cached()` applies a recorded result to a new plan of the same
+key.
 
 The cache is a JSON file: $DXG2_TUNING_CACHE, or ~/.cache/dynamix_amd/gram_tuning.json.
 """

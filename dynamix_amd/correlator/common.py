@@ -144,8 +144,9 @@ class Plan(object):
                 "kchunk": t.kchunk}
 
     def set_tuning(self, tile, band, group, queue, kchunk=0):
-        """Rebuild the Gram work lists for a tuning (waits for the device); kchunk 0 is
-        the dtype's default."""
+        """Rebuild the Gram work lists for a tuning (waits for the device); group and kchunk
+        are the most that a list may have (less where it is short), kchunk 0 is the dtype's
+        default."""
         t = _lib.Tuning(int(tile), int(band), int(group), int(queue), int(kchunk))
         _lib.check(self.lib.dxg2_plan_set_tuning(self.handle, ctypes.byref(t)),
                    "dxg2_plan_set_tuning")

@@ -825,6 +825,11 @@ using Plan16384 = FftPlan<16384, 1024, 16, 8, 8, 16>;
     X(2560, 4) X(3200, 4) X(4096, 4) X(5120, 4) X(6400, 4) X(8192, 4) X(10240, 4)        \
     X(12800, 4) X(16384, 4) X(10240, 8) X(16384, 8) X(10240, 16) X(16384, 16)
 
+#define DXG2_FFT_CHECK(HH, GG) \
+    static_assert(HH % (256 / PM_KPB / (GG / 2)) == 0, "a gather workgroup's points divide H");
+DXG2_FFT_SHAPES(DXG2_FFT_CHECK)
+#undef DXG2_FFT_CHECK
+
 bool fft_shape(int n, FftShape* out) {
     int best = 0;
 #define DXG2_FFT_SHAPE(HH, GG)                                     \
@@ -842,7 +847,7 @@ static void gather_pm_typed(const uint8_t* frames, int64_t hw, int nframes, int 
                             const int32_t* pix_idx, const int32_t* quad_kb, const BinDev* bins,
                             const KbWork* work, int n_work, uint8_t* xs, int64_t* sums,
                             hipStream_t s) {
-    constexpr int SEG = 256 / PM_KPB / (G / 2);  // divides every plan length (multiples of 128)
+    constexpr int SEG = 256 / PM_KPB / (G / 2);  // divides every H (checked above)
     gather_pm_kernel<E, SGN, PM_KPB, G>
         <<<dim3((unsigned)n_work, (unsigned)(H / SEG)), 256, 0, s>>>(
             frames, hw, nframes, H, pix_idx, quad_kb, bins, work, xs, sums);

@@ -160,10 +160,12 @@ int dxg2_correlate_dense_graph(dxg2_plan* plan, const void* d_frames, int64_t* d
                                int64_t* d_sums, double* d_den, float* d_g2, void* stream);
 
 /* Gram launch tuning of a plan: tile size (128 or 256 frames), raster band (tile rows),
- * XCD chunk (consecutive items per XCD, 0 = none), launch form (1 = persistent
- * workgroups over per-XCD work queues, 0 = one workgroup per tile) and k-chunk (k-blocks
+ * XCD chunk (most consecutive items per XCD, 0 = none; fewer where a list is too short for
+ * every XCD to have a share), launch form (1 = persistent
+ * workgroups over per-XCD work queues, 0 = one workgroup per tile) and k-chunk (most k-blocks
  * of 64 pixels per work item, 1..2047; 0 on set = the dtype's default: 512 for uint16,
- * 2047 otherwise).  set_tuning waits for the device, rebuilds the work lists and drops
+ * 2047 otherwise; items are shorter where longer ones are too few or too uneven for the
+ * chip).  get_tuning returns the values as they were set.  set_tuning waits for the device, rebuilds the work lists and drops
  * the plan's graph and calc_std workspaces.  Used by the autotuner
  * (dynamix_amd.autotune).  No reference counterpart: the reference takes block_size for
  * its OpenCL kernels (dense.py:153,163). */
