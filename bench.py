@@ -589,8 +589,8 @@ def main():
         "gather": gather_roofline(q, shape, n, gather_ms, wide_share is not None),
         "roofline": {"bound": "mfma", "achieved": achieved, "peak": peak,
                      "unit": "TOP/s", "frac": achieved / peak,
-                     "traffic": (read_traffic("gram_i8_%s_traffic.txt" % args.workload)
-                                 if wide_share is None else None),
+                     "traffic": read_traffic("gram_%s_%s_traffic.txt" % (
+                         "i8" if wide_share is None else "f4", args.workload)),
                      "kernel": ("gram_f4_queue_kernel + gram_i8_queue_kernel"
                                 if wide_share is not None and plan.get_tuning()["queue"] else
                                 "gram_i8_queue_kernel" if plan.get_tuning()["queue"]

@@ -20,8 +20,8 @@
 // four waves would need in full at the MFMA rate).  Three buffers of GRAM_UNITS units form a
 // ring; everything is spread over the unit's 16 MFMAs, four at a time: two or three fragment
 // reads of the next unit and one DMA of the unit two stages ahead (DMAs issued in a burst
-// hold back the wave's MFMAs behind them: 17.0 ms against 13.3 for this order; 15.7 for
-// fragments loaded straight into registers, 480,000 pixels x 10,000 frames).  One barrier a
+// hold back the wave's MFMAs behind them, a quarter of the time; 480,000 pixels x 10,000 frames
+// 14.9 ms, 15.6 for fragments loaded straight into registers).  One barrier a
 // stage, ahead of its last unit: by then that unit's fragments are in registers, so the
 // buffer is free, and the next stage has landed (the wait leaves this stage's DMAs in
 // flight), so its first fragments are read under the last unit's MFMAs and no latency is
