@@ -478,14 +478,18 @@ static int sums_window(int nframes) {
 // Whether the pair kernel adds each event to its frame's sum by a global atomic (add_sum) and
 // event_sums_item()'s launch is left out.  So few events that their atomics, at about 21e9/s
 // beside the pairs, take less than that launch, and that LDS counters (`counters`: frames of every
-// item) would join none of them.  Pairs and sums with the launch -> without: 8-bit, 128 x 128 x
-// 400,000 (1.6e6 events, 13 windows) 264 -> 233 us, 514 x 1030 x 40,000 (2.1e6, 2 windows) 167 ->
-// 166, 300 x 300 x 40,000 (3.6e6) 165 -> 191; 16-bit, whose pairs take longer, 512 x 512 x 100,000
-// (5.2e6) 1,327 -> 1,234, 300 x 300 x 30,000 (2.7e6) 286 -> 264, 514 x 1030 x 5,000 (1.3e7)
-// 692 -> 720.
+// item) would join none of them.  Both costs beside the atomics, the pairs that hide them and the
+// launch's repeated reads, grow with the lag windows.  Pairs and sums with the launch -> without:
+// 8-bit, 128 x 128 x 400,000 (1.6e6 events, 13 windows) 264 -> 233 us, 514 x 1030 x 40,000 (2.1e6,
+// 2 windows) 167 -> 166, 300 x 300 x 40,000 (3.6e6, 2) 165 -> 191, 512 x 512 x 100,000 (5.2e6, 4)
+// 295 -> 324, x 200,000 (7) 455 -> 432, 1030 x 1065 x 250,000 (2.7e7, 8) 1,899 -> 2,376; 16-bit,
+// whose pairs take longer, 512 x 512 x 100,000 (5.2e6) 1,327 -> 1,234, 514 x 1030 x 5,000 (1.3e7, 1)
+// 692 -> 720, 1030 x 1065 x 50,000 (5.5e7, 4) 4,397 -> 5,317.
 template <typename T>
-static bool sums_with_pairs(int64_t counters, int64_t nnz) {
-    return nnz <= std::min<int64_t>(counters, sizeof(T) == 1 ? 2000000 : 7000000);
+static bool sums_with_pairs(int64_t counters, int64_t nnz, int windows) {
+    const int64_t most = sizeof(T) == 1 ? std::max<int64_t>(2000000, 1200000ll * windows)
+                                        : 7000000ll * std::max(1, windows / 4);
+    return nnz <= std::min(counters, most);
 }
 // Threads: two workgroups share a CU's threads where their counters leave room for it.
 static int sums_threads(int window) { return window > SUMS_WINDOW / 2 ? 1024 : 512; }
@@ -781,7 +785,7 @@ template <typename T, int NW>
 void pairs_jobs_launch(const EventJob* jobs, const EventWork* work, int n_work, int max_frames,
                        int64_t counters, int64_t nnz, hipStream_t s) {
     constexpr int WS = EvHist<T>::window(NW);
-    const bool with_sums = sums_with_pairs<T>(counters, nnz);
+    const bool with_sums = sums_with_pairs<T>(counters, nnz, (max_frames + WS - 1) / WS);
     const int win = sums_window(max_frames);
     if (!with_sums)
         event_sums_jobs_kernel<T><<<dim3((unsigned)n_work, (unsigned)((max_frames + win - 1) / win)),
@@ -831,7 +835,7 @@ void pairs_launch(const int32_t* times, const void* data, const uint32_t* offset
                   int nframes, int64_t nnz, int64_t* num, int64_t* sums, int* err, hipStream_t s) {
     constexpr int WS = EvHist<T>::window(NW);
     int64_t* psums = nullptr;  // frame sums of the pair kernel
-    if (sums_with_pairs<T>((int64_t)n_work * nframes, nnz)) {
+    if (sums_with_pairs<T>((int64_t)n_work * nframes, nnz, (nframes + WS - 1) / WS)) {
         psums = sums;
     } else {
         const int win = sums_window(nframes);
