@@ -820,6 +820,12 @@ using Plan16384 = FftPlan<16384, 1024, 16, 8, 8, 16>;
 // A finer set than the powers of two and five quarters of them: 490 x 694 x 229 0.74 -> 0.38 ms
 // a call (1,024 -> 512), 333 x 335 x 6,000 2.8 -> 2.5 (8,192 -> 6,400), 201 x 203 x 12,000
 // 3.2 -> 2.9 (16,384 -> 12,800).
+// A call of 8-bit frames at N = L, 256 x 256 pixels in 5 bins, ms, whole transforms at their finest
+// length -> these: 512 0.38 -> 0.15, 640 0.38 -> 0.19, 1,024 0.39 -> 0.22, 1,280 0.51 -> 0.33, 2,048 0.53 ->
+// 0.38, 2,560 0.79 -> 0.54, 3,200 0.93 -> 0.72, 4,096 0.99 -> 0.72, 5,120 2.20 -> 1.04, 6,400 2.52 -> 1.36,
+// 8,192 2.61 -> 1.59, 10,240 3.25 -> 2.13, 12,800 4.73 -> 3.32, 16,384 4.92 -> 3.62, 20,480 16.0 -> 4.65,
+// 25,600 18.4 -> 5.92; 160 x 160: 32,768 11.7 -> 3.37, 40,960 14.8 -> 4.22, 65,536 26.0 -> 7.03, 81,920
+// 33.9 -> 9.22, 131,072 64.9 -> 19.8.
 #define DXG2_FFT_SHAPES(X)                                                               \
     X(256, 4) X(320, 4) X(512, 4) X(640, 4) X(1024, 4) X(1280, 4) X(1600, 4) X(2048, 4)  \
     X(2560, 4) X(3200, 4) X(4096, 4) X(5120, 4) X(6400, 4) X(8192, 4) X(10240, 4)        \
