@@ -489,9 +489,7 @@ int gram_kchunk(const std::vector<const dxg2_plan*>& plans, int only = -1,
             for (int b = 0; b < p->n_bins; ++b)
                 if (only < 0 || b == only) f(*p, p->bins[b].nkb);
     };
-    each_bin([&](const dxg2_plan& p, int nkb) {
-        most = std::max(most, std::min(p.tune_kchunk, nkb));
-    });
+    each_bin([&](const dxg2_plan&, int nkb) { most = std::max(most, nkb); });
     int best = MAX_KBLOCKS_PER_ITEM;
     double best_t = 0.0;
     for (int parts = 1; parts <= 64; parts = parts < 4 ? parts + 1 : parts + parts / 2) {
