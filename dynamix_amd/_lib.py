@@ -67,6 +67,7 @@ _SIGNATURES = {
     "dxg2_plan_destroy_async": (c_int, [c_void_p, c_void_p]),
     "dxg2_plan_query": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p]),
     "dxg2_plan_footprint": (c_int, [c_void_p, c_int, ctypes.POINTER(c_size_t)]),
+    "dxg2_plan_set_narrow": (c_int, [c_void_p, c_int]),
     "dxg2_correlate_dense": (c_int, [c_void_p] * 7),
     "dxg2_correlate_dense_std": (c_int, [c_void_p] * 8),
     "dxg2_correlate_dense_graph": (c_int, [c_void_p] * 7),

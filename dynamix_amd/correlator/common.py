@@ -156,6 +156,10 @@ class Plan(object):
         _lib.check(self.lib.dxg2_plan_footprint(self.handle, path, ctypes.byref(out)))
         return out.value
 
+    def set_narrow(self, on=True):
+        """Whether dense calls may have a narrow slab (an option; see footprint(5))."""
+        _lib.check(self.lib.dxg2_plan_set_narrow(self.handle, 1 if on else 0))
+
     def set_profiling(self, on=True):
         _lib.check(self.lib.dxg2_plan_set_profiling(self.handle, 1 if on else 0))
 

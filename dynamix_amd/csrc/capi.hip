@@ -266,6 +266,7 @@ struct dxg2_plan {
     bool last_narrow = false;      // the last dense call was a narrow call
     bool graph_narrow = false;     // the captured one is
     bool narrow_refused = false;   // its memory could not be had
+    bool narrow_declined = false;  // its owner does without (dxg2_plan_set_narrow)
     int64_t* d_wsums = nullptr;    // its wide pixels' frame sums, n_bins rows
     int64_t* d_ugram = nullptr;
     int64_t* d_sums = nullptr;
@@ -1046,7 +1047,8 @@ int ensure_event_buffers(dxg2_plan* p, int64_t nnz_coo, hipStream_t s) {
 constexpr double NARROW_MIN_WORK = 5e11;
 constexpr int HEAD_INTS = 24;
 bool narrow_applies(const dxg2_plan* p) {
-    if (p->dtype == DXG2_U16 || p->gband.empty() || !p->use_queue || p->gram_tile != 256)
+    if (p->dtype == DXG2_U16 || p->gband.empty() || !p->use_queue || p->gram_tile != 256 ||
+        p->narrow_declined)
         return false;
     return p->narrow_opt == 2 ||
            (p->narrow_opt && (double)p->pix_idx.size() * p->N * p->N >= NARROW_MIN_WORK);
@@ -1382,8 +1384,9 @@ int dxg2_plan_dry_run(const dxg2_plan_desc* desc, int64_t* summary, int32_t n) {
     build_tile_work(p, -1, std_scratch_cap(), tw);
     int64_t items = 0;
     for (const auto& c : tw.chunks) items += (c.m1 - c.m0) + (c.x1 - c.x0);
-    size_t dense_bytes = 0, event_bytes = 0;
+    size_t dense_bytes = 0, event_bytes = 0, needed_bytes = 0;
     (void)dxg2_plan_footprint(p, 0, &dense_bytes);
+    (void)dxg2_plan_footprint(p, 5, &needed_bytes);
     (void)dxg2_plan_footprint(p, 3, &event_bytes);
     const int64_t v[] = {p->n_bins,
                          (int64_t)p->pix_idx.size(),
@@ -1398,7 +1401,8 @@ int dxg2_plan_dry_run(const dxg2_plan_desc* desc, int64_t* summary, int32_t n) {
                          (int64_t)tw.tiles.size(),
                          items,
                          (int64_t)dense_bytes,
-                         (int64_t)event_bytes};
+                         (int64_t)event_bytes,
+                         (int64_t)needed_bytes};
     for (int32_t i = 0; i < n && i < (int32_t)(sizeof(v) / sizeof(v[0])); ++i) summary[i] = v[i];
     delete p;
     return DXG2_OK;
@@ -1661,9 +1665,20 @@ int dxg2_plan_footprint(const dxg2_plan* p, int32_t path, size_t* bytes) {
         case 4:
             *bytes = std_footprint(p);
             return DXG2_OK;
+        case 5: {
+            const int rc = dxg2_plan_footprint(p, 0, bytes);
+            *bytes -= narrow_bytes(p);
+            return rc;
+        }
         default:
             return set_error(DXG2_EINVAL, "unknown path %d", path);
     }
+}
+
+int dxg2_plan_set_narrow(dxg2_plan* p, int32_t on) {
+    if (!p) return set_error(DXG2_EINVAL, "null plan");
+    p->narrow_declined = on == 0;
+    return DXG2_OK;
 }
 
 int dxg2_plan_set_profiling(dxg2_plan* p, int32_t on) {

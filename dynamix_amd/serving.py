@@ -38,6 +38,7 @@ jobs share its launch: tests compare each job in the mix with the same job run a
 import collections
 import ctypes
 import functools
+import threading
 import time
 from concurrent.futures import ThreadPoolExecutor
 from dataclasses import dataclass, field
@@ -50,7 +51,6 @@ from .correlator.common import Plan
 SERVE_SHAPES = ((256, 256), (514, 1030), (1030, 1065))
 DENSE_MEAN = 0.02     # counts per pixel per frame of dense jobs
 EVENT_MEAN = 1e-3     # counts per pixel per frame of event jobs
-NARROW_MIN_WORK = 5e11   # list entries x frames^2 from which a plan may have a narrow slab
 
 
 @dataclass
@@ -158,7 +158,8 @@ class Job:
     qmask: np.ndarray = None
     inputs: dict = field(default_factory=dict)
     outputs: tuple = ()
-    footprint: int = 0
+    footprint: int = 0        # device bytes it cannot do without
+    option: int = 0           # more of them that it can use (charged when they are granted)
     t_admit: float = 0.0
     t_dispatch: float = 0.0
     t_done: float = 0.0
@@ -366,6 +367,9 @@ class Scheduler(object):
                 others = staged_bytes - holds.get(job.spec.id, 0)
                 if n_resident > 0 and resident_bytes + others + job.footprint > ex.budget:
                     break
+                if resident_bytes + others + job.footprint + job.option > ex.budget:
+                    job.option = 0       # the job does without
+                job.footprint += job.option
                 waiting.popleft()
                 job.t_admit = clock()
                 try:
@@ -454,7 +458,6 @@ class GpuExecutor(object):
 
     def __init__(self, hbm_budget=None, reserve_bytes=8 << 30, n_streams=2, depth=2,
                  keep_results=False, persistent_gram=True):
-        import threading
         import torch
         self.torch = torch
         self.lib = _lib.load()
@@ -522,8 +525,8 @@ class GpuExecutor(object):
         event with probability below EVENT_MEAN), the outputs and per-bin frame rows
         (numerators, sums, denominators, two prefix sums and the denominator's two digit
         planes), the pixel lists, and for dense jobs the slab (every pixel binned, each bin
-        padded to whole 64-pixel k-blocks, slab rows padded by up to 256), from
-        NARROW_MIN_WORK on the narrow slab of half its size with its lists, flags and sums,
+        padded to whole 64-pixel k-blocks, slab rows padded by up to 256; not the narrow slab,
+        an option that a job gets at admission where the budget has room)
         and the Gram work lists.  An item costs 10 us and a k-block of it 0.5, and a plan's
         items are cut along k only where that ends the launch sooner: beyond one item per
         256-frame tile pair, bin and 2,047 k-blocks, no more of them than cost 256 CUs what
@@ -538,11 +541,7 @@ class GpuExecutor(object):
             nt = (n + 255) // 256
             items = nt * (nt + 1) // 2 * (nb + nkb // 2047 + 1) + 256 * (1 + nkb // 20) + 512
             lists = 2 * 40 * items + 10 * nkb + (1 << 14)
-            slab = entries * (n + 256)
-            # a plan has no narrow slab where the band gather cannot address the i8 slab
-            if float(entries) * n * n >= NARROW_MIN_WORK and hw * n < 1 << 34:
-                slab += slab // 2 + nb * n * 8 + 4 * entries + hw + 16 + 4 * (2 * nb + 1)
-            return n * hw + slab + rows + lists
+            return n * hw + entries * (n + 256) + rows + lists
         return int(1.25 * EVENT_MEAN * n * hw) * 5 + 4 * (hw + 1) * 3 + hw // 128 + 16 * 1100 + rows
 
     def prepare(self, spec, staged=None):
@@ -568,7 +567,8 @@ class GpuExecutor(object):
         out_bytes = nb * n * (8 + 8 + 8 + 4)
         h, w = spec.shape
         if spec.layout == "dense":
-            job.footprint = job.plan.footprint(0) + out_bytes + n * h * w
+            job.footprint = job.plan.footprint(5) + out_bytes + n * h * w
+            job.option = job.plan.footprint(0) - job.plan.footprint(5)
         else:
             job.footprint = job.plan.footprint(3) + out_bytes + job.inputs["nnz"] * 5 + \
                 (h * w + 1) * 4
@@ -580,6 +580,7 @@ class GpuExecutor(object):
         torch = self.torch
         spec = job.spec
         nb, n = job.plan.n_bins, spec.nframes
+        job.plan.set_narrow(job.option > 0)
         s = self.admit_stream
         with torch.cuda.stream(s):
             job.outputs = (torch.empty((nb, n), dtype=torch.int64, device="cuda"),

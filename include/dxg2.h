@@ -85,7 +85,7 @@ int dxg2_plan_create(const dxg2_plan_desc* desc, dxg2_plan** out);
  * every work list) with no device call, and writes up to n of: n_bins, padded pixel
  * count, slab bytes, gather items, band items, band k-blocks, k-blocks on the band
  * gather's fallback, Gram items, Gram items of the queue schedule, event items, calc_std
- * tiles, calc_std chunk items, footprint of the dense path, of the event path (bytes, as
+ * tiles, calc_std chunk items, footprints of paths 0, 3 and 5 (bytes, as
  * dxg2_plan_footprint tells them of a new plan).  Returns the error dxg2_plan_create would return for the description.
  * For checking the plan builder off the GPU (sanitizers, fuzzing).  No reference
  * counterpart. */
@@ -109,9 +109,15 @@ int dxg2_plan_query(const dxg2_plan* plan, int32_t* n_bins, int64_t* pixel_count
                     double* scale);
 
 /* Device bytes the plan holds for a path (0 dense, 1 plain, 2 fft, 3 events, 4 the
- * extra workspaces of dense calc_std), for admission control by memory footprint.
+ * extra workspaces of dense calc_std, 5 dense without the narrow slab, which a call does
+ * without where it cannot be had), for admission control by memory footprint.
  * No reference counterpart. */
 int dxg2_plan_footprint(const dxg2_plan* plan, int32_t path, size_t* bytes);
+/* on = 0: the plan's dense calls from here on keep every pixel in i8 and allocate no narrow
+ * slab (path 0's footprint is then path 5's); 1, as a plan is created: they may have one.
+ * Results are the same integers.  A graph replay keeps the route it was captured with.  No
+ * reference counterpart. */
+int dxg2_plan_set_narrow(dxg2_plan* plan, int32_t on);
 
 /* Dense batched path: qmask gather into per-bin i8 slabs (+ S_b(t)), one grouped
  * i8-MFMA Gram launch over every bin with the diagonal (tau) reduction fused, exact

@@ -182,3 +182,24 @@ def test_settings_are_read_when_the_plan_is_created(monkeypatch):
         assert (_slab4(q) in a.sizes) == (made == "2")
         plan.close()
     assert size["2"] > size["0"] + _slab4(q)
+
+
+def test_a_plan_that_declines_the_narrow_slab(monkeypatch):
+    """set_narrow(False): no narrow slab, the footprint without it, the same integers; and back."""
+    import torch
+    print("[case] narrow slab declined", flush=True)
+    monkeypatch.setenv("DXG2_NARROW", "2")
+    q, f = _inputs()
+    ref, outs, d = og.dense_g2(f, q), _outs(3), torch.from_numpy(f).cuda()
+    a = _Allocator()
+    plan = a.plan(q, np.uint8)
+    assert plan.footprint(0) >= plan.footprint(5) + _slab4(q)
+    for k, on in enumerate((False, True, False)):
+        plan.set_narrow(on)
+        assert (plan.footprint(0) > plan.footprint(5)) == on
+        _call(plan, d, outs)
+        _check(outs, ref)
+        assert on or plan.dense_route() == (False, 0)
+        assert a.sizes.count(_slab4(q)) == (k > 0)
+    plan.close()
+    assert a.live == 0

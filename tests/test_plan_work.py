@@ -8,7 +8,7 @@ import pytest
 from dynamix_amd import _lib
 from dynamix_amd.synth import annular_qmask
 
-GRAM_ITEMS, EVENT_ITEMS, DENSE_BYTES, EVENT_BYTES = 8, 9, 12, 13   # indexes of the summary
+GRAM_ITEMS, EVENT_ITEMS, DENSE_BYTES, EVENT_BYTES, NEEDED_BYTES = 8, 9, 12, 13, 14  # of the summary
 
 
 def _desc(shape, nframes, q, dtype=_lib.DXG2_U8, flags=0):
@@ -18,8 +18,8 @@ def _desc(shape, nframes, q, dtype=_lib.DXG2_U8, flags=0):
 def _dry_run(shape, nframes, q, dtype=_lib.DXG2_U8, flags=0):
     q = np.ascontiguousarray(q, dtype=np.int32)
     d = _desc(shape, nframes, q, dtype, flags)
-    s = (ctypes.c_int64 * 14)()
-    _lib.check(_lib.load().dxg2_plan_dry_run(ctypes.byref(d), s, 14))
+    s = (ctypes.c_int64 * 15)()
+    _lib.check(_lib.load().dxg2_plan_dry_run(ctypes.byref(d), s, 15))
     return list(s)
 
 
@@ -85,8 +85,8 @@ def test_grouped_items_of_uint16_plans_and_empty_masks():
 
 @pytest.mark.parametrize("flags", [0, _lib.DXG2_FLAG_NO_QUEUE])
 def test_serving_reserves_at_least_what_a_job_takes(flags):
-    """GpuExecutor.footprint_bound() against the footprint of the plan it stands for, outputs and
-    input included, on both sides of the line from which a plan has a narrow slab."""
+    """GpuExecutor.footprint_bound() against what the plan it stands for cannot do without, outputs
+    and input included, on both sides of the line from which a plan may have a narrow slab."""
     from dynamix_amd import serving
     specs = serving.make_jobs(14, 10.0, 17)
     specs += serving.make_jobs(20, 10.0, 18, shapes=((64, 48), (96, 96), (131, 77)),
@@ -101,8 +101,9 @@ def test_serving_reserves_at_least_what_a_job_takes(flags):
         out = nb * n * 28
         bound = serving.GpuExecutor.footprint_bound(None, spec)
         if spec.layout == "dense":
-            need = s[DENSE_BYTES] + out + n * h * w
-            seen.add(s[DENSE_BYTES] > 1.3 * s[2])     # a narrow slab beside the i8 slab
+            need = s[NEEDED_BYTES] + out + n * h * w
+            seen.add(s[DENSE_BYTES] >= s[NEEDED_BYTES] + s[2] // 2)   # a narrow slab beside it
+            assert s[DENSE_BYTES] >= s[NEEDED_BYTES] > s[2]
             if min(spec.shape) >= 256:
                 assert bound <= 1.25 * need or flags
         else:

@@ -237,3 +237,33 @@ def test_overload_keeps_staged_inputs_within_budget():
     assert big not in ex.staged_ids and len(ex.staged_ids) == 39
     assert ex.peak <= ex.budget, (ex.peak, ex.budget)
     assert ex.held == 0 and ex.resident == 0
+
+
+@pytest.mark.parametrize("budget_mib,granted", [(1 << 20, True), (700, None), (330, False)])
+def test_optional_memory_is_granted_only_where_the_budget_has_room(budget_mib, granted):
+    """A job needs 300 MiB and can use 100 more: with room every job gets them, without it none
+    does, and a job is never refused or held back for them."""
+    ex = FakeExecutor(budget=budget_mib << 20, footprint=lambda s: 300 << 20)
+    orig, options = ex.prepare, []
+
+    def prepare(spec, staged=None):
+        job = orig(spec, staged)
+        job.option = 100 << 20
+        return job
+
+    def admit(job, run=ex.admit):
+        options.append(job.option)
+        assert job.footprint == (300 << 20) + job.option
+        run(job)
+
+    ex.prepare, ex.admit = prepare, admit
+    sch = Scheduler(ex, max_batch=4, n_streams=2, depth=2)
+    try:
+        st = sch.run(_specs(30))
+    finally:
+        sch.close()
+    assert st["failed"] == 0 and st["jobs"] == 30 and len(options) == 30
+    assert ex.peak <= ex.budget and ex.resident == 0
+    assert set(options) <= {0, 100 << 20}
+    if granted is not None:
+        assert set(options) == {(100 << 20) if granted else 0}
