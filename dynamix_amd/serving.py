@@ -51,6 +51,7 @@ from .correlator.common import Plan
 SERVE_SHAPES = ((256, 256), (514, 1030), (1030, 1065))
 DENSE_MEAN = 0.02     # counts per pixel per frame of dense jobs
 EVENT_MEAN = 1e-3     # counts per pixel per frame of event jobs
+RUNTIME_BYTES = 2 << 30   # device memory left to the HIP runtime while a server is open
 
 
 @dataclass
@@ -453,6 +454,34 @@ class TorchAllocator(object):
         return False
 
 
+class _AllocatorLimit(object):
+    """A bound on the share of the device that torch's allocator may take, until close(); the
+    least of those open at a time holds, and the process's own returns with the last."""
+
+    _open, _own, _lock = [], None, threading.Lock()
+
+    def __init__(self, fraction):
+        import torch
+        self.fraction, cls = fraction, _AllocatorLimit
+        with cls._lock:
+            if not cls._open:
+                cls._own = torch.cuda.get_per_process_memory_fraction()
+            cls._open.append(self)
+            self._apply()
+
+    @classmethod
+    def _apply(cls):
+        import torch
+        torch.cuda.set_per_process_memory_fraction(
+            min([cls._own] + [x.fraction for x in cls._open]))
+
+    def close(self):
+        with _AllocatorLimit._lock:
+            if self in _AllocatorLimit._open:
+                _AllocatorLimit._open.remove(self)
+                self._apply()
+
+
 class GpuExecutor(object):
     """Device side of the serving loop (see module docstring)."""
 
@@ -463,10 +492,16 @@ class GpuExecutor(object):
         self.lib = _lib.load()
         # Job memory comes from torch's caching allocator (TorchAllocator): what the
         # device has free plus what torch holds but is not using.
-        free, _total = torch.cuda.mem_get_info()
-        idle = torch.cuda.memory_reserved() - torch.cuda.memory_allocated()
+        free, total = torch.cuda.mem_get_info()
+        held, live = torch.cuda.memory_reserved(), torch.cuda.memory_allocated()
         self.budget = int(hbm_budget) if hbm_budget else \
-            max(0, int(free) + int(idle) - int(reserve_bytes))
+            max(0, int(free) + int(held - live) - int(reserve_bytes))
+        # The budget counts what jobs hold; the allocator also keeps what they gave back, and
+        # would grow to the last byte of the device.  RUNTIME_BYTES of the reserve stay out of
+        # its reach until close(): the HIP runtime allocates a kernel's scratch memory when it is
+        # launched, up to 200 MB a hardware queue here, and aborts the process where it cannot.
+        limit = max(held + int(free) - min(int(reserve_bytes), RUNTIME_BYTES), live + self.budget)
+        self.limit = _AllocatorLimit(limit / total)
         # A persistent Gram launch holds every CU until its queues drain, so kernels of
         # jobs on the other streams wait behind it; persistent_gram=False gives single
         # dense jobs one workgroup per tile instead, which the hardware interleaves with
@@ -499,6 +534,7 @@ class GpuExecutor(object):
             while q:
                 self.lib.dxg2_batch_destroy(q.popleft())
         self.allocator.__exit__(None, None, None)
+        self.limit.close()
 
     def stage(self, spec):
         """A job's input made resident before the job arrives (the frames or events a

@@ -129,3 +129,23 @@ def test_tight_memory_budget_and_failing_job():
     assert stats["failed"] == 1 and stats["failures"][0][0] == 99
     assert "MemoryError" in stats["failures"][0][1]
     check_mix_equals_alone(stats["records"], oracle_layouts=())
+
+
+def test_the_allocator_leaves_the_runtime_its_share():
+    """What jobs gave back stays in torch's allocator, which must not grow to the last byte of
+    the device: the HIP runtime allocates kernels' scratch memory at their launch.  The bound
+    holds for every server open, and goes with the last."""
+    import torch
+    from dynamix_amd.serving import RUNTIME_BYTES, Server
+    _announce("serving allocator bound")
+    torch.cuda.empty_cache()
+    own = torch.cuda.get_per_process_memory_fraction()
+    first, second = Server(), Server(reserve_bytes=16 << 30)
+    for srv in (first, second):
+        free, total = torch.cuda.mem_get_info()
+        allowed = torch.cuda.get_per_process_memory_fraction() * total
+        assert allowed - torch.cuda.memory_reserved() <= free - RUNTIME_BYTES // 2
+        with pytest.raises(torch.cuda.OutOfMemoryError):
+            torch.empty(free - RUNTIME_BYTES // 2, dtype=torch.uint8, device="cuda")
+        srv.close()
+    assert torch.cuda.get_per_process_memory_fraction() == own
