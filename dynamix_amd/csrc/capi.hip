@@ -868,7 +868,8 @@ int ensure_fft_buffers(dxg2_plan* p, hipStream_t s) {
             p->twiddles[H + r * stride + b] = root((int64_t)r * b, H);
     for (int m = 0; m <= L; ++m) p->twiddles[2 * H + m] = root(m, 2 * (int64_t)L);
     // The series of every k-block at once, or where that memory cannot be had (a series takes up to
-    // 1.6 times its frames' bytes) of half of them, a quarter and so on, one part after the other.
+    // 1.6 times its frames' bytes) of a quarter of them, a sixteenth and so on, one part after the
+    // other (a quarter, not half: the kernels' own scratch memory has to fit beside them).
     // A failure releases what was allocated, so a later call starts again from nothing.
     // d_power is set last: it marks the workspace complete.
     uint8_t* xs = nullptr;
@@ -881,7 +882,7 @@ int ensure_fft_buffers(dxg2_plan* p, hipStream_t s) {
     int32_t* qkb = nullptr;
     const size_t nb = (size_t)std::max(p->n_bins, 1);
     const int total = (int)p->kb_work.size();
-    for (int parts = 1;; parts *= 2) {
+    for (int parts = 1;; parts *= 4) {
         fft_partition(p, parts);
         const size_t entries = (size_t)((total + parts - 1) / parts) * KB;
         auto have = [&](auto** ptr, size_t bytes) {
@@ -904,7 +905,7 @@ int ensure_fft_buffers(dxg2_plan* p, hipStream_t s) {
         drop(xs), drop(pixf), drop(qkb), drop(tw), drop(fnum), drop(finv), drop(kbw), drop(kbg);
         power = nullptr;  // the last one asked for
         (void)hipGetLastError();
-        if (2 * parts > std::min(total, 64))
+        if (4 * parts > std::max(4, std::min(total, 64)))
             return set_error(DXG2_ENOMEM, "cannot allocate FFT workspace");
     }
     p->d_pixfft = pixf;
